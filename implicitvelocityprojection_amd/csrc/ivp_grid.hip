@@ -298,6 +298,7 @@ __device__ __forceinline__ void scan_ids(const Grid& g, const int* __restrict__ 
 struct BuildArgs {
     int nd, ns, C, Cs;
     float h, h2_lo, h2_hi;
+    float h2;       // h^2 rounded to float32 (the matrix-core distances)
     float kc, ks;   // cubic and spiky kernel constants
     float inv_h;    // 1 / h rounded to nearest (div_rn)
     float inv_gs;   // 1 / scale of float16 gradW records (a power of two)
@@ -485,35 +486,65 @@ __global__ __launch_bounds__(BLOCK) void k_scan(BuildArgs a) {
     }
 }
 
-// Candidate scan by cells (ids-only and float16 rows; one grid or a grid per scene).  Every row of
-// one cell visits the same nine candidate runs (scan_ids: the runs of the 3x3 (y, z) neighbour
-// cells, each over the cells x - 1 .. x + 1), so a wave takes SCAN_ROWS consecutive rows of its
-// block's 64-row tile, cuts them into segments of equal cell, and for each segment loads the
-// segment's candidates once -- the nine runs laid end to end in scan_ids' visiting order, 64 per
-// batch, up to SCAN_BATCHES batches in registers -- and tests each row of the segment against them.
-// The row's hits of a batch are ranked by the batch's wave mask, so slots fill in the one-lane
-// order.  The slots are collected in LDS (per row Cs words and 4 spare against bank conflicts; each
-// wave owns its rows, so no block barrier) and written out as whole 8-slot blocks of the paired
+// Candidate scan by cells (ids-only and float16 rows; one grid or a grid per scene).  A wave takes
+// SCAN_ROWS consecutive rows of its block's 64-row tile and cuts them into segments: rows of one
+// (y, z) cell row (and scene) within SCAN_SPAN + 1 cells along x.  The rows of a segment share nine
+// candidate runs (scan_ids' runs of the 3x3 (y, z) neighbour cells, each widened to the cells
+// x_first - 1 .. x_last + 1): a candidate outside a row's own 3x3x3 cells lies a cell width > h away,
+// so the wider runs add no neighbour, and the runs end to end keep scan_ids' visiting order.
+//
+// Distances come from the matrix cores: with a = x_row - o and b = x_candidate - o about the
+// segment's centre o, e = |x_row - x_cand|^2 - h^2 = |b|^2 - 2 a.b + (|a|^2 - h^2) is one
+// 16x16x4 float32 product of candidates (b, |b|^2) and rows (-2 a, 1) with |a|^2 - h^2 as the
+// accumulator's start.  Lane (q, n) of the wave then holds e of row n against 16 candidates per
+// batch of 64 -- the candidates of its quarter q of the chunk -- and collects the sign bits.  The
+// product's rounding is below 2e-5 h^2 (coordinates within 4 h of o; a segment that holds a
+// farther one takes the exact test throughout), so outside |e| < 2^-14 h^2 the sign decides
+// sqrtf(d^2) < h as scan_ids does; inside the band the candidate's unfused d^2 and its correctly
+// rounded root decide.  A row's quarters are ranked by their hit counts, so the slots fill in the
+// one-lane order.
+//
+// What bounds it: vector instruction issue.  One row at a time with a candidate per lane the scan
+// took 14 vector instructions per 64 candidate tests (differences, square, two compares, rank,
+// store address); here a test is one sixteenth of a matrix instruction, one funnel shift for the
+// mask and half a minimum for the band, and only hits cost a store: 112 -> 75 million vector
+// instructions per 1M-row build, 196 -> 150 us (102k rows 33 -> 29, 64 scenes of 1.25M rows 235 ->
+// 200).
+//
+// The slots are collected in LDS (per row Cs words and 4 spare against bank conflicts; each wave
+// owns its rows, so no block barrier) and written out as whole 8-slot blocks of the paired
 // layout, 512 contiguous bytes per wave and block; words of a written block between the row's
 // dynamic [0, cnt) and static [Cs - cs, Cs) ranges get the row's own id, as the exact pass pads.
 constexpr int SCAN_ROWS = 16;     // rows per wave: a block's four waves cover its tile
 constexpr int SCAN_BATCHES = 4;   // candidate batches of 64 held in registers per chunk
+constexpr int SCAN_SPAN = 3;      // a segment's last cell lies at most this many cells past its first
+// LDS words of one wave: candidate ids of a chunk, then one batch's candidate records
+// (x, y, z, |b|^2), 16 per quarter with the quarters 80 words apart: the 64 lanes' reads of one
+// component (candidate 4 t + (n & 3) of quarter n >> 2, component q) hit 64 different banks
+constexpr int SCAN_IDS = WAVE * SCAN_BATCHES;
+constexpr int SCAN_QUARTER = 80;
+constexpr int SCAN_WAVE_LDS = SCAN_IDS + 4 * SCAN_QUARTER;
 
-// The candidate runs of a segment's cell, both populations at once: lane 16 p + k (k < 9) loads
-// population p's run k = 3 (dz + 1) + (dy + 1), the cells x - 1 .. x + 1 of row y + dy, layer
-// z + dz (empty outside the grid).  Returns, per lane, the exclusive prefix of the run lengths
-// within its population (rp) and the run's first particle minus it (rb: candidate v of run k is
-// particle v + rb); lane 16 p + 8 also returns the population's total in T.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The candidate runs of a segment's cells (cx0 .. cx1, cy, cz), both populations at once: lane
+// 16 p + k (k < 9) loads population p's run k = 3 (dz + 1) + (dy + 1), the cells cx0 - 1 .. cx1 + 1 of
+// row y + dy, layer z + dz (empty outside the grid).  Returns, per lane, the exclusive prefix of
+// the run lengths within its population (rp) and the run's first particle minus it (rb: candidate
+// v of run k is particle v + rb); lane 16 p + 8 also returns the population's total in T.
 struct SegRuns {
     int rp, rb, T;
 };
-__device__ __forceinline__ SegRuns seg_runs(const BuildArgs& a, const Grid& g, int cx, int cy, int cz) {
+__device__ __forceinline__ SegRuns seg_runs(const BuildArgs& a, const Grid& g, int cx0, int cx1, int cy, int cz) {
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     const int pop = lane >> 4, k = lane & 15;
     const int zz = cz + k / 3 - 1, yy = cy + k % 3 - 1;
     const bool live = pop < 2 && k < 9 && zz >= 0 && zz < g.dims[2] && yy >= 0 && yy < g.dims[1];
-    const int x0 = cx > 0 ? cx - 1 : 0;
-    const int x1 = cx < g.dims[0] - 1 ? cx + 1 : g.dims[0] - 1;
+    const int x0 = cx0 > 0 ? cx0 - 1 : 0;
+    const int x1 = cx1 < g.dims[0] - 1 ? cx1 + 1 : g.dims[0] - 1;
     int s0 = 0, n = 0;
     if (live) {
         const int* start = pop == 0 ? a.dstart : a.sstart;
@@ -530,175 +561,193 @@ __device__ __forceinline__ SegRuns seg_runs(const BuildArgs& a, const Grid& g, i
     return SegRuns{inc - n, s0 - (inc - n), inc};
 }
 
-// One row (position pr, global index row) against NBU batches of candidates (qx, qy, qz, qj; ok =
-// lanes holding a candidate): hit k of the row goes to slot k (dynamic population; an overflowing
-// row's hits past C all go to slot C, which no reader uses) or to slot Cs - 1 - k while k < lim
-// (static population), lanes without a stored hit write their own word of dum.  Returns the
-// row's hit count after these batches.  Without EXACT, candidates in the band [h2_lo, h2_hi) count
-// as misses and are flagged in near (the row is then done again with EXACT, which decides them by
-// the correctly rounded root as scan_group does).
-template <bool DYN, int NBU, bool EXACT>
-__device__ __forceinline__ int cell_row(const BuildArgs& a, const float (&qx)[SCAN_BATCHES],
-                                        const float (&qy)[SCAN_BATCHES], const float (&qz)[SCAN_BATCHES],
-                                        const int (&qj)[SCAN_BATCHES], const unsigned long long (&ok)[SCAN_BATCHES],
-                                        float3 pr, int row, int before, int lim, uint32_t* srow, uint32_t* dum,
-                                        unsigned long long& near) {
-#pragma unroll
-    for (int u = 0; u < NBU; ++u) {
-        const float dx = pr.x - qx[u], dy = pr.y - qy[u], dz = pr.z - qz[u];
-        const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        unsigned long long valid = ok[u];
-        if (DYN) valid &= __builtin_amdgcn_uicmp((unsigned)qj[u], (unsigned)row, ICMP_NE);
-        const unsigned long long lo = __builtin_amdgcn_fcmpf(d2, a.h2_lo, FCMP_OLT);
-        const unsigned long long hi = __builtin_amdgcn_fcmpf(d2, a.h2_hi, FCMP_OLT);
-        unsigned long long hit = lo & valid;
-        if (EXACT) {
-            const unsigned long long band = (hi & valid) & ~lo;
-            if (band) {
-                bool in = false;
-                if (__builtin_amdgcn_inverse_ballot_w64(band)) {
-                    float d = dx * dx + dy * dy + dz * dz;
-                    asm volatile("" : "+v"(d));
-                    in = sqrtf(d) < a.h;
-                }
-                hit |= __builtin_amdgcn_ballot_w64(in);
-            }
-        } else {
-            near |= hi ^ lo;
-        }
-        const int k = before + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hit >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)hit, 0u));
-        uint32_t* p;
-        if (DYN) p = srow + (k < a.C ? k : a.C);
-        else p = k < lim ? srow + (a.Cs - 1 - k) : dum;
-        if (!__builtin_amdgcn_inverse_ballot_w64(hit)) p = dum;
-        *p = (uint32_t)qj[u];
-        before += (int)__popcll(hit);
-    }
-    return before;
-}
-
-// Rows rs .. re - 1 of a segment (global row row0 + r) against the chunk's NBU batches.  found
-// (lane r) counts row r's hits of the population; lim is C for the dynamic population and C - ndf
-// (lane r's dynamic total) for the static one.
-template <bool DYN, int NBU>
-__device__ __forceinline__ void cell_rows(const BuildArgs& a, const float (&qx)[SCAN_BATCHES],
-                                          const float (&qy)[SCAN_BATCHES], const float (&qz)[SCAN_BATCHES],
-                                          const int (&qj)[SCAN_BATCHES], const unsigned long long (&ok)[SCAN_BATCHES],
-                                          int cb, int rs, int re, int row0, float px, float py, float pz, int& found,
-                                          int ndf, uint32_t* st, uint32_t* dum, int S) {
-    for (int r = rs; r < re; ++r) {
-        const float3 pr = make_float3(
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, px), r)),
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, py), r)),
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pz), r)));
-        // a row's first chunk of a population starts at 0 (each row is in one segment)
-        const int before = cb == 0 ? 0 : __builtin_amdgcn_readlane(found, r);
-        int lim = DYN ? a.C : a.C - __builtin_amdgcn_readlane(ndf, r);
-        lim = lim > 0 ? lim : 0;
-        uint32_t* srow = st + r * S;
-        unsigned long long near = 0ull;
-        int after = cell_row<DYN, NBU, false>(a, qx, qy, qz, qj, ok, pr, row0 + r, before, lim, srow, dum, near);
-        if (near)   // a candidate in the band (rare): the row again, deciding the band exactly
-            after = cell_row<DYN, NBU, true>(a, qx, qy, qz, qj, ok, pr, row0 + r, before, lim, srow, dum, near);
-        found = (int)(threadIdx.x & (WAVE - 1)) == r ? after : found;
-    }
-}
-
-// One population of a segment: rows rs .. re - 1 of the wave (global row row0 + r) in the cell
-// (cx, cy, cz).  found (lane r) counts row r's hits of this population; the dynamic population
-// stores hit k at slot k while k < C, the static one at slot Cs - 1 - k while ndf + k < C (ndf =
-// lane r's dynamic total), as k_scan / scan_ids do.
+// One population of a segment: rows rs .. re - 1 of the wave, whose positions lanes (q, n) hold for
+// row n.  found (every lane of row n) counts row n's hits of this population; the dynamic
+// population stores hit k at slot k while k < C (an overflowing row's hits past C all go to slot C,
+// which no reader uses), the static one at slot Cs - 1 - k while ndf + k < C (ndf = the row's dynamic
+// total; other hits go to the row's spare words).
 template <bool DYN>
-__device__ __forceinline__ void cell_pop_scan(const BuildArgs& a, const SegRuns& R, int T, int rs, int re, int row0,
-                                              float px, float py, float pz, int& found, int ndf, uint32_t* st,
-                                              uint32_t* dum, int S) {
+__device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& R, int T, int rs, int re, int row0,
+                                             float px, float py, float pz, float3 o, int& found, int ndf,
+                                             uint32_t* st, uint32_t* wl, int S) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
     constexpr int NB = SCAN_BATCHES;
     constexpr int pl = DYN ? 0 : 16;
     const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const int q = lane >> 4, n = lane & 15;
     const float4* __restrict__ ppos = DYN ? a.pos : a.pos + a.nd;
+    uint32_t* ids = wl;
+    float* cand = reinterpret_cast<float*>(wl + SCAN_IDS);
     int rb[9], rp[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
         rp[k] = __builtin_amdgcn_readlane(R.rp, pl + k);
         rb[k] = __builtin_amdgcn_readlane(R.rb, pl + k);
     }
-    // a particle of the population for lanes without a candidate (masked by ok)
-    const int jsafe = DYN ? row0 : a.ns - 1;
+    const bool mine = n >= rs && n < re;
+    // the row's operand (component q of (-2 a, 1)) and the accumulator's start
+    const float ax = px - o.x, ay = py - o.y, az = pz - o.z;
+    const float a2 = fmaf(az, az, fmaf(ay, ay, ax * ax));
+    const float rowop = q == 0 ? -2.0f * ax : q == 1 ? -2.0f * ay : q == 2 ? -2.0f * az : 1.0f;
+    const float c0 = a2 - a.h2;
+    const f32x4 acc0 = {c0, c0, c0, c0};
+    const float far2 = 16.0f * a.h2, eps = a.h2 * (1.0f / 16384.0f);
+    const bool row_far = __builtin_amdgcn_ballot_w64(mine && !(a2 <= far2)) != 0ull;
+    // lane (q, n) writes the record of candidate n of quarter q, and reads component q of candidate
+    // 4 t + (n & 3) of quarter n >> 2
+    float* cw = cand + SCAN_QUARTER * q + 4 * n;
+    const float* cr = cand + SCAN_QUARTER * (n >> 2) + 4 * (n & 3) + q;
+    const int lim = DYN ? a.C : (a.C - ndf > 0 ? a.C - ndf : 0);
+    uint32_t* srow = st + n * S;
     for (int cb = 0; cb < T; cb += WAVE * NB) {
-        float qx[NB], qy[NB], qz[NB];
-        int qj[NB];
-        unsigned long long ok[NB];
+        const int left = T - cb < WAVE * NB ? T - cb : WAVE * NB;
+        const int nb = (left + WAVE - 1) / WAVE;
+        // the chunk's candidate ids in visiting order, run by run
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            const int v1 = k < 8 ? rp[k + 1] : T;
+            const int hi = v1 < cb + left ? v1 : cb + left;
+            for (int v = (rp[k] > cb ? rp[k] : cb) + lane; v < hi; v += WAVE) ids[v - cb] = (uint32_t)(v + rb[k]);
+        }
+        wave_lds_sync();
+        const int base = 16 * nb * q;   // the quarter's first candidate, relative to cb
+        float4 p[NB];
+        // all batches' loads in flight together (past the end: the last candidate, never a hit)
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            // candidate v = base + lane: the particle v + rb[k] of the last run k with rp[k] <= v
-            const int v = cb + WAVE * u + lane;
-            int off = rb[0];
-#pragma unroll
-            for (int k = 1; k < 9; ++k) off = v >= rp[k] ? rb[k] : off;
-            const bool in = v < T;
-            ok[u] = __builtin_amdgcn_ballot_w64(in);
-            qj[u] = in ? v + off : jsafe;
+            const int c = base + 16 * u + n;
+            if (u < nb) p[u] = ppos[ids[c < left ? c : left - 1]];
         }
-        // every batch's loads in flight together (a batch past the candidates reads jsafe)
+        uint32_t W[2] = {0u, 0u};   // hits, first candidate in the highest bit, 32 per word
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            const float4 q = ppos[qj[u]];
-            qx[u] = q.x; qy[u] = q.y; qz[u] = q.z;
+            uint32_t w = W[u >> 1] << 16;
+            if (u < nb) {
+                const float bx = p[u].x - o.x, by = p[u].y - o.y, bz = p[u].z - o.z;
+                const float b2 = fmaf(bz, bz, fmaf(by, by, bx * bx));
+                const f32x4 rec = {bx, by, bz, base + 16 * u + n < left ? b2 : 1e30f};
+                *reinterpret_cast<f32x4*>(cw) = rec;
+                wave_lds_sync();
+                f32x4 d[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    d[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[16 * t], rowop, acc0, 0, 0, 0);
+                wave_lds_sync();
+                uint32_t h = 0u;
+                float nearest = 1e30f;
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    const float e = d[k >> 2][k & 3];
+                    h = __builtin_amdgcn_alignbit(h, __float_as_uint(e), 31);   // h << 1 | sign
+                    nearest = fminf(nearest, fabsf(e));
+                }
+                const bool far = !(b2 <= far2) || row_far;
+                if (__builtin_amdgcn_ballot_w64((mine && nearest < eps) || far)) {
+                    // candidates in the band (or, with far coordinates, all of them) by the exact test
+                    const bool all = __builtin_amdgcn_ballot_w64(far) != 0ull;
+                    uint32_t band = 0u;
+#pragma unroll
+                    for (int k = 0; k < 16; ++k)
+                        band = __builtin_amdgcn_alignbit(band, __float_as_uint(fabsf(d[k >> 2][k & 3]) - eps), 31);
+                    const int valid = left - base - 16 * u;   // candidates of this lane's 16
+                    const uint32_t in = valid >= 16 ? 0xffffu : valid > 0 ? 0xffffu & ~(0xffffu >> valid) : 0u;
+                    h = all ? 0u : h;
+                    band = mine ? (all ? in : band & in) : 0u;
+                    while (__builtin_amdgcn_ballot_w64(band != 0u)) {
+                        if (band) {
+                            const int k = __clz((int)band) - 16;
+                            const uint32_t bit = 0x8000u >> k;
+                            band &= ~bit;
+                            const float4 pj = ppos[ids[base + 16 * u + k]];
+                            const float rx = px - pj.x, ry = py - pj.y, rz = pz - pj.z;
+                            const float dd = rx * rx + ry * ry + rz * rz;
+                            h = sqrtf(dd) < a.h ? (h | bit) : (h & ~bit);
+                        }
+                    }
+                }
+                w |= h;
+            }
+            W[u >> 1] = w;
         }
-        const int nbu = (T - cb + WAVE - 1) / WAVE;
-        if (nbu >= 4)
-            cell_rows<DYN, 4>(a, qx, qy, qz, qj, ok, cb, rs, re, row0, px, py, pz, found, ndf, st, dum, S);
-        else if (nbu == 3)
-            cell_rows<DYN, 3>(a, qx, qy, qz, qj, ok, cb, rs, re, row0, px, py, pz, found, ndf, st, dum, S);
-        else if (nbu == 2)
-            cell_rows<DYN, 2>(a, qx, qy, qz, qj, ok, cb, rs, re, row0, px, py, pz, found, ndf, st, dum, S);
-        else
-            cell_rows<DYN, 1>(a, qx, qy, qz, qj, ok, cb, rs, re, row0, px, py, pz, found, ndf, st, dum, S);
+        if (!mine) W[0] = W[1] = 0u;
+        if (DYN) {   // the row itself: in run 4
+            const int li = row0 + n - rb[4] - cb - base;
+            if (li >= 0 && li < 32) W[0] &= ~(0x80000000u >> li);
+            if (li >= 32 && li < 64) W[1] &= ~(0x80000000u >> (li - 32));
+        }
+        // rank the row's quarters
+        const int H = __popc(W[0]) + __popc(W[1]);
+        const int h0 = __shfl(H, n, WAVE), h1 = __shfl(H, n + 16, WAVE), h2 = __shfl(H, n + 32, WAVE),
+                  h3 = __shfl(H, n + 48, WAVE);
+        int k = found + (q > 0 ? h0 : 0) + (q > 1 ? h1 : 0) + (q > 2 ? h2 : 0);
+        found += h0 + h1 + h2 + h3;
+        auto slot = [&](int k) { return DYN ? (k < a.C ? k : a.C) : (k < lim ? a.Cs - 1 - k : a.Cs + 1); };
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            uint32_t w = W[g];
+            const uint32_t* src = ids + base + 32 * g;
+            while (__builtin_amdgcn_ballot_w64(w != 0u)) {
+                if (w) {   // two hits a round, so that their ids' reads overlap
+                    const int c = __clz((int)w);
+                    w &= ~(0x80000000u >> c);
+                    const uint32_t j0 = src[c], j1 = src[w ? __clz((int)w) : c];
+                    srow[slot(k)] = j0;
+                    k++;
+                    if (w) {
+                        w &= ~(0x80000000u >> __clz((int)w));
+                        srow[slot(k)] = j1;
+                        k++;
+                    }
+                }
+            }
+        }
+        wave_lds_sync();
     }
 }
 
-// LDS of one k_scan_cells block: its tile's 64 rows of Cs + 4 words, then a discard word per
-// thread
-inline size_t scan_cells_lds(int Cs) { return ((size_t)WAVE * (size_t)(Cs + 4) + BLOCK) * sizeof(uint32_t); }
+// LDS of one k_scan_cells block: its tile's 64 rows of Cs + 4 words, then each wave's scratch
+inline size_t scan_cells_lds(int Cs) {
+    return ((size_t)WAVE * (size_t)(Cs + 4) + WAVES_PER_BLOCK * SCAN_WAVE_LDS) * sizeof(uint32_t);
+}
 constexpr size_t SCAN_CELLS_LDS_MAX = 64 * 1024;
 
+// (at least four waves per SIMD: within 128 registers the matrix results stay in vector registers)
 template <int FMT, bool SCENES>
-__global__ __launch_bounds__(BLOCK) void k_scan_cells(BuildArgs a) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_scan_cells(BuildArgs a) {
     static_assert(rec_words<FMT>() == 64u, "the cell scan writes the paired ids-only layout");
-    extern __shared__ uint32_t scan_stage[];
+    extern __shared__ __align__(16) uint32_t scan_stage[];
     const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)), lane = (int)(threadIdx.x & (WAVE - 1));
     const int row0 = tile * WAVE + wv * SCAN_ROWS;
     if (row0 >= a.nd) return;   // whole waves; the block has no barrier
     const int nrw = a.nd - row0 < SCAN_ROWS ? a.nd - row0 : SCAN_ROWS;
     const int C = a.C, Cs = a.Cs, S = Cs + 4;
-    uint32_t* st = scan_stage + wv * SCAN_ROWS * S;
-    uint32_t* dum = scan_stage + WAVE * S + wv * WAVE + lane;   // the lane's discard word
-    // lane r < nrw: row row0 + r, its position and cell (independent scenes: in its scene's
-    // grid, whose keys follow the previous scene's, so a segment never spans two scenes)
-    float px = 0.0f, py = 0.0f, pz = 0.0f;
-    int cx = 0, cy = 0, cz = 0, key = -1 - lane, sid = 0;
-    if (lane < nrw) {
-        const float4 p = a.pos[row0 + lane];
-        px = p.x; py = p.y; pz = p.z;
-        if (SCENES) sid = a.sid[row0 + lane];
-        const Grid& g = SCENES ? a.grids[sid] : a.g;
-        cx = cell_coord(g, px, 0); cy = cell_coord(g, py, 1); cz = cell_coord(g, pz, 2);
-        key = cell_key(g, cx, cy, cz);
-    }
-    int fd = 0, fs = 0;   // lane r: row r's dynamic and static hits
+    uint32_t* wl = scan_stage + wv * SCAN_WAVE_LDS;
+    uint32_t* st = scan_stage + WAVES_PER_BLOCK * SCAN_WAVE_LDS + wv * SCAN_ROWS * S;
+    // lane (q, n): row row0 + n (the last row again past the end), its position and cell
+    // (independent scenes: in its scene's grid)
+    const int n = lane & 15;
+    const int row = row0 + (n < nrw ? n : nrw - 1);
+    const float4 p = a.pos[row];
+    const int sid = SCENES ? a.sid[row] : 0;
+    const Grid& g = SCENES ? a.grids[sid] : a.g;
+    const int cx = cell_coord(g, p.x, 0), cy = cell_coord(g, p.y, 1), cz = cell_coord(g, p.z, 2);
+    int fd = 0, fs = 0;   // row n's dynamic and static hits
     for (int s = 0; s < nrw;) {
-        const int k0 = __builtin_amdgcn_readlane(key, s);
-        const unsigned long long diff = __builtin_amdgcn_ballot_w64(lane > s && lane < nrw && key != k0);
-        const int e = diff ? (int)__builtin_ctzll(diff) : nrw;
         const int scx = __builtin_amdgcn_readlane(cx, s), scy = __builtin_amdgcn_readlane(cy, s),
-                  scz = __builtin_amdgcn_readlane(cz, s);
-        const Grid& sg = SCENES ? a.grids[__builtin_amdgcn_readlane(sid, s)] : a.g;
-        const SegRuns R = seg_runs(a, sg, scx, scy, scz);
+                  scz = __builtin_amdgcn_readlane(cz, s), ssid = __builtin_amdgcn_readlane(sid, s);
+        const bool other = cy != scy || cz != scz || cx > scx + SCAN_SPAN || (SCENES && sid != ssid);
+        const unsigned long long diff = __builtin_amdgcn_ballot_w64(lane > s && lane < nrw && other);
+        const int e = diff ? (int)__builtin_ctzll(diff) : nrw;
+        const int ecx = __builtin_amdgcn_readlane(cx, e - 1);
+        const Grid& sg = SCENES ? a.grids[ssid] : a.g;
+        const float w = 1.0f / sg.inv_w;
+        const float3 o = make_float3(sg.origin[0] + 0.5f * (float)(scx + ecx + 1) * w,
+                                     sg.origin[1] + ((float)scy + 0.5f) * w, sg.origin[2] + ((float)scz + 0.5f) * w);
+        const SegRuns R = seg_runs(a, sg, scx, ecx, scy, scz);
         const int Td = __builtin_amdgcn_readlane(R.T, 8), Ts = __builtin_amdgcn_readlane(R.T, 24);
-        if (Td > 0) cell_pop_scan<true>(a, R, Td, s, e, row0, px, py, pz, fd, 0, st, dum, S);
-        if (Ts > 0) cell_pop_scan<false>(a, R, Ts, s, e, row0, px, py, pz, fs, fd, st, dum, S);
+        if (Td > 0) seg_pop_scan<true>(a, R, Td, s, e, row0, p.x, p.y, p.z, o, fd, 0, st, wl, S);
+        if (Ts > 0) seg_pop_scan<false>(a, R, Ts, s, e, row0, p.x, p.y, p.z, o, fs, fd, st, wl, S);
         s = e;
     }
     int cnt = 0, cs = 0;
@@ -710,8 +759,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_cells(BuildArgs a) {
         a.rowtot[row0 + lane] = tot;
         if (tot > C) atomicOr(a.err_flag, 1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     // write-out: lane (q, sub) writes slots 8 b + sub and 8 b + sub + 4 of row q (words
     // 512 b + 8 (row's place in the tile) + 2 sub), every block of [0, ceil8(cnt)) and of
     // [floor8(Cs - cs), Cs); the slots of those blocks between the two ranges get the row's own id
@@ -1339,14 +1387,16 @@ int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m,
 // 145 -> 115 with 4 lanes; 1M rows 501 -> 404 with 2 lanes and 4 batches in flight.  Fewer rows
 // leave fewer waves per SIMD, and the one-lane scan is then a chain of dependent load rounds.
 // 64 is the scan by cells (k_scan_cells), for ids-only and float16 rows (one scene or many) whose
-// staged rows fit the LDS: scan alone 1M rows 225 -> 186 us, 102k rows 32 -> 28 us, 8k rows 12-14 ->
-// 15 us (16 lanes stay there); where it does not apply, the count's lanes per row.
-static int lanes_by_count(int nd) { return nd >= (1 << 18) ? 2 : nd >= (1 << 15) ? 4 : nd >= (1 << 12) ? 8 : 16; }
+// staged rows fit the LDS, from 16k rows: scan alone, lanes per row (best count) against by cells,
+// us: 4k rows 15.8 / 16.7, 8k 16.1 / 16.4, 23k 19.1 / 18.4, 36k 24.7 / 19.1, 102k 43 / 29, 262k 83 /
+// 50, 1M 225 / 149; where it does not apply, the count's lanes per row (16 below 32k rows: 8 lanes
+// took 20 us from 1k to 23k rows against 16).
+static int lanes_by_count(int nd) { return nd >= (1 << 18) ? 2 : nd >= (1 << 15) ? 4 : 16; }
 
 int build_lanes_for(const ivp_ctx* c) {
     const int nd = c->nd;
     const bool cells = c->rec_words == 64 && scan_cells_lds(c->Cs) <= SCAN_CELLS_LDS_MAX;
-    int G = c->build_lanes > 0 ? c->build_lanes : cells && nd >= (1 << 15) ? 64 : lanes_by_count(nd);
+    int G = c->build_lanes > 0 ? c->build_lanes : cells && nd >= (1 << 14) ? 64 : lanes_by_count(nd);
     if (G == 64 && !cells) G = lanes_by_count(nd);
     return G;
 }
@@ -1382,7 +1432,7 @@ int grid_build(ivp_ctx* c) {
         const double hh = (double)c->h * (double)c->h;
         float h2_lo = std::nextafter((float)(hh * (1.0 - 1.0 / 1048576.0)), 0.0f);
         float h2_hi = std::nextafter((float)(hh * (1.0 + 1.0 / 1048576.0)), 1.0f);
-        BuildArgs ba{c->nd, c->ns, c->C, c->Cs, c->h, h2_lo, h2_hi, c->kcubic, c->kspiky, 1.0f / c->h, 1.0f / c->gscale, c->grid,
+        BuildArgs ba{c->nd, c->ns, c->C, c->Cs, c->h, h2_lo, h2_hi, (float)hh, c->kcubic, c->kspiky, 1.0f / c->h, 1.0f / c->gscale, c->grid,
                      c->grids, c->sid, c->pos, c->minv, c->dstart, c->sstart, c->nb, c->g16, c->tile_len,
                      c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag, c->partials, c->max_blocks};
         // bytes (pair count of the previous build): the pair records written, the ids read back
