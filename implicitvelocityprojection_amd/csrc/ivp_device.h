@@ -65,21 +65,18 @@ __device__ __forceinline__ float div_rn(float x, float b, float y) {
     return fmaf(fmaf(-b, q, x), y, q);
 }
 
-// cubic_kernel with q = r_norm / h formed by div_rn from inv_h = 1 / h (rounded to nearest)
+// cubic_kernel with q = r_norm / h formed by div_rn from inv_h = 1 / h (rounded to nearest); both
+// polynomials are formed and one is chosen (a wave's pairs take both anyway; the empty asm keeps
+// the choice a select, so that a pair's arithmetic stays one basic block)
 __device__ __forceinline__ float cubic_kernel_rn(float r_norm, float h, float inv_h, float k) {
-    float res = 0.0f;
-    float q = div_rn(r_norm, h, inv_h);
-    if (q <= 1.0f) {
-        if (q <= 0.5f) {
-            float q2 = q * q;
-            float q3 = q2 * q;
-            res = k * (6.0f * q3 - 6.0f * q2 + 1.0f);
-        } else {
-            float factor = 1.0f - q;
-            res = k * 2.0f * factor * factor * factor;
-        }
-    }
-    return res;
+    const float q = div_rn(r_norm, h, inv_h);
+    const float q2 = q * q;
+    const float q3 = q2 * q;
+    float near = k * (6.0f * q3 - 6.0f * q2 + 1.0f);
+    const float factor = 1.0f - q;
+    float far = k * 2.0f * factor * factor * factor;
+    asm("" : "+v"(near), "+v"(far));
+    return q <= 0.5f ? near : q <= 1.0f ? far : 0.0f;
 }
 
 __device__ __forceinline__ float len3(float x, float y, float z) {

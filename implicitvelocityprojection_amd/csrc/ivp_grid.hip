@@ -780,8 +780,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     }
 }
 
-// Phase B after k_scan: one thread per row, the counts from k_scan
-template <int FMT>
+// Phase B after k_scan for float32-gradient rows: one thread per row, the counts from k_scan
 __global__ __launch_bounds__(BLOCK) void k_eval(BuildArgs a) {
     int blk = xcd_block(blockIdx.x, gridDim.x);
     int i = blk * BLOCK + threadIdx.x;
@@ -795,7 +794,7 @@ __global__ __launch_bounds__(BLOCK) void k_eval(BuildArgs a) {
         tot = a.rowtot[i];
     }
     int cs = (tot < a.C ? tot : a.C) - cnt;
-    build_eval<FMT>(a, i, lane, i >> 6, valid, pi, cnt, cs, tot);
+    build_eval<IVP_ROWS_F32>(a, i, lane, i >> 6, valid, pi, cnt, cs, tot);
 }
 
 template <int FMT>
@@ -966,6 +965,172 @@ __device__ __forceinline__ void build_eval(const BuildArgs& a, int i, int lane, 
     if (lane == 0) a.tile_len[tile] = tlp;
 }
 
+// Four lanes of a row, one term each: acc + t0 + t1 + t2 + t3 in that order on every lane (the
+// one-thread accumulation order; adding an unused slot's 0 changes no bit).  The quad broadcast is
+// a modifier of the add.
+template <int K>
+__device__ __forceinline__ float quad_bcast(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), K * 0x55, 0xf, 0xf, true));
+}
+__device__ __forceinline__ void quad_add(float& acc, float t) {
+    acc = acc + quad_bcast<0>(t);
+    acc = acc + quad_bcast<1>(t);
+    acc = acc + quad_bcast<2>(t);
+    acc = acc + quad_bcast<3>(t);
+}
+__device__ __forceinline__ void quad_sub(float& acc, float t) {
+    acc = acc - quad_bcast<0>(t);
+    acc = acc - quad_bcast<1>(t);
+    acc = acc - quad_bcast<2>(t);
+    acc = acc - quad_bcast<3>(t);
+}
+
+// Phase B of the build with four lanes per row (ids-only and float16 rows): lane g takes slots g and
+// g + 4 of every 8-slot block (one 8-byte id load), forms their terms with the expressions of
+// build_eval, and the row's sums take the four lanes' terms in slot order, so rho, Aii, S and k are
+// bitwise those of the one-thread pass.  A block is one 64-row tile; block partials are per tile.
+// The neighbours of block b + 1 and the ids of block b + 2 are in flight while block b is summed.
+// Bound by vector instruction issue from about 250k rows (the correctly rounded root, reciprocal
+// and quotients; 109 instructions per 64 slots, 20 of them the ordered adds), by the chain of load
+// rounds below, where one thread per row leaves most SIMDs idle: us per build with one thread per
+// row and with four lanes, ids-only rows: 8k 20.5 / 10, 102k 24 / 18, 262k 34 / 33, 1M 104 / 94;
+// float16 rows 1M 235 / 190.
+template <int FMT>
+__global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
+    static_assert(rec_words<FMT>() == 64u, "four lanes per row read the paired ids-only layout");
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    __shared__ int wmax[WAVES_PER_BLOCK];
+    const int tile = xcd_block(blockIdx.x, gridDim.x);
+    const int r = (int)(threadIdx.x >> 2), g = (int)(threadIdx.x & 3), i = tile * WAVE + r;
+    const bool valid = i < a.nd;
+    int cnt = 0, cs = 0;
+    float4 pi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (valid) {
+        pi = a.pos[i];
+        cnt = a.rowcnt[i];
+        const int tot = a.rowtot[i];
+        cs = (tot < a.C ? tot : a.C) - cnt;
+    }
+    const float h = a.h;
+    const size_t w_row = (size_t)tile * (size_t)a.Cs * 64u + 8u * (uint32_t)r;
+    uint32_t* row = a.nb + w_row;
+    const int wl = wave_max(cnt), ws = wave_max(cs);
+    if ((threadIdx.x & (WAVE - 1)) == 0) wmax[threadIdx.x >> 6] = wl;
+    float rho = 0.0f, aii = 0.0f, jx = 0.0f, jy = 0.0f, jz = 0.0f, sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    rho = rho + pi.w * cubic_kernel(0.0f, h, a.kc);
+    const float rho_self = rho;
+    const int self = valid ? i : 0;
+    // An unused slot takes the row itself with mass and 1/m zero: r = 0, and every term is exactly 0
+    // (a row whose position is not finite uses no slot at all: its sums are reset below).
+    struct Nb {
+        float4 p;
+        float m;
+    };
+    uint32_t top = 0u;   // largest id used: below nd, phase A stored dynamic ids
+    auto fetch = [&](uint32_t j, bool use) {
+        j = use ? j : (uint32_t)self;
+        top = j > top ? j : top;
+        const uint32_t c = j < (uint32_t)a.nd ? j : (uint32_t)a.nd - 1u;
+        Nb q = {a.pos[c], a.minv[c]};
+        return q;
+    };
+    auto slots = [&](Nb q, bool use, uint32_t& h0, uint32_t& h1) {
+        q.p.w = use ? q.p.w : 0.0f;
+        q.m = use ? q.m : 0.0f;
+        const float rx = pi.x - q.p.x, ry = pi.y - q.p.y, rz = pi.z - q.p.z;
+        const float rn = len3_rn(rx, ry, rz);
+        const float3 gw = spiky_grad_rn(rx, ry, rz, rn, h, a.ks);
+        if (FMT == IVP_ROWS_F16) {   // (r = 0 gives gradient words of 0; a negative zero is cleared)
+            const uint32_t keep = use ? 0xffffffffu : 0u;
+            h0 = pack_half2(gw.x * a.inv_gs, gw.y * a.inv_gs) & keep;
+            h1 = pack_half2(gw.z * a.inv_gs, 0.0f) & keep;
+        }
+        const float Jx = q.p.w * gw.x, Jy = q.p.w * gw.y, Jz = q.p.w * gw.z;
+        quad_add(rho, q.p.w * cubic_kernel_rn(rn, h, a.inv_h, a.kc));
+        quad_add(aii, (Jx * Jx + Jy * Jy + Jz * Jz) * q.m);
+        quad_sub(jx, Jx);
+        quad_sub(jy, Jy);
+        quad_sub(jz, Jz);
+    };
+    const u32x2* ids2 = reinterpret_cast<const u32x2*>(row + 2 * g);
+    const int nblk = (wl + 7) >> 3;   // <= Cs / 8: wl <= C
+    const u32x2 none = {(uint32_t)self, (uint32_t)self};
+    u32x2 id1 = nblk > 0 && valid ? ids2[0] : none;
+    Nb c0 = fetch(id1.x, g < cnt), c1 = fetch(id1.y, g + 4 < cnt);
+    id1 = nblk > 1 && valid ? ids2[256] : none;
+    for (int b = 0; b < nblk; ++b) {
+        const int k = 8 * b + g;
+        const Nb n0 = fetch(id1.x, k + 8 < cnt), n1 = fetch(id1.y, k + 12 < cnt);
+        id1 = b + 2 < nblk && valid ? ids2[(b + 2) * 256] : none;
+        uint32_t hq[4] = {0u, 0u, 0u, 0u};
+        slots(c0, k < cnt, hq[0], hq[1]);
+        slots(c1, k + 4 < cnt, hq[2], hq[3]);
+        if (FMT == IVP_ROWS_F16 && valid)
+            *reinterpret_cast<u32x4*>(a.g16 + 2 * (w_row + 2 * (size_t)g + 512u * (uint32_t)b)) = u32x4{hq[0], hq[1], hq[2], hq[3]};
+        c0 = n0;
+        c1 = n1;
+    }
+    if (cnt == 0) {
+        rho = rho_self;
+        aii = jx = jy = jz = 0.0f;
+    }
+    bool bad = top >= (uint32_t)a.nd;   // never
+    // static slots Cs - 1, Cs - 2, ...: lane g the (4 s + g)-th
+    for (int s = 0; s < ws; s += 4) {
+        const bool use = s + g < cs;
+        const int j = use ? (int)row[slot_word<64u>(a.Cs - 1 - s - g)] : 0;
+        bad = bad || (use && (unsigned)j >= (unsigned)a.ns);   // never: phase A stored a static id
+        const float4 q = a.pos[a.nd + ((unsigned)j < (unsigned)a.ns ? j : 0)];
+        const float rx = pi.x - q.x, ry = pi.y - q.y, rz = pi.z - q.z;
+        const float rn = len3_rn(rx, ry, rz);
+        const float3 gw = spiky_grad_rn(rx, ry, rz, rn, h, a.ks);
+        const float Jx = use ? q.w * gw.x : 0.0f, Jy = use ? q.w * gw.y : 0.0f, Jz = use ? q.w * gw.z : 0.0f;
+        quad_add(rho, use ? q.w * cubic_kernel_rn(rn, h, a.inv_h, a.kc) : 0.0f);
+        quad_sub(jx, Jx);
+        quad_sub(jy, Jy);
+        quad_sub(jz, Jz);
+        quad_add(sx, Jx);
+        quad_add(sy, Jy);
+        quad_add(sz, Jz);
+    }
+    if (bad) atomicOr(a.err_flag, 4);
+    __syncthreads();
+    const int tl = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    const int tlp = (tl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;   // <= Cs
+    // pad only after the static ids have been consumed (the padded range can reach into them; the
+    // row's four lanes are in one wave)
+    if (valid) {
+        for (int b = cnt >> 3; b < (tlp >> 3); ++b) {
+            const int k = 8 * b + g;
+            uint32_t* w = row + 2 * g + 512 * b;
+            if (k >= cnt) w[0] = (uint32_t)i;
+            if (k + 4 >= cnt) w[1] = (uint32_t)i;
+            // (the wave's own blocks were written above; the tile's longest row may have more)
+            if (FMT == IVP_ROWS_F16 && b >= nblk)
+                *reinterpret_cast<u32x4*>(a.g16 + 2 * (w_row + 2 * (size_t)g + 512u * (uint32_t)b)) = u32x4{0u, 0u, 0u, 0u};
+        }
+        if (g == 0) {
+            aii += (jx * jx + jy * jy + jz * jz) * a.minv[i];
+            a.kk[i] = 1.0f / (aii + 1e-3f);
+            a.density[i] = rho;
+            a.Ss[3 * i + 0] = sx;
+            a.Ss[3 * i + 1] = sy;
+            a.Ss[3 * i + 2] = sz;
+            a.rowcnt[i] = cnt;
+        }
+    }
+    if (threadIdx.x == 0) a.tile_len[tile] = tlp;
+    // row 1 starts at zero: the window pass adds its tile's window size there
+    double v[2] = {valid && g == 0 ? (double)cnt : 0.0, 0.0};
+    __shared__ double lds[WAVES_PER_BLOCK];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const double s = block_sum(v[q], lds);
+        if (threadIdx.x == 0) a.partials[q * a.stride + tile] = s;
+    }
+}
+
 struct WinArgs {
     int nd, Cs;
     int cap;   // largest window kept, <= WIN_MAX
@@ -976,6 +1141,7 @@ struct WinArgs {
     int* win_n;
     double* partials;   // the build's partials (row 1: window sizes)
     int stride;
+    int tiles_per_block;   // of the pass that wrote those partials
 };
 
 // Tile windows of ids-only rows, one block per 64-row tile.  The window is the ascending list of
@@ -1082,9 +1248,9 @@ __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
         }
     if (threadIdx.x == 0) {
         a.win_n[t] = total;
-        // the build's partial row 1 (zeroed by the build's blocks of four tiles; the sums are
-        // integers, exact in any order)
-        atomicAdd(&a.partials[a.stride + t / WAVES_PER_BLOCK], (double)total);
+        // the build's partial row 1 (zeroed by the build's blocks; the sums are integers, exact in
+        // any order)
+        atomicAdd(&a.partials[a.stride + t / a.tiles_per_block], (double)total);
     }
 }
 
@@ -1427,6 +1593,7 @@ int grid_build(ivp_ctx* c) {
         IVP_HIP(hipMemsetAsync(c->dstart, 0, sizeof(int) * (size_t)(c->ncell + 1), c->stream));
         IVP_HIP(hipMemsetAsync(c->err_flag, 0, sizeof(int), c->stream));   // (else cleared by the sort)
     }
+    int tiles_per_block = WAVES_PER_BLOCK;   // of the pass that writes the build's partials
     if (c->nd > 0) {
         // float h2_lo <= h^2 (1 - 2^-20) and h2_hi >= h^2 (1 + 2^-20): the predicate bounds of scan_ids
         const double hh = (double)c->h * (double)c->h;
@@ -1460,12 +1627,17 @@ int grid_build(ivp_ctx* c) {
                 IVP_TRY((launch_scan<IVP_ROWS_F16, false>(c, G, ba)));
             else
                 IVP_TRY((launch_scan<IVP_ROWS_IDS, false>(c, G, ba)));
-            if (c->row_fmt == IVP_ROWS_F32 && c->S == 0)
-                IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval<IVP_ROWS_F32>, nb, ba));
-            else if (c->row_fmt == IVP_ROWS_F16 && c->S == 0)
-                IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval<IVP_ROWS_F16>, nb, ba));
-            else
-                IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval<IVP_ROWS_IDS>, nb, ba));
+            // exact pass: float32-gradient rows one thread per row, the paired layout four lanes
+            if (c->row_fmt == IVP_ROWS_F32) {
+                IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval, nb, ba));
+            } else {
+                tiles_per_block = 1;
+                const dim3 tiles((c->nd + WAVE - 1) / WAVE);
+                if (c->row_fmt == IVP_ROWS_F16)
+                    IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval4<IVP_ROWS_F16>, tiles, ba));
+                else
+                    IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval4<IVP_ROWS_IDS>, tiles, ba));
+            }
         }
     }
     c->win_built = false;
@@ -1476,7 +1648,7 @@ int grid_build(ivp_ctx* c) {
     // step on 256 columns)
     if (c->nd > 0 && c->windows && c->rec_words == 64 && c->S == 0 && ppt <= 32) {
         WinArgs wa{c->nd, c->Cs, c->win_cap, c->nb, c->tile_len, c->loc, c->win_ids, c->win_n, c->partials,
-                   c->max_blocks};
+                   c->max_blocks, tiles_per_block};
         const dim3 grid((c->nd + WAVE - 1) / WAVE);
         if (ppt <= 8)
             IVP_TRY(launch(c, KC_WINDOW, -1, 0.0, k_window<8>, grid, wa));
@@ -1487,7 +1659,8 @@ int grid_build(ivp_ctx* c) {
         c->win_built = true;
     }
     // pair count (row 0) and window sizes (row 1) of the build's blocks
-    if (c->nd > 0) IVP_TRY(finalize<FIN_BUILD>(c, (int)blocks_for(c->nd)));
+    if (c->nd > 0)
+        IVP_TRY(finalize<FIN_BUILD>(c, tiles_per_block == 1 ? (c->nd + WAVE - 1) / WAVE : blocks_for(c->nd)));
     c->built = true;
     return IVP_OK;
 }
