@@ -69,7 +69,7 @@ void free_all(ivp_ctx* c) {
     dfree(c->rho0); dfree(c->rho0_b); dfree(c->mat); dfree(c->mat_b); dfree(c->uid); dfree(c->uid_b);
     dfree(c->inv); dfree(c->density); dfree(c->kk); dfree(c->Ss); dfree(c->divg); dfree(c->divg_b);
     dfree(c->rowcnt); dfree(c->rowtot); dfree(c->nb); dfree(c->tile_len); dfree(c->dstart); dfree(c->sstart);
-    dfree(c->ccount); dfree(c->key); dfree(c->tmp_src); dfree(c->order); dfree(c->scan_bsum);
+    dfree(c->ccount); dfree(c->key); dfree(c->tmp_src); dfree(c->order); dfree(c->scan_bsum); dfree(c->cell_bsum);
     dfree(c->d4); dfree(c->q4); dfree(c->b); dfree(c->sol); dfree(c->r); dfree(c->Ap); dfree(c->p4); dfree(c->y2);
     dfree(c->cc); dfree(c->sfac); dfree(c->jd); dfree(c->xs4); dfree(c->nbact);
     dfree(c->w_pinv); dfree(c->w_p4); dfree(c->w_v4); dfree(c->w_dv); dfree(c->w_r); dfree(c->w_z);
@@ -115,7 +115,7 @@ int alloc_all(ivp_ctx* c) {
     A(key, cap); A(tmp_src, cap + 1); A(order, cap);
     size_t scan_n = std::max((size_t)c->ncell, cap) + 1;
     c->nscan_blocks = (int)((scan_n + 2047) / 2048) + 2;
-    A(scan_bsum, (size_t)c->nscan_blocks + 1);
+    A(scan_bsum, (size_t)c->nscan_blocks + 1); A(cell_bsum, (size_t)c->nscan_blocks);
     A(d4, cap); A(q4, cap); A(b, 3 * cap); A(sol, 3 * cap); A(r, 3 * cap); A(Ap, 3 * cap); A(p4, cap); A(y2, cap);
     A(cc, cap); A(sfac, cap); A(jd, cap); A(xs4, cap); A(nbact, cap);
     A(w_pinv, 9 * cap); A(w_p4, cap); A(w_v4, cap); A(w_dv, 3 * cap); A(w_r, 3 * cap); A(w_z, 3 * cap);
@@ -130,6 +130,7 @@ int alloc_all(ivp_ctx* c) {
 
     memset(c->state_host, 0, sizeof(SolverState));
     IVP_HIP(hipMemsetAsync(c->ccount, 0, sizeof(int) * (size_t)c->ncell, c->stream));
+    IVP_HIP(hipMemsetAsync(c->cell_bsum, 0, sizeof(int) * (size_t)c->nscan_blocks, c->stream));
     IVP_HIP(hipMemsetAsync(c->state, 0, sizeof(SolverState), c->stream));
     IVP_HIP(hipMemsetAsync(c->tile_len, 0, sizeof(int) * tiles, c->stream));
     // the pads past cap are read by the candidate scan (and masked); keep them defined
@@ -255,14 +256,14 @@ int scenes_set(ivp_ctx* c, int S, const ivp_scene* sc) {
     c->loaded = false;
     c->built = false;
     const size_t cap = (size_t)c->cap;
-    dfree(c->dstart); dfree(c->sstart); dfree(c->ccount); dfree(c->scan_bsum);
+    dfree(c->dstart); dfree(c->sstart); dfree(c->ccount); dfree(c->scan_bsum); dfree(c->cell_bsum);
     c->ncell = (int)base;
     size_t scan_n = std::max((size_t)c->ncell, cap) + 1;
     c->nscan_blocks = (int)((scan_n + 2047) / 2048) + 2;
     int rc = IVP_OK;
 #define A(p, n) if ((rc = dalloc(&c->p, (n))) != IVP_OK) return rc
     A(dstart, (size_t)c->ncell + 1); A(sstart, (size_t)c->ncell + 1); A(ccount, (size_t)c->ncell);
-    A(scan_bsum, (size_t)c->nscan_blocks + 1);
+    A(scan_bsum, (size_t)c->nscan_blocks + 1); A(cell_bsum, (size_t)c->nscan_blocks);
     A(grids, (size_t)S); A(sid, cap); A(sdomain, 3 * (size_t)S); A(ss, (size_t)S); A(sprm, 1);
     A(shist_err, (size_t)S * SCENE_HIST); A(shist_pcg, (size_t)S * SCENE_HIST);
     A(spartials, 8 * (size_t)c->max_blocks); A(sactive, 1);
@@ -275,6 +276,7 @@ int scenes_set(ivp_ctx* c, int S, const ivp_scene* sc) {
     for (int s = 0; s < S; ++s)
         for (int a = 0; a < 3; ++a) dom[3 * s + a] = sc[s].domain_size[a];
     IVP_HIP(hipMemsetAsync(c->ccount, 0, sizeof(int) * (size_t)c->ncell, c->stream));
+    IVP_HIP(hipMemsetAsync(c->cell_bsum, 0, sizeof(int) * (size_t)c->nscan_blocks, c->stream));
     IVP_HIP(hipMemsetAsync(c->shist_err, 0, sizeof(double) * (size_t)S * SCENE_HIST, c->stream));
     IVP_HIP(hipMemsetAsync(c->shist_pcg, 0, sizeof(int) * (size_t)S * SCENE_HIST, c->stream));
     IVP_HIP(hipMemsetAsync(c->ss, 0, sizeof(SceneState) * (size_t)S, c->stream));
@@ -728,10 +730,9 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
     rc = prm->pressure_method == 0 ? prj_solve(c, prm->dt, &prm->prj, stats, PRJ_BOTH)
                                    : ip_solve(c, prm->dt, &prm->ip, stats, true);
     if (rc != IVP_OK) return truncated(rc);
-    rc = glue_advect_boundary(c, prm->dt);
-    // the rebuild that ends the step, not waited for: the step's results come from the rows built
-    // before it, and a row of the new build over the capacity stops the next step (above)
-    if (rc == IVP_OK) rc = grid_build(c);
+    // advection and the rebuild that ends the step, not waited for: the step's results come from the
+    // rows built before it, and a row of the new build over the capacity stops the next step (above)
+    rc = grid_build(c, &prm->dt);
     const int rw = ip_solve_wait(c, stats);
     return rc != IVP_OK ? rc : rw;
 }
@@ -761,9 +762,7 @@ int ivp_step_scenes(ivp_ctx* c, const ivp_step_params* prm, ivp_scene_stats* sta
         stats[s].final_density_error = q.final_err;
         if (status == IVP_OK && q.status != IVP_OK) status = q.status;
     }
-    rc = glue_advect_boundary(c, prm->dt);
-    if (rc != IVP_OK) return rc;
-    rc = grid_build(c);
+    rc = grid_build(c, &prm->dt);
     if (rc != IVP_OK) return rc;
     return status;
 }

@@ -4,8 +4,9 @@
 // neighbour_search.py:10-155) and PressureBase.compute_density / compute_Aii
 // (scripts/sim/forces/pressure/pressure_base.py:12-87).
 //
-// Sort: a deterministic counting sort over cell keys.  count (atomic), exclusive scan,
-// scatter (atomic slot), then every particle ranks itself inside its cell by user id, so the
+// Sort: a deterministic counting sort over cell keys.  count (atomic; a step's advection runs in
+// the same pass), exclusive scan, scatter (atomic slot), then every particle ranks itself inside
+// its cell by user id and moves to its place, so the
 // resulting order -- (cell key, user id) -- depends on the positions only.  Cell keys are
 // x-fastest linear, so the three cells (cx-1..cx+1, cy, cz) of a stencil row are one contiguous
 // particle range: a query visits 9 ranges per population.
@@ -102,6 +103,54 @@ __global__ __launch_bounds__(BLOCK) void k_scan3(int n, int* __restrict__ start,
     if (blockIdx.x == 0 && threadIdx.x == 0) start[n] = bsum[nb];
 }
 
+// Cell starts in one launch: start[i] = sum(cnt[0..i)), given the chunk totals bsum (k_keys counts
+// them with the cells).  Every block sums the totals before its chunk itself; with at most
+// CELL_SCAN_CHUNKS of them (16 KB, in L2) that costs less than the two launches it saves: three
+// launches took 9.2 us at 8k rows and 14 us at 1M (30k and 860k cells), this one 3.0 and 4.3.
+constexpr int CELL_SCAN_CHUNKS = 4096;
+__global__ __launch_bounds__(BLOCK) void k_cell_starts(int n, int nb, const int* __restrict__ cnt,
+                                                       const int* __restrict__ bsum, int* __restrict__ start) {
+    __shared__ int psum[WAVES_PER_BLOCK];
+    const int base = blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_PER_THREAD;
+    int v[SCAN_PER_THREAD];
+    int sum = 0;
+    if (base + SCAN_PER_THREAD <= n) {   // chunks start on 8-word boundaries of a 256-byte aligned table
+        const int4 lo = *reinterpret_cast<const int4*>(cnt + base), hi = *reinterpret_cast<const int4*>(cnt + base + 4);
+        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+    } else {
+#pragma unroll
+        for (int q = 0; q < SCAN_PER_THREAD; ++q) v[q] = base + q < n ? cnt[base + q] : 0;
+    }
+    int before = 0;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += BLOCK) before += bsum[k];
+#pragma unroll
+    for (int q = 0; q < SCAN_PER_THREAD; ++q) sum += v[q];
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
+    if ((threadIdx.x & (WAVE - 1)) == 0) psum[threadIdx.x >> 6] = before;
+    int tot;
+    int run = block_excl_scan(sum, &tot);   // (its barriers also publish psum)
+    before = (psum[0] + psum[1]) + (psum[2] + psum[3]);
+    run += before;
+    if (base + SCAN_PER_THREAD <= n) {
+        int w[SCAN_PER_THREAD];
+#pragma unroll
+        for (int q = 0; q < SCAN_PER_THREAD; ++q) {
+            w[q] = run;
+            run += v[q];
+        }
+        *reinterpret_cast<int4*>(start + base) = make_int4(w[0], w[1], w[2], w[3]);
+        *reinterpret_cast<int4*>(start + base + 4) = make_int4(w[4], w[5], w[6], w[7]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < SCAN_PER_THREAD; ++q) {
+            if (base + q < n) start[base + q] = run;
+            run += v[q];
+        }
+    }
+    if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0) start[n] = before + tot;
+}
+
 // Runs of equal keys among the valid lanes of a wave (valid lanes form a prefix of the wave).
 // Particles arrive in the previous step's cell order, so runs are ~ one cell long and one
 // atomic per run replaces one per particle.
@@ -127,25 +176,99 @@ __device__ __forceinline__ KeyRun key_run(int k, bool valid) {
     return r;
 }
 
-// SCENES: particle i uses the grid of its scene, grids[sid[i]].  clear_flag (if set) is zeroed:
-// the build's overflow flags, set only by passes after this one.
-template <bool SCENES>
-__global__ __launch_bounds__(BLOCK) void k_keys(int count, const float4* __restrict__ pos, Grid g,
-                                                const Grid* __restrict__ grids, const int* __restrict__ sid,
-                                                int* __restrict__ key, int* __restrict__ ccount,
-                                                int* __restrict__ clear_flag) {
+// Position of a particle after dt and its domain clamp: advect_position (framework.py:117-136) +
+// enforce_boundary (boundary.py:27-91); p and the velocity are updated in place.
+struct AdvectArgs {
+    float dt, L0, L1, L2, pad;
+    float* vel;
+    const float* sdom;   // independent scenes: domain size of each scene
+};
+__device__ __forceinline__ void advect(const AdvectArgs& a, int i, int scene, float4& p) {
+    float v[3] = {a.vel[3 * i + 0], a.vel[3 * i + 1], a.vel[3 * i + 2]};
+    float x[3] = {p.x + a.dt * v[0], p.y + a.dt * v[1], p.z + a.dt * v[2]};
+    float L[3] = {a.L0, a.L1, a.L2};
+    if (a.sdom) {
+        L[0] = a.sdom[3 * scene + 0]; L[1] = a.sdom[3 * scene + 1]; L[2] = a.sdom[3 * scene + 2];
+    }
+    float nrm[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        if (x[q] > L[q] - a.pad) { nrm[q] = nrm[q] + 1.0f; x[q] = L[q] - a.pad; }
+        if (x[q] <= a.pad) { nrm[q] = nrm[q] + -1.0f; x[q] = a.pad; }
+    }
+    float len = len3(nrm[0], nrm[1], nrm[2]);
+    if (len > 1e-6f) {
+        float c0 = nrm[0] / len, c1 = nrm[1] / len, c2 = nrm[2] / len;
+        float s = (1.0f + 0.5f) * (v[0] * c0 + v[1] * c1 + v[2] * c2);
+        a.vel[3 * i + 0] = v[0] - s * c0;
+        a.vel[3 * i + 1] = v[1] - s * c1;
+        a.vel[3 * i + 2] = v[2] - s * c2;
+    }
+    p = make_float4(x[0], x[1], x[2], p.w);
+}
+
+__global__ __launch_bounds__(BLOCK) void k_advect_boundary(int nd, AdvectArgs a, float4* __restrict__ pos,
+                                                           const int* __restrict__ sid) {
     int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (clear_flag && i == 0) *clear_flag = 0;
-    bool valid = i < count;
+    if (i >= nd) return;
+    float4 p = pos[i];
+    advect(a, i, a.sdom ? sid[i] : 0, p);
+    pos[i] = p;
+}
+
+struct KeysArgs {
+    int count;
+    float4* pos;
+    Grid g;
+    const Grid* grids;   // independent scenes: particle i uses the grid of its scene, grids[sid[i]]
+    const int* sid;
+    int* key;
+    int* ccount;
+    int* bsum;           // particles per SCAN_CHUNK cells (k_cell_starts), or nullptr
+    int* clear_flag;     // zeroed if set: the build's overflow flags, set only by passes after this one
+    AdvectArgs adv;
+};
+
+// Cell keys and counts; with ADVECT the particle first moves (the step's advection reads and writes
+// the position that its key needs).
+template <bool SCENES, bool ADVECT>
+__global__ __launch_bounds__(BLOCK) void k_keys(KeysArgs a) {
+    int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (a.clear_flag && i == 0) *a.clear_flag = 0;
+    bool valid = i < a.count;
     int k = -1;
     if (valid) {
-        if (SCENES) g = grids[sid[i]];
-        float4 p = pos[i];
+        const int scene = SCENES ? a.sid[i] : 0;
+        const Grid g = SCENES ? a.grids[scene] : a.g;
+        float4 p = a.pos[i];
+        if (ADVECT) {
+            advect(a.adv, i, scene, p);
+            a.pos[i] = p;
+        }
         k = cell_key(g, cell_coord(g, p.x, 0), cell_coord(g, p.y, 1), cell_coord(g, p.z, 2));
-        key[i] = k;
+        a.key[i] = k;
     }
     KeyRun r = key_run(k, valid);
-    if (r.head) atomicAdd(&ccount[k], r.len);
+    if (r.head) atomicAdd(&a.ccount[k], r.len);
+    if (a.bsum) {
+        // chunk totals: a block's particles mostly share the chunk of its first one, so that chunk
+        // takes one atomic per block (one per wave serialised on few addresses: 6 -> 26 us at 1M
+        // rows) and other chunks one per run
+        __shared__ int first, same[WAVES_PER_BLOCK];
+        const int c = valid ? k / SCAN_CHUNK : -1;
+        if (threadIdx.x == 0) first = c;
+        __syncthreads();
+        const bool in = valid && c == first;
+        const int n = __popcll(__ballot(in));
+        if ((threadIdx.x & (WAVE - 1)) == 0) same[threadIdx.x >> 6] = n;
+        const unsigned long long rest = __ballot(valid && !in);
+        if (rest) {
+            KeyRun t = key_run(c, valid);
+            if (t.head && !in) atomicAdd(&a.bsum[c], t.len);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) atomicAdd(&a.bsum[first], (same[0] + same[1]) + (same[2] + same[3]));
+    }
 }
 
 // slot = start[key] + (remaining count - 1); leaves ccount at zero for the next sort.  A run's
@@ -168,24 +291,13 @@ __global__ __launch_bounds__(BLOCK) void k_scatter(int count, const int* __restr
     }
 }
 
-// final position = cell start + number of cell members with a smaller user id
-__global__ __launch_bounds__(BLOCK) void k_rank(int count, const int* __restrict__ key,
-                                                const int* __restrict__ start, const int* __restrict__ cell_uid,
-                                                const int* __restrict__ uid, int* __restrict__ order) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= count) return;
-    int k = key[i];
-    int lo = start[k], hi = start[k + 1];
-    int u = uid[i];
-    int rank = 0;
-#pragma unroll 4
-    for (int s = lo; s < hi; ++s) rank += cell_uid[s] < u ? 1 : 0;
-    order[lo + rank] = i;
-}
-
-struct GatherArgs {
+struct PlaceArgs {
     int count, offset;
-    const int* order;
+    const int* key;
+    const int* start;
+    const int* cell_uid;
+    int* bsum;   // chunk totals cleared for the next sort (nullptr: not used)
+    int nb;
     const float4* pos; float4* pos_b;
     const float* vel; float* vel_b;
     const float* minv; float* minv_b;
@@ -196,23 +308,42 @@ struct GatherArgs {
     const float* divg; float* divg_b;
 };
 
+// Final place of particle i = cell start + number of cell members with a smaller user id, and its
+// arrays moved there.  Particles arrive in the previous step's cell order, so the writes of a wave
+// stay close together; ranking and a gather by the inverse order took two launches and the order
+// array (1M rows: 7 + 27 us against 25; 8k rows 3.2 + 4.0 against 3.7).
 template <bool VEL>
-__global__ __launch_bounds__(BLOCK) void k_gather(GatherArgs a) {
-    int s = blockIdx.x * BLOCK + threadIdx.x;
-    if (s >= a.count) return;
-    int src = a.offset + a.order[s];
-    int dst = a.offset + s;
-    a.pos_b[dst] = a.pos[src];
+__global__ __launch_bounds__(BLOCK) void k_place(PlaceArgs a) {
+    int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (a.bsum)
+        for (int q = i; q < a.nb; q += (int)gridDim.x * BLOCK) a.bsum[q] = 0;
+    if (i >= a.count) return;
+    const int src = a.offset + i;
+    const int u = a.uid[src];
+    const int k = a.key[i];
+    const float4 p = a.pos[src];
+    const float minv = a.minv[src], rho0 = a.rho0[src];
+    const int mat = a.mat[src];
+    float v0 = 0.0f, v1 = 0.0f, v2 = 0.0f, dv = 0.0f;
     if (VEL) {
-        a.vel_b[3 * dst + 0] = a.vel[3 * src + 0];
-        a.vel_b[3 * dst + 1] = a.vel[3 * src + 1];
-        a.vel_b[3 * dst + 2] = a.vel[3 * src + 2];
-        a.divg_b[dst] = a.divg[src];
+        v0 = a.vel[3 * src + 0]; v1 = a.vel[3 * src + 1]; v2 = a.vel[3 * src + 2];
+        dv = a.divg[src];
     }
-    a.minv_b[dst] = a.minv[src];
-    a.rho0_b[dst] = a.rho0[src];
-    a.mat_b[dst] = a.mat[src];
-    int u = a.uid[src];
+    const int lo = a.start[k], hi = a.start[k + 1];
+    int rank = 0;
+#pragma unroll 4
+    for (int s = lo; s < hi; ++s) rank += a.cell_uid[s] < u ? 1 : 0;
+    const int dst = a.offset + lo + rank;
+    a.pos_b[dst] = p;
+    if (VEL) {
+        a.vel_b[3 * dst + 0] = v0;
+        a.vel_b[3 * dst + 1] = v1;
+        a.vel_b[3 * dst + 2] = v2;
+        a.divg_b[dst] = dv;
+    }
+    a.minv_b[dst] = minv;
+    a.rho0_b[dst] = rho0;
+    a.mat_b[dst] = mat;
     a.uid_b[dst] = u;
     a.inv[u] = dst;
 }
@@ -1412,6 +1543,11 @@ int scan(ivp_ctx* c, const int* cnt, int* start, int n) {
     return IVP_OK;
 }
 
+AdvectArgs advect_args(ivp_ctx* c, float dt) {
+    return AdvectArgs{dt, c->cfg.domain_size[0], c->cfg.domain_size[1], c->cfg.domain_size[2], c->h, c->vel,
+                      c->S > 0 ? c->sdomain : nullptr};
+}
+
 template <class T>
 void swap_ptr(T*& a, T*& b) {
     T* t = a;
@@ -1424,35 +1560,44 @@ void swap_ptr(T*& a, T*& b) {
 namespace ivp {
 
 // Sort one population [offset, offset + count) of the store by (cell key, user id) and fill
-// its cell table `start_table` (ncell + 1 entries, relative to offset).
-int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bool dynamic) {
+// its cell table `start_table` (ncell + 1 entries, relative to offset).  With adv the particles are
+// advected first.
+int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bool dynamic, const float* adv_dt) {
     if (count <= 0) {
         IVP_HIP(hipMemsetAsync(start_table, 0, sizeof(int) * (size_t)(c->ncell + 1), c->stream));
         return IVP_OK;
     }
     const dim3 nb(blocks_for(count));
-    // bytes: keys (read x 16, write key 4), scatter (key 4 + slot 4), rank (key, uid, cell members
-    // ~ 3 x 4), gather (index 4 + every per-particle array read and written)
-    const double per = dynamic ? 4 + 2 * (16 + 12 + 4 + 4 + 4 + 4 + 4) + 4 : 4 + 2 * (16 + 4 + 4 + 4 + 4) + 4;
-    // the dynamic population's sort starts a rebuild: its first pass clears the overflow flags
-    int* clear = dynamic ? c->err_flag : nullptr;
+    // bytes: keys (read x 16, write key 4; advection: v read, x written), scatter (key 4 + slot 4),
+    // placing (key, uid, cell members ~ 3 x 4, and every per-particle array read and written)
+    const double per = 20 + (dynamic ? 2 * (16 + 12 + 4 + 4 + 4 + 4 + 4) + 4 : 2 * (16 + 4 + 4 + 4 + 4) + 4);
+    const int chunks = (c->ncell + SCAN_CHUNK - 1) / SCAN_CHUNK;
+    int* bsum = chunks <= CELL_SCAN_CHUNKS ? c->cell_bsum : nullptr;
+    KeysArgs ka{count, c->pos + offset, c->grid, c->grids, c->sid ? c->sid + offset : nullptr, c->key, c->ccount, bsum,
+                // the dynamic population's sort starts a rebuild: its first pass clears the overflow flags
+                dynamic ? c->err_flag : nullptr, advect_args(c, adv_dt ? *adv_dt : 0.0f)};
+    const double kb = (c->S > 0 ? 24.0 : 20.0) * count + (adv_dt ? 28.0 * count : 0.0);
     if (c->S > 0)
-        IVP_TRY(launch(c, KC_SORT, -1, 24.0 * count, k_keys<true>, nb, count, (const float4*)(c->pos + offset), c->grid,
-                       (const Grid*)c->grids, (const int*)(c->sid + offset), c->key, c->ccount, clear));
+        IVP_TRY(adv_dt ? launch(c, KC_SORT, -1, kb, k_keys<true, true>, nb, ka)
+                       : launch(c, KC_SORT, -1, kb, k_keys<true, false>, nb, ka));
     else
-        IVP_TRY(launch(c, KC_SORT, -1, 20.0 * count, k_keys<false>, nb, count, (const float4*)(c->pos + offset),
-                       c->grid, (const Grid*)nullptr, (const int*)nullptr, c->key, c->ccount, clear));
-    IVP_TRY(scan(c, c->ccount, start_table, c->ncell));
+        IVP_TRY(adv_dt ? launch(c, KC_SORT, -1, kb, k_keys<false, true>, nb, ka)
+                       : launch(c, KC_SORT, -1, kb, k_keys<false, false>, nb, ka));
+    if (bsum) {
+        hipLaunchKernelGGL(k_cell_starts, dim3(chunks), dim3(BLOCK), 0, c->stream, c->ncell, chunks,
+                           (const int*)c->ccount, (const int*)bsum, start_table);
+        IVP_HIP(hipGetLastError());
+    } else {
+        IVP_TRY(scan(c, c->ccount, start_table, c->ncell));
+    }
     IVP_TRY(launch(c, KC_SORT, -1, 16.0 * count, k_scatter, nb, count, (const int*)c->key, (const int*)start_table,
                    c->ccount, (const int*)(c->uid + offset), c->tmp_src));
-    IVP_TRY(launch(c, KC_SORT, -1, 20.0 * count, k_rank, nb, count, (const int*)c->key, (const int*)start_table,
-                   (const int*)c->tmp_src, (const int*)(c->uid + offset), c->order));
-    GatherArgs ga{count, offset, c->order, c->pos, c->pos_b, c->vel, c->vel_b, c->minv, c->minv_b,
-                  c->rho0, c->rho0_b, c->mat, c->mat_b, c->uid, c->uid_b, c->inv, c->divg, c->divg_b};
+    PlaceArgs pa{count, offset, c->key, start_table, c->tmp_src, bsum, chunks, c->pos, c->pos_b, c->vel, c->vel_b,
+                 c->minv, c->minv_b, c->rho0, c->rho0_b, c->mat, c->mat_b, c->uid, c->uid_b, c->inv, c->divg, c->divg_b};
     if (dynamic)
-        IVP_TRY(launch(c, KC_SORT, -1, per * count, k_gather<true>, nb, ga));
+        IVP_TRY(launch(c, KC_SORT, -1, per * count, k_place<true>, nb, pa));
     else
-        IVP_TRY(launch(c, KC_SORT, -1, per * count, k_gather<false>, nb, ga));
+        IVP_TRY(launch(c, KC_SORT, -1, per * count, k_place<false>, nb, pa));
     swap_ptr(c->pos, c->pos_b);
     swap_ptr(c->minv, c->minv_b);
     swap_ptr(c->rho0, c->rho0_b);
@@ -1520,7 +1665,7 @@ int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m,
     // so afterwards the staged dynamic segment [0, nd) lives in the reorder buffers and the
     // sorted static segment in the primary ones: copy each segment across so both copies of
     // every per-particle array are complete and identical.
-    rc = grid_sort_population(c, c->nd, c->ns, c->sstart, false);
+    rc = grid_sort_population(c, c->nd, c->ns, c->sstart, false, nullptr);
     if (rc != IVP_OK) return rc;
     size_t off = (size_t)c->nd, cnt = (size_t)c->ns;
     if (cnt > 0) {
@@ -1584,10 +1729,21 @@ int launch_scan(ivp_ctx* c, int G, const BuildArgs& ba) {
     }
 }
 
-int grid_build(ivp_ctx* c) {
+// advect_position + enforce_boundary of the dynamic particles on their own
+int glue_advect_boundary(ivp_ctx* c, float dt) {
     if (!c->loaded) return IVP_ERR_STATE;
+    if (c->nd == 0) return IVP_OK;
+    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_advect_boundary, dim3(blocks_for(c->nd)), c->nd, advect_args(c, dt), c->pos,
+                   (const int*)c->sid));
+    c->built = false;
+    return IVP_OK;
+}
+
+int grid_build(ivp_ctx* c, const float* adv_dt) {
+    if (!c->loaded) return IVP_ERR_STATE;
+    if (adv_dt && c->nd > 0) c->built = false;
     if (c->nd > 0) {
-        int rc = grid_sort_population(c, 0, c->nd, c->dstart, true);
+        int rc = grid_sort_population(c, 0, c->nd, c->dstart, true, adv_dt);
         if (rc != IVP_OK) return rc;
     } else {
         IVP_HIP(hipMemsetAsync(c->dstart, 0, sizeof(int) * (size_t)(c->ncell + 1), c->stream));

@@ -214,6 +214,7 @@ struct ivp_ctx {
     int* key = nullptr;
     int* tmp_src = nullptr;
     int* order = nullptr;
+    int* cell_bsum = nullptr;   // particles per chunk of cells, all zero between sorts
     int* scan_bsum = nullptr;
     int nscan_blocks = 0;
 
@@ -336,8 +337,10 @@ int iter_mark(ivp_ctx* c, int k);
 void iter_costs(ivp_ctx* c, int n, ivp_ip_stats* st);
 
 // ivp_grid.hip
-int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bool dynamic);
-int grid_build(ivp_ctx* c);
+int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bool dynamic, const float* adv_dt);
+// adv_dt (if set): the dynamic particles are advected by *adv_dt and clamped first (a step's advection)
+int grid_build(ivp_ctx* c, const float* adv_dt = nullptr);
+int glue_advect_boundary(ivp_ctx* c, float dt);
 int grid_export(ivp_ctx* c, int cache_size, int* count, int* ids, float* gradW);
 int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m, const float* m_inv,
               const float* density0, const int* is_dynamic, const int* material);
@@ -361,7 +364,6 @@ enum PrjPart { PRJ_BOTH = 0, PRJ_CD = 1, PRJ_DF = 2 };   // solve (+ solve_df if
 int prj_solve(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* st, int part);
 int prj_buffers(ivp_ctx* c, int passes);   // ivp_api.hip: PRJ buffers, history for `passes`
 int glue_gravity(ivp_ctx* c, const float g[3], float dt);
-int glue_advect_boundary(ivp_ctx* c, float dt);
 
 inline int blocks_for(int n) { return (n + BLOCK - 1) / BLOCK; }
 

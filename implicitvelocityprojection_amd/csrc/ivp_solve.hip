@@ -1698,39 +1698,6 @@ __global__ __launch_bounds__(BLOCK) void k_gravity(int nd, float gx, float gy, f
     vout[3 * i + 2] = vin[3 * i + 2] + gz;
 }
 
-// advect_position (framework.py:117-136) + enforce_boundary (boundary.py:27-91); with SC each
-// particle is clamped to its scene's domain size sdom[3 sid[i] ..].
-template <bool SC>
-__global__ __launch_bounds__(BLOCK) void k_advect_boundary(int nd, float dt, float L0, float L1, float L2, float pad,
-                                                           float4* __restrict__ pos, float* __restrict__ vel,
-                                                           const float* __restrict__ sdom, const int* __restrict__ sid) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    float4 p = pos[i];
-    float v[3] = {vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2]};
-    float x[3] = {p.x + dt * v[0], p.y + dt * v[1], p.z + dt * v[2]};
-    float L[3] = {L0, L1, L2};
-    if (SC) {
-        const int s = sid[i];
-        L[0] = sdom[3 * s + 0]; L[1] = sdom[3 * s + 1]; L[2] = sdom[3 * s + 2];
-    }
-    float nrm[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        if (x[q] > L[q] - pad) { nrm[q] = nrm[q] + 1.0f; x[q] = L[q] - pad; }
-        if (x[q] <= pad) { nrm[q] = nrm[q] + -1.0f; x[q] = pad; }
-    }
-    float len = len3(nrm[0], nrm[1], nrm[2]);
-    if (len > 1e-6f) {
-        float c0 = nrm[0] / len, c1 = nrm[1] / len, c2 = nrm[2] / len;
-        float s = (1.0f + 0.5f) * (v[0] * c0 + v[1] * c1 + v[2] * c2);
-        vel[3 * i + 0] = v[0] - s * c0;
-        vel[3 * i + 1] = v[1] - s * c1;
-        vel[3 * i + 2] = v[2] - s * c2;
-    }
-    pos[i] = make_float4(x[0], x[1], x[2], p.w);
-}
-
 Rows rows_of(ivp_ctx* c) {
     const bool win = c->win_built && c->windows;
     return Rows{c->nb, c->g16, c->tile_len, c->Cs, c->nd, c->pos, c->h, c->kspiky, c->gscale,
@@ -2610,20 +2577,6 @@ int glue_gravity(ivp_ctx* c, const float g[3], float dt) {
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_gravity, dim3(blocks_for(c->nd)), c->nd, g[0] * dt, g[1] * dt, g[2] * dt,
                    (const float*)c->vel, c->vel_b));
     std::swap(c->vel, c->vel_b);
-    return IVP_OK;
-}
-
-int glue_advect_boundary(ivp_ctx* c, float dt) {
-    if (!c->loaded) return IVP_ERR_STATE;
-    if (c->nd == 0) return IVP_OK;
-    if (c->S > 0)
-        IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_advect_boundary<true>, dim3(blocks_for(c->nd)), c->nd, dt, 0.0f, 0.0f,
-                       0.0f, c->h, c->pos, c->vel, (const float*)c->sdomain, (const int*)c->sid));
-    else
-        IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_advect_boundary<false>, dim3(blocks_for(c->nd)), c->nd, dt,
-                       c->cfg.domain_size[0], c->cfg.domain_size[1], c->cfg.domain_size[2], c->h, c->pos, c->vel,
-                       (const float*)nullptr, (const int*)nullptr));
-    c->built = false;
     return IVP_OK;
 }
 
