@@ -75,7 +75,7 @@ void free_all(ivp_ctx* c) {
     dfree(c->w_pinv); dfree(c->w_p4); dfree(c->w_v4); dfree(c->w_dv); dfree(c->w_r); dfree(c->w_z);
     dfree(c->w_Ap); dfree(c->w_rhs); dfree(c->w_fac); dfree(c->v4); dfree(c->w_dv_prev);
     dfree(c->st_gt); dfree(c->st_div); dfree(c->st_b);
-    dfree(c->prj_v0); dfree(c->prj_lam); dfree(c->prj_prev); dfree(c->prj_df_prev); dfree(c->prj_hist);
+    dfree(c->prj_v0); dfree(c->prj_lam); dfree(c->prj_prev); dfree(c->prj_df_prev); hfree(c->prj_hist);
     c->prj_hist_cap = 0;
     dfree(c->partials); dfree(c->state); dfree(c->err_flag); dfree(c->speed_max);
     if (c->state_host) (void)hipHostFree(c->state_host);
@@ -92,8 +92,8 @@ void free_all(ivp_ctx* c) {
     c->prof_pending.clear();
     for (auto e : c->prof_free) (void)hipEventDestroy(e);
     c->prof_free.clear();
-    for (auto e : c->iter_ev) (void)hipEventDestroy(e);
-    c->iter_ev.clear();
+    hfree(c->marks);
+    c->marks_cap = 0;
     if (c->ip_end_ev) (void)hipEventDestroy(c->ip_end_ev);
     c->ip_end_ev = nullptr;
     if (c->wait_ev) (void)hipEventDestroy(c->wait_ev);
@@ -124,11 +124,14 @@ int alloc_all(ivp_ctx* c) {
     A(partials, 4 * (size_t)c->max_blocks);
     A(state, 1); A(err_flag, 1); A(speed_max, 1);
 #undef A
-    IVP_HIP(hipHostMalloc((void**)&c->state_host, sizeof(SolverState), hipHostMallocDefault));
+    IVP_HIP(hipHostMalloc((void**)&c->state_host, 2 * sizeof(SolverState), hipHostMallocDefault));
     IVP_HIP(hipHostMalloc((void**)&c->err_host, sizeof(int), hipHostMallocDefault));
     IVP_HIP(hipHostMalloc((void**)&c->count_host, 4 * sizeof(int), hipHostMallocDefault));
 
-    memset(c->state_host, 0, sizeof(SolverState));
+    memset(c->state_host, 0, 2 * sizeof(SolverState));
+    int khz = 0;
+    IVP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device));
+    c->ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
     IVP_HIP(hipMemsetAsync(c->ccount, 0, sizeof(int) * (size_t)c->ncell, c->stream));
     IVP_HIP(hipMemsetAsync(c->cell_bsum, 0, sizeof(int) * (size_t)c->nscan_blocks, c->stream));
     IVP_HIP(hipMemsetAsync(c->state, 0, sizeof(SolverState), c->stream));
@@ -211,9 +214,9 @@ int prj_buffers(ivp_ctx* c, int passes) {
     }
     if (passes > c->prj_hist_cap) {
         IVP_HIP(hipStreamSynchronize(c->stream));
-        dfree(c->prj_hist);
+        hfree(c->prj_hist);
         c->prj_hist_cap = 0;
-        IVP_TRY(dalloc(&c->prj_hist, (size_t)passes));
+        IVP_HIP(hipHostMalloc((void**)&c->prj_hist, sizeof(double) * (size_t)passes, hipHostMallocDefault));
         c->prj_hist_cap = passes;
     }
     return IVP_OK;
@@ -336,25 +339,25 @@ void prof_set_bytes(ivp_ctx* c, int epoch, int kclass, double bytes) {
         if (e.epoch == epoch && e.kclass == kclass) e.bytes = bytes;
 }
 
-int iter_mark(ivp_ctx* c, int k) {
-    while ((int)c->iter_ev.size() <= k) {
-        hipEvent_t e = nullptr;
-        // read after the stream is synchronised: no system-scope fence needed
-        IVP_HIP(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
-        c->iter_ev.push_back(e);
-    }
-    IVP_HIP(hipEventRecord(c->iter_ev[(size_t)k], c->stream));
+int marks_buffer(ivp_ctx* c, int n) {
+    if (n + 2 <= c->marks_cap) return IVP_OK;
+    const int cap = std::max(256, 2 * (n + 2));
+    unsigned long long* m = nullptr;
+    IVP_HIP(hipStreamSynchronize(c->stream));   // the old marks are complete
+    IVP_HIP(hipHostMalloc((void**)&m, sizeof(unsigned long long) * (size_t)cap, hipHostMallocDefault));
+    memset(m, 0, sizeof(unsigned long long) * (size_t)cap);
+    if (c->marks) memcpy(m, c->marks, sizeof(unsigned long long) * (size_t)c->marks_cap);
+    hfree(c->marks);
+    c->marks = m;
+    c->marks_cap = cap;
     return IVP_OK;
 }
 
 void iter_costs(ivp_ctx* c, int n, ivp_ip_stats* st) {
     st->n_iter_costs = n;
     if (!st->iter_costs) return;
-    for (int k = 0; k < n && k < st->capacity && k + 1 < (int)c->iter_ev.size(); ++k) {
-        float ms = 0.0f;
-        if (hipEventElapsedTime(&ms, c->iter_ev[(size_t)k], c->iter_ev[(size_t)k + 1]) != hipSuccess) ms = 0.0f;
-        st->iter_costs[k] = (double)ms;
-    }
+    for (int k = 0; k < n && k < st->capacity && k + 1 < c->marks_cap; ++k)
+        st->iter_costs[k] = (double)(c->marks[k + 1] - c->marks[k]) * c->ms_per_tick;
 }
 
 int prof_collect(ivp_ctx* c, int cg_iters_done, int epoch) {
@@ -381,11 +384,6 @@ int prof_collect(ivp_ctx* c, int cg_iters_done, int epoch) {
 }
 
 }  // namespace ivp
-
-static int build_code(int err) {
-    if (err & 4) return IVP_ERR_INTERNAL;
-    return (err & 1) ? IVP_NEIGHBOR_OVERFLOW : IVP_OK;
-}
 
 // Status of the neighbour build last enqueued, read with one synchronisation: its error flags
 // (and the solver state, whose pair count the byte figures of the following passes use).
@@ -632,9 +630,11 @@ int ivp_read(ivp_ctx* c, int field, void* dst) {
 
 int ivp_neighbors_build(ivp_ctx* c) {
     if (!c) return IVP_ERR_ARG;
-    int rc = grid_build(c);
+    int rc = grid_build(c, nullptr, true);
     if (rc != IVP_OK) return rc;
-    return build_status(c);
+    if (c->nd == 0) return build_status(c);
+    IVP_HIP(hipStreamSynchronize(c->stream));
+    return build_code(c->state_host->flags);
 }
 
 int ivp_neighbors_export(ivp_ctx* c, int cache_size, int* count, int* ids, float* gradW) {
@@ -659,8 +659,6 @@ int ivp_viscosity_explicit(ivp_ctx* c, float coeff, float dt) {
 int ivp_viscosity_weiler18(ivp_ctx* c, float coeff, float dt, ivp_cg_stats* stats) {
     if (!c) return IVP_ERR_ARG;
     if (c->S > 0) return IVP_ERR_STATE;
-    // rows that the last rebuild truncated are refused before v changes
-    if (c->built) IVP_TRY(build_status(c));
     return visc_weiler18(c, coeff, dt, stats);
 }
 
@@ -679,8 +677,9 @@ int ivp_prj_solve_df(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_sta
 int ivp_surface_tension_jeske23(ivp_ctx* c, float sigma, float dt, ivp_cg_stats* stats) {
     if (!c) return IVP_ERR_ARG;
     if (c->S > 0) return IVP_ERR_STATE;
-    // rows that the last rebuild truncated are refused before v changes
-    if (c->built) IVP_TRY(build_status(c));
+    // (a solve refuses rows that the last rebuild truncated when it reads the flags, v unchanged; a
+    // call that solves nothing reads them here)
+    if (c->built && (c->nd == 0 || sigma == 0.0f || c->static_fluid)) IVP_TRY(build_status(c));
     return st_jeske23(c, sigma, dt, stats);
 }
 
@@ -699,9 +698,10 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
     if (!c->built || c->S > 0) return IVP_ERR_STATE;
     if (prm->surface_tension_coeff != 0.0f && prm->surface_tension_method != 1) return IVP_ERR_ARG;
     if (prm->pressure_method != 0 && prm->pressure_method != 1) return IVP_ERR_ARG;
+    stats_zero(stats);
     // gravity writes the step's velocities into the second buffer; a stage that finds the rows
-    // truncated by the last rebuild (the pressure solve's first synchronisation reads its flags)
-    // swaps the first one back, so such a step leaves v and x as they were
+    // truncated by the last rebuild (the first solve's first read-back brings its flags) swaps the
+    // first one back, so such a step leaves v and x as they were
     int rc = glue_gravity(c, prm->gravity, prm->dt);
     if (rc != IVP_OK) return rc;
     auto truncated = [&](int r) {
@@ -713,7 +713,7 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
     // compute_non_pressure_forces order (framework.py:400-421): gravity, surface tension, viscosity
     if (prm->surface_tension_coeff != 0.0f) {
         rc = st_jeske23(c, prm->surface_tension_coeff, prm->dt, st);
-        if (rc != IVP_OK) return rc;
+        if (rc != IVP_OK) return truncated(rc);
     }
     // coefficient 0 makes either viscosity model an exact no-op (the rhs v - A v is 0, and the
     // explicit force is scaled by the coefficient)
@@ -722,7 +722,7 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
             rc = visc_weiler18(c, prm->viscosity_coeff, prm->dt, visc);
         else
             rc = visc_explicit(c, prm->viscosity_coeff, prm->dt);
-        if (rc != IVP_OK) return rc;
+        if (rc != IVP_OK) return truncated(rc);
     }
     // pressure solve (framework.py:481-487; PRJ's divergence-free pass runs inside prj_solve).
     // The IP solve's closing wait (its wall time and stats_iter_costs) comes after the rest of

@@ -1739,7 +1739,7 @@ int glue_advect_boundary(ivp_ctx* c, float dt) {
     return IVP_OK;
 }
 
-int grid_build(ivp_ctx* c, const float* adv_dt) {
+int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
     if (!c->loaded) return IVP_ERR_STATE;
     if (adv_dt && c->nd > 0) c->built = false;
     if (c->nd > 0) {
@@ -1816,7 +1816,8 @@ int grid_build(ivp_ctx* c, const float* adv_dt) {
     }
     // pair count (row 0) and window sizes (row 1) of the build's blocks
     if (c->nd > 0)
-        IVP_TRY(finalize<FIN_BUILD>(c, tiles_per_block == 1 ? (c->nd + WAVE - 1) / WAVE : blocks_for(c->nd)));
+        IVP_TRY(finalize<FIN_BUILD>(c, tiles_per_block == 1 ? (c->nd + WAVE - 1) / WAVE : blocks_for(c->nd), 0.0, 0,
+                                    false, report ? c->state_host : nullptr));
     c->built = true;
     return IVP_OK;
 }

@@ -68,6 +68,7 @@ struct SolverState {
     long long active_pairs;
     long long total_pairs;  // stored (dynamic-dynamic) neighbour pairs of the last build
     long long win_entries;  // neighbour ids in the tile windows of the last build
+    int flags;              // the build's error flags, as of the last report to the host
 };
 
 // Independent scenes in one context.  Each scene has its own cell grid (keys of scene s follow
@@ -256,7 +257,7 @@ struct ivp_ctx {
     float2* prj_lam = nullptr;    // (dt^2 lambda, m) per dynamic row
     float* prj_prev = nullptr;    // p_previous, user order
     float* prj_df_prev = nullptr; // dt2_lam_df_previous, user order
-    double* prj_hist = nullptr;   // density error per pass
+    double* prj_hist = nullptr;   // density error per pass (pinned, written by the device)
     int prj_hist_cap = 0;
     int prj_guess = 8;            // first launch chunk of the next pass loop
 
@@ -264,7 +265,10 @@ struct ivp_ctx {
     double* partials = nullptr;   // 4 * max_blocks
     int max_blocks = 0;
     ivp::SolverState* state = nullptr;      // device
-    ivp::SolverState* state_host = nullptr; // pinned
+    // pinned, written by the device: a kernel that ends a stage stores the state there itself, and the
+    // host reads it after waiting for that kernel.  [0] the last report taken, [1] the report of a
+    // constraint pass queued behind another one's wait
+    ivp::SolverState* state_host = nullptr;
     int* err_flag = nullptr;                // device: bit 0 neighbour overflow, bit 2 a kernel's
                                             // consistency guard (set by the build)
     unsigned* speed_max = nullptr;          // device: bits of max |v|^2 (ivp_max_speed2)
@@ -302,8 +306,11 @@ struct ivp_ctx {
     int sgraph_next = 0;
     long long scene_replays = 0;          // replays of the last batched solve
 
-    // stream marks at outer-iteration / pass boundaries (stats_iter_costs)
-    std::vector<hipEvent_t> iter_ev;
+    // device clock at outer-iteration / pass boundaries (stats_iter_costs): pinned, written by the
+    // passes themselves
+    unsigned long long* marks = nullptr;
+    int marks_cap = 0;
+    double ms_per_tick = 0.0;
     // an IP solve whose closing wait was left to the caller (ivp_step enqueues the rest of the
     // step first): its end mark, start time and outer-loop evaluation count
     hipEvent_t ip_end_ev = nullptr;
@@ -331,15 +338,17 @@ int prof_take(ivp_ctx* c, int kclass, int tag, double bytes, ProfEvent* ev);
 int prof_push(ivp_ctx* c, ProfEvent* ev);
 int prof_collect(ivp_ctx* c, int cg_iters_done, int epoch);
 void prof_set_bytes(ivp_ctx* c, int epoch, int kclass, double bytes);
-// stats_iter_costs: mark k on the stream at the start of outer-loop evaluation k (mark n after the
-// last); iter_costs fills the n intervals once the stream has been synchronised
-int iter_mark(ivp_ctx* c, int k);
+// stats_iter_costs: the passes store the device clock at the start of outer-loop evaluation k in
+// mark k (mark n after the last), kept for `n` evaluations at least; iter_costs fills the n intervals
+// once the stream has been synchronised
+int marks_buffer(ivp_ctx* c, int n);
 void iter_costs(ivp_ctx* c, int n, ivp_ip_stats* st);
 
 // ivp_grid.hip
 int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bool dynamic, const float* adv_dt);
 // adv_dt (if set): the dynamic particles are advected by *adv_dt and clamped first (a step's advection)
-int grid_build(ivp_ctx* c, const float* adv_dt = nullptr);
+// report: the build's pair counts and error flags go to state_host (for nd > 0)
+int grid_build(ivp_ctx* c, const float* adv_dt = nullptr, bool report = false);
 int glue_advect_boundary(ivp_ctx* c, float dt);
 int grid_export(ivp_ctx* c, int cache_size, int* count, int* ids, float* gradW);
 int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m, const float* m_inv,
@@ -355,6 +364,7 @@ int ip_solve_scenes(ivp_ctx* c, float dt, const ivp_ip_params* prm);
 // ip_solve_wait, so that the caller can enqueue more work first
 int ip_solve(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* st, bool defer = false);
 int ip_solve_wait(ivp_ctx* c, ivp_ip_stats* st);
+void stats_zero(ivp_ip_stats* st);   // every result field (not the caller's arrays)
 int visc_explicit(ivp_ctx* c, float coeff, float dt);
 int visc_weiler18(ivp_ctx* c, float coeff, float dt, ivp_cg_stats* st);
 int st_jeske23(ivp_ctx* c, float sigma, float dt, ivp_cg_stats* st);
@@ -364,6 +374,11 @@ enum PrjPart { PRJ_BOTH = 0, PRJ_CD = 1, PRJ_DF = 2 };   // solve (+ solve_df if
 int prj_solve(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* st, int part);
 int prj_buffers(ivp_ctx* c, int passes);   // ivp_api.hip: PRJ buffers, history for `passes`
 int glue_gravity(ivp_ctx* c, const float g[3], float dt);
+
+// status of a build from its error flags
+inline int build_code(int flags) {
+    return (flags & 4) ? IVP_ERR_INTERNAL : (flags & 1) ? IVP_NEIGHBOR_OVERFLOW : IVP_OK;
+}
 
 inline int blocks_for(int n) { return (n + BLOCK - 1) / BLOCK; }
 

@@ -32,7 +32,17 @@ struct FinArgs {
     double tol;
     int max_iter;
     int gated;   // FIN_PACK queued behind a CG read-back: only once that CG stopped without failing
+    SolverState* host;           // pinned copy of the state for the host (nullptr: none)
+    const int* flags;            // the build's error flags, reported with it
+    unsigned long long* mark;    // device clock after the reduction (nullptr: none)
 };
+
+// Report to the host: the state, with the build's error flags, into pinned memory.  The host waits
+// for the kernel; no copy command follows it.
+__device__ __forceinline__ void report_state(SolverState* st, SolverState* host, const int* flags) {
+    st->flags = *flags;
+    *host = *st;
+}
 
 constexpr int FIN_BLOCK = 1024;
 constexpr int FIN_UNROLL = 4;  // the fold below adds exactly four loads per row
@@ -192,20 +202,25 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
     // the p pass before this one applied the last iteration's dv update, if any (iterations
     // enqueued past the stop must not apply it again)
     if (OP == FIN_W18_PAP && threadIdx.x == 0) st->dv_apply = 0;
-    if (OP == FIN_PACK && a.gated && (st->active != 0 || st->status != 0)) return;
-    if (OP == FIN_CG_PAP || OP == FIN_CG_UPDATE || OP == FIN_W18_PAP || OP == FIN_W18_UPDATE || OP == FIN_CG_REPLACE) {
-        if (st->active == 0) return;
+    const bool skip = (OP == FIN_PACK && a.gated && (st->active != 0 || st->status != 0)) ||
+                      ((OP == FIN_CG_PAP || OP == FIN_CG_UPDATE || OP == FIN_W18_PAP || OP == FIN_W18_UPDATE ||
+                        OP == FIN_CG_REPLACE) && st->active == 0);
+    if (!skip) {
+        double t[3] = {0.0, 0.0, 0.0};
+        fold_partials<NV>(a.partials, a.stride, a.nblocks, t);
+        if (threadIdx.x == 0) {
+            fin_apply<OP>(st, t, a.tol, a.max_iter);
+            if (a.mark) *a.mark = wall_clock64();
+        }
     }
-    double t[3] = {0.0, 0.0, 0.0};
-    fold_partials<NV>(a.partials, a.stride, a.nblocks, t);
-    if (threadIdx.x != 0) return;
-    fin_apply<OP>(st, t, a.tol, a.max_iter);
+    if (a.host && threadIdx.x == 0) report_state(st, a.host, a.flags);
 }
 
 
 template <int OP>
-inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0, bool gated = false) {
-    FinArgs fa{c->partials, c->max_blocks, nblocks, c->state, tol, max_iter, gated ? 1 : 0};
+inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0, bool gated = false,
+                    SolverState* host = nullptr, unsigned long long* mark = nullptr) {
+    FinArgs fa{c->partials, c->max_blocks, nblocks, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
     hipLaunchKernelGGL(k_finalize<OP>, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
     IVP_HIP(hipGetLastError());
     return IVP_OK;

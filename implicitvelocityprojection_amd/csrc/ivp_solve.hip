@@ -384,6 +384,7 @@ struct PackArgs {
     // when set: the pass runs only if the CG of this state has stopped without failing (a pass
     // queued behind a CG chunk's read-back)
     const SolverState* gate = nullptr;
+    unsigned long long* mark = nullptr;   // device clock at the pass's start (stats_iter_costs)
 };
 
 // A CG of state st has stopped, and not on a non-positive p.Ap
@@ -395,6 +396,7 @@ __device__ __forceinline__ bool cg_stopped(const SolverState* st) { return st->a
 template <class FM, bool SC, int G = lanes_for<SC>()>
 __global__ __launch_bounds__(BLOCK) void k_ip_pack(PackArgs a) {
     if (!SC && a.gate && !cg_stopped(a.gate)) return;
+    if (!SC && a.mark && blockIdx.x == 0 && threadIdx.x == 0) *a.mark = wall_clock64();
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
     Gate gt = gate_all(i, a.R.nd);
@@ -797,6 +799,7 @@ struct PrjArgs {
     double* partials;
     int stride;
     const SolverState* st;
+    unsigned long long* mark0;   // device clock at the head's start (nullptr: not recorded)
 };
 
 // PRJ.solve prologue (prj.py:307-324): c = rho - rho0 (constant-density loop only),
@@ -807,8 +810,16 @@ __global__ __launch_bounds__(BLOCK) void k_prj_init(int nd, float dt, const floa
                                                     const float* __restrict__ rho0, const float* __restrict__ vel,
                                                     const float4* __restrict__ pos, const int* __restrict__ uid,
                                                     const float* __restrict__ prev, int warm, float* __restrict__ cc,
-                                                    float* __restrict__ v0, float2* __restrict__ lam) {
+                                                    float* __restrict__ v0, float2* __restrict__ lam,
+                                                    SolverState* __restrict__ st) {
     int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i == 0) {   // the pass loop's state
+        st->iter = 0;
+        st->active = 1;
+        st->status = 0;
+        st->rr0 = 0.0;
+        st->rr_last = 0.0;
+    }
     if (i >= nd) return;
     if (!DF) cc[i] = density[i] - rho0[i];
     v0[3 * i + 0] = dt * vel[3 * i + 0];
@@ -823,6 +834,7 @@ __global__ __launch_bounds__(BLOCK) void k_prj_init(int nd, float dt, const floa
 template <class FM>
 __global__ __launch_bounds__(BLOCK) void k_prj_head(PrjArgs a) {
     if (a.st->active == 0) return;
+    if (a.mark0 && blockIdx.x == 0 && threadIdx.x == 0) *a.mark0 = wall_clock64();
     constexpr int G = PASS_LANES;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
@@ -918,8 +930,11 @@ struct PrjFinArgs {
     int max_pass;
     int fixed;
     int nd;
-    double* hist;      // density error per pass (nullptr: not recorded)
+    double* hist;      // density error per pass, in pinned memory (nullptr: not recorded)
     int hist_cap;
+    unsigned long long* marks;   // device clock at the end of each pass (nullptr: not recorded)
+    SolverState* host;           // the state for the host after the last pass of a chunk
+    const int* flags;
 };
 
 // The stop test of the pass loop (prj.py:197-206, 277-281): err = avg(max(r / rho0, 0)); stop when
@@ -927,11 +942,15 @@ struct PrjFinArgs {
 // (stats_outer_iters once the loop has stopped); rr0 / rr_last hold the first and the last err.
 __global__ __launch_bounds__(FIN_BLOCK) void k_fin_prj(PrjFinArgs a) {
     SolverState* st = a.st;
-    if (st->active == 0) return;
+    if (st->active == 0) {
+        if (a.host && threadIdx.x == 0) report_state(st, a.host, a.flags);
+        return;
+    }
     double t[3] = {0.0, 0.0, 0.0};
     fold_partials<1>(a.partials, a.stride, a.nblocks, t);
     if (threadIdx.x != 0) return;
     const int pass = st->iter;
+    if (a.marks) a.marks[pass + 1] = wall_clock64();
     const double err = t[0] / (double)a.nd;
     if (a.hist && pass < a.hist_cap) a.hist[pass] = err;
     if (pass == 0) st->rr0 = err;
@@ -941,14 +960,7 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_fin_prj(PrjFinArgs a) {
         st->active = 0;
     else
         st->iter = pass + 1;
-}
-
-__global__ void k_prj_state_init(SolverState* st) {
-    st->iter = 0;
-    st->active = 1;
-    st->status = 0;
-    st->rr0 = 0.0;
-    st->rr_last = 0.0;
+    if (a.host) report_state(st, a.host, a.flags);
 }
 
 // wp.copy(p_previous, dt2_lam) (prj.py:204, 280), into user order
@@ -1267,8 +1279,8 @@ __global__ __launch_bounds__(BLOCK) void k_w18_warm_init(W18Args a, const float*
 // the internal row found through inv (static particles keep their zero)
 __global__ __launch_bounds__(BLOCK) void k_w18_save(int n, int nd, const float* __restrict__ dv,
                                                     const int* __restrict__ inv, float* __restrict__ dv_prev,
-                                                    const SolverState* __restrict__ st) {
-    if (st && st->active != 0) return;   // the solve continues: a later launch saves
+                                                    const SolverState* __restrict__ st, const int* __restrict__ flags) {
+    if (st->active != 0 || (*flags & 5)) return;   // the solve continues (a later launch saves), or truncated rows
     int u = blockIdx.x * BLOCK + threadIdx.x;
     if (u >= n) return;
     const int i = inv[u];
@@ -1370,10 +1382,11 @@ __global__ __launch_bounds__(BLOCK) void k_w18_p(int nd, const float* __restrict
     }
 }
 
-// v += dv (weiler18.py:399-401), once the solve has stopped
+// v += dv (weiler18.py:399-401), once the solve has stopped; rows that the last build truncated
+// leave v as it was (the host refuses them when it reads the flags)
 __global__ __launch_bounds__(BLOCK) void k_w18_apply(int n3, const float* __restrict__ dv, float* __restrict__ vel,
-                                                     const SolverState* __restrict__ st) {
-    if (st && st->active != 0) return;   // nullptr: unconditional
+                                                     const SolverState* __restrict__ st, const int* __restrict__ flags) {
+    if (st->active != 0 || (*flags & 5)) return;
     int i = blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n3) return;
     vel[i] = vel[i] + 1.0f * dv[i];
@@ -1832,47 +1845,35 @@ int scene_graph(ivp_ctx* c, float omega, int K, hipGraphExec_t* out) {
     return IVP_OK;
 }
 
-int read_state(ivp_ctx* c) {
-    IVP_HIP(hipMemcpyAsync(c->state_host, c->state, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
-    IVP_HIP(hipStreamSynchronize(c->stream));
-    return IVP_OK;
-}
+__global__ void k_report(SolverState* st, SolverState* host, const int* flags) { report_state(st, host, flags); }
 
-// Enqueue CG iterations in chunks until the device-side state says stop.  `launch_it(tag)`
-// enqueues one iteration.  Returns the iteration count in *iters.
-// The solver state copied back after the work enqueued so far, then `tail` enqueued (work that
-// follows a finished solve and returns at once while it continues), then a wait for the copy
-// alone: the device runs the tail while the host takes the state.
-template <class T>
-int read_state_then(ivp_ctx* c, T&& tail) {
-    IVP_HIP(hipMemcpyAsync(c->state_host, c->state, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
-    if (!c->wait_ev) IVP_HIP(hipEventCreateWithFlags(&c->wait_ev, hipEventDisableTiming));
-    IVP_HIP(hipEventRecord(c->wait_ev, c->stream));
-    IVP_TRY(tail());
-    IVP_HIP(hipEventSynchronize(c->wait_ev));
-    return IVP_OK;
-}
-
-// With a tail, every chunk's read-back is followed by the tail; it has run on a finished solve
-// when the returned state is inactive.
+// Enqueue CG iterations in chunks until the device-side state says stop.  `launch_it(tag, host)`
+// enqueues one iteration; the last one of a chunk reports the state to `host`.  After each chunk
+// `tail` is enqueued (work that follows a finished solve and returns at once while it continues),
+// then the host waits for the report alone: the device runs the tail while the host takes the
+// state.  The tail has run on a finished solve when the reported state is inactive.
 template <class L, class T>
 int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, int* chunks, T&& tail) {
     int issued = 0;
     int chunk = std::max(2, std::min(guess, 64));
+    if (!c->wait_ev) IVP_HIP(hipEventCreateWithFlags(&c->wait_ev, hipEventDisableTiming));
     for (;;) {
         int todo = std::min(chunk, max_iter - issued);
         if (todo <= 0) {
-            // no iteration allowed at all: the set-up left the solve stopped; read it back (and
-            // run the tail) all the same
-            if (issued == 0) IVP_TRY(read_state_then(c, tail));
-            break;
+            if (issued > 0) break;
+            // no iteration allowed at all: the set-up left the solve stopped; report it all the same
+            todo = 0;
+            hipLaunchKernelGGL(k_report, dim3(1), dim3(1), 0, c->stream, c->state, c->state_host, (const int*)c->err_flag);
+            IVP_HIP(hipGetLastError());
         }
-        for (int q = 0; q < todo; ++q) IVP_TRY(launch_it(issued + q));
+        for (int q = 0; q < todo; ++q) IVP_TRY(launch_it(issued + q, q == todo - 1 ? c->state_host : nullptr));
         issued += todo;
-        IVP_TRY(read_state_then(c, tail));
+        IVP_HIP(hipEventRecord(c->wait_ev, c->stream));
+        IVP_TRY(tail());
+        IVP_HIP(hipEventSynchronize(c->wait_ev));
         (*chunks)++;
         const SolverState& s = *c->state_host;
-        if (s.active == 0) break;
+        if (s.active == 0 || todo == 0 || build_code(s.flags) != IVP_OK) break;   // (truncated rows: refused)
         const double rr0 = s.rr0;
         // geometric extrapolation of r.r to the tolerance
         double rate = s.iter > 0 && rr0 > 0.0 && s.rr_last > 0.0 ? pow(s.rr_last / rr0, 1.0 / s.iter) : 0.5;
@@ -1883,11 +1884,6 @@ int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, i
     }
     *iters = c->state_host->iter;
     return IVP_OK;
-}
-
-template <class L>
-int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, int* chunks) {
-    return run_chunks(c, max_iter, guess, launch_it, iters, chunks, []() { return (int)IVP_OK; });
 }
 
 // Bytes a pass of format FM reads from the pair stream: the id (4 B), plus 12 B of float32 or
@@ -1926,28 +1922,27 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
     bool finish_queued = false; // and k_ip_finish with them
     const float inv_dt = (float)(1.0 / (double)dt);
     double err = 0.0;
-    IVP_TRY(iter_mark(c, 0));
     for (;;) {
+        IVP_TRY(marks_buffer(c, opt_iter + 2));
         PackArgs pa{R, d4, c->Ss, c->cc, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, c->partials, stride};
         double total_pairs = (double)c->state_host->total_pairs;
-        // the constraint pass, its finalize and the flags' copy-back (queued in one piece)
-        auto queue_pack = [&](const SolverState* gate) -> int {
+        // the constraint pass of evaluation k and its finalize, which reports the state
+        auto queue_pack = [&](int k, const SolverState* gate) -> int {
             PackArgs pg = pa;
             pg.gate = gate;
+            pg.mark = c->marks + k;
             IVP_TRY(launch(c, KC_IP_PACK, -1, stream_bytes<FP>(c, total_pairs) + 68.0 * nd, k_ip_pack<FP, false>, np, pg));
-            IVP_TRY(finalize<FIN_PACK>(c, np.x, 0.0, 0, gate != nullptr));
-            IVP_HIP(hipMemcpyAsync(c->err_host, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-            return IVP_OK;
+            return finalize<FIN_PACK>(c, np.x, 0.0, 0, gate != nullptr, c->state_host + 1, c->marks + k + 1);
         };
-        if (!pack_queued) IVP_TRY(queue_pack(nullptr));
+        if (!pack_queued) IVP_TRY(queue_pack(opt_iter, nullptr));
         pack_queued = false;
         // The first evaluation never ends the loop (the stop needs opt_iter >= 1, ip.py:374-376),
         // so the first CG follows without a wait: its first chunk's synchronisation brings back the
         // overflow flags and this pass's error sum and active counts (no later finalize writes them)
         // before anything reads them.
         auto record = [&]() -> int {
-            if (*c->err_host & 4) return IVP_ERR_INTERNAL;
-            if (*c->err_host & 1) return IVP_NEIGHBOR_OVERFLOW;
+            if (c->state_host->flags & 4) return IVP_ERR_INTERNAL;
+            if (c->state_host->flags & 1) return IVP_NEIGHBOR_OVERFLOW;
             err = c->state_host->err_sum / (double)nd;
             if (st.n_density_errors < st.capacity && st.density_errors) st.density_errors[st.n_density_errors] = err;
             st.n_density_errors++;
@@ -1967,13 +1962,11 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
                 IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_finish, nb, nd, inv_dt, (const float4*)d4, (const float*)c->jd,
                                c->vel, c->divg));
             finish_queued = false;
-            IVP_TRY(read_state(c));
+            IVP_HIP(hipStreamSynchronize(c->stream));
+            *c->state_host = c->state_host[1];
             IVP_TRY(record());
             bool converged = err < prm->tol_opt && !prm->use_fixed_iters;
-            if ((converged && opt_iter >= 1) || opt_iter >= prm->max_iteration_opt) {
-                IVP_TRY(iter_mark(c, opt_iter + 1));
-                break;
-            }
+            if ((converged && opt_iter >= 1) || opt_iter >= prm->max_iteration_opt) break;
             spec_finish = false;
             act_pairs = c->state_host->active_pairs;
             act_rows = c->state_host->n_active_rows;
@@ -2010,7 +2003,7 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             // (its x.Ax partials go to row 2, clear of the update's r.r in row 0)
             CGJTArgs tx{R, c->xs4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials + 2 * stride, stride,
                         c->state};
-            auto one_iter = [&](int tag) -> int {
+            auto one_iter = [&](int tag, SolverState* host) -> int {
                 IVP_TRY(launch(c, KC_CG_J, tag, bJ, k_cg_J<FC, false>, np, ja));
                 IVP_TRY(launch(c, KC_CG_JT, tag, bJT, k_cg_JT<FC, false>, np, ta));
                 IVP_TRY(finalize<FIN_CG_PAP>(c, np.x));
@@ -2025,9 +2018,9 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_refresh, nb, nd, (const float*)c->b,
                                    (const float*)c->Ap, c->r, c->partials + stride, stride,
                                    (const SolverState*)c->state));
-                    IVP_TRY(finalize<FIN_CG_REPLACE>(c, nb.x));
+                    IVP_TRY(finalize<FIN_CG_REPLACE>(c, nb.x, 0.0, 0, false, host));
                 } else {
-                    IVP_TRY(finalize<FIN_CG_UPDATE>(c, nb.x));
+                    IVP_TRY(finalize<FIN_CG_UPDATE>(c, nb.x, 0.0, 0, false, host));
                 }
                 return launch(c, KC_CG_P, tag, bP, k_cg_p<false>, nb, nd, (const float*)c->r, c->p4,
                               (const SolverState*)c->state, SceneRef{});
@@ -2042,8 +2035,7 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
                 const SolverState* gate = c->state;
                 IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_dupdate<false>, nb, nd, d4, (const float*)c->sol, SceneRef{},
                                gate));
-                IVP_TRY(iter_mark(c, opt_iter + 1));
-                IVP_TRY(queue_pack(gate));
+                IVP_TRY(queue_pack(opt_iter + 1, gate));
                 if (fin_next)
                     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_finish, nb, nd, inv_dt, (const float4*)d4,
                                    (const float*)c->jd, c->vel, c->divg));
@@ -2141,11 +2133,11 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         cg.v4 = c->w_p4;
         cg.out = c->w_Ap;
         const double bAv = stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 48.0 * nd;
-        auto one_iter = [&](int tag) -> int {
+        auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_W18_AV, tag, bAv, k_w18_Av<FM, ALLFLUID>, pass_grid(nd), cg));
             IVP_TRY(finalize<FIN_W18_PAP>(c, pass_grid(nd).x));
             IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, cg));
-            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x));
+            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x, 0.0, 0, false, host));
             return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, nd, (const float*)c->w_z, c->w_p4, c->w_dv,
                           (const SolverState*)c->state);
         };
@@ -2153,9 +2145,9 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         // solve has stopped (while the host reads the state)
         auto tail = [&]() -> int {
             IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_w18_save, dim3(blocks_for(c->n)), c->n, nd, (const float*)c->w_dv,
-                           (const int*)c->inv, c->w_dv_prev, (const SolverState*)c->state));
+                           (const int*)c->inv, c->w_dv_prev, (const SolverState*)c->state, (const int*)c->err_flag));
             return launch(c, KC_GLUE, -1, 0.0, k_w18_apply, dim3(blocks_for(3 * nd)), 3 * nd, (const float*)c->w_dv,
-                          c->vel, (const SolverState*)c->state);
+                          c->vel, (const SolverState*)c->state, (const int*)c->err_flag);
         };
         c->prof_epoch++;
         int epoch = c->prof_epoch;
@@ -2166,6 +2158,7 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         c->w18_guess = std::max(2, iters);
         // the device stops the solve at the same 1000 iterations, so the last read-back shows it
         // stopped and the tail after it has run
+        IVP_TRY(build_code(c->state_host->flags));
         if (c->state_host->active != 0) return IVP_ERR_INTERNAL;
     }
     *iters_out = iters;
@@ -2207,24 +2200,30 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
         cg.v4 = c->w_p4;
         cg.out = c->w_Ap;
         const double bAv = stream_bytes<FM>(c, pairs) + 4.0 * pairs + 28.0 * nd;
-        auto one_iter = [&](int tag) -> int {
+        auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_ST_AV, tag, bAv, k_st_Av<FM, ALLFLUID, false>, np, cga));
             IVP_TRY(finalize<FIN_W18_PAP>(c, np.x));
             IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, cg));
-            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x));
+            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x, 0.0, 0, false, host));
             return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, nd, (const float*)c->w_z, c->w_p4, c->w_dv,
                           (const SolverState*)c->state);
         };
+        // v += dv follows each chunk, running once the solve has stopped (unless rows were truncated)
+        auto tail = [&]() -> int {
+            return launch(c, KC_GLUE, -1, 0.0, k_w18_apply, dim3(blocks_for(3 * nd)), 3 * nd, (const float*)c->w_dv,
+                          c->vel, (const SolverState*)c->state, (const int*)c->err_flag);
+        };
         c->prof_epoch++;
         int epoch = c->prof_epoch;
-        IVP_TRY(run_chunks(c, 100, c->st_guess, one_iter, &iters, &chunks));
+        IVP_TRY(run_chunks(c, 100, c->st_guess, one_iter, &iters, &chunks, tail));
         prof_set_bytes(c, epoch, KC_ST_AV, stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 4.0 * (double)c->state_host->total_pairs + 28.0 * nd);
         prof_collect(c, iters, epoch);
         c->st_guess = std::max(2, iters);
+        IVP_TRY(build_code(c->state_host->flags));
+        if (c->state_host->active != 0) return IVP_ERR_INTERNAL;
     }
     *iters_out = iters;
-    return launch(c, KC_GLUE, -1, 0.0, k_w18_apply, dim3(blocks_for(3 * nd)), 3 * nd, (const float*)c->w_dv, c->vel,
-                  (const SolverState*)nullptr);
+    return IVP_OK;
 }
 
 // One pass loop of PRJ (solve_PJ, prj.py:162-211; DF: solve_df's loop, prj.py:238-281) on the
@@ -2236,12 +2235,11 @@ int prj_loop(ivp_ctx* c, const ivp_prj_params* prm, double tol, int* passes, dou
     const int nd = c->nd;
     const dim3 np = pass_grid(nd);
     const double pb = pair_bytes<FM>(), pairs = (double)c->state_host->total_pairs;
-    hipLaunchKernelGGL(k_prj_state_init, dim3(1), dim3(1), 0, c->stream, c->state);
-    IVP_HIP(hipGetLastError());
     PrjArgs pa{rows_of(c), c->Ss, c->prj_v0, c->prj_lam, c->d4, c->cc, c->kk, c->rho0, c->rowtot, c->jd,
-               prm->omega, c->C, prm->df_num_threshold, c->partials, c->max_blocks, c->state};
+               prm->omega, c->C, prm->df_num_threshold, c->partials, c->max_blocks, c->state, nullptr};
     PrjFinArgs fa{c->partials, c->max_blocks, (int)np.x, c->state, tol, prm->max_iteration_opt,
-                  prm->use_fixed_iters ? 1 : 0, nd, DF ? nullptr : c->prj_hist, DF ? 0 : c->prj_hist_cap};
+                  prm->use_fixed_iters ? 1 : 0, nd, DF ? nullptr : c->prj_hist, DF ? 0 : c->prj_hist_cap, nullptr, nullptr,
+                  c->err_flag};
     // algorithmic bytes: the pair stream once, the gathered per-particle data once per row
     const double bH = stream_bytes<FM>(c, pairs) + (double)nd * (8 + 12 + 12 + 16);
     const double bT = stream_bytes<FM>(c, pairs) + (double)nd * (16 + 12 + 4 + 4 + 4 + 8 + 4 + 8 + (DF ? 4 : 0));
@@ -2250,22 +2248,29 @@ int prj_loop(ivp_ctx* c, const ivp_prj_params* prm, double tol, int* passes, dou
     const int total = prm->max_iteration_opt + 1;
     int issued = 0;
     int chunk = std::max(2, std::min(c->prj_guess, 128));
-    if (!DF) IVP_TRY(iter_mark(c, 0));
     for (;;) {
         const int todo = std::min(chunk, total - issued);
         if (todo <= 0) break;
+        if (!DF) {
+            IVP_TRY(marks_buffer(c, issued + todo));
+            pa.mark0 = issued == 0 ? c->marks : nullptr;
+            fa.marks = c->marks;
+        }
         for (int q = 0; q < todo; ++q) {
             const int tag = issued + q;
+            if (q == 1) pa.mark0 = nullptr;
+            fa.host = q == todo - 1 ? c->state_host : nullptr;
             IVP_TRY(launch(c, KC_PRJ_HEAD, tag, bH, k_prj_head<FM>, np, pa));
             IVP_TRY(launch(c, KC_PRJ_TAIL, tag, bT, k_prj_tail<FM, DF>, np, pa));
             hipLaunchKernelGGL(k_fin_prj, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
             IVP_HIP(hipGetLastError());
-            if (!DF) IVP_TRY(iter_mark(c, tag + 1));
         }
         issued += todo;
-        IVP_TRY(read_state(c));
+        IVP_HIP(hipStreamSynchronize(c->stream));
         (*chunks)++;
         const SolverState& s = *c->state_host;
+        // rows that the last build truncated: v, the kept multipliers and x are still as they were
+        if (build_code(s.flags) != IVP_OK) return build_code(s.flags);
         if (s.active == 0) break;
         // geometric extrapolation of the density error to the tolerance
         const int done = s.iter;   // passes completed
@@ -2291,7 +2296,7 @@ int prj_solve_body(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats
     auto t0 = std::chrono::steady_clock::now();
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_prj_init<false>, nb, nd, dt, (const float*)c->density,
                    (const float*)c->rho0, (const float*)c->vel, (const float4*)c->pos, (const int*)c->uid,
-                   (const float*)c->prj_prev, prm->warm_start ? 1 : 0, c->cc, c->prj_v0, c->prj_lam));
+                   (const float*)c->prj_prev, prm->warm_start ? 1 : 0, c->cc, c->prj_v0, c->prj_lam, c->state));
     int passes = 0;
     double err = 0.0;
     IVP_TRY((prj_loop<FM, false>(c, prm, prm->tol_opt, &passes, &err, &st.cg_launch_chunks)));
@@ -2299,9 +2304,7 @@ int prj_solve_body(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats
                    c->prj_prev));
     const int n_err = passes + 1;
     const int n_copy = std::min(std::min(n_err, c->prj_hist_cap), st.density_errors ? st.capacity : 0);
-    if (n_copy > 0)
-        IVP_HIP(hipMemcpyAsync(st.density_errors, c->prj_hist, sizeof(double) * (size_t)n_copy,
-                               hipMemcpyDeviceToHost, c->stream));
+    for (int k = 0; k < n_copy; ++k) st.density_errors[k] = c->prj_hist[k];
     st.n_density_errors = n_err;
     st.outer_iters = passes;
     const long long tp = c->state_host->total_pairs;
@@ -2337,7 +2340,7 @@ int prj_df_body(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* s
     auto t1 = std::chrono::steady_clock::now();
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_prj_init<true>, nb, nd, dt, (const float*)c->density,
                    (const float*)c->rho0, (const float*)c->vel, (const float4*)c->pos, (const int*)c->uid,
-                   (const float*)c->prj_df_prev, prm->warm_start ? 1 : 0, c->cc, c->prj_v0, c->prj_lam));
+                   (const float*)c->prj_df_prev, prm->warm_start ? 1 : 0, c->cc, c->prj_v0, c->prj_lam, c->state));
     int df_passes = 0;
     double df_err = 0.0;
     IVP_TRY((prj_loop<FM, true>(c, prm, prm->df_tol_opt, &df_passes, &df_err, &st.cg_launch_chunks)));
@@ -2388,24 +2391,29 @@ int st_jeske23(ivp_ctx* c, float sigma, float dt, ivp_cg_stats* out) {
     return IVP_OK;
 }
 
+void stats_zero(ivp_ip_stats* st) {
+    st->n_density_errors = 0;
+    st->n_pcg = 0;
+    st->outer_iters = 0;
+    st->final_density_error = 0.0;
+    st->pAp_bad = 0.0;
+    st->pcg_iter_bad = 0;
+    st->pairs_traversed = 0;
+    st->rows_traversed = 0;
+    st->cg_launch_chunks = 0;
+    st->solve_ms = 0.0;
+    st->df_outer_iters = 0;
+    st->df_ms = 0.0;
+    st->n_iter_costs = 0;
+}
+
 // IP.solve with its wall-clock cost (stats_total_cost_ms, ip.py:335, 403-404: the reference
 // synchronises before reading the clock, and so does this).
 int ip_solve(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* stats, bool defer) {
     if (!c->built) return IVP_ERR_STATE;
     if (!prm || !stats) return IVP_ERR_ARG;
     ivp_ip_stats& st = *stats;
-    st.n_density_errors = 0;
-    st.n_pcg = 0;
-    st.outer_iters = 0;
-    st.final_density_error = 0.0;
-    st.pAp_bad = 0.0;
-    st.pcg_iter_bad = 0;
-    st.pairs_traversed = 0;
-    st.rows_traversed = 0;
-    st.cg_launch_chunks = 0;
-    st.df_outer_iters = 0;
-    st.df_ms = 0.0;
-    st.n_iter_costs = 0;
+    stats_zero(stats);
     auto t0 = std::chrono::steady_clock::now();
     int rc;
     switch (c->row_fmt) {
@@ -2448,27 +2456,8 @@ int prj_solve(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* sta
     if (!c->built) return IVP_ERR_STATE;
     if (!prm || !stats) return IVP_ERR_ARG;
     if (prm->max_iteration_opt < 0 || prm->df_num_threshold < 0) return IVP_ERR_ARG;
-    ivp_ip_stats& st = *stats;
-    st.n_density_errors = 0;
-    st.n_pcg = 0;
-    st.outer_iters = 0;
-    st.final_density_error = 0.0;
-    st.pAp_bad = 0.0;
-    st.pcg_iter_bad = 0;
-    st.pairs_traversed = 0;
-    st.rows_traversed = 0;
-    st.cg_launch_chunks = 0;
-    st.solve_ms = 0.0;
-    st.df_outer_iters = 0;
-    st.df_ms = 0.0;
-    st.n_iter_costs = 0;
+    stats_zero(stats);
     IVP_TRY(prj_buffers(c, prm->max_iteration_opt + 1));
-    // a row that overflowed the neighbour capacity at the last build (the IP solve reads the
-    // same flag at its first synchronisation)
-    IVP_HIP(hipMemcpyAsync(c->err_host, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    IVP_HIP(hipStreamSynchronize(c->stream));
-    if (*c->err_host & 4) return IVP_ERR_INTERNAL;
-    if (*c->err_host & 1) return IVP_NEIGHBOR_OVERFLOW;
     const int fmt = c->row_fmt;
     if (part != PRJ_DF) {
         int rc = fmt == IVP_ROWS_F32   ? prj_solve_body<FmtF32>(c, dt, prm, stats)
