@@ -1572,7 +1572,10 @@ int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bo
     // placing (key, uid, cell members ~ 3 x 4, and every per-particle array read and written)
     const double per = 20 + (dynamic ? 2 * (16 + 12 + 4 + 4 + 4 + 4 + 4) + 4 : 2 * (16 + 4 + 4 + 4 + 4) + 4);
     const int chunks = (c->ncell + SCAN_CHUNK - 1) / SCAN_CHUNK;
-    int* bsum = chunks <= CELL_SCAN_CHUNKS ? c->cell_bsum : nullptr;
+    // Particles in the caller's order (the first sort after a load, and the statics') rarely share a
+    // chunk within a wave: counting the totals would cost an atomic each (1M rows: 0.1 ms), so those
+    // sorts scan in three launches.
+    int* bsum = dynamic && c->dyn_sorted && chunks <= CELL_SCAN_CHUNKS ? c->cell_bsum : nullptr;
     KeysArgs ka{count, c->pos + offset, c->grid, c->grids, c->sid ? c->sid + offset : nullptr, c->key, c->ccount, bsum,
                 // the dynamic population's sort starts a rebuild: its first pass clears the overflow flags
                 dynamic ? c->err_flag : nullptr, advect_args(c, adv_dt ? *adv_dt : 0.0f)};
@@ -1606,6 +1609,7 @@ int grid_sort_population(ivp_ctx* c, int offset, int count, int* start_table, bo
     if (dynamic) {
         swap_ptr(c->vel, c->vel_b);
         swap_ptr(c->divg, c->divg_b);
+        c->dyn_sorted = true;
     }
     return IVP_OK;
 }
@@ -1616,6 +1620,7 @@ int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m,
     if (n > 0 && (!x || !v || !m || !m_inv || !density0 || !is_dynamic || !material)) return IVP_ERR_ARG;
     c->loaded = false;
     c->built = false;
+    c->dyn_sorted = false;
     c->n = n;
     if (n == 0) {
         c->nd = c->ns = 0;

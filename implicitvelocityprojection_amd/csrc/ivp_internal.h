@@ -165,6 +165,7 @@ struct ivp_ctx {
     int nd_alloc_tiles = 0;
     bool loaded = false;
     bool built = false;
+    bool dyn_sorted = false;     // the dynamic particles have been sorted since they were loaded
     bool all_dyn_fluid = true;
     bool static_fluid = false;   // some static particle has the fluid material
     // neighbour-row format (IVP_ROWS_*): ids only, the operator passes evaluating gradW from
