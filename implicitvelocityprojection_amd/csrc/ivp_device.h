@@ -185,41 +185,85 @@ __device__ __forceinline__ int xcd_block(int b, int nblocks) {
     return start + idx;
 }
 
+// Wave reductions with the lane exchanges inside the vector unit: swap of the wave's halves and of
+// its odd and even 16-lane rows, rotations of a row by 8 and 4, quad permutes -- the lanes of an
+// xor tree with strides 32, 16, 8, 4, 2, 1.  (An exchange through ds_bpermute takes an LDS round
+// trip: a 64-bit sum paid twelve of them, one after another, at the end of every block.)
+// Called by whole waves.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+constexpr int DPP_ROR8 = 0x128, DPP_ROR4 = 0x124, DPP_QUAD_XOR2 = 0x4E, DPP_QUAD_XOR1 = 0xB1;
+
+// f(own, other) over the pairs of lanes that are O apart, on 32-bit words
+template <int O>
+__device__ __forceinline__ void lane_pair(uint32_t v, uint32_t& x, uint32_t& y) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    if constexpr (O == 32) {
+        const u32x2 s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        x = s.x; y = s.y;
+    } else if constexpr (O == 16) {
+        const u32x2 s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        x = s.x; y = s.y;
+    } else {
+        x = v;
+        y = O == 8 ? dpp<DPP_ROR8>(v) : O == 4 ? dpp<DPP_ROR4>(v) : O == 2 ? dpp<DPP_QUAD_XOR2>(v) : dpp<DPP_QUAD_XOR1>(v);
+    }
+}
+
+// One step of the xor tree at stride O on a value that is equal on lanes whose indices differ by
+// a larger stride only (the rotations need that): f is commutative.
+template <int O, class F>
+__device__ __forceinline__ double pair_step(double v, F&& f) {
+    const uint64_t w = __builtin_bit_cast(uint64_t, v);
+    uint32_t xl, yl, xh, yh;
+    lane_pair<O>((uint32_t)w, xl, yl);
+    lane_pair<O>((uint32_t)(w >> 32), xh, yh);
+    return f(__builtin_bit_cast(double, (uint64_t)xh << 32 | xl), __builtin_bit_cast(double, (uint64_t)yh << 32 | yl));
+}
+template <int O, class F>
+__device__ __forceinline__ int pair_step(int v, F&& f) {
+    uint32_t x, y;
+    lane_pair<O>((uint32_t)v, x, y);
+    return f((int)x, (int)y);
+}
+template <class T, class F>
+__device__ __forceinline__ T wave_fold(T v, F&& f) {
+    v = pair_step<32>(v, f);
+    v = pair_step<16>(v, f);
+    v = pair_step<8>(v, f);
+    v = pair_step<4>(v, f);
+    v = pair_step<2>(v, f);
+    return pair_step<1>(v, f);
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+    return wave_fold(v, [](double x, double y) { return x + y; });
 }
-
+__device__ __forceinline__ int wave_sum(int v) {
+    return wave_fold(v, [](int x, int y) { return x + y; });
+}
 __device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        int u = __shfl_xor(v, o, WAVE);
-        v = u < v ? u : v;
-    }
-    return v;
+    return wave_fold(v, [](int x, int y) { return x < y ? x : y; });
 }
-
 __device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        int u = __shfl_xor(v, o, WAVE);
-        v = u > v ? u : v;
-    }
-    return v;
+    return wave_fold(v, [](int x, int y) { return x > y ? x : y; });
 }
 
-// Sum of one double per thread over a 256-thread block, in a fixed order.  Result valid in
-// thread 0.
-__device__ __forceinline__ double block_sum(double v, double* lds4) {
-    v = wave_sum(v);
-    int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
-    if (lane == 0) lds4[w] = v;
+// Sums of NV doubles per thread over a 256-thread block, in a fixed order.  Results valid in
+// thread 0.  lds is not reused before a barrier of the caller's.
+template <int NV>
+__device__ __forceinline__ void block_sums(const double (&v)[NV], double (&s)[NV], double (&lds)[NV][WAVES_PER_BLOCK]) {
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const double x = wave_sum(v[q]);
+        if (lane == 0) lds[q][w] = x;
+    }
     __syncthreads();
-    double r = 0.0;
-    if (threadIdx.x == 0) r = (lds4[0] + lds4[1]) + (lds4[2] + lds4[3]);
-    __syncthreads();
-    return r;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) s[q] = threadIdx.x == 0 ? (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]) : 0.0;
 }
 
 }  // namespace ivp

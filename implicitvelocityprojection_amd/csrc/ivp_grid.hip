@@ -126,7 +126,7 @@ __global__ __launch_bounds__(BLOCK) void k_cell_starts(int n, int nb, const int*
     for (int k = threadIdx.x; k < (int)blockIdx.x; k += BLOCK) before += bsum[k];
 #pragma unroll
     for (int q = 0; q < SCAN_PER_THREAD; ++q) sum += v[q];
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
+    before = wave_sum(before);
     if ((threadIdx.x & (WAVE - 1)) == 0) psum[threadIdx.x >> 6] = before;
     int tot;
     int run = block_excl_scan(sum, &tot);   // (its barriers also publish psum)
@@ -1253,12 +1253,12 @@ __global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
     }
     if (threadIdx.x == 0) a.tile_len[tile] = tlp;
     // row 1 starts at zero: the window pass adds its tile's window size there
-    double v[2] = {valid && g == 0 ? (double)cnt : 0.0, 0.0};
-    __shared__ double lds[WAVES_PER_BLOCK];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const double s = block_sum(v[q], lds);
-        if (threadIdx.x == 0) a.partials[q * a.stride + tile] = s;
+    double v[1] = {valid && g == 0 ? (double)cnt : 0.0}, s[1];
+    __shared__ double lds[1][WAVES_PER_BLOCK];
+    block_sums<1>(v, s, lds);
+    if (threadIdx.x == 0) {
+        a.partials[tile] = s[0];
+        a.partials[a.stride + tile] = 0.0;
     }
 }
 

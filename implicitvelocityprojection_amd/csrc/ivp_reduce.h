@@ -11,12 +11,12 @@ namespace ivp {
 // so no device-scope fence (an L2 write-back on a multi-XCD part) is issued per block.
 template <int NV>
 __device__ __forceinline__ void block_partials(const double (&v)[NV], double* partials, int stride) {
-    __shared__ double lds[WAVES_PER_BLOCK];
+    __shared__ double lds[NV][WAVES_PER_BLOCK];
+    double s[NV];
+    block_sums<NV>(v, s, lds);
+    if (threadIdx.x == 0)
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = block_sum(v[q], lds);
-        if (threadIdx.x == 0) partials[q * stride + blockIdx.x] = s;
-    }
+        for (int q = 0; q < NV; ++q) partials[q * stride + blockIdx.x] = s[q];
 }
 
 enum FinOp {
@@ -235,15 +235,21 @@ inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0,
 template <int NV>
 __device__ __forceinline__ void block_partials_seg(const double (&v)[NV], int seg, bool two, double* partials,
                                                    int stride, int blk) {
-    __shared__ double lds[WAVES_PER_BLOCK];
+    __shared__ double lds[2][NV][WAVES_PER_BLOCK];
+    double x[NV], s[NV];
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s0 = block_sum(seg == 0 ? v[q] : 0.0, lds);
-        if (threadIdx.x == 0) partials[(2 * q) * stride + blk] = s0;
-        if (two) {
-            double s1 = block_sum(seg == 1 ? v[q] : 0.0, lds);
-            if (threadIdx.x == 0) partials[(2 * q + 1) * stride + blk] = s1;
-        }
+    for (int q = 0; q < NV; ++q) x[q] = seg == 0 ? v[q] : 0.0;
+    block_sums<NV>(x, s, lds[0]);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) partials[(2 * q) * stride + blk] = s[q];
+    if (two) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) x[q] = seg == 1 ? v[q] : 0.0;
+        block_sums<NV>(x, s, lds[1]);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) partials[(2 * q + 1) * stride + blk] = s[q];
     }
 }
 

@@ -146,19 +146,21 @@ static_assert(PASS_LANES <= MAX_PASS_LANES, "partials are sized for MAX_PASS_LAN
 
 inline dim3 pass_grid(int nd) { return dim3(blocks_for(nd * PASS_LANES)); }
 
+// Sum over the G lanes of a row (strides 1, then 2), by quad permutes; the lanes of a row branch together
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o, WAVE);
+    static_assert(G == 1 || G == 2 || G == 4, "a row's lanes are within one quad");
+    if constexpr (G >= 2) v += __builtin_bit_cast(float, dpp<DPP_QUAD_XOR1>(__builtin_bit_cast(uint32_t, v)));
+    if constexpr (G >= 4) v += __builtin_bit_cast(float, dpp<DPP_QUAD_XOR2>(__builtin_bit_cast(uint32_t, v)));
     return v;
 }
 
 template <int G>
 __device__ __forceinline__ bool group_any(bool b) {
-    int v = b ? 1 : 0;
-#pragma unroll
-    for (int o = 1; o < G; o <<= 1) v |= __shfl_xor(v, o, WAVE);
-    return v != 0;
+    uint32_t v = b ? 1u : 0u;
+    if constexpr (G >= 2) v |= dpp<DPP_QUAD_XOR1>(v);
+    if constexpr (G >= 4) v |= dpp<DPP_QUAD_XOR2>(v);
+    return v != 0u;
 }
 
 // Row and lane of this thread in a pair pass with G lanes per row, over row block blk
@@ -1739,7 +1741,7 @@ __global__ __launch_bounds__(BLOCK) void k_scene_init(int S, SceneState* __restr
 // End of a replay (one block): scenes whose displacement was just updated start their next
 // outer iteration (ip.py:389-391); *active = scenes not done.
 __global__ __launch_bounds__(BLOCK) void k_scene_advance(int S, SceneState* __restrict__ ss, int* __restrict__ active) {
-    __shared__ double lds[WAVES_PER_BLOCK];
+    __shared__ double lds[1][WAVES_PER_BLOCK];
     int cnt = 0;
     for (int s = threadIdx.x; s < S; s += BLOCK) {
         SceneState& q = ss[s];
@@ -1749,8 +1751,9 @@ __global__ __launch_bounds__(BLOCK) void k_scene_advance(int S, SceneState* __re
         }
         cnt += q.phase != PH_DONE ? 1 : 0;
     }
-    double t = block_sum((double)cnt, lds);
-    if (threadIdx.x == 0) *active = (int)t;
+    double v[1] = {(double)cnt}, t[1];
+    block_sums<1>(v, t, lds);
+    if (threadIdx.x == 0) *active = (int)t[0];
 }
 
 // One replay of the batched outer iteration on stream `st`: constraint pass for scenes starting
