@@ -69,7 +69,7 @@ void free_all(ivp_ctx* c) {
     dfree(c->rho0); dfree(c->rho0_b); dfree(c->mat); dfree(c->mat_b); dfree(c->uid); dfree(c->uid_b);
     dfree(c->inv); dfree(c->density); dfree(c->kk); dfree(c->Ss); dfree(c->divg); dfree(c->divg_b);
     dfree(c->rowcnt); dfree(c->rowtot); dfree(c->nb); dfree(c->tile_len); dfree(c->dstart); dfree(c->sstart);
-    dfree(c->ccount); dfree(c->key); dfree(c->tmp_src); dfree(c->order); dfree(c->scan_bsum); dfree(c->cell_bsum);
+    dfree(c->ccount); dfree(c->key); dfree(c->tmp_src); dfree(c->order); dfree(c->scan_bsum);
     dfree(c->d4); dfree(c->q4); dfree(c->b); dfree(c->sol); dfree(c->r); dfree(c->Ap); dfree(c->p4); dfree(c->y2);
     dfree(c->cc); dfree(c->sfac); dfree(c->jd); dfree(c->xs4); dfree(c->nbact);
     dfree(c->w_pinv); dfree(c->w_p4); dfree(c->w_v4); dfree(c->w_dv); dfree(c->w_r); dfree(c->w_z);
@@ -92,7 +92,8 @@ void free_all(ivp_ctx* c) {
     c->prof_pending.clear();
     for (auto e : c->prof_free) (void)hipEventDestroy(e);
     c->prof_free.clear();
-    hfree(c->marks);
+    if (c->marks_cap > MARKS) hfree(c->marks);
+    c->marks = nullptr;
     c->marks_cap = 0;
     if (c->ip_end_ev) (void)hipEventDestroy(c->ip_end_ev);
     c->ip_end_ev = nullptr;
@@ -115,7 +116,8 @@ int alloc_all(ivp_ctx* c) {
     A(key, cap); A(tmp_src, cap + 1); A(order, cap);
     size_t scan_n = std::max((size_t)c->ncell, cap) + 1;
     c->nscan_blocks = (int)((scan_n + 2047) / 2048) + 2;
-    A(scan_bsum, (size_t)c->nscan_blocks + 1); A(cell_bsum, (size_t)c->nscan_blocks);
+    A(scan_bsum, 2 * (size_t)c->nscan_blocks + 1);
+    c->cell_bsum = c->scan_bsum + c->nscan_blocks + 1;
     A(d4, cap); A(q4, cap); A(b, 3 * cap); A(sol, 3 * cap); A(r, 3 * cap); A(Ap, 3 * cap); A(p4, cap); A(y2, cap);
     A(cc, cap); A(sfac, cap); A(jd, cap); A(xs4, cap); A(nbact, cap);
     A(w_pinv, 9 * cap); A(w_p4, cap); A(w_v4, cap); A(w_dv, 3 * cap); A(w_r, 3 * cap); A(w_z, 3 * cap);
@@ -124,11 +126,15 @@ int alloc_all(ivp_ctx* c) {
     A(partials, 4 * (size_t)c->max_blocks);
     A(state, 1); A(err_flag, 1); A(speed_max, 1);
 #undef A
-    IVP_HIP(hipHostMalloc((void**)&c->state_host, 2 * sizeof(SolverState), hipHostMallocDefault));
+    // the two state copies, then the first MARKS pass times: one pinned allocation
+    IVP_HIP(hipHostMalloc((void**)&c->state_host, 2 * sizeof(SolverState) + sizeof(unsigned long long) * MARKS,
+                          hipHostMallocDefault));
+    c->marks = reinterpret_cast<unsigned long long*>(c->state_host + 2);
+    c->marks_cap = MARKS;
     IVP_HIP(hipHostMalloc((void**)&c->err_host, sizeof(int), hipHostMallocDefault));
     IVP_HIP(hipHostMalloc((void**)&c->count_host, 4 * sizeof(int), hipHostMallocDefault));
 
-    memset(c->state_host, 0, 2 * sizeof(SolverState));
+    memset(c->state_host, 0, 2 * sizeof(SolverState) + sizeof(unsigned long long) * MARKS);
     int khz = 0;
     IVP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device));
     c->ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
@@ -259,14 +265,15 @@ int scenes_set(ivp_ctx* c, int S, const ivp_scene* sc) {
     c->loaded = false;
     c->built = false;
     const size_t cap = (size_t)c->cap;
-    dfree(c->dstart); dfree(c->sstart); dfree(c->ccount); dfree(c->scan_bsum); dfree(c->cell_bsum);
+    dfree(c->dstart); dfree(c->sstart); dfree(c->ccount); dfree(c->scan_bsum);
     c->ncell = (int)base;
     size_t scan_n = std::max((size_t)c->ncell, cap) + 1;
     c->nscan_blocks = (int)((scan_n + 2047) / 2048) + 2;
     int rc = IVP_OK;
 #define A(p, n) if ((rc = dalloc(&c->p, (n))) != IVP_OK) return rc
     A(dstart, (size_t)c->ncell + 1); A(sstart, (size_t)c->ncell + 1); A(ccount, (size_t)c->ncell);
-    A(scan_bsum, (size_t)c->nscan_blocks + 1); A(cell_bsum, (size_t)c->nscan_blocks);
+    A(scan_bsum, 2 * (size_t)c->nscan_blocks + 1);
+    c->cell_bsum = c->scan_bsum + c->nscan_blocks + 1;
     A(grids, (size_t)S); A(sid, cap); A(sdomain, 3 * (size_t)S); A(ss, (size_t)S); A(sprm, 1);
     A(shist_err, (size_t)S * SCENE_HIST); A(shist_pcg, (size_t)S * SCENE_HIST);
     A(spartials, 8 * (size_t)c->max_blocks); A(sactive, 1);
@@ -341,13 +348,13 @@ void prof_set_bytes(ivp_ctx* c, int epoch, int kclass, double bytes) {
 
 int marks_buffer(ivp_ctx* c, int n) {
     if (n + 2 <= c->marks_cap) return IVP_OK;
-    const int cap = std::max(256, 2 * (n + 2));
+    const int cap = 2 * (n + 2);   // > MARKS
     unsigned long long* m = nullptr;
     IVP_HIP(hipStreamSynchronize(c->stream));   // the old marks are complete
     IVP_HIP(hipHostMalloc((void**)&m, sizeof(unsigned long long) * (size_t)cap, hipHostMallocDefault));
     memset(m, 0, sizeof(unsigned long long) * (size_t)cap);
     if (c->marks) memcpy(m, c->marks, sizeof(unsigned long long) * (size_t)c->marks_cap);
-    hfree(c->marks);
+    if (c->marks_cap > MARKS) hfree(c->marks);   // (the first MARKS are part of the state's allocation)
     c->marks = m;
     c->marks_cap = cap;
     return IVP_OK;

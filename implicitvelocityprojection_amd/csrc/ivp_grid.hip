@@ -451,6 +451,11 @@ struct BuildArgs {
     int* err_flag;
     double* partials;
     int stride;
+    // tile windows (k_eval4 with PPT > 0)
+    int win_cap;   // largest window kept, <= WIN_MAX
+    uint32_t* loc;
+    int* win_ids;
+    int* win_n;
 };
 
 // One thread per dynamic row, one wave per 64-row tile, two phases.
@@ -1096,6 +1101,78 @@ __device__ __forceinline__ void build_eval(const BuildArgs& a, int i, int lane, 
     if (lane == 0) a.tile_len[tile] = tlp;
 }
 
+// LDS of the window search: the bitmap and the marks before each of its words
+struct WinBitmap {
+    uint32_t bm[WIN_SPAN_WORDS];
+    uint16_t pre[WIN_SPAN_WORDS];
+};
+
+// Tile window of a 64-row tile by its 256 threads.  The window is the ascending list of the distinct
+// ids in the walked slots [0, tile_len) of the tile's valid rows (padding slots name the row
+// itself); v / on are the thread's word pairs of the tile, ix their ids' places in that list, 16 bits
+// each.  The ids are marked in an LDS bitmap over [lo, hi] of the tile's ids, and an id's place is
+// the number of marks below it.  Returns the list's length, or -1 for a tile whose range exceeds
+// WIN_SPAN_WORDS words or whose window exceeds the cap (at most WIN_MAX ids).  The result is
+// block-uniform; every thread of the block calls it.
+template <int PPT>
+__device__ __forceinline__ int tile_window(const uint32_t (&vx)[PPT], const uint32_t (&vy)[PPT], const bool (&on)[PPT],
+                                           int cap, WinBitmap& s, uint32_t (&ix)[PPT]) {
+    __shared__ int red[2 * WAVES_PER_BLOCK];
+    int lo = 0x7fffffff, hi = -1;
+#pragma unroll
+    for (int k = 0; k < PPT; ++k)
+        if (on[k]) {
+            lo = min(lo, (int)min(vx[k], vy[k]));
+            hi = max(hi, (int)max(vx[k], vy[k]));
+        }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        red[w] = lo;
+        red[WAVES_PER_BLOCK + w] = hi;
+    }
+    __syncthreads();
+    lo = min(min(red[0], red[1]), min(red[2], red[3]));
+    hi = max(max(red[4], red[5]), max(red[6], red[7]));
+    if (hi < 0) return 0;   // no walked slot
+    const int words = ((hi - lo) >> 5) + 1;
+    if (words > WIN_SPAN_WORDS) return -1;
+    for (int k = threadIdx.x; k < words; k += BLOCK) s.bm[k] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PPT; ++k)
+        if (on[k]) {
+            const uint32_t p0 = vx[k] - (uint32_t)lo, p1 = vy[k] - (uint32_t)lo;
+            // an id repeats in many rows of a tile, and atomics on one LDS word serialise: mark
+            // only what is not yet marked
+            const uint32_t m0 = s.bm[p0 >> 5], m1 = s.bm[p1 >> 5];
+            if (!(m0 & (1u << (p0 & 31)))) atomicOr(&s.bm[p0 >> 5], 1u << (p0 & 31));
+            if (!(m1 & (1u << (p1 & 31)))) atomicOr(&s.bm[p1 >> 5], 1u << (p1 & 31));
+        }
+    __syncthreads();
+    // thread k counts the marks of words [w0, w1); exclusive scan over the block
+    const int per = (words + BLOCK - 1) / BLOCK;
+    const int w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
+    int cnt = 0;
+    for (int k = w0; k < w1; ++k) cnt += __popc(s.bm[k]);
+    int total;
+    int off = block_excl_scan(cnt, &total);
+    if (total > cap) return -1;
+    for (int k = w0; k < w1; ++k) {
+        s.pre[k] = (uint16_t)off;
+        off += __popc(s.bm[k]);
+    }
+    __syncthreads();
+    auto index = [&](uint32_t j) {
+        const uint32_t p = j - (uint32_t)lo;
+        return (uint32_t)s.pre[p >> 5] + (uint32_t)__popc(s.bm[p >> 5] & ((1u << (p & 31)) - 1u));
+    };
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) ix[k] = on[k] ? index(vx[k]) | (index(vy[k]) << 16) : 0u;
+    return total;
+}
+
 // Four lanes of a row, one term each: acc + t0 + t1 + t2 + t3 in that order on every lane (the
 // one-thread accumulation order; adding an unused slot's 0 changes no bit).  The quad broadcast is
 // a modifier of the add.
@@ -1120,14 +1197,20 @@ __device__ __forceinline__ void quad_sub(float& acc, float t) {
 // g + 4 of every 8-slot block (one 8-byte id load), forms their terms with the expressions of
 // build_eval, and the row's sums take the four lanes' terms in slot order, so rho, Aii, S and k are
 // bitwise those of the one-thread pass.  A block is one 64-row tile; block partials are per tile.
-// The neighbours of block b + 1 and the ids of block b + 2 are in flight while block b is summed.
+// With PPT > 0 (one scene, rows of at most 8 PPT slots) the block also finds its tile's window
+// (tile_window): the thread's ids, loaded at once, are the word pairs that the search needs, the
+// window's (x, m) and 1/m go to the LDS, where the pairs read them, and the pass writes the list and
+// the slots' indices.  As two passes the ids were read twice and every pair gathered 20 B from
+// memory: us per build at 1M rows 102 + 63 apart, 138 together; a whole 4k-particle rebuild 67 / 59.
+// With PPT = 0 the neighbours of block b + 1 and the ids of block b + 2 are in flight while block b
+// is summed.
 // Bound by vector instruction issue from about 250k rows (the correctly rounded root, reciprocal
 // and quotients; 109 instructions per 64 slots, 20 of them the ordered adds), by the chain of load
 // rounds below, where one thread per row leaves most SIMDs idle: us per build with one thread per
 // row and with four lanes, ids-only rows: 8k 20.5 / 10, 102k 24 / 18, 262k 34 / 33, 1M 104 / 94;
 // float16 rows 1M 235 / 190.
-template <int FMT>
-__global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
+template <int FMT, int PPT>
+__global__ __launch_bounds__(BLOCK, 8) void k_eval4(BuildArgs a) {
     static_assert(rec_words<FMT>() == 64u, "four lanes per row read the paired ids-only layout");
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -1146,7 +1229,7 @@ __global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
     const float h = a.h;
     const size_t w_row = (size_t)tile * (size_t)a.Cs * 64u + 8u * (uint32_t)r;
     uint32_t* row = a.nb + w_row;
-    const int wl = wave_max(cnt), ws = wave_max(cs);
+    const int wl = __builtin_amdgcn_readfirstlane(wave_max(cnt)), ws = __builtin_amdgcn_readfirstlane(wave_max(cs));
     if ((threadIdx.x & (WAVE - 1)) == 0) wmax[threadIdx.x >> 6] = wl;
     float rho = 0.0f, aii = 0.0f, jx = 0.0f, jy = 0.0f, jz = 0.0f, sx = 0.0f, sy = 0.0f, sz = 0.0f;
     rho = rho + pi.w * cubic_kernel(0.0f, h, a.kc);
@@ -1187,20 +1270,91 @@ __global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
     const u32x2* ids2 = reinterpret_cast<const u32x2*>(row + 2 * g);
     const int nblk = (wl + 7) >> 3;   // <= Cs / 8: wl <= C
     const u32x2 none = {(uint32_t)self, (uint32_t)self};
-    u32x2 id1 = nblk > 0 && valid ? ids2[0] : none;
-    Nb c0 = fetch(id1.x, g < cnt), c1 = fetch(id1.y, g + 4 < cnt);
-    id1 = nblk > 1 && valid ? ids2[256] : none;
-    for (int b = 0; b < nblk; ++b) {
-        const int k = 8 * b + g;
-        const Nb n0 = fetch(id1.x, k + 8 < cnt), n1 = fetch(id1.y, k + 12 < cnt);
-        id1 = b + 2 < nblk && valid ? ids2[(b + 2) * 256] : none;
-        uint32_t hq[4] = {0u, 0u, 0u, 0u};
-        slots(c0, k < cnt, hq[0], hq[1]);
-        slots(c1, k + 4 < cnt, hq[2], hq[3]);
+    auto store_h = [&](int b, uint32_t (&hq)[4]) {
         if (FMT == IVP_ROWS_F16 && valid)
             *reinterpret_cast<u32x4*>(a.g16 + 2 * (w_row + 2 * (size_t)g + 512u * (uint32_t)b)) = u32x4{hq[0], hq[1], hq[2], hq[3]};
-        c0 = n0;
-        c1 = n1;
+    };
+    int nwin = -1;
+    int tl = 0, tlp = 0;   // the tile's longest row, and that rounded up to ROW_PAD (<= Cs)
+    if constexpr (PPT > 0) {
+        // the search's bitmap, then in its place the window's records and list
+        union Lds {
+            WinBitmap s;
+            struct {
+                float4 x[WIN_MAX];
+                float m[WIN_MAX];
+                int id[WIN_MAX];
+            } w;
+        };
+        __shared__ Lds lds_w;
+        uint32_t vx[PPT], vy[PPT], ix[PPT];
+        bool on[PPT];
+#pragma unroll
+        for (int b = 0; b < PPT; ++b) {
+            const u32x2 v = b < nblk && valid ? ids2[b * 256] : none;
+            vx[b] = v.x;
+            vy[b] = v.y;
+        }
+        __syncthreads();   // wmax
+        tl = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+        tlp = (tl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;
+        const uint32_t last = (uint32_t)a.nd - 1u;
+#pragma unroll
+        for (int b = 0; b < PPT; ++b) {
+            on[b] = valid && 8 * b < tlp;
+            vx[b] = 8 * b + g < cnt ? vx[b] : (uint32_t)self;
+            vy[b] = 8 * b + g + 4 < cnt ? vy[b] : (uint32_t)self;
+            top = max(top, max(vx[b], vy[b]));
+            vx[b] = min(vx[b], last);
+            vy[b] = min(vy[b], last);
+        }
+        nwin = tile_window<PPT>(vx, vy, on, a.win_cap, lds_w.s, ix);
+        if (threadIdx.x == 0) a.win_n[tile] = nwin;
+        if (nwin >= 0) {
+            __syncthreads();   // the bitmap has been read
+            uint32_t* l32 = a.loc + (size_t)tile * (size_t)a.Cs * (WAVE / 2) + threadIdx.x;
+#pragma unroll
+            for (int b = 0; b < PPT; ++b)
+                if (on[b]) {
+                    lds_w.w.id[ix[b] & 0xffffu] = (int)vx[b];   // (slots of one id write the same word)
+                    lds_w.w.id[ix[b] >> 16] = (int)vy[b];
+                    l32[b * 256] = ix[b];
+                }
+            __syncthreads();
+            for (int k = threadIdx.x; k < nwin; k += BLOCK) {
+                const int j = lds_w.w.id[k];
+                a.win_ids[(size_t)tile * WIN_MAX + k] = j;
+                lds_w.w.x[k] = a.pos[j];
+                lds_w.w.m[k] = a.minv[j];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < PPT; ++b) {
+                if (8 * b >= wl) break;
+                const int k = 8 * b + g;
+                uint32_t hq[4] = {0u, 0u, 0u, 0u};
+                const uint32_t i0 = ix[b] & 0xffffu, i1 = ix[b] >> 16;
+                slots(Nb{lds_w.w.x[i0], lds_w.w.m[i0]}, k < cnt, hq[0], hq[1]);
+                if (8 * b + 4 < wl) slots(Nb{lds_w.w.x[i1], lds_w.w.m[i1]}, k + 4 < cnt, hq[2], hq[3]);
+                store_h(b, hq);
+            }
+        }
+    }
+    if (nwin < 0) {
+        u32x2 id1 = nblk > 0 && valid ? ids2[0] : none;
+        Nb c0 = fetch(id1.x, g < cnt), c1 = fetch(id1.y, g + 4 < cnt);
+        id1 = nblk > 1 && valid ? ids2[256] : none;
+        for (int b = 0; b < nblk; ++b) {
+            const int k = 8 * b + g;
+            const Nb n0 = fetch(id1.x, k + 8 < cnt), n1 = fetch(id1.y, k + 12 < cnt);
+            id1 = b + 2 < nblk && valid ? ids2[(b + 2) * 256] : none;
+            uint32_t hq[4] = {0u, 0u, 0u, 0u};
+            slots(c0, k < cnt, hq[0], hq[1]);
+            if (8 * b + 4 < wl) slots(c1, k + 4 < cnt, hq[2], hq[3]);
+            store_h(b, hq);
+            c0 = n0;
+            c1 = n1;
+        }
     }
     if (cnt == 0) {
         rho = rho_self;
@@ -1226,9 +1380,11 @@ __global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
         quad_add(sz, Jz);
     }
     if (bad) atomicOr(a.err_flag, 4);
-    __syncthreads();
-    const int tl = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-    const int tlp = (tl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;   // <= Cs
+    if constexpr (PPT == 0) {
+        __syncthreads();
+        tl = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+        tlp = (tl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;
+    }
     // pad only after the static ids have been consumed (the padded range can reach into them; the
     // row's four lanes are in one wave)
     if (valid) {
@@ -1252,13 +1408,13 @@ __global__ __launch_bounds__(BLOCK) void k_eval4(BuildArgs a) {
         }
     }
     if (threadIdx.x == 0) a.tile_len[tile] = tlp;
-    // row 1 starts at zero: the window pass adds its tile's window size there
+    // row 1: the tile's window size (a window pass of its own adds it)
     double v[1] = {valid && g == 0 ? (double)cnt : 0.0}, s[1];
     __shared__ double lds[1][WAVES_PER_BLOCK];
     block_sums<1>(v, s, lds);
     if (threadIdx.x == 0) {
         a.partials[tile] = s[0];
-        a.partials[a.stride + tile] = 0.0;
+        a.partials[a.stride + tile] = nwin > 0 ? (double)nwin : 0.0;
     }
 }
 
@@ -1275,96 +1431,33 @@ struct WinArgs {
     int tiles_per_block;   // of the pass that wrote those partials
 };
 
-// Tile windows of ids-only rows, one block per 64-row tile.  The window is the ascending list of
-// the distinct ids in the walked slots [0, tile_len) of the tile's valid rows (padding slots name
-// the row itself); each such slot gets the index of its id in that list, 16 bits at the slot's id
-// word (the 8-byte word pair of slots g, g + 4 becomes one 32-bit word).  The ids are marked in
-// an LDS bitmap over [lo, hi] of the tile's ids, and an id's index is the number of marks below
-// it; every slot then writes its id at its index into the list.  A tile whose range exceeds
-// WIN_SPAN_WORDS words, or whose window exceeds the cap (at most WIN_MAX ids), gets win_n = -1
-// and no indices.  Each thread keeps its PPT word pairs of the tile in registers from one
-// coalesced load.  Measured on the 1M dam break after 20 steps: 69 us per build (107 us with an
-// atomic for every slot; a bit loop writing the list, thread-contiguous pairs, per-word merged
-// marks or the list staged in LDS were no faster).
+// Tile windows in a pass of their own (rows of more than 64 slots, and rows that the one-lane build
+// wrote), one block per 64-row tile; each walked slot's index goes 16 bits wide to the slot's id
+// word (the 8-byte word pair of slots g, g + 4 becomes one 32-bit word).  Each thread keeps its PPT
+// word pairs of the tile in registers from one coalesced load.
 template <int PPT>
 __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    __shared__ uint32_t bm[WIN_SPAN_WORDS];
-    __shared__ uint16_t pre[WIN_SPAN_WORDS];
-    __shared__ int red[2 * WAVES_PER_BLOCK];
+    __shared__ WinBitmap s;
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int nrow = min(WAVE, a.nd - t * WAVE);
     const int npair = a.tile_len[t] * (WAVE / 2);
     const size_t base = (size_t)t * (size_t)a.Cs * WAVE;
     const u32x2* ids2 = reinterpret_cast<const u32x2*>(a.nb + base);
     // word pair q of a tile: block q >> 8, row (q >> 2) & 63; thread pairs q = thread + BLOCK k
-    u32x2 v[PPT];
+    uint32_t vx[PPT], vy[PPT], ix[PPT];
     bool on[PPT];
-    int lo = 0x7fffffff, hi = -1;
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
         const int q = (int)threadIdx.x + BLOCK * k;
         on[k] = q < npair && ((q >> 2) & (WAVE - 1)) < nrow;
-        v[k] = on[k] ? ids2[q] : u32x2{0u, 0u};
+        const u32x2 v = on[k] ? ids2[q] : u32x2{0u, 0u};
+        vx[k] = v.x;
+        vy[k] = v.y;
     }
-#pragma unroll
-    for (int k = 0; k < PPT; ++k)
-        if (on[k]) {
-            lo = min(lo, (int)min(v[k].x, v[k].y));
-            hi = max(hi, (int)max(v[k].x, v[k].y));
-        }
-    lo = wave_min(lo);
-    hi = wave_max(hi);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & (WAVE - 1)) == 0) {
-        red[w] = lo;
-        red[WAVES_PER_BLOCK + w] = hi;
-    }
-    __syncthreads();
-    lo = min(min(red[0], red[1]), min(red[2], red[3]));
-    hi = max(max(red[4], red[5]), max(red[6], red[7]));
-    if (hi < 0) {   // no walked slot
-        if (threadIdx.x == 0) a.win_n[t] = 0;
-        return;
-    }
-    const int words = ((hi - lo) >> 5) + 1;
-    if (words > WIN_SPAN_WORDS) {
-        if (threadIdx.x == 0) a.win_n[t] = -1;
-        return;
-    }
-    for (int k = threadIdx.x; k < words; k += BLOCK) bm[k] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < PPT; ++k)
-        if (on[k]) {
-            const uint32_t p0 = v[k].x - (uint32_t)lo, p1 = v[k].y - (uint32_t)lo;
-            // an id repeats in many rows of a tile, and atomics on one LDS word serialise: mark
-            // only what is not yet marked
-            const uint32_t m0 = bm[p0 >> 5], m1 = bm[p1 >> 5];
-            if (!(m0 & (1u << (p0 & 31)))) atomicOr(&bm[p0 >> 5], 1u << (p0 & 31));
-            if (!(m1 & (1u << (p1 & 31)))) atomicOr(&bm[p1 >> 5], 1u << (p1 & 31));
-        }
-    __syncthreads();
-    // thread k counts the marks of words [w0, w1); exclusive scan over the block
-    const int per = (words + BLOCK - 1) / BLOCK;
-    const int w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
-    int cnt = 0;
-    for (int k = w0; k < w1; ++k) cnt += __popc(bm[k]);
-    int total;
-    int off = block_excl_scan(cnt, &total);
-    if (total > a.cap) {
-        if (threadIdx.x == 0) a.win_n[t] = -1;
-        return;
-    }
-    for (int k = w0; k < w1; ++k) {
-        pre[k] = (uint16_t)off;
-        off += __popc(bm[k]);
-    }
-    __syncthreads();
-    auto index = [&](uint32_t j) {
-        const uint32_t p = j - (uint32_t)lo;
-        return (uint32_t)pre[p >> 5] + (uint32_t)__popc(bm[p >> 5] & ((1u << (p & 31)) - 1u));
-    };
+    const int total = tile_window<PPT>(vx, vy, on, a.cap, s, ix);
+    if (threadIdx.x == 0) a.win_n[t] = total;
+    if (total <= 0) return;
     // every window id is named by some walked slot: each slot writes its id at its index (slots
     // of one id write the same word)
     int* wid = a.win_ids + (size_t)t * WIN_MAX;
@@ -1372,17 +1465,13 @@ __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
 #pragma unroll
     for (int k = 0; k < PPT; ++k)
         if (on[k]) {
-            const uint32_t i0 = index(v[k].x), i1 = index(v[k].y);
-            wid[i0] = (int)v[k].x;
-            wid[i1] = (int)v[k].y;
-            l32[threadIdx.x + BLOCK * k] = i0 | (i1 << 16);
+            wid[ix[k] & 0xffffu] = (int)vx[k];
+            wid[ix[k] >> 16] = (int)vy[k];
+            l32[threadIdx.x + BLOCK * k] = ix[k];
         }
-    if (threadIdx.x == 0) {
-        a.win_n[t] = total;
-        // the build's partial row 1 (zeroed by the build's blocks; the sums are integers, exact in
-        // any order)
-        atomicAdd(&a.partials[a.stride + t / a.tiles_per_block], (double)total);
-    }
+    // the build's partial row 1 (zeroed by the build's blocks; the sums are integers, exact in
+    // any order)
+    if (threadIdx.x == 0) atomicAdd(&a.partials[a.stride + t / a.tiles_per_block], (double)total);
 }
 
 struct ExportArgs {
@@ -1754,6 +1843,13 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         IVP_HIP(hipMemsetAsync(c->dstart, 0, sizeof(int) * (size_t)(c->ncell + 1), c->stream));
         IVP_HIP(hipMemsetAsync(c->err_flag, 0, sizeof(int), c->stream));   // (else cleared by the sort)
     }
+    // tile windows, where a tile's walked slots fit the search (Cs * 32 word pairs, PPT per thread); not
+    // for independent scenes: their passes run late in a batched solve on few active blocks, and
+    // windows over every scene's rows cost more than they saved (4.28 -> 4.48 ms per step on 256
+    // columns)
+    const int ppt = (c->Cs * (WAVE / 2) + BLOCK - 1) / BLOCK;
+    const bool windows = c->nd > 0 && c->windows && c->rec_words == 64 && c->S == 0 && ppt <= 32;
+    bool fused = false;   // the exact pass finds the windows
     int tiles_per_block = WAVES_PER_BLOCK;   // of the pass that writes the build's partials
     if (c->nd > 0) {
         // float h2_lo <= h^2 (1 - 2^-20) and h2_hi >= h^2 (1 + 2^-20): the predicate bounds of scan_ids
@@ -1762,7 +1858,8 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         float h2_hi = std::nextafter((float)(hh * (1.0 + 1.0 / 1048576.0)), 1.0f);
         BuildArgs ba{c->nd, c->ns, c->C, c->Cs, c->h, h2_lo, h2_hi, (float)hh, c->kcubic, c->kspiky, 1.0f / c->h, 1.0f / c->gscale, c->grid,
                      c->grids, c->sid, c->pos, c->minv, c->dstart, c->sstart, c->nb, c->g16, c->tile_len,
-                     c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag, c->partials, c->max_blocks};
+                     c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag, c->partials, c->max_blocks,
+                     c->win_cap, c->loc, c->win_ids, c->win_n};
         // bytes (pair count of the previous build): the pair records written, the ids read back
         // once, x and m of every particle once, the per-row outputs (rho, k, S, counts)
         double pairs = (double)c->state_host->total_pairs;
@@ -1794,20 +1891,14 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
             } else {
                 tiles_per_block = 1;
                 const dim3 tiles((c->nd + WAVE - 1) / WAVE);
-                if (c->row_fmt == IVP_ROWS_F16)
-                    IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval4<IVP_ROWS_F16>, tiles, ba));
-                else
-                    IVP_TRY(launch(c, KC_BUILD, -1, bytes, k_eval4<IVP_ROWS_IDS>, tiles, ba));
+                fused = windows && ppt <= 8;
+                auto k = c->row_fmt == IVP_ROWS_F16 ? (fused ? k_eval4<IVP_ROWS_F16, 8> : k_eval4<IVP_ROWS_F16, 0>)
+                                                    : (fused ? k_eval4<IVP_ROWS_IDS, 8> : k_eval4<IVP_ROWS_IDS, 0>);
+                IVP_TRY(launch(c, KC_BUILD, -1, bytes, k, tiles, ba));
             }
         }
     }
-    c->win_built = false;
-    // a tile walks at most Cs slots: Cs * 32 word pairs, PPT per thread
-    const int ppt = (c->Cs * (WAVE / 2) + BLOCK - 1) / BLOCK;
-    // (not for independent scenes: their passes run late in a batched solve on few active blocks,
-    // and the window pass over every scene's rows cost more than it saved -- 4.28 -> 4.48 ms per
-    // step on 256 columns)
-    if (c->nd > 0 && c->windows && c->rec_words == 64 && c->S == 0 && ppt <= 32) {
+    if (windows && !fused) {
         WinArgs wa{c->nd, c->Cs, c->win_cap, c->nb, c->tile_len, c->loc, c->win_ids, c->win_n, c->partials,
                    c->max_blocks, tiles_per_block};
         const dim3 grid((c->nd + WAVE - 1) / WAVE);
@@ -1817,8 +1908,8 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
             IVP_TRY(launch(c, KC_WINDOW, -1, 0.0, k_window<16>, grid, wa));
         else
             IVP_TRY(launch(c, KC_WINDOW, -1, 0.0, k_window<32>, grid, wa));
-        c->win_built = true;
     }
+    c->win_built = windows;
     // pair count (row 0) and window sizes (row 1) of the build's blocks
     if (c->nd > 0)
         IVP_TRY(finalize<FIN_BUILD>(c, tiles_per_block == 1 ? (c->nd + WAVE - 1) / WAVE : blocks_for(c->nd), 0.0, 0,

@@ -110,6 +110,7 @@ struct SceneParams {
     int max_opt, max_pcg, fixed;
 };
 
+constexpr int MARKS = 256;        // pass times that every context holds (more are allocated when needed)
 constexpr int ROW_PAD = 8;        // tile lengths are padded to a multiple of this many slots
 // slot_word's 8-slot blocks and the paired (g, g + 4) id loads of the pair passes assume both
 static_assert(ROW_PAD % 8 == 0, "ids-only rows are stored in 8-slot blocks");
