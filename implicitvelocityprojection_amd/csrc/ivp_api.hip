@@ -111,7 +111,8 @@ int alloc_all(ivp_ctx* c) {
     A(pos, cap + POS_PAD); A(pos_b, cap + POS_PAD); A(vel, 3 * cap); A(vel_b, 3 * cap); A(minv, cap); A(minv_b, cap);
     A(rho0, cap); A(rho0_b, cap); A(mat, cap); A(mat_b, cap); A(uid, cap); A(uid_b, cap); A(inv, cap);
     A(density, cap); A(kk, cap); A(Ss, 3 * cap); A(divg, cap); A(divg_b, cap); A(rowcnt, cap); A(rowtot, cap);
-    A(tile_len, tiles);
+    A(tile_len, 5 * tiles);
+    c->wave_len = c->tile_len + tiles;
     A(dstart, (size_t)c->ncell + 1); A(sstart, (size_t)c->ncell + 1); A(ccount, (size_t)c->ncell);
     A(key, cap); A(tmp_src, cap + 1); A(order, cap);
     size_t scan_n = std::max((size_t)c->ncell, cap) + 1;
@@ -141,7 +142,7 @@ int alloc_all(ivp_ctx* c) {
     IVP_HIP(hipMemsetAsync(c->ccount, 0, sizeof(int) * (size_t)c->ncell, c->stream));
     IVP_HIP(hipMemsetAsync(c->cell_bsum, 0, sizeof(int) * (size_t)c->nscan_blocks, c->stream));
     IVP_HIP(hipMemsetAsync(c->state, 0, sizeof(SolverState), c->stream));
-    IVP_HIP(hipMemsetAsync(c->tile_len, 0, sizeof(int) * tiles, c->stream));
+    IVP_HIP(hipMemsetAsync(c->tile_len, 0, sizeof(int) * 5 * tiles, c->stream));
     // the pads past cap are read by the candidate scan (and masked); keep them defined
     IVP_HIP(hipMemsetAsync(c->pos, 0, sizeof(float4) * (cap + POS_PAD), c->stream));
     IVP_HIP(hipMemsetAsync(c->pos_b, 0, sizeof(float4) * (cap + POS_PAD), c->stream));

@@ -251,6 +251,12 @@ __device__ __forceinline__ int wave_max(int v) {
     return wave_fold(v, [](int x, int y) { return x > y ? x : y; });
 }
 
+// Largest value over each 16 consecutive lanes
+__device__ __forceinline__ int row16_max(int v) {
+    auto f = [](int x, int y) { return x > y ? x : y; };
+    return pair_step<1>(pair_step<2>(pair_step<4>(pair_step<8>(v, f), f), f), f);
+}
+
 // Sums of NV doubles per thread over a 256-thread block, in a fixed order.  Results valid in
 // thread 0.  lds is not reused before a barrier of the caller's.
 template <int NV>

@@ -443,6 +443,7 @@ struct BuildArgs {
     uint32_t* nb;
     uint32_t* g16;   // float16 format: gradW / scale as two half-pair words at twice each id's word
     int* tile_len;
+    int* wave_len;
     int* rowcnt;
     int* rowtot;
     float* density;
@@ -1099,6 +1100,8 @@ __device__ __forceinline__ void build_eval(const BuildArgs& a, int i, int lane, 
     double v[2] = {(double)cnt, 0.0};
     block_partials<2>(v, a.partials, a.stride);
     if (lane == 0) a.tile_len[tile] = tlp;
+    const int wl = row16_max(cnt);
+    if ((lane & 15) == 0) a.wave_len[4 * tile + (lane >> 4)] = (wl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;
 }
 
 // LDS of the window search: the bitmap and the marks before each of its words
@@ -1230,7 +1233,10 @@ __global__ __launch_bounds__(BLOCK, 8) void k_eval4(BuildArgs a) {
     const size_t w_row = (size_t)tile * (size_t)a.Cs * 64u + 8u * (uint32_t)r;
     uint32_t* row = a.nb + w_row;
     const int wl = __builtin_amdgcn_readfirstlane(wave_max(cnt)), ws = __builtin_amdgcn_readfirstlane(wave_max(cs));
-    if ((threadIdx.x & (WAVE - 1)) == 0) wmax[threadIdx.x >> 6] = wl;
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        wmax[threadIdx.x >> 6] = wl;
+        a.wave_len[4 * tile + (int)(threadIdx.x >> 6)] = (wl + ROW_PAD - 1) / ROW_PAD * ROW_PAD;
+    }
     float rho = 0.0f, aii = 0.0f, jx = 0.0f, jy = 0.0f, jz = 0.0f, sx = 0.0f, sy = 0.0f, sz = 0.0f;
     rho = rho + pi.w * cubic_kernel(0.0f, h, a.kc);
     const float rho_self = rho;
@@ -1857,7 +1863,7 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         float h2_lo = std::nextafter((float)(hh * (1.0 - 1.0 / 1048576.0)), 0.0f);
         float h2_hi = std::nextafter((float)(hh * (1.0 + 1.0 / 1048576.0)), 1.0f);
         BuildArgs ba{c->nd, c->ns, c->C, c->Cs, c->h, h2_lo, h2_hi, (float)hh, c->kcubic, c->kspiky, 1.0f / c->h, 1.0f / c->gscale, c->grid,
-                     c->grids, c->sid, c->pos, c->minv, c->dstart, c->sstart, c->nb, c->g16, c->tile_len,
+                     c->grids, c->sid, c->pos, c->minv, c->dstart, c->sstart, c->nb, c->g16, c->tile_len, c->wave_len,
                      c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag, c->partials, c->max_blocks,
                      c->win_cap, c->loc, c->win_ids, c->win_n};
         // bytes (pair count of the previous build): the pair records written, the ids read back

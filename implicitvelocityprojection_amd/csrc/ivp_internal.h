@@ -19,7 +19,8 @@
 //   * cached gradW (REC = 256 float32: id, gx, gy, gz; REC = 192 float16: id, (gx, gy), (gz, 0)):
 //     slot-major records, word k REC + c 64 + lane for component c, one contiguous record per
 //     (tile, slot) read by one wave.
-// The tile length is the tile's longest row rounded up to ROW_PAD; slots past a row's count hold
+// The tile length is the tile's longest row rounded up to ROW_PAD (a pass with four lanes per row
+// walks its 16 rows' longest row, rounded up the same); slots past a row's count hold
 // (id = the row itself, gradW = 0): r_ii = 0 gives gradW = 0 either way, which adds exactly 0 to
 // every operator, so the hot loops run a wave-uniform trip count.
 #pragma once
@@ -199,6 +200,7 @@ struct ivp_ctx {
     uint32_t* g16 = nullptr;   // float16 format: gradW / gscale, two half-pair words per slot at
                                // twice the word index of the slot's id
     int* tile_len = nullptr;
+    int* wave_len = nullptr;   // slots to walk per 16 rows (after the tile lengths in one allocation)
     // tile windows (ids-only layout, one scene): per 64-row tile its distinct neighbour ids in
     // ascending order (win_ids, WIN_MAX per tile) and their count (win_n, -1: the tile has no
     // window); per walked slot of a valid row the index of its id in the window, 16 bits at the

@@ -66,6 +66,7 @@ struct Rows {
     const uint32_t* nb;
     const uint32_t* g16;   // float16 gradW side array (float16 format): words 2w, 2w + 1 for id word w
     const int* tile_len;   // per tile: slots to walk, a multiple of ROW_PAD, padded with the row itself
+    const int* wave_len;   // the same per 16 rows: a wave's, with four lanes per row
     int Cs;                // slots per row in the tile layout
     int nd;
     const float4* pos;   // particle positions (x, y, z, m), for evaluated gradients
@@ -201,7 +202,8 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
     static_assert(FM::GS != GS_F16 || REC == 64u, "float16 gradients live beside the ids-only layout");
     const size_t w_row = (size_t)(i >> 6) * (size_t)R.Cs * REC + row_word0<REC>(i & (WAVE - 1));
     const uint32_t* e = R.nb + w_row;
-    const int tl = __builtin_amdgcn_readfirstlane(R.tile_len[i >> 6]);   // one tile per wave
+    // one tile, or a quarter of one, per wave
+    const int tl = __builtin_amdgcn_readfirstlane(REC == 64u && G == 4 ? R.wave_len[i >> 4] : R.tile_len[i >> 6]);
     // gw: the slot's gradient words (float32 x, y, z at 64-word strides, or two float16 words)
     auto visit = [&](int j, const uint32_t* gw) {
         float4 Aj = loadA(j);
@@ -1528,7 +1530,7 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
     const uint32_t* e = a.R.nb + (size_t)(i >> 6) * (size_t)a.R.Cs * REC + row_word0<REC>(i & (WAVE - 1));
     // the per-pair g-tilde array has one word per slot in the layout of ids-only rows
     float* eg = a.gt + (size_t)(i >> 6) * (size_t)a.R.Cs * 64u + row_word0<64u>(i & (WAVE - 1));
-    const int tl = __builtin_amdgcn_readfirstlane(a.R.tile_len[i >> 6]);
+    const int tl = __builtin_amdgcn_readfirstlane(REC == 64u ? a.R.wave_len[i >> 4] : a.R.tile_len[i >> 6]);
     const float4 xi = a.R.pos[i];
     const float4 ui = a.u4[i];
     const float m_i = ui.w, rho_i = a.density[i], div_i = a.div[i];
@@ -1627,7 +1629,7 @@ __global__ __launch_bounds__(BLOCK) void k_st_Av(StArgs a) {
         if (ALLFLUID || a.mat[i] == a.fluid) {
             const uint32_t* e = a.R.nb + (size_t)(i >> 6) * (size_t)a.R.Cs * REC + row_word0<REC>(i & (WAVE - 1));
             const float* eg = a.gt + (size_t)(i >> 6) * (size_t)a.R.Cs * 64u + row_word0<64u>(i & (WAVE - 1));
-            const int tl = __builtin_amdgcn_readfirstlane(a.R.tile_len[i >> 6]);
+            const int tl = __builtin_amdgcn_readfirstlane(REC == 64u ? a.R.wave_len[i >> 4] : a.R.tile_len[i >> 6]);
             const float m_i = ui.w;
             float sx = 0.0f, sy = 0.0f, sz = 0.0f;
             auto visit_u = [&](const float4& uj, float gt) {
@@ -1715,7 +1717,7 @@ __global__ __launch_bounds__(BLOCK) void k_gravity(int nd, float gx, float gy, f
 
 Rows rows_of(ivp_ctx* c) {
     const bool win = c->win_built && c->windows;
-    return Rows{c->nb, c->g16, c->tile_len, c->Cs, c->nd, c->pos, c->h, c->kspiky, c->gscale,
+    return Rows{c->nb, c->g16, c->tile_len, c->wave_len, c->Cs, c->nd, c->pos, c->h, c->kspiky, c->gscale,
                 c->loc, c->win_ids, win ? c->win_n : nullptr};
 }
 
