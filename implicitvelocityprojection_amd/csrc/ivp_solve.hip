@@ -195,9 +195,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #endif
 constexpr int LOC_PF = IVP_LOC_PF;   // window-index words requested at once per lane
 // With LOC (tile windows, four lanes per row) the lane reads its two slots' window indices as
-// one 32-bit word at half the word index of their ids, and loadA / loadB take window indices.
+// one 32-bit word at half the word index of their ids, and loadA / loadB take window indices; the
+// words of the first LOC_PF blocks are in lp (loc_prefetch).
+struct LocPre {
+    uint32_t q[LOC_PF];
+};
 template <class FM, int NB, int G = 1, int U = 4, bool LOC = false, class LA, class LB, class F>
-__device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& loadA, LB&& loadB, F&& f, int g = 0) {
+__device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& loadA, LB&& loadB, F&& f, int g = 0,
+                                          const LocPre& lp = LocPre()) {
     constexpr unsigned REC = FM::REC;
     static_assert(FM::GS != GS_F16 || REC == 64u, "float16 gradients live beside the ids-only layout");
     const size_t w_row = (size_t)(i >> 6) * (size_t)R.Cs * REC + row_word0<REC>(i & (WAVE - 1));
@@ -224,38 +229,25 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
         f(Aj, Bj, gx, gy, gz);
     };
     static_assert(!LOC || (REC == 64u && G == 4), "tile windows index the paired ids-only layout");
-    if constexpr (LOC && FM::GS != GS_F16) {
-        // all index words of up to LOC_PF blocks are requested before the first is used (the
-        // words come from HBM; the neighbours from LDS)
+    if constexpr (LOC) {
         const uint32_t* l = R.loc + ((w_row + 2 * g) >> 1);
-        for (int b0 = 0; b0 < tl; b0 += 8 * LOC_PF) {
-            uint32_t q[LOC_PF];
+        const u32x4* g4 = FM::GS == GS_F16 ? reinterpret_cast<const u32x4*>(R.g16 + 2 * (w_row + 2 * g)) : nullptr;
+        // (float16 rows: the next block's gradient words in flight while a block is visited)
+        u32x4 h = {0u, 0u, 0u, 0u};
+        auto grads = [&](int b) {
+            if constexpr (FM::GS == GS_F16) h = __builtin_nontemporal_load(g4 + b * 256);
+        };
+        auto block = [&](uint32_t q, int b) {
+            const uint32_t w0[2] = {h.x, h.y}, w1[2] = {h.z, h.w};
+            if (8 * (b + 1) < tl) grads(b + 1);
+            visit((int)(q & 0xffffu), w0);
+            visit((int)(q >> 16), w1);
+        };
+        if (tl > 0) grads(0);
 #pragma unroll
-            for (int k = 0; k < LOC_PF; ++k)
-                q[k] = b0 + 8 * k < tl ? __builtin_nontemporal_load(l + ((b0 >> 3) + k) * 256) : 0u;
-#pragma unroll
-            for (int k = 0; k < LOC_PF; ++k)
-                if (b0 + 8 * k < tl) {
-                    visit((int)(q[k] & 0xffffu), nullptr);
-                    visit((int)(q[k] >> 16), nullptr);
-                }
-        }
-    } else if constexpr (LOC) {
-        const uint32_t* l = R.loc + ((w_row + 2 * g) >> 1);
-#pragma unroll((U + 1) / 2)
-        for (int b = 0; b < tl; b += 8) {
-            const uint32_t q = __builtin_nontemporal_load(l + (b >> 3) * 256);
-            if constexpr (FM::GS == GS_F16) {
-                const u32x4* g4 = reinterpret_cast<const u32x4*>(R.g16 + 2 * (w_row + 2 * g));
-                const u32x4 h = __builtin_nontemporal_load(g4 + (b >> 3) * 256);
-                const uint32_t w0[2] = {h.x, h.y}, w1[2] = {h.z, h.w};
-                visit((int)(q & 0xffffu), w0);
-                visit((int)(q >> 16), w1);
-            } else {
-                visit((int)(q & 0xffffu), nullptr);
-                visit((int)(q >> 16), nullptr);
-            }
-        }
+        for (int k = 0; k < LOC_PF; ++k)
+            if (8 * k < tl) block(lp.q[k], k);
+        for (int b = LOC_PF; 8 * b < tl; ++b) block(__builtin_nontemporal_load(l + b * 256), b);
     } else if constexpr (REC == 64u && G == 4) {
         // tl is a multiple of ROW_PAD = 8: whole blocks; block b's pair for this lane is the
         // 8-byte word pair 2 g of the row's 8 words in block b (512 words per block), and its
@@ -301,20 +293,76 @@ struct WinLds {
     float4 B[N];
 };
 
+// A pass block waits for memory more than it computes: walked one after another, the window's length,
+// its ids, their records, the index words, the row's own data and what the row's end reads are five
+// round trips, and without any pair at all the passes took 60 to 75 % of their time (1M rows).  So a
+// pass requests everything that depends on nothing first -- win_prefetch, its row's data and
+// loc_prefetch -- and only then stages (1M rows, us before / after: ip_pack
+// 62 / 53, ip_rhs 52 / 47, cg_JT 47 / 42, w18_setup 76 / 71, w18_Av 48 / 46).  The requests cost registers, so the
+// passes are compiled for the eight blocks per CU that the window's LDS allows (64 registers): left at 72 to
+// 80 they gained nothing.
+struct WinPre {
+    int nw;      // ids in the tile's window (-1: none)
+    int id[2];   // the thread's first two (not valid past nw)
+};
+template <class FM, int G>
+__device__ __forceinline__ WinPre win_prefetch(const Rows& R, int tile) {
+    WinPre p = {-1, {0, 0}};
+    if constexpr (has_windows<FM, G>()) {
+        static_assert(BLOCK / G == WAVE, "a four-lane pass block is one tile");
+        static_assert(2 * BLOCK <= WIN_MAX, "the first two ids of a thread are inside the tile's list");
+        if (R.win_n != nullptr) {
+            const int* wid = R.win_ids + (size_t)tile * WIN_MAX + threadIdx.x;
+            p.nw = R.win_n[tile];
+            p.id[0] = wid[0];
+            p.id[1] = wid[BLOCK];
+        }
+    }
+    return p;
+}
+
+// The row's first LOC_PF index words (tile windows); the first LOC_EAGER without waiting for the
+// number of slots to walk
+constexpr int LOC_EAGER = 4;
+template <class FM, int G>
+__device__ __forceinline__ LocPre loc_prefetch(const Rows& R, int i, int g) {
+    LocPre p;
+#pragma unroll
+    for (int k = 0; k < LOC_PF; ++k) p.q[k] = 0u;
+    if constexpr (has_windows<FM, G>()) {
+        if (R.win_n != nullptr) {
+            const uint32_t* l = R.loc + (size_t)(i >> 6) * (size_t)R.Cs * 32u + 4u * (uint32_t)(i & (WAVE - 1)) + (uint32_t)g;
+            const int wl = R.wave_len[i >> 4];
+#pragma unroll
+            for (int k = 0; k < LOC_EAGER; ++k)
+                if (8 * k < R.Cs) p.q[k] = __builtin_nontemporal_load(l + k * 256);
+            const int tl = __builtin_amdgcn_readfirstlane(wl);
+#pragma unroll
+            for (int k = LOC_EAGER; k < LOC_PF; ++k)
+                if (8 * k < tl) p.q[k] = __builtin_nontemporal_load(l + k * 256);
+        }
+    }
+    return p;
+}
+
 template <class FM, int G, class LA, class LB>
-__device__ __forceinline__ bool stage_window(const Rows& R, int tile, WinLds<FM, G>& w, LA&& la, LB&& lb) {
+__device__ __forceinline__ bool stage_window(const Rows& R, int tile, const WinPre& pre, WinLds<FM, G>& w, LA&& la, LB&& lb) {
     if constexpr (!has_windows<FM, G>()) {
         return false;
     } else {
-        static_assert(BLOCK / G == WAVE, "a four-lane pass block is one tile");
         if (R.win_n == nullptr) return false;
-        const int nw = __builtin_amdgcn_readfirstlane(R.win_n[tile]);
+        const int nw = __builtin_amdgcn_readfirstlane(pre.nw);
         if (nw < 0) return false;
-        const int* wid = R.win_ids + (size_t)tile * WIN_MAX;
-        for (int k = threadIdx.x; k < nw; k += BLOCK) {
-            const int j = wid[k];
-            w.A[k] = la(j);
-            w.B[k] = lb(j);
+        const int k = threadIdx.x;
+        float4 A0, B0, A1, B1;
+        if (k < nw) { A0 = la(pre.id[0]); B0 = lb(pre.id[0]); }
+        if (k + BLOCK < nw) { A1 = la(pre.id[1]); B1 = lb(pre.id[1]); }
+        if (k < nw) { w.A[k] = A0; w.B[k] = B0; }
+        if (k + BLOCK < nw) { w.A[k + BLOCK] = A1; w.B[k + BLOCK] = B1; }
+        for (int q = k + 2 * BLOCK; q < nw; q += BLOCK) {
+            const int j = R.win_ids[(size_t)tile * WIN_MAX + q];
+            w.A[q] = la(j);
+            w.B[q] = lb(j);
         }
         __syncthreads();
         return true;
@@ -331,12 +379,12 @@ __device__ __forceinline__ Vec<NB> vec_of(const float4& b) {
 }
 
 template <class FM, int NB, int G, class LA, class LB, class F>
-__device__ __forceinline__ void row_pairs_w(bool win, const WinLds<FM, G>& w, const Rows& R, int i, float4 xi,
-                                            LA&& loadA, LB&& loadB, F&& f, int g) {
+__device__ __forceinline__ void row_pairs_w(bool win, const WinLds<FM, G>& w, const LocPre& lp, const Rows& R, int i,
+                                            float4 xi, LA&& loadA, LB&& loadB, F&& f, int g) {
     if constexpr (has_windows<FM, G>()) {
         if (win) {
             row_pairs<FM, NB, G, PASS_UNROLL, true>(R, i, xi, [&](int k) { return w.A[k]; },
-                                                    [&](int k) { return vec_of<NB>(w.B[k]); }, f, g);
+                                                    [&](int k) { return vec_of<NB>(w.B[k]); }, f, g, lp);
             return;
         }
     }
@@ -398,7 +446,7 @@ __device__ __forceinline__ bool cg_stopped(const SolverState* st) { return st->a
 // (math_utils.py:76-91, pressure_base.py:187-203, 413-423).  J d in the form of
 // compute_J_x_kernel (pressure_base.py:111-127): sum_j m_j dot(d_i - d_j, gradW_ij) + dot(d_i, S_i).
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK) void k_ip_pack(PackArgs a) {
+__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
     if (!SC && a.gate && !cg_stopped(a.gate)) return;
     if (!SC && a.mark && blockIdx.x == 0 && threadIdx.x == 0) *a.mark = wall_clock64();
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -409,12 +457,31 @@ __global__ __launch_bounds__(BLOCK) void k_ip_pack(PackArgs a) {
     auto loadA = [&](int j) { return j_record<FM::EVAL>(a.R.pos, a.d4, j); };
     auto loadB = [&](int j) { return vec3_of(a.d4, j); };
     __shared__ WinLds<FM, G> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.d4[j]; });
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    float4 di, xi;
+    float s0, s1, s2, cc, k, rho0;
+    int cnt;
+    auto own = [&]() {
+        di = a.d4[ic];
+        xi = a.R.pos[ic];
+    };
+    auto tail = [&]() {
+        s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2];
+        cc = a.cc[ic]; k = a.kk[ic]; rho0 = a.rho0[ic];
+        cnt = a.rowcnt[ic];
+    };
+    if (!SC) {   // (scenes have no windows to wait for: their rows load when they need it)
+        own();
+        tail();
+    }
+    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.d4[j]; });
     double err = 0.0, nact = 0.0, npairs = 0.0;
     float acc = 0.0f;
     if (gt.on) {
-        float4 di = a.d4[i];
-        row_pairs_w<FM, 3, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+        if (SC) own();
+        row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                              [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
                                  float dx = di.x - Bj.v[0], dy = di.y - Bj.v[1], dz = di.z - Bj.v[2];
                                  acc = fmaf(Aj.w, fmaf(dz, gz, fmaf(dy, gy, dx * gx)), acc);
@@ -422,22 +489,21 @@ __global__ __launch_bounds__(BLOCK) void k_ip_pack(PackArgs a) {
         acc = group_sum<G>(acc);
     }
     if (gt.on && g == 0) {
-        float4 di = a.d4[i];
-        float jd = acc + (di.x * a.Ss[3 * i + 0] + di.y * a.Ss[3 * i + 1] + di.z * a.Ss[3 * i + 2]);
+        if (SC) tail();
+        float jd = acc + (di.x * s0 + di.y * s1 + di.z * s2);
         a.jd[i] = jd;
-        float t = jd + a.cc[i];
+        float t = jd + cc;
         float f = fmaxf(t, 0.0f);
         float dfdt = t >= 1e-6f ? 1.0f : 0.0f;
-        float k = a.kk[i];
         float sk = dfdt * k;
         a.sfac[i] = sk;
         a.q4[i] = make_float4(f * k, sk, di.w, 0.0f);
-        float denom = a.rho0[i];
+        float denom = rho0;
         if (denom < 1e-6f) denom = 1e-6f;
         err = (double)fmaxf(f / denom, 0.0f);
         if (sk != 0.0f) {
             nact = 1.0;
-            npairs = (double)a.rowcnt[i];
+            npairs = (double)cnt;
         }
     }
     double v[3] = {err, nact, npairs};
@@ -460,7 +526,7 @@ struct RhsArgs {
 // ip_rhs_fused (ip.py:174-215): b = omega J^T (f k); also marks rows whose CG J^T loop can be
 // non-zero (own dfdt > 0 or a dynamic neighbour with dfdt > 0).
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK) void k_ip_rhs(RhsArgs a) {
+__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
     Gate gt = gate_all(i, a.R.nd);
@@ -477,14 +543,32 @@ __global__ __launch_bounds__(BLOCK) void k_ip_rhs(RhsArgs a) {
         return B;
     };
     __shared__ WinLds<FM, G> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.q4[j]; });
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    float4 qi, xi;
+    float s0, s1, s2;
+    int cnt;
+    auto own = [&]() {
+        qi = a.q4[ic];
+        xi = a.R.pos[ic];
+    };
+    auto tail = [&]() {
+        s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2];
+        cnt = a.rowcnt[ic];
+    };
+    if (!SC) {
+        own();
+        tail();
+    }
+    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.q4[j]; });
     double touched = 0.0, tpairs = 0.0;
     if (gt.on) {
-        float4 qi = a.q4[i];
+        if (SC) own();
         float fki = qi.x, mi = qi.z;
         bool act = qi.y != 0.0f;
         float rx = 0.0f, ry = 0.0f, rz = 0.0f;
-        row_pairs_w<FM, 2, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+        row_pairs_w<FM, 2, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                              [&](const float4& Aj, const Vec<2>& Bj, float gx, float gy, float gz) {
                                  float sc = fmaf(Aj.w, fki, mi * Bj.v[0]);
                                  rx = fmaf(sc, gx, rx); ry = fmaf(sc, gy, ry); rz = fmaf(sc, gz, rz);
@@ -495,16 +579,17 @@ __global__ __launch_bounds__(BLOCK) void k_ip_rhs(RhsArgs a) {
         rz = group_sum<G>(rz);
         act = group_any<G>(act);
         if (g == 0) {
-            rx += fki * a.Ss[3 * i + 0];
-            ry += fki * a.Ss[3 * i + 1];
-            rz += fki * a.Ss[3 * i + 2];
+            if (SC) tail();
+            rx += fki * s0;
+            ry += fki * s1;
+            rz += fki * s2;
             a.b[3 * i + 0] = a.omega * rx;
             a.b[3 * i + 1] = a.omega * ry;
             a.b[3 * i + 2] = a.omega * rz;
             a.nbact[i] = act ? 1 : 0;
             if (act) {
                 touched = 1.0;
-                tpairs = (double)a.rowcnt[i];
+                tpairs = (double)cnt;
             }
         }
     }
@@ -559,34 +644,50 @@ struct CGJArgs {
 // compute_Jx_pcg (ip.py:19-60): y_i = dfdt_i k_i (J p)_i on rows with dfdt > 0, J p in the form
 // sum_j dot(p_i - p_j, m_j gradW_ij) + dot(p_i, S_i) (ip.py:51-58)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK) void k_cg_J(CGJArgs a) {
+__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_J(CGJArgs a) {
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
     Gate gt = gate_all(i, a.R.nd);
     if (SC && !gate_block<BLOCK / G>(a.sc, blk, i, a.R.nd, PH_CG, gt)) return;
-    const float sk = gt.on ? a.sfac[i] : 0.0f;
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float sk = gt.on ? a.sfac[ic] : 0.0f;
+    float4 pi, xi;
+    float s0, s1, s2;
+    auto own = [&]() {
+        pi = a.p4[ic];
+        xi = a.R.pos[ic];
+    };
+    auto tail = [&]() { s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2]; };
+    if (!SC) {
+        own();
+        tail();
+    }
     // neighbour record: A = (x, y, z, m), B = p
     auto loadA = [&](int j) { return j_record<FM::EVAL>(a.R.pos, a.p4, j); };
     auto loadB = [&](int j) { return vec3_of(a.p4, j); };
     __shared__ WinLds<FM, G> w;
     bool win = false;
+    LocPre lp;
     if constexpr (has_windows<FM, G>()) {
         // a tile without active rows neither stages nor walks
         if (!__syncthreads_or(sk != 0.0f)) return;
-        win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.p4[j]; });
+        if (sk != 0.0f) lp = loc_prefetch<FM, G>(a.R, i, g);
+        win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.p4[j]; });
     }
     if (sk == 0.0f) return;
-    float4 pi = a.p4[i];
+    if (SC) own();
     float acc = 0.0f;
-    row_pairs_w<FM, 3, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+    row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                          [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
                              float dx = pi.x - Bj.v[0], dy = pi.y - Bj.v[1], dz = pi.z - Bj.v[2];
                              acc = fmaf(Aj.w, fmaf(dz, gz, fmaf(dy, gy, dx * gx)), acc);
                          }, g);
     acc = group_sum<G>(acc);
     if (g != 0) return;
-    acc = acc + (pi.x * a.Ss[3 * i + 0] + pi.y * a.Ss[3 * i + 1] + pi.z * a.Ss[3 * i + 2]);
+    if (SC) tail();
+    acc = acc + (pi.x * s0 + pi.y * s1 + pi.z * s2);
     a.y2[i] = make_float2(acc * sk, pi.w);
 }
 
@@ -607,13 +708,27 @@ struct CGJTArgs {
 // compute_Ax_part1 + compute_Ax_part2 (ip.py:63-121) in gather form, fused with p.Ap
 // (ip.py:307)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK) void k_cg_JT(CGJTArgs a) {
+__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_JT(CGJTArgs a) {
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
     Gate gt = gate_all(i, a.R.nd);
     if (SC && !gate_block<BLOCK / G>(a.sc, blk, i, a.R.nd, PH_CG, gt)) return;
-    const bool touched = gt.on && a.nbact[i] != 0;
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const bool touched = gt.on && a.nbact[ic] != 0;
+    const float4 pi = a.p4[ic];
+    float4 xi;
+    float yi, s0, s1, s2;
+    auto own = [&]() {
+        xi = a.R.pos[ic];
+        yi = a.y2[ic].x;
+    };
+    auto tail = [&]() { s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2]; };
+    if (!SC) {
+        own();
+        tail();
+    }
     // neighbour record: A = (x, y, z, m), B = y; y2 = (y, m)
     auto loadA = [&](int j) {
         return FM::EVAL ? a.R.pos[j] : make_float4(0.0f, 0.0f, 0.0f, a.y2[j].y);
@@ -625,22 +740,24 @@ __global__ __launch_bounds__(BLOCK) void k_cg_JT(CGJTArgs a) {
     };
     __shared__ WinLds<FM, G> w;
     bool win = false;
+    LocPre lp;
     if constexpr (has_windows<FM, G>()) {
         // a tile without touched rows stages nothing (its rows only write m p)
-        if (__syncthreads_or(touched))
-            win = stage_window(a.R, blk, w, loadA, [&](int j) {
+        if (__syncthreads_or(touched)) {
+            if (touched) lp = loc_prefetch<FM, G>(a.R, i, g);
+            win = stage_window(a.R, blk, wp, w, loadA, [&](int j) {
                 const float2 y = a.y2[j];
                 return make_float4(y.x, y.y, 0.0f, 0.0f);
             });
+        }
     }
     double pap = 0.0;
     if (gt.on) {
-        float4 pi = a.p4[i];
         float mi = pi.w;
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         if (touched) {
-            float yi = a.y2[i].x;
-            row_pairs_w<FM, 1, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+            if (SC) own();
+            row_pairs_w<FM, 1, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                                  [&](const float4& Aj, const Vec<1>& Bj, float gx, float gy, float gz) {
                                      float sc = fmaf(Aj.w, yi, mi * Bj.v[0]);
                                      ax = fmaf(sc, gx, ax); ay = fmaf(sc, gy, ay); az = fmaf(sc, gz, az);
@@ -648,9 +765,10 @@ __global__ __launch_bounds__(BLOCK) void k_cg_JT(CGJTArgs a) {
             ax = group_sum<G>(ax);
             ay = group_sum<G>(ay);
             az = group_sum<G>(az);
-            ax += yi * a.Ss[3 * i + 0];
-            ay += yi * a.Ss[3 * i + 1];
-            az += yi * a.Ss[3 * i + 2];
+            if (SC) tail();
+            ax += yi * s0;
+            ay += yi * s1;
+            az += yi * s2;
         }
         float Apx = mi * pi.x + a.omega * ax;
         float Apy = mi * pi.y + a.omega * ay;
@@ -836,7 +954,7 @@ __global__ __launch_bounds__(BLOCK) void k_prj_init(int nd, float dt, const floa
 
 // pj_head_fused (prj.py:17-59); also the head of solve_df (prj.py:243-253)
 template <class FM>
-__global__ __launch_bounds__(BLOCK) void k_prj_head(PrjArgs a) {
+__global__ __launch_bounds__(BLOCK, 8) void k_prj_head(PrjArgs a) {
     if (a.st->active == 0) return;
     if (a.mark0 && blockIdx.x == 0 && threadIdx.x == 0) *a.mark0 = wall_clock64();
     constexpr int G = PASS_LANES;
@@ -852,14 +970,20 @@ __global__ __launch_bounds__(BLOCK) void k_prj_head(PrjArgs a) {
         return B;
     };
     __shared__ WinLds<FM, G> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) {
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float2 li = a.lam[ic];
+    const float4 xi = a.R.pos[ic];
+    const float s0 = a.Ss[3 * ic + 0], s1 = a.Ss[3 * ic + 1], s2 = a.Ss[3 * ic + 2];
+    const float v0 = a.v0[3 * ic + 0], v1 = a.v0[3 * ic + 1], v2 = a.v0[3 * ic + 2];
+    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) {
         const float2 l = a.lam[j];
         return make_float4(l.x, l.y, 0.0f, 0.0f);
     });
     if (i >= a.R.nd) return;   // the G lanes of a row leave together
-    const float2 li = a.lam[i];
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    row_pairs_w<FM, 1, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+    row_pairs_w<FM, 1, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                                      [&](const float4& Aj, const Vec<1>& Bj, float gx, float gy, float gz) {
                                          float s = fmaf(Aj.w, li.x, li.y * Bj.v[0]);
                                          ax = fmaf(s, gx, ax); ay = fmaf(s, gy, ay); az = fmaf(s, gz, az);
@@ -868,18 +992,17 @@ __global__ __launch_bounds__(BLOCK) void k_prj_head(PrjArgs a) {
     ay = group_sum<G>(ay);
     az = group_sum<G>(az);
     if (g != 0) return;
-    ax += li.x * a.Ss[3 * i + 0];
-    ay += li.x * a.Ss[3 * i + 1];
-    az += li.x * a.Ss[3 * i + 2];
+    ax += li.x * s0;
+    ay += li.x * s1;
+    az += li.x * s2;
     const float denom = li.y < 1e-6f ? 1e-6f : li.y;
-    a.d4[i] = make_float4(a.v0[3 * i + 0] - ax / denom, a.v0[3 * i + 1] - ay / denom, a.v0[3 * i + 2] - az / denom,
-                          li.y);
+    a.d4[i] = make_float4(v0 - ax / denom, v1 - ay / denom, v2 - az / denom, li.y);
 }
 
 // pj_tail_fused (prj.py:62-115); DF: the pass of solve_df (prj.py:255-283: J v masked by the
 // active rows, D^-1 J v, lambda + omega D^-1 J v, max(., 0), error of J v / rho0)
 template <class FM, bool DF>
-__global__ __launch_bounds__(BLOCK) void k_prj_tail(PrjArgs a) {
+__global__ __launch_bounds__(BLOCK, 8) void k_prj_tail(PrjArgs a) {
     if (a.st->active == 0) return;
     constexpr int G = PASS_LANES;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -889,34 +1012,40 @@ __global__ __launch_bounds__(BLOCK) void k_prj_tail(PrjArgs a) {
     auto loadA = [&](int j) { return j_record<FM::EVAL>(a.R.pos, a.d4, j); };
     auto loadB = [&](int j) { return vec3_of(a.d4, j); };
     __shared__ WinLds<FM, G> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.d4[j]; });
+    const WinPre wp = win_prefetch<FM, G>(a.R, blk);
+    const int ic = on ? i : a.R.nd - 1;
+    const float4 di = a.d4[ic], xi = a.R.pos[ic];
+    const float s0 = a.Ss[3 * ic + 0], s1 = a.Ss[3 * ic + 1], s2 = a.Ss[3 * ic + 2];
+    const float lam = a.lam[ic].x, kk = a.kk[ic], cc = DF ? 0.0f : a.cc[ic];
+    const int tot = DF ? a.rowtot[ic] : 0;
+    float rho0 = a.rho0[ic];
+    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.d4[j]; });
     double err = 0.0;
     if (on) {
-        const float4 di = a.d4[i];
         float acc = 0.0f;
-        row_pairs_w<FM, 3, G>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+        row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                                          [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
                                              float dx = di.x - Bj.v[0], dy = di.y - Bj.v[1], dz = di.z - Bj.v[2];
                                              acc = fmaf(Aj.w, fmaf(dz, gz, fmaf(dy, gy, dx * gx)), acc);
                                          }, g);
         acc = group_sum<G>(acc);
         if (g == 0) {
-            const float jd = acc + (di.x * a.Ss[3 * i + 0] + di.y * a.Ss[3 * i + 1] + di.z * a.Ss[3 * i + 2]);
+            const float jd = acc + (di.x * s0 + di.y * s1 + di.z * s2);
             a.jd[i] = jd;
-            float l = a.lam[i].x, e;
+            float l = lam, e;
             if (!DF) {
-                const float r = jd + a.cc[i];
-                l = fmaxf(l + a.omega * r * a.kk[i], 0.0f);
+                const float r = jd + cc;
+                l = fmaxf(l + a.omega * r * kk, 0.0f);
                 e = r;
             } else {
-                const int cnt = a.rowtot[i] < a.C ? a.rowtot[i] : a.C;
+                const int cnt = tot < a.C ? tot : a.C;
                 const float dJ = jd * (cnt > a.df_threshold ? 1.0f : 0.0f);
-                const float Dr = dJ * a.kk[i];
+                const float Dr = dJ * kk;
                 l = fmaxf(l + a.omega * Dr, 0.0f);
                 e = dJ;
             }
             a.lam[i] = make_float2(l, di.w);
-            float rho0 = a.rho0[i];
             if (rho0 < 1e-6f) rho0 = 1e-6f;
             err = (double)fmaxf(e / rho0, 0.0f);
         }
@@ -987,14 +1116,17 @@ __global__ __launch_bounds__(BLOCK) void k_v4(int nd, const float* __restrict__ 
 // viscosity.py:62-108 with Jacobi reads.  Neighbour record: A = (x, y, z, m_j), m_j = 0 for a
 // non-fluid neighbour (its term is then exactly 0, as the reference's skip), B = (v_j, rho_j).
 template <class FM, bool ALLFLUID>
-__global__ __launch_bounds__(BLOCK) void k_visc(Rows R, float coeff, float dt, int fluid,
+__global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt, int fluid,
                                                 const float4* __restrict__ v4, const float* __restrict__ rho0,
                                                 const int* __restrict__ mat, float* __restrict__ vel) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
+    // neighbour record: A = (x, y, z, m_j / rho_j), the quotient formed once per record instead of once
+    // per pair (102k rows: 16.4 -> 14.4 us), B = (v, rho)
     auto loadA = [&](int j) {
         float4 A = R.pos[j];
         if (!ALLFLUID && mat[j] != fluid) A.w = 0.0f;
+        A.w = A.w / v4[j].w;
         return A;
     };
     auto loadB = [&](int j) {
@@ -1004,24 +1136,26 @@ __global__ __launch_bounds__(BLOCK) void k_visc(Rows R, float coeff, float dt, i
         return B;
     };
     __shared__ WinLds<FM, PASS_LANES> w;
-    const bool win = stage_window(R, blk, w, loadA, [&](int j) { return v4[j]; });
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(R, blk);
+    const int ic = i < R.nd ? i : R.nd - 1;
+    const float4 xi = R.pos[ic], vi = v4[ic];
+    const float rho_i = vi.w, rho0_i = rho0[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(R, i, g);
+    const bool win = stage_window(R, blk, wp, w, loadA, [&](int j) { return v4[j]; });
     if (i >= R.nd) return;
     if (!ALLFLUID && mat[i] != fluid) return;
-    float4 xi = R.pos[i];
-    float4 vi = v4[i];
-    float rho_i = vi.w, rho0_i = rho0[i];
     float eps2 = (0.01f * R.h) * (0.01f * R.h);
     float k_visc = 2.0f * (3.0f + 2.0f);
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    row_pairs_w<FM, 4, PASS_LANES>(win, w, R, i, xi, loadA, loadB,
+    row_pairs_w<FM, 4, PASS_LANES>(win, w, lp, R, i, xi, loadA, loadB,
                          [&](const float4& xj, const Vec<4>& vj, float gx, float gy, float gz) {
                              float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-                             float rn = len3(rx, ry, rz);
+                             float rn = len3_rn(rx, ry, rz);
                              float vx = vi.x - vj.v[0], vy = vi.y - vj.v[1], vz = vi.z - vj.v[2];
                              float vxy = vx * rx + vy * ry + vz * rz;
                              float rho_j = vj.v[3];
                              float K = 2.0f * rho0_i / (rho_i + rho_j);
-                             float sc = k_visc * coeff * (xj.w / rho_j) * (vxy / (rn * rn + eps2));
+                             float sc = k_visc * coeff * xj.w * (vxy / (rn * rn + eps2));
                              ax = ax + K * (sc * gx);
                              ay = ay + K * (sc * gy);
                              az = az + K * (sc * gz);
@@ -1110,10 +1244,9 @@ __device__ __forceinline__ float4 w18_Av_record(const W18Args& a, int j) {
 // (A u)_i = u_i - factor_i * 10 sum_fluid (m_j/rho_j) (u_ij . x_ij) / (r^2 + 0.01 h^2) gradW_ij
 // (compute_Av_weiler18, weiler18.py:103-172).  The caller stages the block's window.
 template <class FM, bool ALLFLUID, int G, class LA, class LB>
-__device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui, bool win, const WinLds<FM, G>& w,
-                                             LA&& loadA, LB&& loadB, int g = 0) {
+__device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui, float4 xi, float f, bool win,
+                                             const WinLds<FM, G>& w, const LocPre& lp, LA&& loadA, LB&& loadB, int g = 0) {
     if (!ALLFLUID && a.mat[i] != a.fluid) return make_float3(ui.x, ui.y, ui.z);
-    float4 xi = a.R.pos[i];
     float lx = 0.0f, ly = 0.0f, lz = 0.0f;
     float eps2 = 0.01f * a.R.h * a.R.h;
     if constexpr (FM::EVAL) {
@@ -1121,7 +1254,7 @@ __device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui,
         // 10 V_j (u_ij . x_ij) / (r^2 + 0.01 h^2) fold into one scalar per pair, the constant
         // -10 ks carried by the neighbour record's w (w18_Av_record); x_ij is scaled once
         const float h = a.R.h;
-        row_pairs_w<FM, 3, G>(win, w, a.R, i, xi, loadA, loadB,
+        row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                              [&](const float4& xj, const Vec<3>& uj, float, float, float) {
                                  float x0 = xi.x - xj.x, x1 = xi.y - xj.y, x2 = xi.z - xj.z;
                                  float v0 = ui.x - uj.v[0], v1 = ui.y - uj.v[1], v2 = ui.z - uj.v[2];
@@ -1135,11 +1268,10 @@ __device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui,
         lx = group_sum<G>(lx);
         ly = group_sum<G>(ly);
         lz = group_sum<G>(lz);
-        float f = a.fac[i];
         return make_float3(ui.x - f * lx, ui.y - f * ly, ui.z - f * lz);
     }
     float dd = 10.0f;
-    row_pairs_w<FM, 3, G>(win, w, a.R, i, xi, loadA, loadB,
+    row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                          [&](const float4& xj, const Vec<3>& uj, float gx, float gy, float gz) {
                              float x0 = xi.x - xj.x, x1 = xi.y - xj.y, x2 = xi.z - xj.z;
                              float v0 = ui.x - uj.v[0], v1 = ui.y - uj.v[1], v2 = ui.z - uj.v[2];
@@ -1151,7 +1283,6 @@ __device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui,
     lx = group_sum<G>(lx);
     ly = group_sum<G>(ly);
     lz = group_sum<G>(lz);
-    float f = a.fac[i];
     return make_float3(ui.x - f * lx, ui.y - f * ly, ui.z - f * lz);
 }
 
@@ -1165,26 +1296,29 @@ __device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui,
 // from the operator pass on p4 and k_w18_warm_init.  Without the preconditioner the blocks are
 // the identity, so z = P r is r exactly (apply_preconditioner's copy, weiler18.py:279-292).
 template <class FM, bool ALLFLUID, bool WARM = false>
-__global__ __launch_bounds__(BLOCK) void k_w18_setup(W18Args a, float4* __restrict__ p4) {
+__global__ __launch_bounds__(BLOCK, 8) void k_w18_setup(W18Args a, float4* __restrict__ p4) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     auto loadA = [&](int j) { return w18_record<ALLFLUID>(a.R.pos, a.v4, a.mat, a.fluid, j); };
     auto loadB = [&](int j) { return vec3_of(a.v4, j); };
     __shared__ WinLds<FM, PASS_LANES> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.v4[j]; });
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float4 vi = a.v4[ic], xi = a.R.pos[ic];
+    const float f = a.fac[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.v4[j]; });
     double rz = 0.0;
     if (i < a.R.nd) {
-        const float4 vi = a.v4[i];
         const bool fl = ALLFLUID || a.mat[i] == a.fluid;
         float L[9];
 #pragma unroll
         for (int q = 0; q < 9; ++q) L[q] = 0.0f;
         float lx = 0.0f, ly = 0.0f, lz = 0.0f;
         if (fl) {
-            const float4 xi = a.R.pos[i];
             const float eps2 = 0.01f * a.R.h * a.R.h;
             const float dd = 10.0f;
-            row_pairs_w<FM, 3, PASS_LANES>(win, w, a.R, i, xi, loadA, loadB,
+            row_pairs_w<FM, 3, PASS_LANES>(win, w, lp, a.R, i, xi, loadA, loadB,
                 [&](const float4& xj, const Vec<3>& uj, float gx, float gy, float gz) {
                     float x[3] = {xi.x - xj.x, xi.y - xj.y, xi.z - xj.z};
                     float v0 = vi.x - uj.v[0], v1 = vi.y - uj.v[1], v2 = vi.z - uj.v[2];
@@ -1211,7 +1345,6 @@ __global__ __launch_bounds__(BLOCK) void k_w18_setup(W18Args a, float4* __restri
             float P[9];
             float Av0 = vi.x, Av1 = vi.y, Av2 = vi.z;
             if (fl) {
-                const float f = a.fac[i];
                 if (a.precond) {
                     float M[9];
 #pragma unroll
@@ -1317,18 +1450,22 @@ __global__ __launch_bounds__(BLOCK) void k_w18_init(W18Args a, float4* __restric
 // Ap = A p, p.Ap (weiler18.py:337-338).  Without CHECK (the warm-start residual) it runs
 // regardless of the solver state.
 template <class FM, bool ALLFLUID, bool CHECK = true>
-__global__ __launch_bounds__(BLOCK) void k_w18_Av(W18Args a) {
+__global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a) {
     if (CHECK && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     auto loadA = [&](int j) { return w18_Av_record<FM, ALLFLUID>(a, j); };
     auto loadB = [&](int j) { return vec3_of(a.v4, j); };
     __shared__ WinLds<FM, PASS_LANES> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.v4[j]; });
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float4 pi = a.v4[ic], xi = a.R.pos[ic];
+    const float f = a.fac[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.v4[j]; });
     double pap = 0.0;
     if (i < a.R.nd) {
-        float4 pi = a.v4[i];
-        float3 Ap = w18_Av_row<FM, ALLFLUID, PASS_LANES>(a, i, pi, win, w, loadA, loadB, g);
+        float3 Ap = w18_Av_row<FM, ALLFLUID, PASS_LANES>(a, i, pi, xi, f, win, w, lp, loadA, loadB, g);
         if (g == 0) {
             a.out[3 * i + 0] = Ap.x; a.out[3 * i + 1] = Ap.y; a.out[3 * i + 2] = Ap.z;
             pap = (double)(pi.x * Ap.x + pi.y * Ap.y + pi.z * Ap.z);
@@ -1450,7 +1587,7 @@ struct StArgs {
 
 // compute_divergence_jeske23 (jeske23.py:73-112): div_i = sum_fluid m_j (v_i - v_j) . gradW_ij
 template <class FM, bool ALLFLUID>
-__global__ __launch_bounds__(BLOCK) void k_st_div(StArgs a) {
+__global__ __launch_bounds__(BLOCK, 8) void k_st_div(StArgs a) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     auto loadA = [&](int j) {
@@ -1460,15 +1597,18 @@ __global__ __launch_bounds__(BLOCK) void k_st_div(StArgs a) {
     };
     auto loadB = [&](int j) { return vec3_of(a.u4, j); };
     __shared__ WinLds<FM, PASS_LANES> w;
-    const bool win = stage_window(a.R, blk, w, loadA, [&](int j) { return a.u4[j]; });
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float4 ui = a.u4[ic], xi = a.R.pos[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.u4[j]; });
     if (i >= a.R.nd) return;
     if (!ALLFLUID && a.mat[i] != a.fluid) {
         if (g == 0) a.div[i] = 0.0f;
         return;
     }
-    float4 ui = a.u4[i];
     float acc = 0.0f;
-    row_pairs_w<FM, 3, PASS_LANES>(win, w, a.R, i, a.R.pos[i], loadA, loadB,
+    row_pairs_w<FM, 3, PASS_LANES>(win, w, lp, a.R, i, xi, loadA, loadB,
                          [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
                              float vx = ui.x - Bj.v[0], vy = ui.y - Bj.v[1], vz = ui.z - Bj.v[2];
                              acc = acc + Aj.w * (vx * gx + vy * gy + vz * gz);
@@ -1499,22 +1639,27 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
     // the tile window (every thread of the block stages before any row leaves)
     __shared__ StWinLds<FM> w;
     bool win = false;
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float4 xi = a.R.pos[ic], ui = a.u4[ic];
+    const float m_i = ui.w, rho_i = a.density[ic], div_i = a.div[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
     if constexpr (has_windows<FM, PASS_LANES>()) {
-        if (a.R.win_n != nullptr) {
-            const int nw = __builtin_amdgcn_readfirstlane(a.R.win_n[blk]);
-            if (nw >= 0) {
-                const int* wid = a.R.win_ids + (size_t)blk * WIN_MAX;
-                for (int k = threadIdx.x; k < nw; k += BLOCK) {
-                    const int j = wid[k];
-                    const float4 xj = a.R.pos[j];
-                    w.A[k] = make_float4(xj.x, xj.y, xj.z, a.density[j]);
-                    w.B[k] = a.u4[j];
-                    w.C[k] = a.div[j];
-                    w.D[k] = j | ((ALLFLUID || a.mat[j] == a.fluid) ? 0 : (int)0x80000000u);
-                }
-                __syncthreads();
-                win = true;
-            }
+        const int nw = __builtin_amdgcn_readfirstlane(wp.nw);
+        if (a.R.win_n != nullptr && nw >= 0) {
+            auto stage = [&](int k, int j) {
+                const float4 xj = a.R.pos[j];
+                w.A[k] = make_float4(xj.x, xj.y, xj.z, a.density[j]);
+                w.B[k] = a.u4[j];
+                w.C[k] = a.div[j];
+                w.D[k] = j | ((ALLFLUID || a.mat[j] == a.fluid) ? 0 : (int)0x80000000u);
+            };
+            const int k = threadIdx.x;
+            if (k < nw) stage(k, wp.id[0]);
+            if (k + BLOCK < nw) stage(k + BLOCK, wp.id[1]);
+            for (int q = k + 2 * BLOCK; q < nw; q += BLOCK) stage(q, a.R.win_ids[(size_t)blk * WIN_MAX + q]);
+            __syncthreads();
+            win = true;
         }
     }
     if (i >= a.R.nd) return;
@@ -1531,9 +1676,6 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
     // the per-pair g-tilde array has one word per slot in the layout of ids-only rows
     float* eg = a.gt + (size_t)(i >> 6) * (size_t)a.R.Cs * 64u + row_word0<64u>(i & (WAVE - 1));
     const int tl = __builtin_amdgcn_readfirstlane(REC == 64u ? a.R.wave_len[i >> 4] : a.R.tile_len[i >> 6]);
-    const float4 xi = a.R.pos[i];
-    const float4 ui = a.u4[i];
-    const float m_i = ui.w, rho_i = a.density[i], div_i = a.div[i];
     float bx = 0.0f, by = 0.0f, bz = 0.0f, diag = 0.0f;
     // one slot: g~ of the pair (stored by the caller) and the sums; rho_j and div_j are read only
     // for a used pair within h_st
@@ -1578,12 +1720,15 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
             const bool use = (d & 0x7fffffff) != i && d >= 0;
             return pair(A.x, A.y, A.z, w.B[k], use, [&] { return A.w; }, [&] { return w.C[k]; });
         };
-        for (int b = 0; b < tl; b += 8) {
-            const uint32_t q = __builtin_nontemporal_load(l + (b >> 3) * 256);
+        auto block = [&](uint32_t q, int b) {
             const float t0 = from(q & 0xffffu);
             const float t1 = from(q >> 16);
-            g2[(b >> 3) * 256] = f32x2{t0, t1};
-        }
+            g2[b * 256] = f32x2{t0, t1};
+        };
+#pragma unroll
+        for (int k = 0; k < LOC_PF; ++k)
+            if (8 * k < tl) block(lp.q[k], k);
+        for (int b = LOC_PF; 8 * b < tl; ++b) block(__builtin_nontemporal_load(l + b * 256), b);
     } else {
         for (int k = g; k < tl; k += PASS_LANES) {
             const int j = (int)__builtin_nontemporal_load(e + slot_word<REC>(k));
@@ -1613,18 +1758,21 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
 // RHS: out = u - M u + b (jeske23.py:637-647); otherwise out = M u and the block's p.Mp partial.
 // Only the ids and g~ are streamed and (u_j, m_j) gathered: positions are not needed.
 template <class FM, bool ALLFLUID, bool RHS>
-__global__ __launch_bounds__(BLOCK) void k_st_Av(StArgs a) {
+__global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a) {
     if (!RHS && a.st->active == 0) return;
     constexpr unsigned REC = FM::REC;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     // only (u_j, m_j) is read per neighbour: the window's B records
     __shared__ WinLds<FM, PASS_LANES> w;
-    const bool win = stage_window(a.R, blk, w, [](int) { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); },
+    const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
+    const int ic = i < a.R.nd ? i : a.R.nd - 1;
+    const float4 ui = a.u4[ic];
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const bool win = stage_window(a.R, blk, wp, w, [](int) { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); },
                                   [&](int j) { return a.u4[j]; });
     double pap = 0.0;
     if (i < a.R.nd) {
-        const float4 ui = a.u4[i];
         float Mx = ui.x, My = ui.y, Mz = ui.z;
         if (ALLFLUID || a.mat[i] == a.fluid) {
             const uint32_t* e = a.R.nb + (size_t)(i >> 6) * (size_t)a.R.Cs * REC + row_word0<REC>(i & (WAVE - 1));
@@ -1644,13 +1792,19 @@ __global__ __launch_bounds__(BLOCK) void k_st_Av(StArgs a) {
                 typedef float f32x2 __attribute__((ext_vector_type(2)));
                 const uint32_t* l = a.R.loc + ((size_t)(i >> 6) * (size_t)a.R.Cs * 32u + 4u * (i & (WAVE - 1)) + g);
                 const f32x2* g2 = reinterpret_cast<const f32x2*>(eg + 2 * g);
-#pragma unroll((PASS_UNROLL + 1) / 2)
-                for (int b = 0; b < tl; b += 8) {
-                    const uint32_t q = __builtin_nontemporal_load(l + (b >> 3) * 256);
-                    const f32x2 gts = __builtin_nontemporal_load(g2 + (b >> 3) * 256);
-                    visit_u(w.B[q & 0xffffu], gts.x);
-                    visit_u(w.B[q >> 16], gts.y);
-                }
+                // (the next block's g~ in flight while a block is visited)
+                f32x2 gts = {0.0f, 0.0f};
+                if (tl > 0) gts = __builtin_nontemporal_load(g2);
+                auto block = [&](uint32_t q, int b) {
+                    const f32x2 t = gts;
+                    if (8 * (b + 1) < tl) gts = __builtin_nontemporal_load(g2 + (b + 1) * 256);
+                    visit_u(w.B[q & 0xffffu], t.x);
+                    visit_u(w.B[q >> 16], t.y);
+                };
+#pragma unroll
+                for (int k = 0; k < LOC_PF; ++k)
+                    if (8 * k < tl) block(lp.q[k], k);
+                for (int b = LOC_PF; 8 * b < tl; ++b) block(__builtin_nontemporal_load(l + b * 256), b);
             } else if constexpr (REC == 64u && PASS_LANES == 4) {
                 // slots g + 8 b and g + 4 + 8 b: one 8-byte load of ids and one of g-tilde
                 typedef float f32x2 __attribute__((ext_vector_type(2)));
