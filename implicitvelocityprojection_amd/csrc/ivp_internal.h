@@ -61,7 +61,11 @@ struct SolverState {
     int iter;           // CG iterations completed
     int max_iter;
     int active;         // 1 while CG continues
-    int dv_apply;       // Weiler18 / Jeske23: this iteration's dv += alpha p is left to the p pass
+    // Written by an iteration's update pass for its p pass, which advances the state above while its
+    // other blocks still read it: what became of the iteration, and the values it starts from.
+    int ran;            // 0: the solve had stopped, 1: updated, 2: p.Ap ends the solve here
+    int prev_iter, prev_stalls;
+    double prev_rr_old, prev_rr_best;
     int status;         // 0 ok, IVP_NOT_PD
     int n_active_rows;  // rows with dfdt > 0 (per outer iteration)
     int n_touched_rows; // rows whose J^T loop runs (active or with an active neighbour)
@@ -111,6 +115,8 @@ struct SceneParams {
     int max_opt, max_pcg, fixed;
 };
 
+constexpr int PARTIAL_ROWS = 6;   // rows of max_blocks partials
+constexpr int PREFOLD = 64;       // partials per row that k_prefold leaves
 constexpr int MARKS = 256;        // pass times that every context holds (more are allocated when needed)
 constexpr int ROW_PAD = 8;        // tile lengths are padded to a multiple of this many slots
 // slot_word's 8-slot blocks and the paired (g, g + 4) id loads of the pair passes assume both

@@ -1,13 +1,15 @@
-// ivp_reduce.h -- grid reductions: per-block partials plus a one-block finalize kernel that
-// folds them in a fixed order (deterministic) and advances the device-resident solver state.
+// ivp_reduce.h -- grid reductions: per-block partials, folded in a fixed order (deterministic) by a
+// one-block finalize kernel or by every block of the pass that needs the sum, which also advance the
+// device-resident solver state.
 #pragma once
 
 #include "ivp_internal.h"
+#include "ivp_launch.h"
 
 namespace ivp {
 
 // Per-block partial sums of up to 3 doubles (fixed order inside the block).  The grid totals are
-// formed by k_finalize, launched next on the stream: the kernel boundary publishes the partials,
+// formed by a later launch on the stream: the kernel boundary publishes the partials,
 // so no device-scope fence (an L2 write-back on a multi-XCD part) is issued per block.
 template <int NV>
 __device__ __forceinline__ void block_partials(const double (&v)[NV], double* partials, int stride) {
@@ -20,7 +22,7 @@ __device__ __forceinline__ void block_partials(const double (&v)[NV], double* pa
 }
 
 enum FinOp {
-    FIN_BUILD, FIN_PACK, FIN_RHS, FIN_CG_INIT, FIN_CG_PAP, FIN_CG_UPDATE, FIN_W18_INIT, FIN_W18_PAP, FIN_W18_UPDATE,
+    FIN_BUILD, FIN_PACK, FIN_RHS, FIN_FIRST, FIN_CG_PAP, FIN_CG_UPDATE, FIN_W18_INIT, FIN_W18_PAP, FIN_W18_UPDATE,
     FIN_CG_REPLACE
 };
 
@@ -52,7 +54,7 @@ constexpr int FIN_UNROLL = 4;  // the fold below adds exactly four loads per row
 // memory latencies instead of one per loop trip.
 template <int NV>
 __device__ __forceinline__ void fold_partials(const double* __restrict__ partials, int stride, int n,
-                                              double (&t)[3]) {
+                                              double* t) {
     __shared__ double lds[NV][FIN_BLOCK / WAVE];
     double s[NV];
 #pragma unroll
@@ -89,7 +91,7 @@ __device__ __forceinline__ void fold_partials(const double* __restrict__ partial
 // Scalar state update after a reduction (the host logic of ip.py:296-327,
 // pressure_base.py:405-423, weiler18.py:330-365), applied to one solver state.
 template <int OP>
-__device__ __forceinline__ void fin_apply(SolverState* st, const double (&t)[3], double tol, int max_iter) {
+__device__ __forceinline__ void fin_apply(SolverState* st, const double* t, double tol, int max_iter) {
     if (OP == FIN_BUILD) {
         st->total_pairs = (long long)t[0];
         st->win_entries = (long long)t[1];
@@ -97,24 +99,29 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double (&t)[3],
         st->err_sum = t[0];
         st->n_active_rows = (int)t[1];
         st->active_pairs = (long long)t[2];
-    } else if (OP == FIN_RHS) {
-        st->n_touched_rows = (int)t[0];
-        st->touched_pairs = (long long)t[1];
-    } else if (OP == FIN_CG_INIT || OP == FIN_W18_INIT) {
+    } else if (OP == FIN_FIRST) {   // the constraint pass's sums, then the right-hand side's
+        fin_apply<FIN_PACK>(st, t, tol, max_iter);
+        fin_apply<FIN_RHS>(st, t + 3, tol, max_iter);
+    } else if (OP == FIN_RHS || OP == FIN_W18_INIT) {
+        double rr = t[0];
+        if (OP == FIN_RHS) {
+            st->n_touched_rows = (int)t[0];
+            st->touched_pairs = (long long)t[1];
+            rr = t[2];
+        }
         // IP: CG runs when r.r > 1e-30 (ip.py:302); Weiler18: when r.z > 1e-12 (weiler18.py:337)
-        double floor_ = OP == FIN_CG_INIT ? 1e-30 : 1e-12;
-        st->rr_old = t[0];
-        st->rr_new = t[0];
-        st->rr_last = t[0];
-        st->rr0 = t[0];
-        st->rr_best = t[0];
+        double floor_ = OP == FIN_RHS ? 1e-30 : 1e-12;
+        st->rr_old = rr;
+        st->rr_new = rr;
+        st->rr_last = rr;
+        st->rr0 = rr;
+        st->rr_best = rr;
         st->stalls = 0;
         st->tol = tol;
         st->max_iter = max_iter;
         st->iter = 0;
         st->status = 0;
-        st->dv_apply = 0;
-        st->active = (t[0] > floor_ && max_iter > 0) ? 1 : 0;
+        st->active = (rr > floor_ && max_iter > 0) ? 1 : 0;
     } else if (OP == FIN_CG_PAP) {
         // ip.py:307-311
         st->pAp = t[0];
@@ -123,14 +130,6 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double (&t)[3],
             st->active = 0;
         } else {
             st->alpha = st->rr_old / (t[0] > 1e-30 ? t[0] : 1e-30);
-        }
-    } else if (OP == FIN_W18_PAP) {
-        // weiler18.py:338-342: pAp <= 0 ends the iteration
-        st->pAp = t[0];
-        if (t[0] <= 0.0) {
-            st->active = 0;
-        } else {
-            st->alpha = st->rr_old / (t[0] > 1e-12 ? t[0] : 1e-12);
         }
     } else if (OP == FIN_CG_UPDATE) {
         // ip.py:317-327
@@ -171,9 +170,7 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double (&t)[3],
             st->rr_old = t[1];
         }
     } else if (OP == FIN_W18_UPDATE) {
-        // weiler18.py:350-365 (t[0] = r.r, t[1] = r.z); the iteration's dv += alpha p follows in
-        // the p pass, also when this iteration ends the solve
-        st->dv_apply = 1;
+        // weiler18.py:350-365 (t[0] = r.r, t[1] = r.z)
         int it = st->iter + 1;
         st->iter = it;
         st->rr_last = t[0];
@@ -190,7 +187,8 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double (&t)[3],
 
 template <int OP>
 constexpr int fin_nv() {
-    return OP == FIN_PACK ? 3 : (OP == FIN_BUILD || OP == FIN_RHS || OP == FIN_W18_UPDATE || OP == FIN_CG_REPLACE) ? 2 : 1;
+    return OP == FIN_FIRST ? 6 : OP == FIN_PACK || OP == FIN_RHS ? 3
+           : OP == FIN_BUILD || OP == FIN_W18_UPDATE || OP == FIN_CG_REPLACE ? 2 : 1;
 }
 
 // One block: fold the partials of the previous kernel in a fixed order and advance the solver
@@ -199,14 +197,9 @@ template <int OP>
 __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
     constexpr int NV = fin_nv<OP>();
     SolverState* st = a.st;
-    // the p pass before this one applied the last iteration's dv update, if any (iterations
-    // enqueued past the stop must not apply it again)
-    if (OP == FIN_W18_PAP && threadIdx.x == 0) st->dv_apply = 0;
-    const bool skip = (OP == FIN_PACK && a.gated && (st->active != 0 || st->status != 0)) ||
-                      ((OP == FIN_CG_PAP || OP == FIN_CG_UPDATE || OP == FIN_W18_PAP || OP == FIN_W18_UPDATE ||
-                        OP == FIN_CG_REPLACE) && st->active == 0);
+    const bool skip = OP == FIN_PACK && a.gated && (st->active != 0 || st->status != 0);
     if (!skip) {
-        double t[3] = {0.0, 0.0, 0.0};
+        double t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         fold_partials<NV>(a.partials, a.stride, a.nblocks, t);
         if (threadIdx.x == 0) {
             fin_apply<OP>(st, t, a.tol, a.max_iter);
@@ -216,11 +209,169 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
     if (a.host && threadIdx.x == 0) report_state(st, a.host, a.flags);
 }
 
+// ---- folds by the pass that needs the sum ---------------------------------------------------
+//
+// A finalize launch between two passes costs 2 us and the gap before it for a few scalars.  With at
+// most FOLD_MAX partials (16 KB, in L2) every block of the next pass folds them itself, all to the
+// same bits, and one block writes the state; above it a block's fold takes as long as the launch
+// that it saves, and k_prefold first reduces each row to PREFOLD partials in one short launch of
+// many blocks (15 625 partials: 2.4 us; the one-block finalize took 4.6, with two rows 7.9, with three
+// 9.1: the bandwidth of one CU).
+constexpr int FOLD_MAX = 2048;
+
+template <int NV>
+__device__ __forceinline__ void block_fold(const double* __restrict__ p, int stride, int n, double (&t)[NV]) {
+    __shared__ double lds[NV][WAVES_PER_BLOCK];
+    double s[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) s[q] = 0.0;
+    for (int base = 0; base < n; base += 4 * BLOCK) {
+        double v[NV][4];
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = base + u * BLOCK + (int)threadIdx.x;
+                v[q][u] = k < n ? p[(size_t)q * stride + k] : 0.0;
+            }
+#pragma unroll
+        for (int q = 0; q < NV; ++q) s[q] += (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
+    }
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const double x = wave_sum(s[q]);
+        if ((threadIdx.x & (WAVE - 1)) == 0) lds[q][threadIdx.x >> 6] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; ++q) t[q] = (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]);
+}
+
+// Row q of n partials to PREFOLD partials: block b folds the b-th share
+template <int NV>
+__global__ __launch_bounds__(BLOCK) void k_prefold(const double* __restrict__ p, int stride, int n,
+                                                   double* __restrict__ out, const SolverState* __restrict__ gate) {
+    if (gate && gate->active == 0) return;
+    const int per = (n + PREFOLD - 1) / PREFOLD;
+    const int k0 = (int)blockIdx.x * per < n ? (int)blockIdx.x * per : n;
+    double t[NV];
+    block_fold<NV>(p + k0, stride, k0 + per < n ? per : n - k0, t);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) out[q * PREFOLD + (int)blockIdx.x] = t[q];
+}
+
+// Partials to fold: rows `stride` apart, n per row
+struct Fold {
+    const double* p;
+    int stride, n;
+};
+
+// The partials in rows row0 .. row0 + NV - 1, brought down to PREFOLD per row if there are many (gate:
+// skipped once that solve has stopped)
+template <int NV>
+inline int fold_source(ivp_ctx* c, int row0, int n, const SolverState* gate, Fold* f) {
+    const double* p = c->partials + (size_t)row0 * c->max_blocks;
+    *f = Fold{p, c->max_blocks, n};
+    if (n <= FOLD_MAX) return IVP_OK;
+    double* out = c->partials + (size_t)PARTIAL_ROWS * c->max_blocks + row0 * PREFOLD;
+    hipLaunchKernelGGL(k_prefold<NV>, dim3(PREFOLD), dim3(BLOCK), 0, c->stream, p, c->max_blocks, n, out, gate);
+    IVP_HIP(hipGetLastError());
+    *f = Fold{out, PREFOLD, PREFOLD};
+    return IVP_OK;
+}
+
+// In an iteration's update pass: alpha from the operator pass's p.Ap (OP = FIN_CG_PAP, FIN_W18_PAP).
+// Returns false when there is nothing to update.  The state's own fields stay as they are until
+// the p pass; ran and prev_* tell it what happened here.
+template <int OP>
+__device__ __forceinline__ bool fold_alpha(SolverState* st, const Fold& f, float* alpha) {
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    if (st->active == 0) {
+        if (lead) st->ran = 0;
+        return false;
+    }
+    double t[1];
+    block_fold<1>(f.p, f.stride, f.n, t);
+    // ip.py:307-311 fails on p.Ap < 0; weiler18.py:338-342 ends the iteration on p.Ap <= 0
+    const double least = OP == FIN_CG_PAP ? 1e-30 : 1e-12;
+    const bool bad = OP == FIN_CG_PAP ? t[0] < 0.0 : t[0] <= 0.0;
+    const double al = st->rr_old / (t[0] > least ? t[0] : least);
+    *alpha = (float)al;
+    if (lead) {
+        st->pAp = t[0];
+        st->ran = bad ? 2 : 1;
+        if (!bad) {
+            st->alpha = al;
+            st->prev_iter = st->iter;
+            st->prev_rr_old = st->rr_old;
+            st->prev_rr_best = st->rr_best;
+            st->prev_stalls = st->stalls;
+        }
+    }
+    return !bad;
+}
+
+struct Advance {
+    bool ran;        // the iteration updated x and r
+    bool active;     // and the solve goes on
+    bool stopped;    // no further iteration, and not because p.Ap failed
+    float beta;
+};
+
+// In the iteration's p pass: the state after the iteration from the update pass's sums (OP =
+// FIN_CG_UPDATE, FIN_CG_REPLACE, FIN_W18_UPDATE), formed by every block and written by one, which
+// reports it to the host if asked.
+template <int OP>
+__device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, SolverState* host, const int* flags) {
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int ran = st->ran;
+    Advance a = {ran == 1, false, ran == 0 && st->status == 0, 0.0f};
+    if (ran == 1) {
+        double t[fin_nv<OP>()];
+        block_fold<fin_nv<OP>()>(f.p, f.stride, f.n, t);
+        SolverState s;
+        s.iter = st->prev_iter;
+        s.rr_old = st->prev_rr_old;
+        s.rr_best = st->prev_rr_best;
+        s.stalls = st->prev_stalls;
+        s.tol = st->tol;
+        s.max_iter = st->max_iter;
+        s.active = 1;
+        s.beta = 0.0;
+        s.rr_new = 0.0;
+        fin_apply<OP>(&s, t, 0.0, 0);
+        a.active = s.active != 0;
+        a.stopped = !a.active;
+        a.beta = (float)s.beta;
+        if (lead) {
+            st->iter = s.iter;
+            st->rr_old = s.rr_old;
+            if (OP != FIN_W18_UPDATE) st->rr_new = s.rr_new;
+            st->rr_last = s.rr_last;
+            st->rr_best = s.rr_best;
+            st->stalls = s.stalls;
+            if (a.active) st->beta = s.beta;
+            st->active = s.active;
+        }
+    } else if (ran == 2) {
+        if (OP == FIN_W18_UPDATE) a.stopped = true;
+        if (lead) {
+            if (OP != FIN_W18_UPDATE) st->status = IVP_NOT_PD;
+            st->active = 0;
+        }
+    }
+    if (lead && host) report_state(st, host, flags);
+    return a;
+}
 
 template <int OP>
 inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0, bool gated = false,
                     SolverState* host = nullptr, unsigned long long* mark = nullptr) {
-    FinArgs fa{c->partials, c->max_blocks, nblocks, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
+    constexpr int NV = fin_nv<OP>();
+    Fold f{c->partials + (OP == FIN_RHS ? 3 : 0) * (size_t)c->max_blocks, c->max_blocks, nblocks};
+    if (NV > 1) IVP_TRY((fold_source<NV>(c, OP == FIN_RHS ? 3 : 0, nblocks, nullptr, &f)));
+    FinArgs fa{f.p, f.stride, f.n, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
     hipLaunchKernelGGL(k_finalize<OP>, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
     IVP_HIP(hipGetLastError());
     return IVP_OK;
@@ -271,7 +422,7 @@ struct FinScenesArgs {
 template <int OP>
 __global__ __launch_bounds__(BLOCK) void k_fin_scenes(FinScenesArgs a) {
     constexpr int NV = fin_nv<OP>();
-    constexpr int want = OP == FIN_PACK ? PH_PACK : (OP == FIN_RHS || OP == FIN_CG_INIT) ? PH_RHS : PH_CG;
+    constexpr int want = OP == FIN_PACK ? PH_PACK : OP == FIN_RHS ? PH_RHS : PH_CG;
     const int s = blockIdx.x * WAVES_PER_BLOCK + (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & (WAVE - 1);
     if (s >= a.S) return;
@@ -305,8 +456,6 @@ __global__ __launch_bounds__(BLOCK) void k_fin_scenes(FinScenesArgs a) {
             sc->phase = PH_RHS;
         }
     } else if (OP == FIN_RHS) {
-        fin_apply<OP>(&sc->cg, t, 0.0, 0);
-    } else if (OP == FIN_CG_INIT) {
         fin_apply<OP>(&sc->cg, t, p.tol_pcg, p.max_pcg);
         if (sc->cg.active) {
             sc->phase = PH_CG;

@@ -515,7 +515,11 @@ struct RhsArgs {
     const float4* q4;
     const float* Ss;
     float omega;
-    float* b;
+    float* b;        // kept only for residual replacements (nullptr: not)
+    float* sol;
+    float* r;
+    float4* p4;
+    float2* y2;
     int* nbact;
     const int* rowcnt;
     double* partials;
@@ -524,7 +528,9 @@ struct RhsArgs {
 };
 
 // ip_rhs_fused (ip.py:174-215): b = omega J^T (f k); also marks rows whose CG J^T loop can be
-// non-zero (own dfdt > 0 or a dynamic neighbour with dfdt > 0).
+// non-zero (own dfdt > 0 or a dynamic neighbour with dfdt > 0).  The CG prologue (ip.py:292-304:
+// x = 0, r = b, rr = r.r, p = r) is part of the pass; as a launch of its own with its own finalize
+// it took 18 us at 1M rows and 5 at 8k.
 template <class FM, bool SC, int G = lanes_for<SC>()>
 __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -562,7 +568,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
     }
     const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.q4[j]; });
-    double touched = 0.0, tpairs = 0.0;
+    double touched = 0.0, tpairs = 0.0, rr = 0.0;
     if (gt.on) {
         if (SC) own();
         float fki = qi.x, mi = qi.z;
@@ -583,9 +589,15 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
             rx += fki * s0;
             ry += fki * s1;
             rz += fki * s2;
-            a.b[3 * i + 0] = a.omega * rx;
-            a.b[3 * i + 1] = a.omega * ry;
-            a.b[3 * i + 2] = a.omega * rz;
+            const float bx = a.omega * rx, by = a.omega * ry, bz = a.omega * rz;
+            if (a.b) {
+                a.b[3 * i + 0] = bx; a.b[3 * i + 1] = by; a.b[3 * i + 2] = bz;
+            }
+            a.sol[3 * i + 0] = 0.0f; a.sol[3 * i + 1] = 0.0f; a.sol[3 * i + 2] = 0.0f;
+            a.r[3 * i + 0] = bx; a.r[3 * i + 1] = by; a.r[3 * i + 2] = bz;
+            a.p4[i] = make_float4(bx, by, bz, qi.z);
+            a.y2[i] = make_float2(0.0f, qi.z);
+            rr = (double)(bx * bx + by * by + bz * bz);
             a.nbact[i] = act ? 1 : 0;
             if (act) {
                 touched = 1.0;
@@ -593,42 +605,8 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
             }
         }
     }
-    double v[2] = {touched, tpairs};
-    row_partials<SC, 2>(v, gt, a.partials, a.stride, blk);
-}
-
-struct CGInitArgs {
-    int nd;
-    const float* b;
-    const float4* pos;
-    float* sol;
-    float* r;
-    float4* p4;
-    float2* y2;
-    double* partials;
-    int stride;
-    SceneRef sc;
-};
-
-// IP.PCG prologue (ip.py:292-304): x = 0, r = b, rr = r.r, p = r
-template <bool SC>
-__global__ __launch_bounds__(BLOCK) void k_cg_init(CGInitArgs a) {
-    const int blk = blockIdx.x;
-    int i = blk * BLOCK + threadIdx.x;
-    Gate gt = gate_all(i, a.nd);
-    if (SC && !gate_block(a.sc, blk, i, a.nd, PH_RHS, gt)) return;
-    double rr = 0.0;
-    if (gt.on) {
-        float bx = a.b[3 * i + 0], by = a.b[3 * i + 1], bz = a.b[3 * i + 2];
-        float m = a.pos[i].w;
-        a.sol[3 * i + 0] = 0.0f; a.sol[3 * i + 1] = 0.0f; a.sol[3 * i + 2] = 0.0f;
-        a.r[3 * i + 0] = bx; a.r[3 * i + 1] = by; a.r[3 * i + 2] = bz;
-        a.p4[i] = make_float4(bx, by, bz, m);
-        a.y2[i] = make_float2(0.0f, m);
-        rr = (double)(bx * bx + by * by + bz * bz);
-    }
-    double v[1] = {rr};
-    row_partials<SC, 1>(v, gt, a.partials, a.stride, blk);
+    double v[3] = {touched, tpairs, rr};
+    row_partials<SC, 3>(v, gt, a.partials, a.stride, blk);
 }
 
 struct CGJArgs {
@@ -790,19 +768,21 @@ struct CGUpdArgs {
     const float* Ap;
     double* partials;
     int stride;
-    const SolverState* st;
+    SolverState* st;
     SceneRef sc;
+    Fold pap;        // one scene: the operator pass's p.Ap
 };
 
 // pcg_update_x_r_scalar (math_utils.py:180-195) + r.r (ip.py:314-317)
 template <bool SC>
 __global__ __launch_bounds__(BLOCK) void k_cg_update(CGUpdArgs a) {
-    if (!SC && a.st->active == 0) return;
+    float alpha = 0.0f;
+    if (!SC && !fold_alpha<FIN_CG_PAP>(a.st, a.pap, &alpha)) return;
     const int blk = blockIdx.x;
     int i = blk * BLOCK + threadIdx.x;
     Gate gt = gate_all(i, a.nd);
     if (SC && !gate_block(a.sc, blk, i, a.nd, PH_CG, gt)) return;
-    float alpha = (float)(SC ? a.sc.ss[gt.s].cg.alpha : a.st->alpha);
+    if (SC) alpha = (float)a.sc.ss[gt.s].cg.alpha;
     double rr = 0.0;
     if (gt.on) {
         float4 p = a.p4[i];
@@ -820,22 +800,55 @@ __global__ __launch_bounds__(BLOCK) void k_cg_update(CGUpdArgs a) {
     row_partials<SC, 1>(v, gt, a.partials, a.stride, blk);
 }
 
-// p = r + beta p (add_vec3, ip.py:323-326)
-template <bool SC>
-__global__ __launch_bounds__(BLOCK) void k_cg_p(int nd, const float* __restrict__ r, float4* __restrict__ p4,
-                                                const SolverState* __restrict__ st, SceneRef sc) {
-    if (!SC && st->active == 0) return;
+// p = r + beta p of independent scenes (add_vec3, ip.py:323-326)
+__global__ __launch_bounds__(BLOCK) void k_cg_p_scenes(int nd, const float* __restrict__ r, float4* __restrict__ p4,
+                                                       SceneRef sc) {
     const int blk = blockIdx.x;
     int i = blk * BLOCK + threadIdx.x;
     Gate gt = gate_all(i, nd);
-    if (SC && !gate_block(sc, blk, i, nd, PH_CG, gt)) return;
+    if (!gate_block(sc, blk, i, nd, PH_CG, gt)) return;
     if (!gt.on) return;
-    float beta = (float)(SC ? sc.ss[gt.s].cg.beta : st->beta);
+    float beta = (float)sc.ss[gt.s].cg.beta;
     float4 p = p4[i];
     p.x = r[3 * i + 0] + beta * p.x;
     p.y = r[3 * i + 1] + beta * p.y;
     p.z = r[3 * i + 2] + beta * p.z;
     p4[i] = p;
+}
+
+struct CGPArgs {
+    int nd;
+    const float* r;
+    float4* p4;
+    const float* sol;
+    float4* d4;
+    SolverState* st;
+    Fold rr;             // the update pass's r.r (and the replaced residual's)
+    SolverState* host;   // the last iteration of a chunk: the state is reported here
+    const int* flags;
+};
+
+// The end of a CG iteration (OP = FIN_CG_UPDATE or FIN_CG_REPLACE): the stop test, then
+// p = r + beta p (add_vec3, ip.py:323-326) while the solve goes on; in the last iteration of a chunk a
+// solve that has stopped without failing moves d -= x instead (add_vec3 with scale -1, ip.py:389).
+template <int OP>
+__global__ __launch_bounds__(BLOCK) void k_cg_p(CGPArgs a) {
+    const Advance v = fold_advance<OP>(a.st, a.rr, a.host, a.flags);
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= a.nd) return;
+    if (v.active) {
+        float4 p = a.p4[i];
+        p.x = a.r[3 * i + 0] + v.beta * p.x;
+        p.y = a.r[3 * i + 1] + v.beta * p.y;
+        p.z = a.r[3 * i + 2] + v.beta * p.z;
+        a.p4[i] = p;
+    } else if (a.host && v.stopped) {
+        float4 d = a.d4[i];
+        d.x = d.x + -1.0f * a.sol[3 * i + 0];
+        d.y = d.y + -1.0f * a.sol[3 * i + 1];
+        d.z = d.z + -1.0f * a.sol[3 * i + 2];
+        a.d4[i] = d;
+    }
 }
 
 // (x, m) of the CG iterate, the input of the true-residual passes
@@ -866,7 +879,7 @@ __global__ __launch_bounds__(BLOCK) void k_cg_refresh(int nd, const float* __res
     block_partials<1>(v, partials, stride);
 }
 
-// d -= sol (add_vec3 with scale -1, ip.py:389)
+// d -= sol (add_vec3 with scale -1, ip.py:389): independent scenes, and a solve that is allowed no iteration
 template <bool SC>
 __global__ __launch_bounds__(BLOCK) void k_ip_dupdate(int nd, float4* __restrict__ d4, const float* __restrict__ sol,
                                                       SceneRef sc, const SolverState* __restrict__ gate) {
@@ -1226,10 +1239,11 @@ struct W18Args {
     float* dv; float* r; float* z;
     double* partials;
     int stride;
-    const SolverState* st;
+    SolverState* st;
     int precond;            // use_preconditioner: block-Jacobi blocks, else identity (plain CG)
     const int* uid;         // user index of each internal row
     const float* dv_prev;   // the last solve's correction in user order (warm starts)
+    Fold pap{};             // the operator pass's p.Ap (update pass)
 };
 
 // The operator pass's neighbour record: w18_record, with w = -10 ks V_j when the gradients are
@@ -1478,8 +1492,9 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a) {
 // r -= alpha Ap, r.r, z = P r, r.z (weiler18.py:344-360); dv += alpha p of the same lines
 // follows in the p pass, which reads p anyway
 __global__ __launch_bounds__(BLOCK) void k_w18_update(W18Args a) {
-    if (a.st->active == 0) return;
-    float nalpha = (float)(-a.st->alpha);
+    float alpha;
+    if (!fold_alpha<FIN_W18_PAP>(a.st, a.pap, &alpha)) return;
+    const float nalpha = -alpha;
     int i = blockIdx.x * BLOCK + threadIdx.x;
     double rr = 0.0, rz = 0.0;
     if (i < a.R.nd) {
@@ -1499,38 +1514,47 @@ __global__ __launch_bounds__(BLOCK) void k_w18_update(W18Args a) {
     block_partials<2>(v, a.partials, a.stride);
 }
 
-// dv += alpha p (the iteration's update, weiler18.py:344-346), then p = z + beta p while the
-// solve continues
-__global__ __launch_bounds__(BLOCK) void k_w18_p(int nd, const float* __restrict__ z, float4* __restrict__ p4,
-                                                 float* __restrict__ dv, const SolverState* __restrict__ st) {
-    const int apply = st->dv_apply, active = st->active;
-    if (apply == 0 && active == 0) return;
-    float alpha = (float)st->alpha;
-    float beta = (float)st->beta;
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    float4 p = p4[i];
-    if (apply) {
-        dv[3 * i + 0] = dv[3 * i + 0] + alpha * p.x;
-        dv[3 * i + 1] = dv[3 * i + 1] + alpha * p.y;
-        dv[3 * i + 2] = dv[3 * i + 2] + alpha * p.z;
-    }
-    if (active) {
-        p.x = z[3 * i + 0] + beta * p.x;
-        p.y = z[3 * i + 1] + beta * p.y;
-        p.z = z[3 * i + 2] + beta * p.z;
-        p4[i] = p;
-    }
-}
+struct W18PArgs {
+    int nd;
+    const float* z;
+    float4* p4;
+    float* dv;
+    float* vel;
+    SolverState* st;
+    Fold sums;           // the update pass's r.r and r.z
+    SolverState* host;   // the last iteration of a chunk: the state is reported here
+    const int* flags;
+};
 
-// v += dv (weiler18.py:399-401), once the solve has stopped; rows that the last build truncated
-// leave v as it was (the host refuses them when it reads the flags)
-__global__ __launch_bounds__(BLOCK) void k_w18_apply(int n3, const float* __restrict__ dv, float* __restrict__ vel,
-                                                     const SolverState* __restrict__ st, const int* __restrict__ flags) {
-    if (st->active != 0 || (*flags & 5)) return;
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n3) return;
-    vel[i] = vel[i] + 1.0f * dv[i];
+// The end of an iteration: the stop test, dv += alpha p (the iteration's update,
+// weiler18.py:344-346, also of the iteration that ends the solve), then p = z + beta p while the solve
+// goes on.  In the last iteration of a chunk a solve that has stopped also adds v += dv
+// (weiler18.py:399-401), except on rows that the last build truncated (the host refuses them when it
+// reads the flags).
+__global__ __launch_bounds__(BLOCK) void k_w18_p(W18PArgs a) {
+    const Advance v = fold_advance<FIN_W18_UPDATE>(a.st, a.sums, a.host, a.flags);
+    const bool apply = a.host && v.stopped && !(*a.flags & 5);
+    if (!v.ran && !apply) return;
+    const float alpha = (float)a.st->alpha;
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= a.nd) return;
+    float dv[3] = {a.dv[3 * i + 0], a.dv[3 * i + 1], a.dv[3 * i + 2]};
+    if (v.ran) {
+        float4 p = a.p4[i];
+        dv[0] = dv[0] + alpha * p.x;
+        dv[1] = dv[1] + alpha * p.y;
+        dv[2] = dv[2] + alpha * p.z;
+        a.dv[3 * i + 0] = dv[0]; a.dv[3 * i + 1] = dv[1]; a.dv[3 * i + 2] = dv[2];
+        if (v.active) {
+            p.x = a.z[3 * i + 0] + v.beta * p.x;
+            p.y = a.z[3 * i + 1] + v.beta * p.y;
+            p.z = a.z[3 * i + 2] + v.beta * p.z;
+            a.p4[i] = p;
+        }
+    }
+    if (apply)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a.vel[3 * i + q] = a.vel[3 * i + q] + 1.0f * dv[q];
 }
 
 // ---- Jeske23 implicit surface tension (jeske23.py) -----------------------------------------
@@ -1932,23 +1956,19 @@ int enqueue_scene_replay_g(ivp_ctx* c, hipStream_t st, float omega, int K) {
     PackArgs pa{R, c->d4, c->Ss, c->cc, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, P, stride, sc};
     hipLaunchKernelGGL((k_ip_pack<FmtIds, true, G>), np, blk, 0, st, pa);
     hipLaunchKernelGGL(k_fin_scenes<FIN_PACK>, nf, blk, 0, st, fp);
-    RhsArgs ra{R, c->q4, c->Ss, omega, c->b, c->nbact, c->rowcnt, P, stride, sc};
+    RhsArgs ra{R, c->q4, c->Ss, omega, nullptr, c->sol, c->r, c->p4, c->y2, c->nbact, c->rowcnt, P, stride, sc};
     hipLaunchKernelGGL((k_ip_rhs<FmtIds, true, G>), np, blk, 0, st, ra);
     hipLaunchKernelGGL(k_fin_scenes<FIN_RHS>, nf, blk, 0, st, fp);
-    CGInitArgs ia{nd, c->b, c->pos, c->sol, c->r, c->p4, c->y2, P, stride, sc};
-    hipLaunchKernelGGL(k_cg_init<true>, nb, blk, 0, st, ia);
-    hipLaunchKernelGGL(k_fin_scenes<FIN_CG_INIT>, nf, blk, 0, st, fa);
     CGJArgs ja{R, c->p4, c->Ss, c->sfac, c->y2, c->state, sc};
     CGJTArgs ta{R, c->p4, c->y2, c->Ss, c->nbact, omega, c->Ap, P, stride, c->state, sc};
-    CGUpdArgs ua{nd, c->sol, c->r, c->p4, c->Ap, P, stride, c->state, sc};
+    CGUpdArgs ua{nd, c->sol, c->r, c->p4, c->Ap, P, stride, c->state, sc, Fold{}};
     for (int k = 0; k < K; ++k) {
         hipLaunchKernelGGL((k_cg_J<FmtIds, true, G>), np, blk, 0, st, ja);
         hipLaunchKernelGGL((k_cg_JT<FmtIds, true, G>), np, blk, 0, st, ta);
         hipLaunchKernelGGL(k_fin_scenes<FIN_CG_PAP>, nf, blk, 0, st, fp);
         hipLaunchKernelGGL(k_cg_update<true>, nb, blk, 0, st, ua);
         hipLaunchKernelGGL(k_fin_scenes<FIN_CG_UPDATE>, nf, blk, 0, st, fa);
-        hipLaunchKernelGGL(k_cg_p<true>, nb, blk, 0, st, nd, (const float*)c->r, c->p4,
-                           (const SolverState*)c->state, sc);
+        hipLaunchKernelGGL(k_cg_p_scenes, nb, blk, 0, st, nd, (const float*)c->r, c->p4, sc);
     }
     hipLaunchKernelGGL(k_ip_dupdate<true>, nb, blk, 0, st, nd, c->d4, (const float*)c->sol, sc,
                        (const SolverState*)nullptr);
@@ -2008,9 +2028,10 @@ __global__ void k_report(SolverState* st, SolverState* host, const int* flags) {
 
 // Enqueue CG iterations in chunks until the device-side state says stop.  `launch_it(tag, host)`
 // enqueues one iteration; the last one of a chunk reports the state to `host`.  After each chunk
-// `tail` is enqueued (work that follows a finished solve and returns at once while it continues),
-// then the host waits for the report alone: the device runs the tail while the host takes the
-// state.  The tail has run on a finished solve when the reported state is inactive.
+// `tail(none)` is enqueued (work that follows a finished solve and returns at once while it continues;
+// `none` when there was no iteration), then the host waits for the report alone: the device runs the
+// tail while the host takes the state.  The tail has run on a finished solve when the reported state
+// is inactive.
 template <class L, class T>
 int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, int* chunks, T&& tail) {
     int issued = 0;
@@ -2028,7 +2049,7 @@ int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, i
         for (int q = 0; q < todo; ++q) IVP_TRY(launch_it(issued + q, q == todo - 1 ? c->state_host : nullptr));
         issued += todo;
         IVP_HIP(hipEventRecord(c->wait_ev, c->stream));
-        IVP_TRY(tail());
+        IVP_TRY(tail(todo == 0));
         IVP_HIP(hipEventSynchronize(c->wait_ev));
         (*chunks)++;
         const SolverState& s = *c->state_host;
@@ -2085,12 +2106,14 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
         IVP_TRY(marks_buffer(c, opt_iter + 2));
         PackArgs pa{R, d4, c->Ss, c->cc, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, c->partials, stride};
         double total_pairs = (double)c->state_host->total_pairs;
+        const bool deferred = opt_iter == 0 && prm->max_iteration_opt >= 1;
         // the constraint pass of evaluation k and its finalize, which reports the state
         auto queue_pack = [&](int k, const SolverState* gate) -> int {
             PackArgs pg = pa;
             pg.gate = gate;
             pg.mark = c->marks + k;
             IVP_TRY(launch(c, KC_IP_PACK, -1, stream_bytes<FP>(c, total_pairs) + 68.0 * nd, k_ip_pack<FP, false>, np, pg));
+            if (k == 0 && deferred) return IVP_OK;   // its sums are folded with the right-hand side's
             return finalize<FIN_PACK>(c, np.x, 0.0, 0, gate != nullptr, c->state_host + 1, c->marks + k + 1);
         };
         if (!pack_queued) IVP_TRY(queue_pack(opt_iter, nullptr));
@@ -2107,7 +2130,6 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             st.n_density_errors++;
             return IVP_OK;
         };
-        const bool deferred = opt_iter == 0 && prm->max_iteration_opt >= 1;
         long long act_pairs = c->state_host->active_pairs;   // (deferred: the last evaluation's, for
         int act_rows = c->state_host->n_active_rows;         //  the byte model until read back)
         if (!deferred) {
@@ -2131,12 +2153,13 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             act_rows = c->state_host->n_active_rows;
         }
 
-        RhsArgs ra{R, c->q4, c->Ss, prm->omega, c->b, c->nbact, c->rowcnt, c->partials, stride};
+        RhsArgs ra{R, c->q4, c->Ss, prm->omega, FC::GS == GS_F16 ? c->b : nullptr, c->sol, c->r, c->p4, c->y2, c->nbact,
+                   c->rowcnt, c->partials + 3 * (size_t)stride, stride};
         IVP_TRY(launch(c, KC_IP_RHS, -1, stream_bytes<FP>(c, total_pairs) + 48.0 * nd, k_ip_rhs<FP, false>, np, ra));
-        IVP_TRY(finalize<FIN_RHS>(c, np.x));
-        CGInitArgs ia{nd, c->b, c->pos, c->sol, c->r, c->p4, c->y2, c->partials, stride};
-        IVP_TRY(launch(c, -1, -1, 0.0, k_cg_init<false>, nb, ia));
-        IVP_TRY(finalize<FIN_CG_INIT>(c, nb.x, prm->tol_pcg, prm->max_iteration_pcg));
+        if (deferred)
+            IVP_TRY(finalize<FIN_FIRST>(c, np.x, prm->tol_pcg, prm->max_iteration_pcg, false, nullptr, c->marks + 1));
+        else
+            IVP_TRY(finalize<FIN_RHS>(c, np.x, prm->tol_pcg, prm->max_iteration_pcg));
         // The first CG chunk is enqueued without waiting for the set-up: its kernels return at once
         // when there is nothing to solve.  The J^T byte model (touched rows, reported by the set-up)
         // is attached to the launches once the first chunk's state has been read.
@@ -2155,45 +2178,48 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             double bP = (double)nd * (12 + 16 + 16);
             CGJArgs ja{R, c->p4, c->Ss, c->sfac, c->y2, c->state};
             CGJTArgs ta{R, c->p4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials, stride, c->state};
-            CGUpdArgs ua{nd, c->sol, c->r, c->p4, c->Ap, c->partials, stride, c->state};
+            // partial rows: p.Ap 0, the update's r.r 1, a replaced residual's r.r 2 (x.Ax 3)
+            CGUpdArgs ua{nd, c->sol, c->r, c->p4, c->Ap, c->partials + stride, stride, c->state, SceneRef{}, Fold{}};
+            CGPArgs pp{nd, c->r, c->p4, c->sol, d4, c->state, Fold{}, nullptr, c->err_flag};
             // true-residual passes: the same J / J^T kernels on (x, m), gradW evaluated
             using FE = Fmt<FC::REC, GS_EVAL>;
             CGJArgs jx{R, c->xs4, c->Ss, c->sfac, c->y2, c->state};
-            // (its x.Ax partials go to row 2, clear of the update's r.r in row 0)
-            CGJTArgs tx{R, c->xs4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials + 2 * stride, stride,
+            CGJTArgs tx{R, c->xs4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials + 3 * (size_t)stride, stride,
                         c->state};
             auto one_iter = [&](int tag, SolverState* host) -> int {
                 IVP_TRY(launch(c, KC_CG_J, tag, bJ, k_cg_J<FC, false>, np, ja));
                 IVP_TRY(launch(c, KC_CG_JT, tag, bJT, k_cg_JT<FC, false>, np, ta));
-                IVP_TRY(finalize<FIN_CG_PAP>(c, np.x));
+                IVP_TRY(fold_source<1>(c, 0, np.x, c->state, &ua.pap));
                 IVP_TRY(launch(c, KC_CG_UPDATE, tag, bU, k_cg_update<false>, nb, ua));
                 if (FC::GS == GS_F16 && (tag + 1) % REFRESH_EVERY == 0) {
                     // residual replacement: r = b - A x with A in float32 from the positions;
-                    // its r.r (row 1) and the recursive r.r (row 0) go to the stop test and beta
+                    // its r.r and the recursive r.r go to the stop test and beta
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_x4, nb, nd, (const float*)c->sol,
                                    (const float4*)c->pos, c->xs4, (const SolverState*)c->state));
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_J<FE, false>, np, jx));
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_JT<FE, false>, np, tx));
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_refresh, nb, nd, (const float*)c->b,
-                                   (const float*)c->Ap, c->r, c->partials + stride, stride,
+                                   (const float*)c->Ap, c->r, c->partials + 2 * (size_t)stride, stride,
                                    (const SolverState*)c->state));
-                    IVP_TRY(finalize<FIN_CG_REPLACE>(c, nb.x, 0.0, 0, false, host));
-                } else {
-                    IVP_TRY(finalize<FIN_CG_UPDATE>(c, nb.x, 0.0, 0, false, host));
+                    IVP_TRY(fold_source<2>(c, 1, nb.x, c->state, &pp.rr));
+                    pp.host = host;
+                    return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_REPLACE>, nb, pp);
                 }
-                return launch(c, KC_CG_P, tag, bP, k_cg_p<false>, nb, nd, (const float*)c->r, c->p4,
-                              (const SolverState*)c->state, SceneRef{});
+                IVP_TRY(fold_source<1>(c, 1, nb.x, c->state, &pp.rr));
+                pp.host = host;
+                return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_UPDATE>, nb, pp);
             };
-            // Behind each chunk's state copy: d -= x, the outer-iteration mark and the next constraint
-            // pass with its finalize, all returning at once unless the CG has stopped (and not
+            // Behind each chunk's report (d -= x is part of its last launch): the next constraint
+            // pass with its mark and its finalize, all returning at once unless the CG has stopped (and not
             // failed), so the device works while the host reads the state; after the first CG of
             // the solve (whose read-back also checks the rows for overflow) also the closing
             // k_ip_finish that the next evaluation may need (see above).
             fin_next = !deferred && opt_iter + 1 < prm->max_iteration_opt && !prm->use_fixed_iters;
-            auto tail = [&]() -> int {
+            auto tail = [&](bool none) -> int {
                 const SolverState* gate = c->state;
-                IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_dupdate<false>, nb, nd, d4, (const float*)c->sol, SceneRef{},
-                               gate));
+                if (none)
+                    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_dupdate<false>, nb, nd, d4, (const float*)c->sol,
+                                   SceneRef{}, gate));
                 IVP_TRY(queue_pack(opt_iter + 1, gate));
                 if (fin_next)
                     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_finish, nb, nd, inv_dt, (const float4*)d4,
@@ -2256,6 +2282,20 @@ int visc_explicit_body(ivp_ctx* c, float coeff, float dt) {
                   (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel);
 }
 
+// The rest of a Weiler18 / Jeske23 CG iteration after its operator pass (npap blocks); partial rows:
+// p.Ap 0, r.r 1, r.z 2
+int w18_update(ivp_ctx* c, const W18Args& cg, int npap, int tag, SolverState* host) {
+    const int nd = c->nd;
+    const dim3 nb(blocks_for(nd));
+    W18Args u = cg;
+    u.partials = c->partials + c->max_blocks;
+    IVP_TRY(fold_source<1>(c, 0, npap, c->state, &u.pap));
+    IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, u));
+    W18PArgs p{nd, c->w_z, c->w_p4, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag};
+    IVP_TRY(fold_source<2>(c, 1, nb.x, c->state, &p.sums));
+    return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, p);
+}
+
 template <class FM, bool ALLFLUID>
 int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
     const int nd = c->nd;
@@ -2294,19 +2334,13 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         const double bAv = stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 48.0 * nd;
         auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_W18_AV, tag, bAv, k_w18_Av<FM, ALLFLUID>, pass_grid(nd), cg));
-            IVP_TRY(finalize<FIN_W18_PAP>(c, pass_grid(nd).x));
-            IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, cg));
-            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x, 0.0, 0, false, host));
-            return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, nd, (const float*)c->w_z, c->w_p4, c->w_dv,
-                          (const SolverState*)c->state);
+            return w18_update(c, cg, pass_grid(nd).x, tag, host);
         };
-        // the save of the correction and v += dv follow each chunk's state copy, running once the
-        // solve has stopped (while the host reads the state)
-        auto tail = [&]() -> int {
-            IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_w18_save, dim3(blocks_for(c->n)), c->n, nd, (const float*)c->w_dv,
-                           (const int*)c->inv, c->w_dv_prev, (const SolverState*)c->state, (const int*)c->err_flag));
-            return launch(c, KC_GLUE, -1, 0.0, k_w18_apply, dim3(blocks_for(3 * nd)), 3 * nd, (const float*)c->w_dv,
-                          c->vel, (const SolverState*)c->state, (const int*)c->err_flag);
+        // the save of the correction follows each chunk's report, running once the solve has stopped
+        // (while the host reads the state)
+        auto tail = [&](bool) -> int {
+            return launch(c, KC_GLUE, -1, 0.0, k_w18_save, dim3(blocks_for(c->n)), c->n, nd, (const float*)c->w_dv,
+                          (const int*)c->inv, c->w_dv_prev, (const SolverState*)c->state, (const int*)c->err_flag);
         };
         c->prof_epoch++;
         int epoch = c->prof_epoch;
@@ -2361,17 +2395,9 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
         const double bAv = stream_bytes<FM>(c, pairs) + 4.0 * pairs + 28.0 * nd;
         auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_ST_AV, tag, bAv, k_st_Av<FM, ALLFLUID, false>, np, cga));
-            IVP_TRY(finalize<FIN_W18_PAP>(c, np.x));
-            IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, cg));
-            IVP_TRY(finalize<FIN_W18_UPDATE>(c, nb.x, 0.0, 0, false, host));
-            return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, nd, (const float*)c->w_z, c->w_p4, c->w_dv,
-                          (const SolverState*)c->state);
+            return w18_update(c, cg, np.x, tag, host);
         };
-        // v += dv follows each chunk, running once the solve has stopped (unless rows were truncated)
-        auto tail = [&]() -> int {
-            return launch(c, KC_GLUE, -1, 0.0, k_w18_apply, dim3(blocks_for(3 * nd)), 3 * nd, (const float*)c->w_dv,
-                          c->vel, (const SolverState*)c->state, (const int*)c->err_flag);
-        };
+        auto tail = [](bool) { return (int)IVP_OK; };
         c->prof_epoch++;
         int epoch = c->prof_epoch;
         IVP_TRY(run_chunks(c, 100, c->st_guess, one_iter, &iters, &chunks, tail));
