@@ -580,6 +580,92 @@ __device__ __forceinline__ int scan_group(const Grid& g, const int* __restrict__
     return found;
 }
 
+// Lane K of each 16-lane row to the whole row
+template <int K>
+__device__ __forceinline__ int row_bcast(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + K, 0xf, 0xf, true);
+}
+
+// scan_group with 16 lanes per row (one DPP row), for counts that leave a SIMD a few waves: a run after
+// another, the scan waited for two bounds and one or two candidate batches nine times over.  Here
+// lanes 0 to 8 load the nine runs' bounds at once, and the runs end to end -- candidate v of run k is
+// particle v + rb[k], its run found by eight compares -- go through in batches of 16 with UL of them in
+// flight: 4k rows 12.2 -> 8.8 us alone, 8k 13.8 -> 10 (12 or 17 batches in flight: 9.6 and 10 at 4k; more
+// registers and code than the few waves hide).  Same order, same decisions, same ranks.
+constexpr int SCAN16_BATCHES = 8;   // batches in flight
+struct Row16Runs {
+    int s0, end;   // lane k < 9 of the row: run k's candidates [s0, end)
+};
+__device__ __forceinline__ Row16Runs row16_runs(const Grid& g, const int* __restrict__ start, bool on, float4 pi, int gl) {
+    const int cx = cell_coord(g, pi.x, 0), cy = cell_coord(g, pi.y, 1), cz = cell_coord(g, pi.z, 2);
+    const int x0 = cx > 0 ? cx - 1 : 0;
+    const int x1 = cx < g.dims[0] - 1 ? cx + 1 : g.dims[0] - 1;
+    // run gl = 3 (dz + 1) + (dy + 1)
+    const int yy = cy + gl % 3 - 1, zz = cz + gl / 3 - 1;
+    Row16Runs r = {0, 0};
+    if (on && gl < 9 && yy >= 0 && yy < g.dims[1] && zz >= 0 && zz < g.dims[2]) {
+        r.s0 = start[cell_key(g, x0, yy, zz)];
+        r.end = start[cell_key(g, x1, yy, zz) + 1];
+    }
+    return r;
+}
+
+template <int UL, class P>
+__device__ __forceinline__ int scan_row16(const float4* __restrict__ ppos, Row16Runs runs, int self, float4 pi, float h,
+                                          float h2_lo, float h2_hi, int gl, P&& put) {
+    const int wl = (int)(threadIdx.x & (WAVE - 1));
+    const int base = wl & ~15;
+    const uint32_t below = (1u << gl) - 1u;
+    const int s0 = runs.s0, len = runs.end - runs.s0;
+    int end = len;   // inclusive prefix over the row
+    end += __builtin_amdgcn_update_dpp(0, end, 0x111, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x112, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x114, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x118, 0xf, 0xf, true);
+    const int off = s0 - (end - len);
+    const int T = row_bcast<8>(end);
+    const int e[8] = {row_bcast<0>(end), row_bcast<1>(end), row_bcast<2>(end), row_bcast<3>(end),
+                      row_bcast<4>(end), row_bcast<5>(end), row_bcast<6>(end), row_bcast<7>(end)};
+    const int rb[9] = {row_bcast<0>(off), row_bcast<1>(off), row_bcast<2>(off), row_bcast<3>(off), row_bcast<4>(off),
+                       row_bcast<5>(off), row_bcast<6>(off), row_bcast<7>(off), row_bcast<8>(off)};
+    const int most = wave_max(T);   // the wave's four rows go through together
+    int found = 0;
+    for (int cb = 0; cb < most; cb += 16 * UL) {
+        int j[UL];
+        float4 p[UL];
+#pragma unroll
+        for (int u = 0; u < UL; ++u) {
+            const int v = cb + 16 * u + gl;
+            int o = rb[0];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o = v >= e[k] ? rb[k + 1] : o;
+            j[u] = v < T ? v + o : -1;
+            if (j[u] >= 0) p[u] = ppos[j[u]];
+        }
+        __builtin_amdgcn_sched_barrier(0);   // every load of the chunk in flight before the tests
+#pragma unroll
+        for (int u = 0; u < UL; ++u) {
+            if (cb + 16 * u >= most) break;
+            float rx = pi.x - p[u].x, ry = pi.y - p[u].y, rz = pi.z - p[u].z;
+            float d2 = fmaf(rz, rz, fmaf(ry, ry, rx * rx));
+            const bool valid = j[u] >= 0 && j[u] != self;
+            bool in = valid && d2 < h2_lo;
+            const bool band = valid && !in && d2 < h2_hi;
+            if (__builtin_amdgcn_ballot_w64(band)) {
+                if (band) {
+                    float d = rx * rx + ry * ry + rz * rz;
+                    asm volatile("" : "+v"(d));
+                    in = sqrtf(d) < h;
+                }
+            }
+            const uint32_t m = (uint32_t)(__builtin_amdgcn_ballot_w64(in) >> base) & 0xffffu;
+            if (in) put(j[u], __popc(m & below), found);
+            found += __popc(m);
+        }
+    }
+    return found;
+}
+
 // Phase A alone with G lanes per row (threads = rows x G): ids into the rows' slots exactly as
 // k_build's scan stores them, the row's dynamic slot count into rowcnt and its neighbour total
 // into rowtot.  For particle counts that leave few waves per SIMD, where the one-lane scan is a
@@ -591,32 +677,44 @@ __global__ __launch_bounds__(BLOCK) void k_scan(BuildArgs a) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = blk * (BLOCK / G) + (int)(threadIdx.x / G);
     const int gl = (int)(threadIdx.x % G);
-    if (i >= a.nd) return;   // the G lanes of a row leave together
+    const bool on = i < a.nd;
+    if (G != 16 && !on) return;   // the G lanes of a row leave together (scan_row16 takes whole waves)
     const int C = a.C, Cs = a.Cs;
     // the wave's rows share one 64-row tile (64 / G rows from a multiple of 64 / G); slot k of the
     // row is word row_word0(lane) + slot_word(k) of the tile, a 32-bit index from the tile's
     // (uniform) base
     uint32_t* tnb = a.nb + (size_t)__builtin_amdgcn_readfirstlane(i >> 6) * (size_t)Cs * REC;
     const uint32_t w0 = row_word0<REC>(i & (WAVE - 1));
-    const float4 pi = a.pos[i];
-    const Grid g = SCENES ? a.grids[a.sid[i]] : a.g;
+    const int ic = on ? i : a.nd - 1;
+    const float4 pi = a.pos[ic];
+    const Grid g = SCENES ? a.grids[a.sid[ic]] : a.g;
     int tot = 0, cnt = 0, cs = 0;
     // the k-th neighbour found (dynamic ones first) is stored when k < C
-    int nd_found = scan_group<G, U>(g, a.dstart, a.pos, i, pi, a.h, a.h2_lo, a.h2_hi, gl,
-                                    [&](int j, int rank, int before) {
-                                        if (before + rank < C) tnb[slot_word<REC>(before + rank) + w0] = (uint32_t)j;
-                                    });
+    Row16Runs rd = {0, 0}, rs = {0, 0};
+    if constexpr (G == 16) {   // both populations' bounds in flight together
+        rd = row16_runs(g, a.dstart, on, pi, gl);
+        rs = row16_runs(g, a.sstart, on, pi, gl);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    auto scan = [&](const int* start, const float4* ppos, int self, auto&& put) {
+        if constexpr (G == 16)
+            return scan_row16<SCAN16_BATCHES>(ppos, self >= 0 ? rd : rs, self, pi, a.h, a.h2_lo, a.h2_hi, gl, put);
+        else
+            return scan_group<G, U>(g, start, ppos, self, pi, a.h, a.h2_lo, a.h2_hi, gl, put);
+    };
+    int nd_found = scan(a.dstart, a.pos, i, [&](int j, int rank, int before) {
+        if (before + rank < C) tnb[slot_word<REC>(before + rank) + w0] = (uint32_t)j;
+    });
     cnt = nd_found < C ? nd_found : C;
     tot = nd_found;
-    int ns_found = scan_group<G, U>(g, a.sstart, a.pos + a.nd, -1, pi, a.h, a.h2_lo, a.h2_hi, gl,
-                                    [&](int j, int rank, int before) {
-                                        const int k = nd_found + before + rank;
-                                        if (k < C) tnb[slot_word<REC>(Cs - 1 - (before + rank)) + w0] = (uint32_t)j;
-                                    });
+    int ns_found = scan(a.sstart, a.pos + a.nd, -1, [&](int j, int rank, int before) {
+        const int k = nd_found + before + rank;
+        if (k < C) tnb[slot_word<REC>(Cs - 1 - (before + rank)) + w0] = (uint32_t)j;
+    });
     tot += ns_found;
     cs = (tot < C ? tot : C) - cnt;
     (void)cs;
-    if (gl == 0) {
+    if (on && gl == 0) {
         a.rowcnt[i] = cnt;
         a.rowtot[i] = tot;
         if (tot > C) atomicOr(a.err_flag, 1);
@@ -1223,15 +1321,15 @@ __global__ __launch_bounds__(BLOCK, 8) void k_eval4(BuildArgs a) {
     const bool valid = i < a.nd;
     int cnt = 0, cs = 0;
     float4 pi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float h = a.h;
+    const size_t w_row = (size_t)tile * (size_t)a.Cs * 64u + 8u * (uint32_t)r;
+    uint32_t* row = a.nb + w_row;
     if (valid) {
         pi = a.pos[i];
         cnt = a.rowcnt[i];
         const int tot = a.rowtot[i];
         cs = (tot < a.C ? tot : a.C) - cnt;
     }
-    const float h = a.h;
-    const size_t w_row = (size_t)tile * (size_t)a.Cs * 64u + 8u * (uint32_t)r;
-    uint32_t* row = a.nb + w_row;
     const int wl = __builtin_amdgcn_readfirstlane(wave_max(cnt)), ws = __builtin_amdgcn_readfirstlane(wave_max(cs));
     if ((threadIdx.x & (WAVE - 1)) == 0) {
         wmax[threadIdx.x >> 6] = wl;
@@ -1798,16 +1896,16 @@ int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m,
 // 145 -> 115 with 4 lanes; 1M rows 501 -> 404 with 2 lanes and 4 batches in flight.  Fewer rows
 // leave fewer waves per SIMD, and the one-lane scan is then a chain of dependent load rounds.
 // 64 is the scan by cells (k_scan_cells), for ids-only and float16 rows (one scene or many) whose
-// staged rows fit the LDS, from 16k rows: scan alone, lanes per row (best count) against by cells,
-// us: 4k rows 15.8 / 16.7, 8k 16.1 / 16.4, 23k 19.1 / 18.4, 36k 24.7 / 19.1, 102k 43 / 29, 262k 83 /
-// 50, 1M 225 / 149; where it does not apply, the count's lanes per row (16 below 32k rows: 8 lanes
+// staged rows fit the LDS, from 20k rows: scan alone, lanes per row (best count) against by cells,
+// us: 12k rows 12.3 / 14.7, 16k 13.5 / 15.7, 23k 17.5 / 15.2, 32k 21.2 / 16.6, 48k 27.1 / 17.8, 102k 43 /
+// 29, 262k 83 / 50, 1M 225 / 149; where it does not apply, the count's lanes per row (16 below 32k rows: 8 lanes
 // took 20 us from 1k to 23k rows against 16).
 static int lanes_by_count(int nd) { return nd >= (1 << 18) ? 2 : nd >= (1 << 15) ? 4 : 16; }
 
 int build_lanes_for(const ivp_ctx* c) {
     const int nd = c->nd;
     const bool cells = c->rec_words == 64 && scan_cells_lds(c->Cs) <= SCAN_CELLS_LDS_MAX;
-    int G = c->build_lanes > 0 ? c->build_lanes : cells && nd >= (1 << 14) ? 64 : lanes_by_count(nd);
+    int G = c->build_lanes > 0 ? c->build_lanes : cells && nd >= 20480 ? 64 : lanes_by_count(nd);
     if (G == 64 && !cells) G = lanes_by_count(nd);
     return G;
 }
