@@ -219,8 +219,10 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
 // 9.1: the bandwidth of one CU).
 constexpr int FOLD_MAX = 2048;
 
-template <int NV>
-__device__ __forceinline__ void block_fold(const double* __restrict__ p, int stride, int n, double (&t)[NV]) {
+// `meanwhile` runs with the first partials in flight: the caller's own loads, which would otherwise wait
+// for the fold (23k rows: update 3.8 -> 3.4 us, p pass 3.9 -> 3.5).
+template <int NV, class M>
+__device__ __forceinline__ void block_fold(const double* __restrict__ p, int stride, int n, double (&t)[NV], M&& meanwhile) {
     __shared__ double lds[NV][WAVES_PER_BLOCK];
     double s[NV];
 #pragma unroll
@@ -234,6 +236,7 @@ __device__ __forceinline__ void block_fold(const double* __restrict__ p, int str
                 const int k = base + u * BLOCK + (int)threadIdx.x;
                 v[q][u] = k < n ? p[(size_t)q * stride + k] : 0.0;
             }
+        if (base == 0) meanwhile();
 #pragma unroll
         for (int q = 0; q < NV; ++q) s[q] += (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
     }
@@ -255,7 +258,7 @@ __global__ __launch_bounds__(BLOCK) void k_prefold(const double* __restrict__ p,
     const int per = (n + PREFOLD - 1) / PREFOLD;
     const int k0 = (int)blockIdx.x * per < n ? (int)blockIdx.x * per : n;
     double t[NV];
-    block_fold<NV>(p + k0, stride, k0 + per < n ? per : n - k0, t);
+    block_fold<NV>(p + k0, stride, k0 + per < n ? per : n - k0, t, []() {});
     if (threadIdx.x == 0)
 #pragma unroll
         for (int q = 0; q < NV; ++q) out[q * PREFOLD + (int)blockIdx.x] = t[q];
@@ -284,29 +287,31 @@ inline int fold_source(ivp_ctx* c, int row0, int n, const SolverState* gate, Fol
 // In an iteration's update pass: alpha from the operator pass's p.Ap (OP = FIN_CG_PAP, FIN_W18_PAP).
 // Returns false when there is nothing to update.  The state's own fields stay as they are until
 // the p pass; ran and prev_* tell it what happened here.
-template <int OP>
-__device__ __forceinline__ bool fold_alpha(SolverState* st, const Fold& f, float* alpha) {
+template <int OP, class M>
+__device__ __forceinline__ bool fold_alpha(SolverState* st, const Fold& f, float* alpha, M&& meanwhile) {
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (st->active == 0) {
         if (lead) st->ran = 0;
         return false;
     }
+    const double rr_old = st->rr_old, rr_best = st->rr_best;
+    const int iter = st->iter, stalls = st->stalls;
     double t[1];
-    block_fold<1>(f.p, f.stride, f.n, t);
+    block_fold<1>(f.p, f.stride, f.n, t, meanwhile);
     // ip.py:307-311 fails on p.Ap < 0; weiler18.py:338-342 ends the iteration on p.Ap <= 0
     const double least = OP == FIN_CG_PAP ? 1e-30 : 1e-12;
     const bool bad = OP == FIN_CG_PAP ? t[0] < 0.0 : t[0] <= 0.0;
-    const double al = st->rr_old / (t[0] > least ? t[0] : least);
+    const double al = rr_old / (t[0] > least ? t[0] : least);
     *alpha = (float)al;
     if (lead) {
         st->pAp = t[0];
         st->ran = bad ? 2 : 1;
         if (!bad) {
             st->alpha = al;
-            st->prev_iter = st->iter;
-            st->prev_rr_old = st->rr_old;
-            st->prev_rr_best = st->rr_best;
-            st->prev_stalls = st->stalls;
+            st->prev_iter = iter;
+            st->prev_rr_old = rr_old;
+            st->prev_rr_best = rr_best;
+            st->prev_stalls = stalls;
         }
     }
     return !bad;
@@ -322,14 +327,13 @@ struct Advance {
 // In the iteration's p pass: the state after the iteration from the update pass's sums (OP =
 // FIN_CG_UPDATE, FIN_CG_REPLACE, FIN_W18_UPDATE), formed by every block and written by one, which
 // reports it to the host if asked.
-template <int OP>
-__device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, SolverState* host, const int* flags) {
+template <int OP, class M>
+__device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, SolverState* host, const int* flags,
+                                                M&& meanwhile) {
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     const int ran = st->ran;
     Advance a = {ran == 1, false, ran == 0 && st->status == 0, 0.0f};
     if (ran == 1) {
-        double t[fin_nv<OP>()];
-        block_fold<fin_nv<OP>()>(f.p, f.stride, f.n, t);
         SolverState s;
         s.iter = st->prev_iter;
         s.rr_old = st->prev_rr_old;
@@ -340,6 +344,8 @@ __device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, 
         s.active = 1;
         s.beta = 0.0;
         s.rr_new = 0.0;
+        double t[fin_nv<OP>()];
+        block_fold<fin_nv<OP>()>(f.p, f.stride, f.n, t, meanwhile);
         fin_apply<OP>(&s, t, 0.0, 0);
         a.active = s.active != 0;
         a.stopped = !a.active;

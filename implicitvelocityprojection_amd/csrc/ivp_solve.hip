@@ -776,22 +776,34 @@ struct CGUpdArgs {
 // pcg_update_x_r_scalar (math_utils.py:180-195) + r.r (ip.py:314-317)
 template <bool SC>
 __global__ __launch_bounds__(BLOCK) void k_cg_update(CGUpdArgs a) {
-    float alpha = 0.0f;
-    if (!SC && !fold_alpha<FIN_CG_PAP>(a.st, a.pap, &alpha)) return;
     const int blk = blockIdx.x;
     int i = blk * BLOCK + threadIdx.x;
+    float alpha = 0.0f;
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float x[3] = {0.0f, 0.0f, 0.0f}, r[3] = {0.0f, 0.0f, 0.0f}, Ap[3] = {0.0f, 0.0f, 0.0f};
+    auto own = [&]() {
+        if (i >= a.nd) return;
+        p = a.p4[i];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            x[q] = a.sol[3 * i + q];
+            r[q] = a.r[3 * i + q];
+            Ap[q] = a.Ap[3 * i + q];
+        }
+    };
+    if (!SC && !fold_alpha<FIN_CG_PAP>(a.st, a.pap, &alpha, own)) return;
     Gate gt = gate_all(i, a.nd);
     if (SC && !gate_block(a.sc, blk, i, a.nd, PH_CG, gt)) return;
     if (SC) alpha = (float)a.sc.ss[gt.s].cg.alpha;
     double rr = 0.0;
     if (gt.on) {
-        float4 p = a.p4[i];
-        float x0 = a.sol[3 * i + 0] + alpha * p.x;
-        float x1 = a.sol[3 * i + 1] + alpha * p.y;
-        float x2 = a.sol[3 * i + 2] + alpha * p.z;
-        float r0 = a.r[3 * i + 0] - alpha * a.Ap[3 * i + 0];
-        float r1 = a.r[3 * i + 1] - alpha * a.Ap[3 * i + 1];
-        float r2 = a.r[3 * i + 2] - alpha * a.Ap[3 * i + 2];
+        if (SC) own();
+        float x0 = x[0] + alpha * p.x;
+        float x1 = x[1] + alpha * p.y;
+        float x2 = x[2] + alpha * p.z;
+        float r0 = r[0] - alpha * Ap[0];
+        float r1 = r[1] - alpha * Ap[1];
+        float r2 = r[2] - alpha * Ap[2];
         a.sol[3 * i + 0] = x0; a.sol[3 * i + 1] = x1; a.sol[3 * i + 2] = x2;
         a.r[3 * i + 0] = r0; a.r[3 * i + 1] = r1; a.r[3 * i + 2] = r2;
         rr = (double)(r0 * r0 + r1 * r1 + r2 * r2);
@@ -833,14 +845,20 @@ struct CGPArgs {
 // solve that has stopped without failing moves d -= x instead (add_vec3 with scale -1, ip.py:389).
 template <int OP>
 __global__ __launch_bounds__(BLOCK) void k_cg_p(CGPArgs a) {
-    const Advance v = fold_advance<OP>(a.st, a.rr, a.host, a.flags);
     const int i = blockIdx.x * BLOCK + threadIdx.x;
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float r[3] = {0.0f, 0.0f, 0.0f};
+    const Advance v = fold_advance<OP>(a.st, a.rr, a.host, a.flags, [&]() {
+        if (i >= a.nd) return;
+        p = a.p4[i];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[q] = a.r[3 * i + q];
+    });
     if (i >= a.nd) return;
     if (v.active) {
-        float4 p = a.p4[i];
-        p.x = a.r[3 * i + 0] + v.beta * p.x;
-        p.y = a.r[3 * i + 1] + v.beta * p.y;
-        p.z = a.r[3 * i + 2] + v.beta * p.z;
+        p.x = r[0] + v.beta * p.x;
+        p.y = r[1] + v.beta * p.y;
+        p.z = r[2] + v.beta * p.z;
         a.p4[i] = p;
     } else if (a.host && v.stopped) {
         float4 d = a.d4[i];
@@ -1492,17 +1510,27 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a) {
 // r -= alpha Ap, r.r, z = P r, r.z (weiler18.py:344-360); dv += alpha p of the same lines
 // follows in the p pass, which reads p anyway
 __global__ __launch_bounds__(BLOCK) void k_w18_update(W18Args a) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
     float alpha;
-    if (!fold_alpha<FIN_W18_PAP>(a.st, a.pap, &alpha)) return;
+    float r[3] = {0.0f, 0.0f, 0.0f}, Ap[3] = {0.0f, 0.0f, 0.0f}, P[9] = {};
+    auto own = [&]() {
+        if (i >= a.R.nd) return;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            r[q] = a.r[3 * i + q];
+            Ap[q] = a.out[3 * i + q];
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) P[q] = a.pinv[9 * (size_t)i + q];
+    };
+    if (!fold_alpha<FIN_W18_PAP>(a.st, a.pap, &alpha, own)) return;
     const float nalpha = -alpha;
-    int i = blockIdx.x * BLOCK + threadIdx.x;
     double rr = 0.0, rz = 0.0;
     if (i < a.R.nd) {
-        float r0 = a.r[3 * i + 0] + nalpha * a.out[3 * i + 0];
-        float r1 = a.r[3 * i + 1] + nalpha * a.out[3 * i + 1];
-        float r2 = a.r[3 * i + 2] + nalpha * a.out[3 * i + 2];
+        float r0 = r[0] + nalpha * Ap[0];
+        float r1 = r[1] + nalpha * Ap[1];
+        float r2 = r[2] + nalpha * Ap[2];
         a.r[3 * i + 0] = r0; a.r[3 * i + 1] = r1; a.r[3 * i + 2] = r2;
-        const float* P = a.pinv + 9 * (size_t)i;
         float z0 = P[0] * r0 + P[1] * r1 + P[2] * r2;
         float z1 = P[3] * r0 + P[4] * r1 + P[5] * r2;
         float z2 = P[6] * r0 + P[7] * r1 + P[8] * r2;
@@ -1532,23 +1560,33 @@ struct W18PArgs {
 // (weiler18.py:399-401), except on rows that the last build truncated (the host refuses them when it
 // reads the flags).
 __global__ __launch_bounds__(BLOCK) void k_w18_p(W18PArgs a) {
-    const Advance v = fold_advance<FIN_W18_UPDATE>(a.st, a.sums, a.host, a.flags);
-    const bool apply = a.host && v.stopped && !(*a.flags & 5);
-    if (!v.ran && !apply) return;
-    const float alpha = (float)a.st->alpha;
     const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= a.nd) return;
-    float dv[3] = {a.dv[3 * i + 0], a.dv[3 * i + 1], a.dv[3 * i + 2]};
+    const float alpha = (float)a.st->alpha;
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float dv[3] = {0.0f, 0.0f, 0.0f}, z[3] = {0.0f, 0.0f, 0.0f};
+    const Advance v = fold_advance<FIN_W18_UPDATE>(a.st, a.sums, a.host, a.flags, [&]() {
+        if (i >= a.nd) return;
+        p = a.p4[i];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            dv[q] = a.dv[3 * i + q];
+            z[q] = a.z[3 * i + q];
+        }
+    });
+    const bool apply = a.host && v.stopped && !(*a.flags & 5);
+    if ((!v.ran && !apply) || i >= a.nd) return;
+    if (!v.ran)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) dv[q] = a.dv[3 * i + q];
     if (v.ran) {
-        float4 p = a.p4[i];
         dv[0] = dv[0] + alpha * p.x;
         dv[1] = dv[1] + alpha * p.y;
         dv[2] = dv[2] + alpha * p.z;
         a.dv[3 * i + 0] = dv[0]; a.dv[3 * i + 1] = dv[1]; a.dv[3 * i + 2] = dv[2];
         if (v.active) {
-            p.x = a.z[3 * i + 0] + v.beta * p.x;
-            p.y = a.z[3 * i + 1] + v.beta * p.y;
-            p.z = a.z[3 * i + 2] + v.beta * p.z;
+            p.x = z[0] + v.beta * p.x;
+            p.y = z[1] + v.beta * p.y;
+            p.z = z[2] + v.beta * p.z;
             a.p4[i] = p;
         }
     }
