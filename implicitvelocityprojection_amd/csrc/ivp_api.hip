@@ -396,11 +396,23 @@ int prof_collect(ivp_ctx* c, int cg_iters_done, int epoch) {
 // Status of the neighbour build last enqueued, read with one synchronisation: its error flags
 // (and the solver state, whose pair count the byte figures of the following passes use).
 static int build_status(ivp_ctx* c) {
+    IVP_TRY(build_fold(c));
     IVP_HIP(hipMemcpyAsync(c->err_host, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     IVP_HIP(hipMemcpyAsync(c->state_host, c->state, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
     IVP_HIP(hipStreamSynchronize(c->stream));
     return build_code(*c->err_host);
 }
+
+// Within a step each stage leaves the next one its input; nothing of it outlives the step
+struct StepPlan {
+    ivp_ctx* c;
+    explicit StepPlan(ivp_ctx* c) : c(c) { clear(); }
+    ~StepPlan() { clear(); }
+    void clear() {
+        c->next = NextIn{};
+        c->ready = NEXT_NONE;
+    }
+};
 
 static const char* kclass_name(int k) {
     static const char* names[KC_COUNT] = {"sort", "build", "ip_pack", "ip_rhs", "cg_J", "cg_JT", "cg_update", "cg_p",
@@ -710,6 +722,11 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
     // gravity writes the step's velocities into the second buffer; a stage that finds the rows
     // truncated by the last rebuild (the first solve's first read-back brings its flags) swaps the
     // first one back, so such a step leaves v and x as they were
+    const bool tension = prm->surface_tension_coeff != 0.0f, viscous = prm->viscosity_coeff != 0.0f;
+    const NextKind force = prm->viscosity_method == 1 ? NEXT_W18 : NEXT_VISC;
+    const NextKind solve = prm->pressure_method == 0 ? NEXT_NONE : NEXT_IP;
+    StepPlan plan(c);
+    c->next = next_in(c, tension ? NEXT_ST : viscous ? force : solve, prm->dt, prm->viscosity_coeff);
     int rc = glue_gravity(c, prm->gravity, prm->dt);
     if (rc != IVP_OK) return rc;
     auto truncated = [&](int r) {
@@ -719,13 +736,15 @@ int ivp_step(ivp_ctx* c, const ivp_step_params* prm, ivp_ip_stats* stats, ivp_cg
     if (visc) { visc->cg_iters = 0; visc->residual_norm2 = 0.0; }
     if (st) { st->cg_iters = 0; st->residual_norm2 = 0.0; }
     // compute_non_pressure_forces order (framework.py:400-421): gravity, surface tension, viscosity
-    if (prm->surface_tension_coeff != 0.0f) {
+    if (tension) {
+        c->next = next_in(c, viscous ? force : solve, prm->dt, prm->viscosity_coeff);
         rc = st_jeske23(c, prm->surface_tension_coeff, prm->dt, st);
         if (rc != IVP_OK) return truncated(rc);
     }
     // coefficient 0 makes either viscosity model an exact no-op (the rhs v - A v is 0, and the
     // explicit force is scaled by the coefficient)
-    if (prm->viscosity_coeff != 0.0f) {
+    if (viscous) {
+        c->next = next_in(c, solve, prm->dt, 0.0f);
         if (prm->viscosity_method == 1)
             rc = visc_weiler18(c, prm->viscosity_coeff, prm->dt, visc);
         else
@@ -756,6 +775,8 @@ int ivp_step_scenes(ivp_ctx* c, const ivp_step_params* prm, ivp_scene_stats* sta
     // viscosity and surface tension are not part of the scene step, which solves with IP
     if (prm->viscosity_coeff != 0.0f || prm->surface_tension_coeff != 0.0f) return IVP_ERR_ARG;
     if (prm->pressure_method != 1) return IVP_ERR_ARG;
+    StepPlan plan(c);
+    c->next = next_in(c, NEXT_IP, prm->dt, 0.0f);
     int rc = glue_gravity(c, prm->gravity, prm->dt);
     if (rc != IVP_OK) return rc;
     rc = ip_solve_scenes(c, prm->dt, &prm->ip);
@@ -836,6 +857,7 @@ int ivp_counts(ivp_ctx* c, int* n_total, int* n_dynamic, long long* dyn_pairs) {
     if (dyn_pairs) {
         *dyn_pairs = 0;
         if (c->built && c->nd > 0) {
+            IVP_TRY(build_fold(c));
             IVP_HIP(hipMemcpyAsync(c->state_host, c->state, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
             IVP_HIP(hipStreamSynchronize(c->stream));
             *dyn_pairs = c->state_host->total_pairs;

@@ -1937,6 +1937,12 @@ int glue_advect_boundary(ivp_ctx* c, float dt) {
     return IVP_OK;
 }
 
+int build_fold(ivp_ctx* c) {
+    if (!c->build_pending || !c->built || c->nd == 0) return IVP_OK;
+    c->build_pending = false;
+    return finalize<FIN_BUILD>(c, (c->nd + WAVE - 1) / WAVE);
+}
+
 int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
     if (!c->loaded) return IVP_ERR_STATE;
     if (adv_dt && c->nd > 0) c->built = false;
@@ -1962,7 +1968,8 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         float h2_hi = std::nextafter((float)(hh * (1.0 + 1.0 / 1048576.0)), 1.0f);
         BuildArgs ba{c->nd, c->ns, c->C, c->Cs, c->h, h2_lo, h2_hi, (float)hh, c->kcubic, c->kspiky, 1.0f / c->h, 1.0f / c->gscale, c->grid,
                      c->grids, c->sid, c->pos, c->minv, c->dstart, c->sstart, c->nb, c->g16, c->tile_len, c->wave_len,
-                     c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag, c->partials, c->max_blocks,
+                     c->rowcnt, c->rowtot, c->density, c->kk, c->Ss, c->err_flag,
+                     c->partials + (size_t)BUILD_ROW * c->max_blocks, c->max_blocks,
                      c->win_cap, c->loc, c->win_ids, c->win_n};
         // bytes (pair count of the previous build): the pair records written, the ids read back
         // once, x and m of every particle once, the per-row outputs (rho, k, S, counts)
@@ -2003,8 +2010,8 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         }
     }
     if (windows && !fused) {
-        WinArgs wa{c->nd, c->Cs, c->win_cap, c->nb, c->tile_len, c->loc, c->win_ids, c->win_n, c->partials,
-                   c->max_blocks, tiles_per_block};
+        WinArgs wa{c->nd, c->Cs, c->win_cap, c->nb, c->tile_len, c->loc, c->win_ids, c->win_n,
+                   c->partials + (size_t)BUILD_ROW * c->max_blocks, c->max_blocks, tiles_per_block};
         const dim3 grid((c->nd + WAVE - 1) / WAVE);
         if (ppt <= 8)
             IVP_TRY(launch(c, KC_WINDOW, -1, 0.0, k_window<8>, grid, wa));
@@ -2014,10 +2021,14 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
             IVP_TRY(launch(c, KC_WINDOW, -1, 0.0, k_window<32>, grid, wa));
     }
     c->win_built = windows;
-    // pair count (row 0) and window sizes (row 1) of the build's blocks
-    if (c->nd > 0)
+    // pair count and window sizes of the build's blocks: folded here when they are reported, else with the
+    // first sums of the next pressure solve (a launch less per step: 4 us of a small one)
+    c->build_pending = c->nd > 0;
+    if (c->nd > 0 && (report || tiles_per_block != 1)) {
         IVP_TRY(finalize<FIN_BUILD>(c, tiles_per_block == 1 ? (c->nd + WAVE - 1) / WAVE : blocks_for(c->nd), 0.0, 0,
                                     false, report ? c->state_host : nullptr));
+        c->build_pending = false;
+    }
     c->built = true;
     return IVP_OK;
 }

@@ -76,6 +76,25 @@ struct SolverState {
     int flags;              // the build's error flags, as of the last report to the host
 };
 
+// Per-particle input that the next stage of a step reads, formed from the velocities by whichever
+// kernel writes them (gravity, a force's last launch) or, called on its own, by k_next.
+enum NextKind {
+    NEXT_NONE,
+    NEXT_IP,     // (dt v, m)
+    NEXT_W18,    // (v, m / rho) and dt mu / rho, mu = coeff rho0
+    NEXT_ST,     // (v, m)
+    NEXT_VISC    // (v, rho)
+};
+struct NextIn {
+    int kind = NEXT_NONE;
+    float dt = 0.0f, coeff = 0.0f;
+    const float4* pos = nullptr;
+    const float* density = nullptr;
+    const float* rho0 = nullptr;
+    float4* out = nullptr;
+    float* fac = nullptr;
+};
+
 // Independent scenes in one context.  Each scene has its own cell grid (keys of scene s follow
 // those of scene s-1), so the cell sort keeps every scene's particles contiguous: dynamic
 // particles of scene s at internal [row0, row0 + nd), static ones in the same scene order after
@@ -115,7 +134,8 @@ struct SceneParams {
     int max_opt, max_pcg, fixed;
 };
 
-constexpr int PARTIAL_ROWS = 6;   // rows of max_blocks partials
+constexpr int PARTIAL_ROWS = 8;   // rows of max_blocks partials; the build's sums are in the last two
+constexpr int BUILD_ROW = 6;
 constexpr int PREFOLD = 64;       // partials per row that k_prefold leaves
 constexpr int MARKS = 256;        // pass times that every context holds (more are allocated when needed)
 constexpr int ROW_PAD = 8;        // tile lengths are padded to a multiple of this many slots
@@ -215,6 +235,11 @@ struct ivp_ctx {
     int* win_ids = nullptr;
     int* win_n = nullptr;
     bool windows = true;
+    // a step's plan: `next` is what the stage being enqueued leaves for the one after it, `ready` what the
+    // one before it has left
+    ivp::NextIn next;
+    int ready = ivp::NEXT_NONE;
+    bool build_pending = false;   // the last build's sums (pairs, window sizes) are not in the state yet
     int win_cap = ivp::WIN_MAX;   // largest window kept (a smaller cap leaves more tiles without)
     bool win_built = false;
 
@@ -384,6 +409,10 @@ enum PrjPart { PRJ_BOTH = 0, PRJ_CD = 1, PRJ_DF = 2 };   // solve (+ solve_df if
 int prj_solve(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* st, int part);
 int prj_buffers(ivp_ctx* c, int passes);   // ivp_api.hip: PRJ buffers, history for `passes`
 int glue_gravity(ivp_ctx* c, const float g[3], float dt);
+// the input of stage `kind` for this context's particles
+ivp::NextIn next_in(ivp_ctx* c, ivp::NextKind kind, float dt, float coeff);
+// fold the last build's sums into the solver state if no pass has yet (ivp_grid.hip)
+int build_fold(ivp_ctx* c);
 
 // status of a build from its error flags
 inline int build_code(int flags) {

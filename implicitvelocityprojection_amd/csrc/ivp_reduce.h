@@ -22,7 +22,7 @@ __device__ __forceinline__ void block_partials(const double (&v)[NV], double* pa
 }
 
 enum FinOp {
-    FIN_BUILD, FIN_PACK, FIN_RHS, FIN_FIRST, FIN_CG_PAP, FIN_CG_UPDATE, FIN_W18_INIT, FIN_W18_PAP, FIN_W18_UPDATE,
+    FIN_BUILD, FIN_PACK, FIN_RHS, FIN_FIRST, FIN_FIRST_BUILD, FIN_CG_PAP, FIN_CG_UPDATE, FIN_W18_INIT, FIN_W18_PAP, FIN_W18_UPDATE,
     FIN_CG_REPLACE
 };
 
@@ -99,9 +99,11 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double* t, doub
         st->err_sum = t[0];
         st->n_active_rows = (int)t[1];
         st->active_pairs = (long long)t[2];
-    } else if (OP == FIN_FIRST) {   // the constraint pass's sums, then the right-hand side's
+    } else if (OP == FIN_FIRST || OP == FIN_FIRST_BUILD) {
+        // the constraint pass's sums, the right-hand side's, and the last build's if they are left
         fin_apply<FIN_PACK>(st, t, tol, max_iter);
         fin_apply<FIN_RHS>(st, t + 3, tol, max_iter);
+        if (OP == FIN_FIRST_BUILD) fin_apply<FIN_BUILD>(st, t + BUILD_ROW, tol, max_iter);
     } else if (OP == FIN_RHS || OP == FIN_W18_INIT) {
         double rr = t[0];
         if (OP == FIN_RHS) {
@@ -187,7 +189,7 @@ __device__ __forceinline__ void fin_apply(SolverState* st, const double* t, doub
 
 template <int OP>
 constexpr int fin_nv() {
-    return OP == FIN_FIRST ? 6 : OP == FIN_PACK || OP == FIN_RHS ? 3
+    return OP == FIN_FIRST_BUILD ? 8 : OP == FIN_FIRST ? 6 : OP == FIN_PACK || OP == FIN_RHS ? 3
            : OP == FIN_BUILD || OP == FIN_W18_UPDATE || OP == FIN_CG_REPLACE ? 2 : 1;
 }
 
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
     SolverState* st = a.st;
     const bool skip = OP == FIN_PACK && a.gated && (st->active != 0 || st->status != 0);
     if (!skip) {
-        double t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        double t[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         fold_partials<NV>(a.partials, a.stride, a.nblocks, t);
         if (threadIdx.x == 0) {
             fin_apply<OP>(st, t, a.tol, a.max_iter);
@@ -375,8 +377,9 @@ template <int OP>
 inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0, bool gated = false,
                     SolverState* host = nullptr, unsigned long long* mark = nullptr) {
     constexpr int NV = fin_nv<OP>();
-    Fold f{c->partials + (OP == FIN_RHS ? 3 : 0) * (size_t)c->max_blocks, c->max_blocks, nblocks};
-    if (NV > 1) IVP_TRY((fold_source<NV>(c, OP == FIN_RHS ? 3 : 0, nblocks, nullptr, &f)));
+    constexpr int row0 = OP == FIN_RHS ? 3 : OP == FIN_BUILD ? BUILD_ROW : 0;
+    Fold f{c->partials + row0 * (size_t)c->max_blocks, c->max_blocks, nblocks};
+    if (NV > 1) IVP_TRY((fold_source<NV>(c, row0, nblocks, nullptr, &f)));
     FinArgs fa{f.p, f.stride, f.n, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
     hipLaunchKernelGGL(k_finalize<OP>, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
     IVP_HIP(hipGetLastError());

@@ -393,15 +393,25 @@ __device__ __forceinline__ void row_pairs_w(bool win, const WinLds<FM, G>& w, co
 
 // ---- IP ------------------------------------------------------------------------------------
 
-// compute_constraint (pressure_base.py:169-184) and d = dt v (ip.py:343)
-__global__ __launch_bounds__(BLOCK) void k_ip_init(int nd, float dt, const float* __restrict__ density,
-                                                   const float* __restrict__ rho0, const float* __restrict__ vel,
-                                                   const float4* __restrict__ pos, float* __restrict__ cc,
-                                                   float4* __restrict__ d4) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    cc[i] = density[i] - rho0[i];
-    d4[i] = make_float4(dt * vel[3 * i + 0], dt * vel[3 * i + 1], dt * vel[3 * i + 2], pos[i].w);
+// The next stage's input from particle i's velocity: d = dt v (ip.py:343) with the mass, (v, m / rho) and
+// factor = dt mu_i / rho_i, mu_i = coeff rho0_i, of the Weiler18 operator, (v, m) or (v, rho)
+__device__ __forceinline__ void next_input(const NextIn& a, int i, float vx, float vy, float vz) {
+    if (a.kind == NEXT_NONE) return;
+    if (a.kind == NEXT_IP) {
+        a.out[i] = make_float4(a.dt * vx, a.dt * vy, a.dt * vz, a.pos[i].w);
+    } else if (a.kind == NEXT_W18) {
+        const float rho = a.density[i];
+        a.out[i] = make_float4(vx, vy, vz, a.pos[i].w / rho);
+        const float mu = a.coeff * a.rho0[i];
+        a.fac[i] = a.dt * mu / rho;
+    } else {
+        a.out[i] = make_float4(vx, vy, vz, a.kind == NEXT_ST ? a.pos[i].w : a.density[i]);
+    }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_next(int nd, const float* __restrict__ vel, NextIn a) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i < nd) next_input(a, i, vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2]);
 }
 
 // Neighbour record (x, y, z, m) of the J passes: positions are needed only to evaluate gradW;
@@ -423,7 +433,7 @@ struct PackArgs {
     Rows R;
     const float4* d4;
     const float* Ss;
-    const float* cc;
+    const float* density;
     const float* kk;
     const float* rho0;
     const int* rowcnt;
@@ -460,7 +470,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
     const WinPre wp = win_prefetch<FM, G>(a.R, blk);
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
     float4 di, xi;
-    float s0, s1, s2, cc, k, rho0;
+    float s0, s1, s2, density, k, rho0;
     int cnt;
     auto own = [&]() {
         di = a.d4[ic];
@@ -468,7 +478,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
     };
     auto tail = [&]() {
         s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2];
-        cc = a.cc[ic]; k = a.kk[ic]; rho0 = a.rho0[ic];
+        density = a.density[ic]; k = a.kk[ic]; rho0 = a.rho0[ic];
         cnt = a.rowcnt[ic];
     };
     if (!SC) {   // (scenes have no windows to wait for: their rows load when they need it)
@@ -492,7 +502,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
         if (SC) tail();
         float jd = acc + (di.x * s0 + di.y * s1 + di.z * s2);
         a.jd[i] = jd;
-        float t = jd + cc;
+        float t = jd + (density - rho0);   // compute_constraint (pressure_base.py:169-184)
         float f = fmaxf(t, 0.0f);
         float dfdt = t >= 1e-6f ? 1.0f : 0.0f;
         float sk = dfdt * k;
@@ -1137,19 +1147,12 @@ __global__ __launch_bounds__(BLOCK) void k_prj_save(int nd, const float2* __rest
 
 // ---- explicit viscosity (viscosity.py:9-108), Jacobi reads ---------------------------------
 
-__global__ __launch_bounds__(BLOCK) void k_v4(int nd, const float* __restrict__ vel, const float* __restrict__ density,
-                                              float4* __restrict__ v4) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    v4[i] = make_float4(vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2], density[i]);
-}
-
 // viscosity.py:62-108 with Jacobi reads.  Neighbour record: A = (x, y, z, m_j), m_j = 0 for a
 // non-fluid neighbour (its term is then exactly 0, as the reference's skip), B = (v_j, rho_j).
 template <class FM, bool ALLFLUID>
 __global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt, int fluid,
                                                 const float4* __restrict__ v4, const float* __restrict__ rho0,
-                                                const int* __restrict__ mat, float* __restrict__ vel) {
+                                                const int* __restrict__ mat, float* __restrict__ vel, NextIn next) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     // neighbour record: A = (x, y, z, m_j / rho_j), the quotient formed once per record instead of once
@@ -1174,7 +1177,10 @@ __global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt
     const LocPre lp = loc_prefetch<FM, PASS_LANES>(R, i, g);
     const bool win = stage_window(R, blk, wp, w, loadA, [&](int j) { return v4[j]; });
     if (i >= R.nd) return;
-    if (!ALLFLUID && mat[i] != fluid) return;
+    if (!ALLFLUID && mat[i] != fluid) {   // v stays
+        if (g == 0) next_input(next, i, vi.x, vi.y, vi.z);
+        return;
+    }
     float eps2 = (0.01f * R.h) * (0.01f * R.h);
     float k_visc = 2.0f * (3.0f + 2.0f);
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
@@ -1195,25 +1201,14 @@ __global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt
     ay = group_sum<PASS_LANES>(ay);
     az = group_sum<PASS_LANES>(az);
     if (g != 0) return;
-    vel[3 * i + 0] = vi.x + ax * dt;
-    vel[3 * i + 1] = vi.y + ay * dt;
-    vel[3 * i + 2] = vi.z + az * dt;
+    const float vx = vi.x + ax * dt, vy = vi.y + ay * dt, vz = vi.z + az * dt;
+    vel[3 * i + 0] = vx;
+    vel[3 * i + 1] = vy;
+    vel[3 * i + 2] = vz;
+    next_input(next, i, vx, vy, vz);
 }
 
 // ---- Weiler 2018 (weiler18.py) -------------------------------------------------------------
-
-// (v, m / rho) for the operator gathers and factor = dt mu_i / rho_i, mu_i = coeff rho0_i
-__global__ __launch_bounds__(BLOCK) void k_w18_prep(int nd, float coeff, float dt, const float* __restrict__ vel,
-                                                    const float4* __restrict__ pos, const float* __restrict__ density,
-                                                    const float* __restrict__ rho0, float4* __restrict__ v4,
-                                                    float* __restrict__ fac) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    float rho = density[i];
-    v4[i] = make_float4(vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2], pos[i].w / rho);
-    float mu = coeff * rho0[i];
-    fac[i] = dt * mu / rho;
-}
 
 __device__ __forceinline__ void inverse33(const float a[9], float out[9]) {
     float c00 = a[4] * a[8] - a[5] * a[7];
@@ -1552,6 +1547,7 @@ struct W18PArgs {
     Fold sums;           // the update pass's r.r and r.z
     SolverState* host;   // the last iteration of a chunk: the state is reported here
     const int* flags;
+    NextIn next;         // formed from the final velocities
 };
 
 // The end of an iteration: the stop test, dv += alpha p (the iteration's update,
@@ -1590,9 +1586,15 @@ __global__ __launch_bounds__(BLOCK) void k_w18_p(W18PArgs a) {
             a.p4[i] = p;
         }
     }
-    if (apply)
+    if (apply) {
+        float v1[3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) a.vel[3 * i + q] = a.vel[3 * i + q] + 1.0f * dv[q];
+        for (int q = 0; q < 3; ++q) {
+            v1[q] = a.vel[3 * i + q] + 1.0f * dv[q];
+            a.vel[3 * i + q] = v1[q];
+        }
+        next_input(a.next, i, v1[0], v1[1], v1[2]);
+    }
 }
 
 // ---- Jeske23 implicit surface tension (jeske23.py) -----------------------------------------
@@ -1911,24 +1913,15 @@ __global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a) {
     }
 }
 
-// (v, m) of the particles for the surface-tension passes
-__global__ __launch_bounds__(BLOCK) void k_st_prep(int nd, const float* __restrict__ vel, const float4* __restrict__ pos,
-                                                   float4* __restrict__ u4) {
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= nd) return;
-    u4[i] = make_float4(vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2], pos[i].w);
-}
-
-// ---- glue ----------------------------------------------------------------------------------
-
-// apply_gravity (framework.py:26-41)
 __global__ __launch_bounds__(BLOCK) void k_gravity(int nd, float gx, float gy, float gz, const float* __restrict__ vin,
-                                                   float* __restrict__ vout) {
+                                                   float* __restrict__ vout, NextIn next) {
     int i = blockIdx.x * BLOCK + threadIdx.x;
     if (i >= nd) return;
-    vout[3 * i + 0] = vin[3 * i + 0] + gx;
-    vout[3 * i + 1] = vin[3 * i + 1] + gy;
-    vout[3 * i + 2] = vin[3 * i + 2] + gz;
+    const float vx = vin[3 * i + 0] + gx, vy = vin[3 * i + 1] + gy, vz = vin[3 * i + 2] + gz;
+    vout[3 * i + 0] = vx;
+    vout[3 * i + 1] = vy;
+    vout[3 * i + 2] = vz;
+    next_input(next, i, vx, vy, vz);
 }
 
 Rows rows_of(ivp_ctx* c) {
@@ -1991,7 +1984,7 @@ int enqueue_scene_replay_g(ivp_ctx* c, hipStream_t st, float omega, int K) {
     FinScenesArgs fa{P, stride, c->sid, c->ss, c->sprm, c->shist_err, c->shist_pcg, c->S, BLOCK};
     FinScenesArgs fp = fa;   // partials of the pair passes: BLOCK / G rows per block
     fp.rpb = BLOCK / G;
-    PackArgs pa{R, c->d4, c->Ss, c->cc, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, P, stride, sc};
+    PackArgs pa{R, c->d4, c->Ss, c->density, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, P, stride, sc};
     hipLaunchKernelGGL((k_ip_pack<FmtIds, true, G>), np, blk, 0, st, pa);
     hipLaunchKernelGGL(k_fin_scenes<FIN_PACK>, nf, blk, 0, st, fp);
     RhsArgs ra{R, c->q4, c->Ss, omega, nullptr, c->sol, c->r, c->p4, c->y2, c->nbact, c->rowcnt, P, stride, sc};
@@ -2060,6 +2053,23 @@ int scene_graph(ivp_ctx* c, float omega, int K, hipGraphExec_t* out) {
     slot.win = win;
     *out = exec;
     return IVP_OK;
+}
+
+// The stage's own input: left by the stage before it in a step, else formed here
+int stage_input(ivp_ctx* c, NextKind kind, float dt, float coeff) {
+    const bool ready = c->ready == kind;
+    c->ready = NEXT_NONE;
+    if (ready) return IVP_OK;
+    return launch(c, KC_GLUE, -1, 0.0, k_next, dim3(blocks_for(c->nd)), c->nd, (const float*)c->vel,
+                  next_in(c, kind, dt, coeff));
+}
+
+// What the stage being enqueued leaves for the next one
+NextIn take_next(ivp_ctx* c) {
+    const NextIn n = c->next;
+    c->next = NextIn{};
+    c->ready = n.kind;
+    return n;
 }
 
 __global__ void k_report(SolverState* st, SolverState* host, const int* flags) { report_state(st, host, flags); }
@@ -2132,8 +2142,8 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
     const double pb = pair_bytes<FP>(), pbc = pair_bytes<FC>();
     Rows R = rows_of(c);
     float4* d4 = c->d4;
-    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_init, nb, nd, dt, (const float*)c->density, (const float*)c->rho0,
-                   (const float*)c->vel, (const float4*)c->pos, c->cc, d4));
+    IVP_TRY(stage_input(c, NEXT_IP, dt, 0.0f));
+    if (prm->max_iteration_opt < 1 || PASS_LANES != 4) IVP_TRY(build_fold(c));   // (no first solve to fold them with)
     int opt_iter = 0;
     bool spec_finish = false;   // k_ip_finish enqueued before the last read-back
     bool pack_queued = false;   // this evaluation's passes were queued behind the CG's read-back
@@ -2142,7 +2152,7 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
     double err = 0.0;
     for (;;) {
         IVP_TRY(marks_buffer(c, opt_iter + 2));
-        PackArgs pa{R, d4, c->Ss, c->cc, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, c->partials, stride};
+        PackArgs pa{R, d4, c->Ss, c->density, c->kk, c->rho0, c->rowcnt, c->q4, c->sfac, c->jd, c->partials, stride};
         double total_pairs = (double)c->state_host->total_pairs;
         const bool deferred = opt_iter == 0 && prm->max_iteration_opt >= 1;
         // the constraint pass of evaluation k and its finalize, which reports the state
@@ -2194,9 +2204,12 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
         RhsArgs ra{R, c->q4, c->Ss, prm->omega, FC::GS == GS_F16 ? c->b : nullptr, c->sol, c->r, c->p4, c->y2, c->nbact,
                    c->rowcnt, c->partials + 3 * (size_t)stride, stride};
         IVP_TRY(launch(c, KC_IP_RHS, -1, stream_bytes<FP>(c, total_pairs) + 48.0 * nd, k_ip_rhs<FP, false>, np, ra));
-        if (deferred)
+        if (deferred && c->build_pending) {
+            c->build_pending = false;
+            IVP_TRY(finalize<FIN_FIRST_BUILD>(c, np.x, prm->tol_pcg, prm->max_iteration_pcg, false, nullptr, c->marks + 1));
+        } else if (deferred) {
             IVP_TRY(finalize<FIN_FIRST>(c, np.x, prm->tol_pcg, prm->max_iteration_pcg, false, nullptr, c->marks + 1));
-        else
+        } else
             IVP_TRY(finalize<FIN_RHS>(c, np.x, prm->tol_pcg, prm->max_iteration_pcg));
         // The first CG chunk is enqueued without waiting for the set-up: its kernels return at once
         // when there is nothing to solve.  The J^T byte model (touched rows, reported by the set-up)
@@ -2310,26 +2323,27 @@ template <class FM>
 int visc_explicit_body(ivp_ctx* c, float coeff, float dt) {
     const int nd = c->nd;
     const dim3 nb(blocks_for(nd));
-    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_v4, nb, nd, (const float*)c->vel, (const float*)c->density, c->v4));
+    IVP_TRY(stage_input(c, NEXT_VISC, dt, coeff));
+    const NextIn next = take_next(c);
     double bytes = stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 48.0 * nd;
     Rows R = rows_of(c);
     if (c->all_dyn_fluid)
         return launch(c, KC_VISC, -1, bytes, k_visc<FM, true>, pass_grid(nd), R, coeff, dt, c->cfg.material_fluid,
-                      (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel);
+                      (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel, next);
     return launch(c, KC_VISC, -1, bytes, k_visc<FM, false>, pass_grid(nd), R, coeff, dt, c->cfg.material_fluid,
-                  (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel);
+                  (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel, next);
 }
 
 // The rest of a Weiler18 / Jeske23 CG iteration after its operator pass (npap blocks); partial rows:
 // p.Ap 0, r.r 1, r.z 2
-int w18_update(ivp_ctx* c, const W18Args& cg, int npap, int tag, SolverState* host) {
+int w18_update(ivp_ctx* c, const W18Args& cg, int npap, int tag, SolverState* host, const NextIn& next) {
     const int nd = c->nd;
     const dim3 nb(blocks_for(nd));
     W18Args u = cg;
     u.partials = c->partials + c->max_blocks;
     IVP_TRY(fold_source<1>(c, 0, npap, c->state, &u.pap));
     IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, u));
-    W18PArgs p{nd, c->w_z, c->w_p4, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag};
+    W18PArgs p{nd, c->w_z, c->w_p4, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag, next};
     IVP_TRY(fold_source<2>(c, 1, nb.x, c->state, &p.sums));
     return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, p);
 }
@@ -2340,8 +2354,9 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
     const dim3 nb(blocks_for(nd));
     const int stride = c->max_blocks;
     Rows R = rows_of(c);
-    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_w18_prep, nb, nd, coeff, dt, (const float*)c->vel, (const float4*)c->pos,
-                   (const float*)c->density, (const float*)c->rho0, c->w_v4, c->w_fac));
+    IVP_TRY(stage_input(c, NEXT_W18, dt, coeff));
+    const NextIn next = take_next(c);
+    if (c->prof) IVP_TRY(build_fold(c));   // (the byte figures of the timed passes)
     const double pairs = (double)c->state_host->total_pairs;
     const double pb = pair_bytes<FM>();
     W18Args wa{R, c->cfg.material_fluid, c->w_fac, c->mat, c->w_pinv, c->w_v4, c->w_rhs,
@@ -2372,7 +2387,7 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         const double bAv = stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 48.0 * nd;
         auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_W18_AV, tag, bAv, k_w18_Av<FM, ALLFLUID>, pass_grid(nd), cg));
-            return w18_update(c, cg, pass_grid(nd).x, tag, host);
+            return w18_update(c, cg, pass_grid(nd).x, tag, host, next);
         };
         // the save of the correction follows each chunk's report, running once the solve has stopped
         // (while the host reads the state)
@@ -2413,7 +2428,9 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
               c->w_rhs, sigma, dt, d, hst, 1.0f / hst, tn, tnh, c->partials, stride, c->state};
     const double pairs = (double)c->state_host->total_pairs;
     const double pb = pair_bytes<FM>();
-    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_st_prep, nb, nd, (const float*)c->vel, (const float4*)c->pos, c->w_v4));
+    IVP_TRY(stage_input(c, NEXT_ST, dt, 0.0f));
+    const NextIn next = take_next(c);
+    if (c->prof) IVP_TRY(build_fold(c));
     IVP_TRY(launch(c, KC_ST_SETUP, -1, stream_bytes<FM>(c, pairs) + 36.0 * nd, k_st_div<FM, ALLFLUID>, np, sa));
     IVP_TRY(launch(c, KC_ST_SETUP, -1, (pb + 4.0) * pairs + 72.0 * nd, k_st_setup<FM, ALLFLUID>, np, sa));
     IVP_TRY(launch(c, KC_ST_AV, -1, stream_bytes<FM>(c, pairs) + 4.0 * pairs + 40.0 * nd, k_st_Av<FM, ALLFLUID, true>, np, sa));
@@ -2433,7 +2450,7 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
         const double bAv = stream_bytes<FM>(c, pairs) + 4.0 * pairs + 28.0 * nd;
         auto one_iter = [&](int tag, SolverState* host) -> int {
             IVP_TRY(launch(c, KC_ST_AV, tag, bAv, k_st_Av<FM, ALLFLUID, false>, np, cga));
-            return w18_update(c, cg, np.x, tag, host);
+            return w18_update(c, cg, np.x, tag, host, next);
         };
         auto tail = [](bool) { return (int)IVP_OK; };
         c->prof_epoch++;
@@ -2681,6 +2698,7 @@ int prj_solve(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* sta
     if (prm->max_iteration_opt < 0 || prm->df_num_threshold < 0) return IVP_ERR_ARG;
     stats_zero(stats);
     IVP_TRY(prj_buffers(c, prm->max_iteration_opt + 1));
+    IVP_TRY(build_fold(c));   // (its statistics count the pairs)
     const int fmt = c->row_fmt;
     if (part != PRJ_DF) {
         int rc = fmt == IVP_ROWS_F32   ? prj_solve_body<FmtF32>(c, dt, prm, stats)
@@ -2745,8 +2763,7 @@ int ip_solve_scenes(ivp_ctx* c, float dt, const ivp_ip_params* prm) {
     hp.max_pcg = prm->max_iteration_pcg;
     hp.fixed = prm->use_fixed_iters ? 1 : 0;
     IVP_HIP(hipMemcpyAsync(c->sprm, c->sprm_host, sizeof(SceneParams), hipMemcpyHostToDevice, c->stream));
-    IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_init, nb, nd, dt, (const float*)c->density, (const float*)c->rho0,
-                   (const float*)c->vel, (const float4*)c->pos, c->cc, c->d4));
+    IVP_TRY(stage_input(c, NEXT_IP, dt, 0.0f));
     hipLaunchKernelGGL(k_scene_init, dim3((c->S + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, c->stream, c->S, c->ss);
     IVP_HIP(hipGetLastError());
     const int K = std::max(1, c->scene_chunk);
@@ -2783,11 +2800,17 @@ int ip_solve_scenes(ivp_ctx* c, float dt, const ivp_ip_params* prm) {
 
 // v + g dt into the second velocity buffer, which becomes the first; the previous velocities stay
 // in the second until the next re-sort, so a step that must not start can restore them
+NextIn next_in(ivp_ctx* c, NextKind kind, float dt, float coeff) {
+    if (kind == NEXT_NONE) return NextIn{};
+    float4* out = kind == NEXT_IP ? c->d4 : kind == NEXT_VISC ? c->v4 : c->w_v4;
+    return NextIn{kind, dt, coeff, c->pos, c->density, c->rho0, out, c->w_fac};
+}
+
 int glue_gravity(ivp_ctx* c, const float g[3], float dt) {
     if (!c->loaded) return IVP_ERR_STATE;
     if (c->nd == 0) return IVP_OK;
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_gravity, dim3(blocks_for(c->nd)), c->nd, g[0] * dt, g[1] * dt, g[2] * dt,
-                   (const float*)c->vel, c->vel_b));
+                   (const float*)c->vel, c->vel_b, take_next(c)));
     std::swap(c->vel, c->vel_b);
     return IVP_OK;
 }
