@@ -1953,12 +1953,13 @@ int grid_build(ivp_ctx* c, const float* adv_dt, bool report) {
         IVP_HIP(hipMemsetAsync(c->dstart, 0, sizeof(int) * (size_t)(c->ncell + 1), c->stream));
         IVP_HIP(hipMemsetAsync(c->err_flag, 0, sizeof(int), c->stream));   // (else cleared by the sort)
     }
-    // tile windows, where a tile's walked slots fit the search (Cs * 32 word pairs, PPT per thread); not
-    // for independent scenes: their passes run late in a batched solve on few active blocks, and
-    // windows over every scene's rows cost more than they saved (4.28 -> 4.48 ms per step on 256
-    // columns)
+    // tile windows, where a tile's walked slots fit the search (Cs * 32 word pairs, PPT per thread).
+    // Independent scenes whose passes run four lanes per row have them too: found in a pass of their own
+    // they cost more than they saved (256 columns 4.28 -> 4.48 ms per step), found by the exact pass
+    // they save more (64 scenes, two builds and a solve: 1788 -> 1744 us)
     const int ppt = (c->Cs * (WAVE / 2) + BLOCK - 1) / BLOCK;
-    const bool windows = c->nd > 0 && c->windows && c->rec_words == 64 && c->S == 0 && ppt <= 32;
+    const bool windows = c->nd > 0 && c->windows && c->rec_words == 64 &&
+                         (c->S == 0 ? ppt <= 32 : ppt <= 8 && c->scene_lanes == 4 && build_lanes_for(c) != 1);
     bool fused = false;   // the exact pass finds the windows
     int tiles_per_block = WAVES_PER_BLOCK;   // of the pass that writes the build's partials
     if (c->nd > 0) {

@@ -277,7 +277,7 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
     }
 }
 
-// Tile windows: the block of a four-lane pass over one scene is one 64-row tile.  stage_window
+// Tile windows: the block of a four-lane pass is one 64-row tile.  stage_window
 // loads the tile's window into LDS, A[k] = la(win[k]) and B[k] = lb(win[k]) (the pass's B record
 // in the first NB components of a float4), and returns true; it returns false, staging nothing,
 // when the rows have no windows or this tile has none.  Every thread of the block calls it (it
@@ -285,6 +285,12 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
 // the window, or through memory when there is none: the same values in the same order.
 template <class FM, int G>
 constexpr bool has_windows() { return FM::REC == 64u && G == 4; }
+
+// Passes that may stage a window request their rows' data before it; a pass over scenes with fewer
+// lanes has no window to wait for, and its rows load when they need it (the rest of a solve finds most
+// of them in another phase).
+template <class FM, bool SC, int G>
+constexpr bool eager_loads() { return !SC || has_windows<FM, G>(); }
 
 template <class FM, int G>
 struct WinLds {
@@ -456,7 +462,8 @@ __device__ __forceinline__ bool cg_stopped(const SolverState* st) { return st->a
 // (math_utils.py:76-91, pressure_base.py:187-203, 413-423).  J d in the form of
 // compute_J_x_kernel (pressure_base.py:111-127): sum_j m_j dot(d_i - d_j, gradW_ij) + dot(d_i, S_i).
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
+__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_pack(PackArgs a) {
+    constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.gate && !cg_stopped(a.gate)) return;
     if (!SC && a.mark && blockIdx.x == 0 && threadIdx.x == 0) *a.mark = wall_clock64();
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -481,7 +488,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
         density = a.density[ic]; k = a.kk[ic]; rho0 = a.rho0[ic];
         cnt = a.rowcnt[ic];
     };
-    if (!SC) {   // (scenes have no windows to wait for: their rows load when they need it)
+    if (EAGER) {
         own();
         tail();
     }
@@ -490,7 +497,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
     double err = 0.0, nact = 0.0, npairs = 0.0;
     float acc = 0.0f;
     if (gt.on) {
-        if (SC) own();
+        if (!EAGER) own();
         row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                              [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
                                  float dx = di.x - Bj.v[0], dy = di.y - Bj.v[1], dz = di.z - Bj.v[2];
@@ -499,7 +506,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_pack(PackArgs a) {
         acc = group_sum<G>(acc);
     }
     if (gt.on && g == 0) {
-        if (SC) tail();
+        if (!EAGER) tail();
         float jd = acc + (di.x * s0 + di.y * s1 + di.z * s2);
         a.jd[i] = jd;
         float t = jd + (density - rho0);   // compute_constraint (pressure_base.py:169-184)
@@ -542,7 +549,8 @@ struct RhsArgs {
 // x = 0, r = b, rr = r.r, p = r) is part of the pass; as a launch of its own with its own finalize
 // it took 18 us at 1M rows and 5 at 8k.
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
+__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_rhs(RhsArgs a) {
+    constexpr bool EAGER = eager_loads<FM, SC, G>();
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
     Gate gt = gate_all(i, a.R.nd);
@@ -572,7 +580,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
         s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2];
         cnt = a.rowcnt[ic];
     };
-    if (!SC) {
+    if (EAGER) {
         own();
         tail();
     }
@@ -580,7 +588,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.q4[j]; });
     double touched = 0.0, tpairs = 0.0, rr = 0.0;
     if (gt.on) {
-        if (SC) own();
+        if (!EAGER) own();
         float fki = qi.x, mi = qi.z;
         bool act = qi.y != 0.0f;
         float rx = 0.0f, ry = 0.0f, rz = 0.0f;
@@ -595,7 +603,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_ip_rhs(RhsArgs a) {
         rz = group_sum<G>(rz);
         act = group_any<G>(act);
         if (g == 0) {
-            if (SC) tail();
+            if (!EAGER) tail();
             rx += fki * s0;
             ry += fki * s1;
             rz += fki * s2;
@@ -632,7 +640,8 @@ struct CGJArgs {
 // compute_Jx_pcg (ip.py:19-60): y_i = dfdt_i k_i (J p)_i on rows with dfdt > 0, J p in the form
 // sum_j dot(p_i - p_j, m_j gradW_ij) + dot(p_i, S_i) (ip.py:51-58)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_J(CGJArgs a) {
+__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_J(CGJArgs a) {
+    constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
@@ -648,7 +657,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_J(CGJArgs a) {
         xi = a.R.pos[ic];
     };
     auto tail = [&]() { s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2]; };
-    if (!SC) {
+    if (EAGER) {
         own();
         tail();
     }
@@ -665,7 +674,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_J(CGJArgs a) {
         win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.p4[j]; });
     }
     if (sk == 0.0f) return;
-    if (SC) own();
+    if (!EAGER) own();
     float acc = 0.0f;
     row_pairs_w<FM, 3, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                          [&](const float4& Aj, const Vec<3>& Bj, float gx, float gy, float gz) {
@@ -674,7 +683,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_J(CGJArgs a) {
                          }, g);
     acc = group_sum<G>(acc);
     if (g != 0) return;
-    if (SC) tail();
+    if (!EAGER) tail();
     acc = acc + (pi.x * s0 + pi.y * s1 + pi.z * s2);
     a.y2[i] = make_float2(acc * sk, pi.w);
 }
@@ -696,7 +705,8 @@ struct CGJTArgs {
 // compute_Ax_part1 + compute_Ax_part2 (ip.py:63-121) in gather form, fused with p.Ap
 // (ip.py:307)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_JT(CGJTArgs a) {
+__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_JT(CGJTArgs a) {
+    constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
@@ -713,7 +723,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_JT(CGJTArgs a) {
         yi = a.y2[ic].x;
     };
     auto tail = [&]() { s0 = a.Ss[3 * ic + 0]; s1 = a.Ss[3 * ic + 1]; s2 = a.Ss[3 * ic + 2]; };
-    if (!SC) {
+    if (EAGER) {
         own();
         tail();
     }
@@ -744,7 +754,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_JT(CGJTArgs a) {
         float mi = pi.w;
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         if (touched) {
-            if (SC) own();
+            if (!EAGER) own();
             row_pairs_w<FM, 1, G>(win, w, lp, a.R, i, xi, loadA, loadB,
                                  [&](const float4& Aj, const Vec<1>& Bj, float gx, float gy, float gz) {
                                      float sc = fmaf(Aj.w, yi, mi * Bj.v[0]);
@@ -753,7 +763,7 @@ __global__ __launch_bounds__(BLOCK, SC ? 1 : 8) void k_cg_JT(CGJTArgs a) {
             ax = group_sum<G>(ax);
             ay = group_sum<G>(ay);
             az = group_sum<G>(az);
-            if (SC) tail();
+            if (!EAGER) tail();
             ax += yi * s0;
             ay += yi * s1;
             az += yi * s2;

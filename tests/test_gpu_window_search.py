@@ -49,3 +49,25 @@ def test_window_search_in_the_exact_pass(n, C, rows, cap):
         assert stats[1] == stats[0], stats
     for a, b, c in zip(got, ref, off):
         assert np.array_equal(a, b) and np.array_equal(a, c)
+
+
+def test_scene_windows_bitwise():
+    """Independent scenes with four lanes per row: tiles that span two scenes, with and without windows."""
+    from implicitvelocityprojection_amd import _native as N
+    from implicitvelocityprojection_amd.scene_batch import SceneBatch
+    from implicitvelocityprojection_amd.scenes import synthetic_batch
+    out = []
+    for windows in (1, 300, 0):
+        b = SceneBatch(synthetic_batch(5, seed=3, count_range=(300, 2500)), chunk=2, lanes=4)
+        N.check(b.ctx.lib.ivp_set_option(b.ctx.h, N.OPT_TILE_WINDOWS, windows), "ivp_set_option")
+        assert b.ctx.neighbors_build() == N.IVP_OK
+        tiles, windowed, _ = b.ctx.window_stats()
+        assert (windowed == 0) == (windows == 0) and windowed <= tiles
+        for _ in range(3):
+            b.step()
+        f = {N.FIELD_X: (b.n, 3), N.FIELD_V: (b.n, 3), N.FIELD_DENSITY: (b.n,), N.FIELD_DIVERGENCE: (b.n,)}
+        out.append([b.ctx.read(k, torch.zeros(s, device="cuda")).cpu().numpy().view(np.uint32) for k, s in f.items()])
+        b.close()
+    for got in out[:2]:
+        for x, y in zip(got, out[2]):
+            assert np.array_equal(x, y)
