@@ -213,13 +213,18 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
 
 // ---- folds by the pass that needs the sum ---------------------------------------------------
 //
-// A finalize launch between two passes costs 2 us and the gap before it for a few scalars.  With at
-// most FOLD_MAX partials (16 KB, in L2) every block of the next pass folds them itself, all to the
-// same bits, and one block writes the state; above it a block's fold takes as long as the launch
-// that it saves, and k_prefold first reduces each row to PREFOLD partials in one short launch of
-// many blocks (15 625 partials: 2.4 us; the one-block finalize took 4.6, with two rows 7.9, with three
-// 9.1: the bandwidth of one CU).
-constexpr int FOLD_MAX = 2048;
+// A finalize launch between two passes costs 2 us and the gap before it for a few scalars.  While the
+// readers' blocks times the partials stay below FOLD_READS (42 MB a row, from L2) every block of the next
+// pass folds them itself, all to the same bits, and one block writes the state; above it the folds take
+// longer than the launch that they save, and k_prefold first reduces each row to PREFOLD partials in
+// one short launch of many blocks (15 625 partials: 2.4 us; the one-block finalize took 4.6, with two
+// rows 7.9, with three 9.1: the bandwidth of one CU).  p.Ap has nd / 64 partials, an update's sums
+// nd / 256, and both are read by nd / 256 blocks.  us per implicit viscosity solve, prefolded /
+// folded by the readers: p.Ap at 133k rows 420 / 390, 176k 506 / 480, 262k (4.2 million reads) 879 / 861,
+// 350k (7.5 million) 1079 / 1108; the sums at 500k (3.8 million) 1378 / 1359, 750k (8.6 million) 1908 / 1956, 1M
+// 2371 / 2535.
+constexpr long long FOLD_READS = 5ll << 20;
+constexpr int FIN_MAX = 2048;   // partials per row that the one-block finalize folds alone
 
 // `meanwhile` runs with the first partials in flight: the caller's own loads, which would otherwise wait
 // for the fold (23k rows: update 3.8 -> 3.4 us, p pass 3.9 -> 3.5).
@@ -255,8 +260,7 @@ __device__ __forceinline__ void block_fold(const double* __restrict__ p, int str
 // Row q of n partials to PREFOLD partials: block b folds the b-th share
 template <int NV>
 __global__ __launch_bounds__(BLOCK) void k_prefold(const double* __restrict__ p, int stride, int n,
-                                                   double* __restrict__ out, const SolverState* __restrict__ gate) {
-    if (gate && gate->active == 0) return;
+                                                   double* __restrict__ out) {
     const int per = (n + PREFOLD - 1) / PREFOLD;
     const int k0 = (int)blockIdx.x * per < n ? (int)blockIdx.x * per : n;
     double t[NV];
@@ -272,15 +276,15 @@ struct Fold {
     int stride, n;
 };
 
-// The partials in rows row0 .. row0 + NV - 1, brought down to PREFOLD per row if there are many (gate:
-// skipped once that solve has stopped)
+// The partials in rows row0 .. row0 + NV - 1 for `readers` blocks that each fold them, brought down to
+// PREFOLD per row if that is less work
 template <int NV>
-inline int fold_source(ivp_ctx* c, int row0, int n, const SolverState* gate, Fold* f) {
+inline int fold_source(ivp_ctx* c, int row0, int n, int readers, Fold* f) {
     const double* p = c->partials + (size_t)row0 * c->max_blocks;
     *f = Fold{p, c->max_blocks, n};
-    if (n <= FOLD_MAX) return IVP_OK;
+    if ((long long)n * readers <= FOLD_READS) return IVP_OK;
     double* out = c->partials + (size_t)PARTIAL_ROWS * c->max_blocks + row0 * PREFOLD;
-    hipLaunchKernelGGL(k_prefold<NV>, dim3(PREFOLD), dim3(BLOCK), 0, c->stream, p, c->max_blocks, n, out, gate);
+    hipLaunchKernelGGL(k_prefold<NV>, dim3(PREFOLD), dim3(BLOCK), 0, c->stream, p, c->max_blocks, n, out);
     IVP_HIP(hipGetLastError());
     *f = Fold{out, PREFOLD, PREFOLD};
     return IVP_OK;
@@ -379,7 +383,7 @@ inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0,
     constexpr int NV = fin_nv<OP>();
     constexpr int row0 = OP == FIN_RHS ? 3 : OP == FIN_BUILD ? BUILD_ROW : 0;
     Fold f{c->partials + row0 * (size_t)c->max_blocks, c->max_blocks, nblocks};
-    if (NV > 1) IVP_TRY((fold_source<NV>(c, row0, nblocks, nullptr, &f)));
+    if (NV > 1 && nblocks > FIN_MAX) IVP_TRY((fold_source<NV>(c, row0, nblocks, 1 << 20, &f)));
     FinArgs fa{f.p, f.stride, f.n, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
     hipLaunchKernelGGL(k_finalize<OP>, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
     IVP_HIP(hipGetLastError());

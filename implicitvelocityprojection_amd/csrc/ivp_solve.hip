@@ -1484,22 +1484,72 @@ __global__ __launch_bounds__(BLOCK) void k_w18_init(W18Args a, float4* __restric
     block_partials<1>(v, a.partials, a.stride);
 }
 
+// The end of the iteration before, taken into this iteration's operator pass (k_w18_p's work, but for a
+// chunk's last iteration): the stop test, dv += alpha p, and p = z + beta p formed for the row and for
+// each of its neighbours from z and the old p, the row's own stored into the other of two buffers.
+// One launch less per iteration for 12 B more per window entry, so up to FUSE_P_MAX rows (us per implicit
+// viscosity solve, as a pass of its own / here: 4k rows 238 / 202, 12k 256 / 216, 50k 286 / 256, 90k 338 / 292,
+// 133k 397 / 377, 176k 480 / 481, 262k 858 / 903).
+constexpr int FUSE_P_MAX = 5 << 15;
+struct PStep {
+    const float* z;
+    const float4* p;     // the old direction
+    float4* next;
+    float* dv;
+    Fold sums;           // the update pass's r.r and r.z
+    const int* flags;
+
+    __device__ __forceinline__ float4 at(int j, float beta) const {
+        float4 q = p[j];
+        q.x = z[3 * j + 0] + beta * q.x;
+        q.y = z[3 * j + 1] + beta * q.y;
+        q.z = z[3 * j + 2] + beta * q.z;
+        return q;
+    }
+};
+
+// Advances the solve; returns false when the pass has nothing (more) to do.  pi becomes the new p of row i.
+__device__ __forceinline__ bool p_step(const PStep& n, SolverState* st, int i, int nd, int g, float4& pi, float* beta) {
+    const int ic = i < nd ? i : nd - 1;
+    const float alpha = (float)st->alpha;
+    const float z[3] = {n.z[3 * ic + 0], n.z[3 * ic + 1], n.z[3 * ic + 2]};
+    const Advance v = fold_advance<FIN_W18_UPDATE>(st, n.sums, nullptr, n.flags, []() {});
+    if (!v.ran) return false;
+    const bool own = i < nd && g == 0;
+    if (own) {
+        n.dv[3 * i + 0] = n.dv[3 * i + 0] + alpha * pi.x;
+        n.dv[3 * i + 1] = n.dv[3 * i + 1] + alpha * pi.y;
+        n.dv[3 * i + 2] = n.dv[3 * i + 2] + alpha * pi.z;
+    }
+    if (!v.active) return false;
+    pi.x = z[0] + v.beta * pi.x;
+    pi.y = z[1] + v.beta * pi.y;
+    pi.z = z[2] + v.beta * pi.z;
+    if (own) n.next[i] = pi;
+    *beta = v.beta;
+    return true;
+}
+
 // Ap = A p, p.Ap (weiler18.py:337-338).  Without CHECK (the warm-start residual) it runs
 // regardless of the solver state.
-template <class FM, bool ALLFLUID, bool CHECK = true>
-__global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a) {
-    if (CHECK && a.st->active == 0) return;
+template <class FM, bool ALLFLUID, bool CHECK = true, bool NEXT = false>
+__global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a, PStep n) {
+    if (CHECK && !NEXT && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
+    float beta = 0.0f;
+    auto vec = [&](int j) { return NEXT ? n.at(j, beta) : a.v4[j]; };
     auto loadA = [&](int j) { return w18_Av_record<FM, ALLFLUID>(a, j); };
-    auto loadB = [&](int j) { return vec3_of(a.v4, j); };
+    auto loadB = [&](int j) { return vec_of<3>(vec(j)); };
     __shared__ WinLds<FM, PASS_LANES> w;
     const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
-    const float4 pi = a.v4[ic], xi = a.R.pos[ic];
+    float4 pi = a.v4[ic];
+    const float4 xi = a.R.pos[ic];
     const float f = a.fac[ic];
     const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
-    const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.v4[j]; });
+    if (NEXT && !p_step(n, a.st, i, a.R.nd, g, pi, &beta)) return;
+    const bool win = stage_window(a.R, blk, wp, w, loadA, vec);
     double pap = 0.0;
     if (i < a.R.nd) {
         float3 Ap = w18_Av_row<FM, ALLFLUID, PASS_LANES>(a, i, pi, xi, f, win, w, lp, loadA, loadB, g);
@@ -1656,7 +1706,7 @@ struct StArgs {
     float tn, tnh;     // theta * 8/(pi h_st^3), and that times 1/h_st
     double* partials;
     int stride;
-    const SolverState* st;
+    SolverState* st;
 };
 
 // compute_divergence_jeske23 (jeske23.py:73-112): div_i = sum_fluid m_j (v_i - v_j) . gradW_ij
@@ -1831,9 +1881,9 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
 // compute_Av_jeske23 (jeske23.py:245-295): (M u)_i = u_i + dt^2 (sigma/m_i) sum m_bar g~ (u_i - u_j).
 // RHS: out = u - M u + b (jeske23.py:637-647); otherwise out = M u and the block's p.Mp partial.
 // Only the ids and g~ are streamed and (u_j, m_j) gathered: positions are not needed.
-template <class FM, bool ALLFLUID, bool RHS>
-__global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a) {
-    if (!RHS && a.st->active == 0) return;
+template <class FM, bool ALLFLUID, bool RHS, bool NEXT = false>
+__global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a, PStep n) {
+    if (!RHS && !NEXT && a.st->active == 0) return;
     constexpr unsigned REC = FM::REC;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
@@ -1841,10 +1891,12 @@ __global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a) {
     __shared__ WinLds<FM, PASS_LANES> w;
     const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
-    const float4 ui = a.u4[ic];
+    float4 ui = a.u4[ic];
+    float beta = 0.0f;
+    auto vec = [&](int j) { return NEXT ? n.at(j, beta) : a.u4[j]; };
     const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
-    const bool win = stage_window(a.R, blk, wp, w, [](int) { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); },
-                                  [&](int j) { return a.u4[j]; });
+    if (NEXT && !p_step(n, a.st, i, a.R.nd, g, ui, &beta)) return;
+    const bool win = stage_window(a.R, blk, wp, w, [](int) { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); }, vec);
     double pap = 0.0;
     if (i < a.R.nd) {
         float Mx = ui.x, My = ui.y, Mz = ui.z;
@@ -1860,7 +1912,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a) {
                 sy = sy + w * (ui.y - uj.y);
                 sz = sz + w * (ui.z - uj.z);
             };
-            auto visit = [&](int j, float gt) { visit_u(a.u4[j], gt); };
+            auto visit = [&](int j, float gt) { visit_u(vec(j), gt); };
             if (has_windows<FM, PASS_LANES>() && win) {
                 // window indices of slots g + 8 b and g + 4 + 8 b: one 32-bit word
                 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -2084,7 +2136,7 @@ NextIn take_next(ivp_ctx* c) {
 
 __global__ void k_report(SolverState* st, SolverState* host, const int* flags) { report_state(st, host, flags); }
 
-// Enqueue CG iterations in chunks until the device-side state says stop.  `launch_it(tag, host)`
+// Enqueue CG iterations in chunks until the device-side state says stop.  `launch_it(tag, host, first)`
 // enqueues one iteration; the last one of a chunk reports the state to `host`.  After each chunk
 // `tail(none)` is enqueued (work that follows a finished solve and returns at once while it continues;
 // `none` when there was no iteration), then the host waits for the report alone: the device runs the
@@ -2104,7 +2156,7 @@ int run_chunks(ivp_ctx* c, int max_iter, int guess, L&& launch_it, int* iters, i
             hipLaunchKernelGGL(k_report, dim3(1), dim3(1), 0, c->stream, c->state, c->state_host, (const int*)c->err_flag);
             IVP_HIP(hipGetLastError());
         }
-        for (int q = 0; q < todo; ++q) IVP_TRY(launch_it(issued + q, q == todo - 1 ? c->state_host : nullptr));
+        for (int q = 0; q < todo; ++q) IVP_TRY(launch_it(issued + q, q == todo - 1 ? c->state_host : nullptr, q == 0));
         issued += todo;
         IVP_HIP(hipEventRecord(c->wait_ev, c->stream));
         IVP_TRY(tail(todo == 0));
@@ -2247,10 +2299,10 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             CGJArgs jx{R, c->xs4, c->Ss, c->sfac, c->y2, c->state};
             CGJTArgs tx{R, c->xs4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials + 3 * (size_t)stride, stride,
                         c->state};
-            auto one_iter = [&](int tag, SolverState* host) -> int {
+            auto one_iter = [&](int tag, SolverState* host, bool) -> int {
                 IVP_TRY(launch(c, KC_CG_J, tag, bJ, k_cg_J<FC, false>, np, ja));
                 IVP_TRY(launch(c, KC_CG_JT, tag, bJT, k_cg_JT<FC, false>, np, ta));
-                IVP_TRY(fold_source<1>(c, 0, np.x, c->state, &ua.pap));
+                IVP_TRY(fold_source<1>(c, 0, np.x, nb.x, &ua.pap));
                 IVP_TRY(launch(c, KC_CG_UPDATE, tag, bU, k_cg_update<false>, nb, ua));
                 if (FC::GS == GS_F16 && (tag + 1) % REFRESH_EVERY == 0) {
                     // residual replacement: r = b - A x with A in float32 from the positions;
@@ -2262,11 +2314,11 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_refresh, nb, nd, (const float*)c->b,
                                    (const float*)c->Ap, c->r, c->partials + 2 * (size_t)stride, stride,
                                    (const SolverState*)c->state));
-                    IVP_TRY(fold_source<2>(c, 1, nb.x, c->state, &pp.rr));
+                    IVP_TRY(fold_source<2>(c, 1, nb.x, nb.x, &pp.rr));
                     pp.host = host;
                     return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_REPLACE>, nb, pp);
                 }
-                IVP_TRY(fold_source<1>(c, 1, nb.x, c->state, &pp.rr));
+                IVP_TRY(fold_source<1>(c, 1, nb.x, nb.x, &pp.rr));
                 pp.host = host;
                 return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_UPDATE>, nb, pp);
             };
@@ -2344,17 +2396,32 @@ int visc_explicit_body(ivp_ctx* c, float coeff, float dt) {
                   (const float4*)c->v4, (const float*)c->rho0, (const int*)c->mat, c->vel, next);
 }
 
-// The rest of a Weiler18 / Jeske23 CG iteration after its operator pass (npap blocks); partial rows:
-// p.Ap 0, r.r 1, r.z 2
-int w18_update(ivp_ctx* c, const W18Args& cg, int npap, int tag, SolverState* host, const NextIn& next) {
+// One Weiler18 / Jeske23 CG iteration with operator pass av(p, fused, step): av enqueues it on direction p,
+// with the end of the iteration before if `fused`.  first / last: of a chunk.  `cur` is the buffer that
+// holds p, `other` the second one.  Partial rows: p.Ap 0, r.r 1, r.z 2.
+template <class FM, class AV>
+int w18_iter(ivp_ctx* c, const W18Args& cg, int npap, int tag, bool first, SolverState* host, const NextIn& next,
+             float4** cur, float4** other, AV&& av) {
     const int nd = c->nd;
+    // (without windows every pair would gather z as well)
+    const bool fuse = has_windows<FM, PASS_LANES>() && c->win_built && c->windows && nd <= FUSE_P_MAX;
+    PStep step{};
+    if (fuse && !first) {
+        step = PStep{c->w_z, *cur, *other, c->w_dv, Fold{}, c->err_flag};
+        IVP_TRY(fold_source<2>(c, 1, blocks_for(nd), npap, &step.sums));
+        IVP_TRY(av(*cur, true, step));
+        std::swap(*cur, *other);
+    } else {
+        IVP_TRY(av(*cur, false, step));
+    }
     const dim3 nb(blocks_for(nd));
     W18Args u = cg;
     u.partials = c->partials + c->max_blocks;
-    IVP_TRY(fold_source<1>(c, 0, npap, c->state, &u.pap));
+    IVP_TRY(fold_source<1>(c, 0, npap, nb.x, &u.pap));
     IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, u));
-    W18PArgs p{nd, c->w_z, c->w_p4, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag, next};
-    IVP_TRY(fold_source<2>(c, 1, nb.x, c->state, &p.sums));
+    if (fuse && !host) return IVP_OK;
+    W18PArgs p{nd, c->w_z, *cur, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag, next};
+    IVP_TRY(fold_source<2>(c, 1, nb.x, nb.x, &p.sums));
     return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, p);
 }
 
@@ -2384,7 +2451,7 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         res.v4 = c->w_p4;
         res.out = c->w_Ap;
         IVP_TRY(launch(c, KC_W18_PRE, -1, stream_bytes<FM>(c, pairs) + 48.0 * nd, k_w18_Av<FM, ALLFLUID, false>, pass_grid(nd),
-                       res));
+                       res, PStep{}));
         IVP_TRY(launch(c, KC_W18_PRE, -1, 0.0, k_w18_warm_init, nb, res, (const float*)c->w_rhs, c->w_p4));
     }
     IVP_TRY(finalize<FIN_W18_INIT>(c, c->w18_warm ? nb.x : pass_grid(nd).x, 1e-5, 1000));
@@ -2395,9 +2462,15 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
         cg.v4 = c->w_p4;
         cg.out = c->w_Ap;
         const double bAv = stream_bytes<FM>(c, (double)c->state_host->total_pairs) + 48.0 * nd;
-        auto one_iter = [&](int tag, SolverState* host) -> int {
-            IVP_TRY(launch(c, KC_W18_AV, tag, bAv, k_w18_Av<FM, ALLFLUID>, pass_grid(nd), cg));
-            return w18_update(c, cg, pass_grid(nd).x, tag, host, next);
+        float4 *cur = c->w_p4, *other = c->w_v4;   // (w_v4 is free once the set-up has read it)
+        auto one_iter = [&](int tag, SolverState* host, bool first) -> int {
+            auto av = [&](float4* p, bool fused, const PStep& step) {
+                W18Args ca = cg;
+                ca.v4 = p;
+                return launch(c, KC_W18_AV, tag, bAv, fused ? k_w18_Av<FM, ALLFLUID, true, true> : k_w18_Av<FM, ALLFLUID>,
+                              pass_grid(nd), ca, step);
+            };
+            return w18_iter<FM>(c, cg, pass_grid(nd).x, tag, first, host, next, &cur, &other, av);
         };
         // the save of the correction follows each chunk's report, running once the solve has stopped
         // (while the host reads the state)
@@ -2443,7 +2516,7 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
     if (c->prof) IVP_TRY(build_fold(c));
     IVP_TRY(launch(c, KC_ST_SETUP, -1, stream_bytes<FM>(c, pairs) + 36.0 * nd, k_st_div<FM, ALLFLUID>, np, sa));
     IVP_TRY(launch(c, KC_ST_SETUP, -1, (pb + 4.0) * pairs + 72.0 * nd, k_st_setup<FM, ALLFLUID>, np, sa));
-    IVP_TRY(launch(c, KC_ST_AV, -1, stream_bytes<FM>(c, pairs) + 4.0 * pairs + 40.0 * nd, k_st_Av<FM, ALLFLUID, true>, np, sa));
+    IVP_TRY(launch(c, KC_ST_AV, -1, stream_bytes<FM>(c, pairs) + 4.0 * pairs + 40.0 * nd, k_st_Av<FM, ALLFLUID, true>, np, sa, PStep{}));
     W18Args wa{R, c->cfg.material_fluid, c->w_fac, c->mat, c->w_pinv, c->w_v4, c->w_rhs,
                c->w_dv, c->w_r, c->w_z, c->partials, stride, c->state};
     IVP_TRY(launch(c, -1, -1, 0.0, k_w18_init, nb, wa, c->w_p4));
@@ -2458,9 +2531,15 @@ int jeske23_body(ivp_ctx* c, float sigma, float dt, int* iters_out) {
         cg.v4 = c->w_p4;
         cg.out = c->w_Ap;
         const double bAv = stream_bytes<FM>(c, pairs) + 4.0 * pairs + 28.0 * nd;
-        auto one_iter = [&](int tag, SolverState* host) -> int {
-            IVP_TRY(launch(c, KC_ST_AV, tag, bAv, k_st_Av<FM, ALLFLUID, false>, np, cga));
-            return w18_update(c, cg, np.x, tag, host, next);
+        float4 *cur = c->w_p4, *other = c->w_v4;
+        auto one_iter = [&](int tag, SolverState* host, bool first) -> int {
+            auto av = [&](float4* p, bool fused, const PStep& step) {
+                StArgs ca = cga;
+                ca.u4 = p;
+                return launch(c, KC_ST_AV, tag, bAv, fused ? k_st_Av<FM, ALLFLUID, false, true> : k_st_Av<FM, ALLFLUID, false>,
+                              np, ca, step);
+            };
+            return w18_iter<FM>(c, cg, np.x, tag, first, host, next, &cur, &other, av);
         };
         auto tail = [](bool) { return (int)IVP_OK; };
         c->prof_epoch++;
