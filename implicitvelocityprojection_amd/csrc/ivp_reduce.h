@@ -224,7 +224,9 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
 // 350k (7.5 million) 1079 / 1108; the sums at 500k (3.8 million) 1378 / 1359, 750k (8.6 million) 1908 / 1956, 1M
 // 2371 / 2535.
 constexpr long long FOLD_READS = 5ll << 20;
-constexpr int FIN_MAX = 2048;   // partials per row that the one-block finalize folds alone
+// partials (all rows) that the one-block finalize folds alone: three rows of 4096 take it 4.3 us, and 6.9
+// with a prefold; three of 15 625 9.1 and 6.9
+constexpr int FIN_MAX = 16384;
 
 // `meanwhile` runs with the first partials in flight: the caller's own loads, which would otherwise wait
 // for the fold (23k rows: update 3.8 -> 3.4 us, p pass 3.9 -> 3.5).
@@ -383,7 +385,7 @@ inline int finalize(ivp_ctx* c, int nblocks, double tol = 0.0, int max_iter = 0,
     constexpr int NV = fin_nv<OP>();
     constexpr int row0 = OP == FIN_RHS ? 3 : OP == FIN_BUILD ? BUILD_ROW : 0;
     Fold f{c->partials + row0 * (size_t)c->max_blocks, c->max_blocks, nblocks};
-    if (NV > 1 && nblocks > FIN_MAX) IVP_TRY((fold_source<NV>(c, row0, nblocks, 1 << 20, &f)));
+    if (NV > 1 && nblocks * NV > FIN_MAX) IVP_TRY((fold_source<NV>(c, row0, nblocks, 1 << 20, &f)));
     FinArgs fa{f.p, f.stride, f.n, c->state, tol, max_iter, gated ? 1 : 0, host, c->err_flag, mark};
     hipLaunchKernelGGL(k_finalize<OP>, dim3(1), dim3(FIN_BLOCK), 0, c->stream, fa);
     IVP_HIP(hipGetLastError());

@@ -23,9 +23,9 @@
 // expression (in the neighbour build).
 //
 // Control.  CG dot products are reduced in FP64 on the device; alpha, beta and the stop test
-// (ip.py:302-327) are evaluated by a one-block finalize kernel after each reduction, and the
-// host enqueues CG iterations in chunks, synchronising once per chunk instead of twice per
-// iteration.
+// (ip.py:302-327) are formed by every block of the pass that needs them from the partials of the pass
+// before, and written to the device's solver state by one (ivp_reduce.h).  The host enqueues CG
+// iterations in chunks, synchronising once per chunk instead of twice per iteration.
 #include <math.h>
 
 #include <algorithm>
