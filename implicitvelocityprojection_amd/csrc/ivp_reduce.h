@@ -217,16 +217,16 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
 // readers' blocks times the partials stay below FOLD_READS (42 MB a row, from L2) every block of the next
 // pass folds them itself, all to the same bits, and one block writes the state; above it the folds take
 // longer than the launch that they save, and k_prefold first reduces each row to PREFOLD partials in
-// one short launch of many blocks (15 625 partials: 2.4 us; the one-block finalize took 4.6, with two
-// rows 7.9, with three 9.1: the bandwidth of one CU).  p.Ap has nd / 64 partials, an update's sums
+// one short launch of many blocks (15 625 partials: 4.6 us, what the one-block finalize took; the pass
+// that folds the rest is then no dependent launch of its own).  p.Ap has nd / 64 partials, an update's sums
 // nd / 256, and both are read by nd / 256 blocks.  us per implicit viscosity solve, prefolded /
 // folded by the readers: p.Ap at 133k rows 420 / 390, 176k 506 / 480, 262k (4.2 million reads) 879 / 861,
 // 350k (7.5 million) 1079 / 1108; the sums at 500k (3.8 million) 1378 / 1359, 750k (8.6 million) 1908 / 1956, 1M
 // 2371 / 2535.
 constexpr long long FOLD_READS = 5ll << 20;
-// partials (all rows) that the one-block finalize folds alone: three rows of 4096 take it 4.3 us, and 6.9
-// with a prefold; three of 15 625 9.1 and 6.9
-constexpr int FIN_MAX = 16384;
+// Partials (all rows) that the one-block finalize folds alone, us: three rows of 4096 4.3 and 6.9 with a
+// prefold; three of 15 625 9.1 and 9.7; six of 15 625 9.7 with one
+constexpr int FIN_MAX = 1 << 16;
 
 // `meanwhile` runs with the first partials in flight: the caller's own loads, which would otherwise wait
 // for the fold (23k rows: update 3.8 -> 3.4 us, p pass 3.9 -> 3.5).
