@@ -257,10 +257,20 @@ __device__ __forceinline__ int row16_max(int v) {
     return pair_step<1>(pair_step<2>(pair_step<4>(pair_step<8>(v, f), f), f), f);
 }
 
-// Sums of NV doubles per thread over a 256-thread block, in a fixed order.  Results valid in
+// Sums of the waves' values of a T-thread block in a fixed order
+template <int T>
+__device__ __forceinline__ double waves_total(const double* w) {
+    if constexpr (T == 4 * WAVE) return (w[0] + w[1]) + (w[2] + w[3]);
+    double s = w[0];
+#pragma unroll
+    for (int k = 1; k < T / WAVE; ++k) s += w[k];
+    return s;
+}
+
+// Sums of NV doubles per thread over a T-thread block, in a fixed order.  Results valid in
 // thread 0.  lds is not reused before a barrier of the caller's.
-template <int NV>
-__device__ __forceinline__ void block_sums(const double (&v)[NV], double (&s)[NV], double (&lds)[NV][WAVES_PER_BLOCK]) {
+template <int NV, int T = BLOCK>
+__device__ __forceinline__ void block_sums(const double (&v)[NV], double (&s)[NV], double (&lds)[NV][T / WAVE]) {
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
@@ -269,7 +279,7 @@ __device__ __forceinline__ void block_sums(const double (&v)[NV], double (&s)[NV
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NV; ++q) s[q] = threadIdx.x == 0 ? (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]) : 0.0;
+    for (int q = 0; q < NV; ++q) s[q] = threadIdx.x == 0 ? waves_total<T>(lds[q]) : 0.0;
 }
 
 }  // namespace ivp

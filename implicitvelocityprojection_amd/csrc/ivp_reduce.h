@@ -3,6 +3,8 @@
 // device-resident solver state.
 #pragma once
 
+#include <type_traits>
+
 #include "ivp_internal.h"
 #include "ivp_launch.h"
 
@@ -11,11 +13,11 @@ namespace ivp {
 // Per-block partial sums of up to 3 doubles (fixed order inside the block).  The grid totals are
 // formed by a later launch on the stream: the kernel boundary publishes the partials,
 // so no device-scope fence (an L2 write-back on a multi-XCD part) is issued per block.
-template <int NV>
+template <int NV, int T = BLOCK>
 __device__ __forceinline__ void block_partials(const double (&v)[NV], double* partials, int stride) {
-    __shared__ double lds[NV][WAVES_PER_BLOCK];
+    __shared__ double lds[NV][T / WAVE];
     double s[NV];
-    block_sums<NV>(v, s, lds);
+    block_sums<NV, T>(v, s, lds);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int q = 0; q < NV; ++q) partials[q * stride + blockIdx.x] = s[q];
@@ -230,19 +232,19 @@ constexpr int FIN_MAX = 1 << 16;
 
 // `meanwhile` runs with the first partials in flight: the caller's own loads, which would otherwise wait
 // for the fold (23k rows: update 3.8 -> 3.4 us, p pass 3.9 -> 3.5).
-template <int NV, class M>
+template <int NV, int T, class M>
 __device__ __forceinline__ void block_fold(const double* __restrict__ p, int stride, int n, double (&t)[NV], M&& meanwhile) {
-    __shared__ double lds[NV][WAVES_PER_BLOCK];
+    __shared__ double lds[NV][T / WAVE];
     double s[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) s[q] = 0.0;
-    for (int base = 0; base < n; base += 4 * BLOCK) {
+    for (int base = 0; base < n; base += 4 * T) {
         double v[NV][4];
 #pragma unroll
         for (int q = 0; q < NV; ++q)
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int k = base + u * BLOCK + (int)threadIdx.x;
+                const int k = base + u * T + (int)threadIdx.x;
                 v[q][u] = k < n ? p[(size_t)q * stride + k] : 0.0;
             }
         if (base == 0) meanwhile();
@@ -256,7 +258,7 @@ __device__ __forceinline__ void block_fold(const double* __restrict__ p, int str
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NV; ++q) t[q] = (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]);
+    for (int q = 0; q < NV; ++q) t[q] = waves_total<T>(lds[q]);
 }
 
 // Row q of n partials to PREFOLD partials: block b folds the b-th share
@@ -266,10 +268,40 @@ __global__ __launch_bounds__(BLOCK) void k_prefold(const double* __restrict__ p,
     const int per = (n + PREFOLD - 1) / PREFOLD;
     const int k0 = (int)blockIdx.x * per < n ? (int)blockIdx.x * per : n;
     double t[NV];
-    block_fold<NV>(p + k0, stride, k0 + per < n ? per : n - k0, t, []() {});
+    block_fold<NV, BLOCK>(p + k0, stride, k0 + per < n ? per : n - k0, t, []() {});
     if (threadIdx.x == 0)
 #pragma unroll
         for (int q = 0; q < NV; ++q) out[q * PREFOLD + (int)blockIdx.x] = t[q];
+}
+
+// Blocks of a CG's vector passes (update, p): 256 threads of one row each, or between VEC_MIN and VEC_MAX rows at
+// most 256 blocks -- one per CU -- of 1024 threads with as many rows each as that takes, all in flight:
+// then both the partials they write and the blocks that fold the operator pass's are few, and no
+// k_prefold is needed (us per implicit viscosity solve, 256-thread blocks / these: 90k rows 294 /
+// 302, 133k 377 / 371, 262k
+// 860 / 843, 350k 1071 / 1025, 500k 1351 / 1287, 1M 2374 / 2283; IP solve at 262k 331 / 315, 700k 652 (750k) / 609).
+constexpr int VEC_THREADS = 1024, VEC_BLOCKS = 256, VEC_ROWS = 4;
+constexpr int VEC_MIN = 1 << 17, VEC_MAX = VEC_THREADS * VEC_BLOCKS * VEC_ROWS;
+struct VecGrid {
+    int threads, rows, blocks;   // per block; per thread; blocks
+};
+inline VecGrid vec_grid(int nd) {
+    if (nd < VEC_MIN || nd > VEC_MAX) return VecGrid{BLOCK, 1, blocks_for(nd)};
+    const int rows = (nd + VEC_THREADS * VEC_BLOCKS - 1) / (VEC_THREADS * VEC_BLOCKS);
+    return VecGrid{VEC_THREADS, rows, (nd + VEC_THREADS * rows - 1) / (VEC_THREADS * rows)};
+}
+// f(threads, rows) of a grid, as compile-time constants
+template <class F>
+inline int vec_dispatch(const VecGrid& g, F&& f) {
+    using std::integral_constant;
+    if (g.threads == BLOCK) return f(integral_constant<int, BLOCK>{}, integral_constant<int, 1>{});
+    integral_constant<int, VEC_THREADS> t;
+    switch (g.rows) {
+    case 1: return f(t, integral_constant<int, 1>{});
+    case 2: return f(t, integral_constant<int, 2>{});
+    case 3: return f(t, integral_constant<int, 3>{});
+    default: return f(t, integral_constant<int, VEC_ROWS>{});
+    }
 }
 
 // Partials to fold: rows `stride` apart, n per row
@@ -295,7 +327,7 @@ inline int fold_source(ivp_ctx* c, int row0, int n, int readers, Fold* f) {
 // In an iteration's update pass: alpha from the operator pass's p.Ap (OP = FIN_CG_PAP, FIN_W18_PAP).
 // Returns false when there is nothing to update.  The state's own fields stay as they are until
 // the p pass; ran and prev_* tell it what happened here.
-template <int OP, class M>
+template <int OP, int T, class M>
 __device__ __forceinline__ bool fold_alpha(SolverState* st, const Fold& f, float* alpha, M&& meanwhile) {
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (st->active == 0) {
@@ -305,7 +337,7 @@ __device__ __forceinline__ bool fold_alpha(SolverState* st, const Fold& f, float
     const double rr_old = st->rr_old, rr_best = st->rr_best;
     const int iter = st->iter, stalls = st->stalls;
     double t[1];
-    block_fold<1>(f.p, f.stride, f.n, t, meanwhile);
+    block_fold<1, T>(f.p, f.stride, f.n, t, meanwhile);
     // ip.py:307-311 fails on p.Ap < 0; weiler18.py:338-342 ends the iteration on p.Ap <= 0
     const double least = OP == FIN_CG_PAP ? 1e-30 : 1e-12;
     const bool bad = OP == FIN_CG_PAP ? t[0] < 0.0 : t[0] <= 0.0;
@@ -335,7 +367,7 @@ struct Advance {
 // In the iteration's p pass: the state after the iteration from the update pass's sums (OP =
 // FIN_CG_UPDATE, FIN_CG_REPLACE, FIN_W18_UPDATE), formed by every block and written by one, which
 // reports it to the host if asked.
-template <int OP, class M>
+template <int OP, int T, class M>
 __device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, SolverState* host, const int* flags,
                                                 M&& meanwhile) {
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
@@ -353,7 +385,7 @@ __device__ __forceinline__ Advance fold_advance(SolverState* st, const Fold& f, 
         s.beta = 0.0;
         s.rr_new = 0.0;
         double t[fin_nv<OP>()];
-        block_fold<fin_nv<OP>()>(f.p, f.stride, f.n, t, meanwhile);
+        block_fold<fin_nv<OP>(), T>(f.p, f.stride, f.n, t, meanwhile);
         fin_apply<OP>(&s, t, 0.0, 0);
         a.active = s.active != 0;
         a.stopped = !a.active;

@@ -793,43 +793,54 @@ struct CGUpdArgs {
     Fold pap;        // one scene: the operator pass's p.Ap
 };
 
-// pcg_update_x_r_scalar (math_utils.py:180-195) + r.r (ip.py:314-317)
-template <bool SC>
-__global__ __launch_bounds__(BLOCK) void k_cg_update(CGUpdArgs a) {
-    const int blk = blockIdx.x;
-    int i = blk * BLOCK + threadIdx.x;
+// pcg_update_x_r_scalar (math_utils.py:180-195) + r.r (ip.py:314-317); R rows per thread, T apart
+template <bool SC, int T = BLOCK, int R = 1>
+__global__ __launch_bounds__(T) void k_cg_update(CGUpdArgs a) {
+    static_assert(!SC || (T == BLOCK && R == 1), "scenes: one row per thread");
+    const int blk = blockIdx.x, i0 = blk * (T * R) + threadIdx.x;
     float alpha = 0.0f;
-    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float x[3] = {0.0f, 0.0f, 0.0f}, r[3] = {0.0f, 0.0f, 0.0f}, Ap[3] = {0.0f, 0.0f, 0.0f};
+    float4 p[R];
+    float x[R][3], r[R][3], Ap[R][3];
     auto own = [&]() {
-        if (i >= a.nd) return;
-        p = a.p4[i];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            x[q] = a.sol[3 * i + q];
-            r[q] = a.r[3 * i + q];
-            Ap[q] = a.Ap[3 * i + q];
+        for (int k = 0; k < R; ++k) {
+            const int i = i0 + k * T;
+            if (i >= a.nd) continue;
+            p[k] = a.p4[i];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                x[k][q] = a.sol[3 * i + q];
+                r[k][q] = a.r[3 * i + q];
+                Ap[k][q] = a.Ap[3 * i + q];
+            }
         }
     };
-    if (!SC && !fold_alpha<FIN_CG_PAP>(a.st, a.pap, &alpha, own)) return;
-    Gate gt = gate_all(i, a.nd);
-    if (SC && !gate_block(a.sc, blk, i, a.nd, PH_CG, gt)) return;
+    if constexpr (!SC)
+        if (!fold_alpha<FIN_CG_PAP, T>(a.st, a.pap, &alpha, own)) return;
+    Gate gt = gate_all(i0, a.nd);
+    if (SC && !gate_block(a.sc, blk, i0, a.nd, PH_CG, gt)) return;
     if (SC) alpha = (float)a.sc.ss[gt.s].cg.alpha;
+    if (SC && gt.on) own();
     double rr = 0.0;
-    if (gt.on) {
-        if (SC) own();
-        float x0 = x[0] + alpha * p.x;
-        float x1 = x[1] + alpha * p.y;
-        float x2 = x[2] + alpha * p.z;
-        float r0 = r[0] - alpha * Ap[0];
-        float r1 = r[1] - alpha * Ap[1];
-        float r2 = r[2] - alpha * Ap[2];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = i0 + k * T;
+        if (SC ? !gt.on : i >= a.nd) continue;
+        float x0 = x[k][0] + alpha * p[k].x;
+        float x1 = x[k][1] + alpha * p[k].y;
+        float x2 = x[k][2] + alpha * p[k].z;
+        float r0 = r[k][0] - alpha * Ap[k][0];
+        float r1 = r[k][1] - alpha * Ap[k][1];
+        float r2 = r[k][2] - alpha * Ap[k][2];
         a.sol[3 * i + 0] = x0; a.sol[3 * i + 1] = x1; a.sol[3 * i + 2] = x2;
         a.r[3 * i + 0] = r0; a.r[3 * i + 1] = r1; a.r[3 * i + 2] = r2;
-        rr = (double)(r0 * r0 + r1 * r1 + r2 * r2);
+        rr += (double)(r0 * r0 + r1 * r1 + r2 * r2);
     }
     double v[1] = {rr};
-    row_partials<SC, 1>(v, gt, a.partials, a.stride, blk);
+    if constexpr (SC)
+        row_partials<SC, 1>(v, gt, a.partials, a.stride, blk);
+    else
+        block_partials<1, T>(v, a.partials, a.stride);
 }
 
 // p = r + beta p of independent scenes (add_vec3, ip.py:323-326)
@@ -863,29 +874,37 @@ struct CGPArgs {
 // The end of a CG iteration (OP = FIN_CG_UPDATE or FIN_CG_REPLACE): the stop test, then
 // p = r + beta p (add_vec3, ip.py:323-326) while the solve goes on; in the last iteration of a chunk a
 // solve that has stopped without failing moves d -= x instead (add_vec3 with scale -1, ip.py:389).
-template <int OP>
-__global__ __launch_bounds__(BLOCK) void k_cg_p(CGPArgs a) {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float r[3] = {0.0f, 0.0f, 0.0f};
-    const Advance v = fold_advance<OP>(a.st, a.rr, a.host, a.flags, [&]() {
-        if (i >= a.nd) return;
-        p = a.p4[i];
+template <int OP, int T, int R>
+__global__ __launch_bounds__(T) void k_cg_p(CGPArgs a) {
+    const int i0 = blockIdx.x * (T * R) + threadIdx.x;
+    float4 p[R];
+    float r[R][3];
+    const Advance v = fold_advance<OP, T>(a.st, a.rr, a.host, a.flags, [&]() {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) r[q] = a.r[3 * i + q];
+        for (int k = 0; k < R; ++k) {
+            const int i = i0 + k * T;
+            if (i >= a.nd) continue;
+            p[k] = a.p4[i];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) r[k][q] = a.r[3 * i + q];
+        }
     });
-    if (i >= a.nd) return;
-    if (v.active) {
-        p.x = r[0] + v.beta * p.x;
-        p.y = r[1] + v.beta * p.y;
-        p.z = r[2] + v.beta * p.z;
-        a.p4[i] = p;
-    } else if (a.host && v.stopped) {
-        float4 d = a.d4[i];
-        d.x = d.x + -1.0f * a.sol[3 * i + 0];
-        d.y = d.y + -1.0f * a.sol[3 * i + 1];
-        d.z = d.z + -1.0f * a.sol[3 * i + 2];
-        a.d4[i] = d;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = i0 + k * T;
+        if (i >= a.nd) continue;
+        if (v.active) {
+            p[k].x = r[k][0] + v.beta * p[k].x;
+            p[k].y = r[k][1] + v.beta * p[k].y;
+            p[k].z = r[k][2] + v.beta * p[k].z;
+            a.p4[i] = p[k];
+        } else if (a.host && v.stopped) {
+            float4 d = a.d4[i];
+            d.x = d.x + -1.0f * a.sol[3 * i + 0];
+            d.y = d.y + -1.0f * a.sol[3 * i + 1];
+            d.z = d.z + -1.0f * a.sol[3 * i + 2];
+            a.d4[i] = d;
+        }
     }
 }
 
@@ -899,22 +918,25 @@ __global__ __launch_bounds__(BLOCK) void k_x4(int nd, const float* __restrict__ 
 }
 
 // Residual replacement: r = b - A x with A applied in float32 from positions, and r.r
-__global__ __launch_bounds__(BLOCK) void k_cg_refresh(int nd, const float* __restrict__ b,
-                                                      const float* __restrict__ Ax, float* __restrict__ r,
-                                                      double* __restrict__ partials, int stride,
-                                                      const SolverState* __restrict__ st) {
+template <int T, int R>
+__global__ __launch_bounds__(T) void k_cg_refresh(int nd, const float* __restrict__ b,
+                                                  const float* __restrict__ Ax, float* __restrict__ r,
+                                                  double* __restrict__ partials, int stride,
+                                                  const SolverState* __restrict__ st) {
     if (st->active == 0) return;
-    int i = blockIdx.x * BLOCK + threadIdx.x;
     double rr = 0.0;
-    if (i < nd) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = ((int)blockIdx.x * R + k) * T + (int)threadIdx.x;
+        if (i >= nd) continue;
         float r0 = b[3 * i + 0] - Ax[3 * i + 0];
         float r1 = b[3 * i + 1] - Ax[3 * i + 1];
         float r2 = b[3 * i + 2] - Ax[3 * i + 2];
         r[3 * i + 0] = r0; r[3 * i + 1] = r1; r[3 * i + 2] = r2;
-        rr = (double)(r0 * r0 + r1 * r1 + r2 * r2);
+        rr += (double)(r0 * r0 + r1 * r1 + r2 * r2);
     }
     double v[1] = {rr};
-    block_partials<1>(v, partials, stride);
+    block_partials<1, T>(v, partials, stride);
 }
 
 // d -= sol (add_vec3 with scale -1, ip.py:389): independent scenes, and a solve that is allowed no iteration
@@ -1513,7 +1535,7 @@ __device__ __forceinline__ bool p_step(const PStep& n, SolverState* st, int i, i
     const int ic = i < nd ? i : nd - 1;
     const float alpha = (float)st->alpha;
     const float z[3] = {n.z[3 * ic + 0], n.z[3 * ic + 1], n.z[3 * ic + 2]};
-    const Advance v = fold_advance<FIN_W18_UPDATE>(st, n.sums, nullptr, n.flags, []() {});
+    const Advance v = fold_advance<FIN_W18_UPDATE, BLOCK>(st, n.sums, nullptr, n.flags, []() {});
     if (!v.ran) return false;
     const bool own = i < nd && g == 0;
     if (own) {
@@ -1564,37 +1586,45 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a, PStep n) {
 
 // r -= alpha Ap, r.r, z = P r, r.z (weiler18.py:344-360); dv += alpha p of the same lines
 // follows in the p pass, which reads p anyway
-__global__ __launch_bounds__(BLOCK) void k_w18_update(W18Args a) {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
+template <int T, int R>
+__global__ __launch_bounds__(T) void k_w18_update(W18Args a) {
+    const int i0 = blockIdx.x * (T * R) + threadIdx.x;
     float alpha;
-    float r[3] = {0.0f, 0.0f, 0.0f}, Ap[3] = {0.0f, 0.0f, 0.0f}, P[9] = {};
+    float r[R][3], Ap[R][3], P[R][9];
     auto own = [&]() {
-        if (i >= a.R.nd) return;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            r[q] = a.r[3 * i + q];
-            Ap[q] = a.out[3 * i + q];
+        for (int k = 0; k < R; ++k) {
+            const int i = i0 + k * T;
+            if (i >= a.R.nd) continue;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                r[k][q] = a.r[3 * i + q];
+                Ap[k][q] = a.out[3 * i + q];
+            }
+#pragma unroll
+            for (int q = 0; q < 9; ++q) P[k][q] = a.pinv[9 * (size_t)i + q];
         }
-#pragma unroll
-        for (int q = 0; q < 9; ++q) P[q] = a.pinv[9 * (size_t)i + q];
     };
-    if (!fold_alpha<FIN_W18_PAP>(a.st, a.pap, &alpha, own)) return;
+    if (!fold_alpha<FIN_W18_PAP, T>(a.st, a.pap, &alpha, own)) return;
     const float nalpha = -alpha;
     double rr = 0.0, rz = 0.0;
-    if (i < a.R.nd) {
-        float r0 = r[0] + nalpha * Ap[0];
-        float r1 = r[1] + nalpha * Ap[1];
-        float r2 = r[2] + nalpha * Ap[2];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = i0 + k * T;
+        if (i >= a.R.nd) continue;
+        float r0 = r[k][0] + nalpha * Ap[k][0];
+        float r1 = r[k][1] + nalpha * Ap[k][1];
+        float r2 = r[k][2] + nalpha * Ap[k][2];
         a.r[3 * i + 0] = r0; a.r[3 * i + 1] = r1; a.r[3 * i + 2] = r2;
-        float z0 = P[0] * r0 + P[1] * r1 + P[2] * r2;
-        float z1 = P[3] * r0 + P[4] * r1 + P[5] * r2;
-        float z2 = P[6] * r0 + P[7] * r1 + P[8] * r2;
+        float z0 = P[k][0] * r0 + P[k][1] * r1 + P[k][2] * r2;
+        float z1 = P[k][3] * r0 + P[k][4] * r1 + P[k][5] * r2;
+        float z2 = P[k][6] * r0 + P[k][7] * r1 + P[k][8] * r2;
         a.z[3 * i + 0] = z0; a.z[3 * i + 1] = z1; a.z[3 * i + 2] = z2;
-        rr = (double)(r0 * r0 + r1 * r1 + r2 * r2);
-        rz = (double)(r0 * z0 + r1 * z1 + r2 * z2);
+        rr += (double)(r0 * r0 + r1 * r1 + r2 * r2);
+        rz += (double)(r0 * z0 + r1 * z1 + r2 * z2);
     }
     double v[2] = {rr, rz};
-    block_partials<2>(v, a.partials, a.stride);
+    block_partials<2, T>(v, a.partials, a.stride);
 }
 
 struct W18PArgs {
@@ -1615,45 +1645,55 @@ struct W18PArgs {
 // goes on.  In the last iteration of a chunk a solve that has stopped also adds v += dv
 // (weiler18.py:399-401), except on rows that the last build truncated (the host refuses them when it
 // reads the flags).
-__global__ __launch_bounds__(BLOCK) void k_w18_p(W18PArgs a) {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
+template <int T, int R>
+__global__ __launch_bounds__(T) void k_w18_p(W18PArgs a) {
+    const int i0 = blockIdx.x * (T * R) + threadIdx.x;
     const float alpha = (float)a.st->alpha;
-    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float dv[3] = {0.0f, 0.0f, 0.0f}, z[3] = {0.0f, 0.0f, 0.0f};
-    const Advance v = fold_advance<FIN_W18_UPDATE>(a.st, a.sums, a.host, a.flags, [&]() {
-        if (i >= a.nd) return;
-        p = a.p4[i];
+    float4 p[R];
+    float dv[R][3], z[R][3];
+    const Advance v = fold_advance<FIN_W18_UPDATE, T>(a.st, a.sums, a.host, a.flags, [&]() {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            dv[q] = a.dv[3 * i + q];
-            z[q] = a.z[3 * i + q];
+        for (int k = 0; k < R; ++k) {
+            const int i = i0 + k * T;
+            if (i >= a.nd) continue;
+            p[k] = a.p4[i];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                dv[k][q] = a.dv[3 * i + q];
+                z[k][q] = a.z[3 * i + q];
+            }
         }
     });
     const bool apply = a.host && v.stopped && !(*a.flags & 5);
-    if ((!v.ran && !apply) || i >= a.nd) return;
-    if (!v.ran)
+    if (!v.ran && !apply) return;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) dv[q] = a.dv[3 * i + q];
-    if (v.ran) {
-        dv[0] = dv[0] + alpha * p.x;
-        dv[1] = dv[1] + alpha * p.y;
-        dv[2] = dv[2] + alpha * p.z;
-        a.dv[3 * i + 0] = dv[0]; a.dv[3 * i + 1] = dv[1]; a.dv[3 * i + 2] = dv[2];
-        if (v.active) {
-            p.x = z[0] + v.beta * p.x;
-            p.y = z[1] + v.beta * p.y;
-            p.z = z[2] + v.beta * p.z;
-            a.p4[i] = p;
-        }
-    }
-    if (apply) {
-        float v1[3];
+    for (int k = 0; k < R; ++k) {
+        const int i = i0 + k * T;
+        if (i >= a.nd) continue;
+        if (!v.ran)
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            v1[q] = a.vel[3 * i + q] + 1.0f * dv[q];
-            a.vel[3 * i + q] = v1[q];
+            for (int q = 0; q < 3; ++q) dv[k][q] = a.dv[3 * i + q];
+        if (v.ran) {
+            dv[k][0] = dv[k][0] + alpha * p[k].x;
+            dv[k][1] = dv[k][1] + alpha * p[k].y;
+            dv[k][2] = dv[k][2] + alpha * p[k].z;
+            a.dv[3 * i + 0] = dv[k][0]; a.dv[3 * i + 1] = dv[k][1]; a.dv[3 * i + 2] = dv[k][2];
+            if (v.active) {
+                p[k].x = z[k][0] + v.beta * p[k].x;
+                p[k].y = z[k][1] + v.beta * p[k].y;
+                p[k].z = z[k][2] + v.beta * p[k].z;
+                a.p4[i] = p[k];
+            }
         }
-        next_input(a.next, i, v1[0], v1[1], v1[2]);
+        if (apply) {
+            float v1[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                v1[q] = a.vel[3 * i + q] + 1.0f * dv[k][q];
+                a.vel[3 * i + q] = v1[q];
+            }
+            next_input(a.next, i, v1[0], v1[1], v1[2]);
+        }
     }
 }
 
@@ -2292,6 +2332,7 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             CGJArgs ja{R, c->p4, c->Ss, c->sfac, c->y2, c->state};
             CGJTArgs ta{R, c->p4, c->y2, c->Ss, c->nbact, prm->omega, c->Ap, c->partials, stride, c->state};
             // partial rows: p.Ap 0, the update's r.r 1, a replaced residual's r.r 2 (x.Ax 3)
+            const VecGrid vg = vec_grid(nd);
             CGUpdArgs ua{nd, c->sol, c->r, c->p4, c->Ap, c->partials + stride, stride, c->state, SceneRef{}, Fold{}};
             CGPArgs pp{nd, c->r, c->p4, c->sol, d4, c->state, Fold{}, nullptr, c->err_flag};
             // true-residual passes: the same J / J^T kernels on (x, m), gradW evaluated
@@ -2302,8 +2343,10 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
             auto one_iter = [&](int tag, SolverState* host, bool) -> int {
                 IVP_TRY(launch(c, KC_CG_J, tag, bJ, k_cg_J<FC, false>, np, ja));
                 IVP_TRY(launch(c, KC_CG_JT, tag, bJT, k_cg_JT<FC, false>, np, ta));
-                IVP_TRY(fold_source<1>(c, 0, np.x, nb.x, &ua.pap));
-                IVP_TRY(launch(c, KC_CG_UPDATE, tag, bU, k_cg_update<false>, nb, ua));
+                IVP_TRY(fold_source<1>(c, 0, np.x, vg.blocks, &ua.pap));
+                IVP_TRY(vec_dispatch(vg, [&](auto t, auto r) {
+                    return launch_any(c, KC_CG_UPDATE, tag, bU, k_cg_update<false, t.value, r.value>, dim3(vg.blocks), vg.threads, 0u, ua);
+                }));
                 if (FC::GS == GS_F16 && (tag + 1) % REFRESH_EVERY == 0) {
                     // residual replacement: r = b - A x with A in float32 from the positions;
                     // its r.r and the recursive r.r go to the stop test and beta
@@ -2311,16 +2354,22 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
                                    (const float4*)c->pos, c->xs4, (const SolverState*)c->state));
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_J<FE, false>, np, jx));
                     IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_JT<FE, false>, np, tx));
-                    IVP_TRY(launch(c, KC_CG_REFRESH, tag, 0.0, k_cg_refresh, nb, nd, (const float*)c->b,
-                                   (const float*)c->Ap, c->r, c->partials + 2 * (size_t)stride, stride,
-                                   (const SolverState*)c->state));
-                    IVP_TRY(fold_source<2>(c, 1, nb.x, nb.x, &pp.rr));
+                    IVP_TRY(vec_dispatch(vg, [&](auto t, auto r) {
+                        return launch_any(c, KC_CG_REFRESH, tag, 0.0, k_cg_refresh<t.value, r.value>, dim3(vg.blocks),
+                                          vg.threads, 0u, nd, (const float*)c->b, (const float*)c->Ap, c->r,
+                                          c->partials + 2 * (size_t)stride, stride, (const SolverState*)c->state);
+                    }));
+                    IVP_TRY(fold_source<2>(c, 1, vg.blocks, vg.blocks, &pp.rr));
                     pp.host = host;
-                    return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_REPLACE>, nb, pp);
+                    return vec_dispatch(vg, [&](auto t, auto r) {
+                        return launch_any(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_REPLACE, t.value, r.value>, dim3(vg.blocks), vg.threads, 0u, pp);
+                    });
                 }
-                IVP_TRY(fold_source<1>(c, 1, nb.x, nb.x, &pp.rr));
+                IVP_TRY(fold_source<1>(c, 1, vg.blocks, vg.blocks, &pp.rr));
                 pp.host = host;
-                return launch(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_UPDATE>, nb, pp);
+                return vec_dispatch(vg, [&](auto t, auto r) {
+                    return launch_any(c, KC_CG_P, tag, bP, k_cg_p<FIN_CG_UPDATE, t.value, r.value>, dim3(vg.blocks), vg.threads, 0u, pp);
+                });
             };
             // Behind each chunk's report (d -= x is part of its last launch): the next constraint
             // pass with its mark and its finalize, all returning at once unless the CG has stopped (and not
@@ -2405,24 +2454,28 @@ int w18_iter(ivp_ctx* c, const W18Args& cg, int npap, int tag, bool first, Solve
     const int nd = c->nd;
     // (without windows every pair would gather z as well)
     const bool fuse = has_windows<FM, PASS_LANES>() && c->win_built && c->windows && nd <= FUSE_P_MAX;
+    const VecGrid vg = vec_grid(nd);
     PStep step{};
     if (fuse && !first) {
         step = PStep{c->w_z, *cur, *other, c->w_dv, Fold{}, c->err_flag};
-        IVP_TRY(fold_source<2>(c, 1, blocks_for(nd), npap, &step.sums));
+        IVP_TRY(fold_source<2>(c, 1, vg.blocks, npap, &step.sums));
         IVP_TRY(av(*cur, true, step));
         std::swap(*cur, *other);
     } else {
         IVP_TRY(av(*cur, false, step));
     }
-    const dim3 nb(blocks_for(nd));
     W18Args u = cg;
     u.partials = c->partials + c->max_blocks;
-    IVP_TRY(fold_source<1>(c, 0, npap, nb.x, &u.pap));
-    IVP_TRY(launch(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update, nb, u));
+    IVP_TRY(fold_source<1>(c, 0, npap, vg.blocks, &u.pap));
+    IVP_TRY(vec_dispatch(vg, [&](auto t, auto r) {
+        return launch_any(c, KC_W18_UPDATE, tag, 84.0 * nd, k_w18_update<t.value, r.value>, dim3(vg.blocks), vg.threads, 0u, u);
+    }));
     if (fuse && !host) return IVP_OK;
     W18PArgs p{nd, c->w_z, *cur, c->w_dv, c->vel, c->state, Fold{}, host, c->err_flag, next};
-    IVP_TRY(fold_source<2>(c, 1, nb.x, nb.x, &p.sums));
-    return launch(c, KC_W18_P, tag, 68.0 * nd, k_w18_p, nb, p);
+    IVP_TRY(fold_source<2>(c, 1, vg.blocks, vg.blocks, &p.sums));
+    return vec_dispatch(vg, [&](auto t, auto r) {
+        return launch_any(c, KC_W18_P, tag, 68.0 * nd, k_w18_p<t.value, r.value>, dim3(vg.blocks), vg.threads, 0u, p);
+    });
 }
 
 template <class FM, bool ALLFLUID>
