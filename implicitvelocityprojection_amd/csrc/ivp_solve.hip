@@ -196,7 +196,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int LOC_PF = IVP_LOC_PF;   // window-index words requested at once per lane
 // With LOC (tile windows, four lanes per row) the lane reads its two slots' window indices as
 // one 32-bit word at half the word index of their ids, and loadA / loadB take window indices; the
-// words of the first LOC_PF blocks are in lp (loc_prefetch).
+// words of the first LOC_PF blocks are in lp (loc_prefetch).  U: slots in flight per lane where pairs are
+// gathered from memory (2 in the passes whose accumulators and records leave no registers for 4).
 struct LocPre {
     uint32_t q[LOC_PF];
 };
@@ -210,9 +211,7 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
     // one tile, or a quarter of one, per wave
     const int tl = __builtin_amdgcn_readfirstlane(REC == 64u && G == 4 ? R.wave_len[i >> 4] : R.tile_len[i >> 6]);
     // gw: the slot's gradient words (float32 x, y, z at 64-word strides, or two float16 words)
-    auto visit = [&](int j, const uint32_t* gw) {
-        float4 Aj = loadA(j);
-        Vec<NB> Bj = loadB(j);
+    auto pair = [&](const float4& Aj, const Vec<NB>& Bj, const uint32_t* gw) {
         float gx, gy, gz;
         if (FM::GS == GS_EVAL) {
             float rx = xi.x - Aj.x, ry = xi.y - Aj.y, rz = xi.z - Aj.z;
@@ -227,6 +226,11 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
             gx = R.gs * half_lo(w1); gy = R.gs * half_hi(w1); gz = R.gs * half_lo(w2);
         }
         f(Aj, Bj, gx, gy, gz);
+    };
+    auto visit = [&](int j, const uint32_t* gw) {
+        float4 Aj = loadA(j);
+        Vec<NB> Bj = loadB(j);
+        pair(Aj, Bj, gw);
     };
     static_assert(!LOC || (REC == 64u && G == 4), "tile windows index the paired ids-only layout");
     if constexpr (LOC) {
@@ -253,19 +257,43 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
         // 8-byte word pair 2 g of the row's 8 words in block b (512 words per block), and its
         // float16 gradients the 16-byte quad at twice that word index
         const u32x2* e2 = reinterpret_cast<const u32x2*>(e + 2 * g);
-#pragma unroll((U + 1) / 2)
-        for (int b = 0; b < tl; b += 8) {
-            const u32x2 ids = __builtin_nontemporal_load(e2 + (b >> 3) * 256);
-            if constexpr (FM::GS == GS_F16) {
-                const u32x4* g4 = reinterpret_cast<const u32x4*>(R.g16 + 2 * (w_row + 2 * g));
-                const u32x4 q = __builtin_nontemporal_load(g4 + (b >> 3) * 256);
-                const uint32_t w0[2] = {q.x, q.y}, w1[2] = {q.z, q.w};
-                visit((int)ids.x, w0);
-                visit((int)ids.y, w1);
-            } else {
-                visit((int)ids.x, nullptr);
-                visit((int)ids.y, nullptr);
+        // A tile without a window gathers every pair's records: U / 2 blocks' ids, then their records, are
+        // in flight together before the first pair is formed (left to the compiler, 64 registers per
+        // lane kept two records in flight: a 256 x 256 x 16 block, us per pass, ip_pack 110 / 87, cg_J
+        // 73 / 62, prj_tail 103 / 81)
+        auto blocks = [&](int b, auto count) {
+            constexpr int P = count.value;
+            u32x2 ids[P];
+            u32x4 q[P] = {};
+            float4 A[2 * P];
+            Vec<NB> B[2 * P];
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                ids[k] = __builtin_nontemporal_load(e2 + ((b >> 3) + k) * 256);
+                if constexpr (FM::GS == GS_F16)
+                    q[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(R.g16 + 2 * (w_row + 2 * g)) +
+                                                      ((b >> 3) + k) * 256);
             }
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                A[2 * k] = loadA((int)ids[k].x); B[2 * k] = loadB((int)ids[k].x);
+                A[2 * k + 1] = loadA((int)ids[k].y); B[2 * k + 1] = loadB((int)ids[k].y);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                const uint32_t w0[2] = {q[k].x, q[k].y}, w1[2] = {q[k].z, q[k].w};
+                pair(A[2 * k], B[2 * k], w0);
+                pair(A[2 * k + 1], B[2 * k + 1], w1);
+            }
+        };
+        using std::integral_constant;
+        int b = 0;
+        if constexpr (U >= 4) {
+            for (; b + 16 <= tl; b += 16) blocks(b, integral_constant<int, 2>{});
+            if (b < tl) blocks(b, integral_constant<int, 1>{});
+        } else {
+            for (; b < tl; b += 8) blocks(b, integral_constant<int, 1>{});
         }
     } else {
 #pragma unroll(U)
@@ -286,6 +314,12 @@ __device__ __forceinline__ void row_pairs(const Rows& R, int i, float4 xi, LA&& 
 template <class FM, int G>
 constexpr bool has_windows() { return FM::REC == 64u && G == 4; }
 
+// Blocks per CU that a pair pass is compiled for: the eight that the window's LDS allows (64 registers);
+// without windows nothing else asks for them (float32-gradient rows: w18_setup's 78 registers cut to 64
+// cost 9 %, 1M rows 226 -> 244 us)
+template <class FM, int G = PASS_LANES>
+constexpr int pass_blocks() { return has_windows<FM, G>() ? 8 : 1; }
+
 // Passes that may stage a window request their rows' data before it; a pass over scenes with fewer
 // lanes has no window to wait for, and its rows load when they need it (the rest of a solve finds most
 // of them in another phase).
@@ -302,11 +336,11 @@ struct WinLds {
 // A pass block waits for memory more than it computes: walked one after another, the window's length,
 // its ids, their records, the index words, the row's own data and what the row's end reads are five
 // round trips, and without any pair at all the passes took 60 to 75 % of their time (1M rows).  So a
-// pass requests everything that depends on nothing first -- win_prefetch, its row's data and
-// loc_prefetch -- and only then stages (1M rows, us before / after: ip_pack
-// 62 / 53, ip_rhs 52 / 47, cg_JT 47 / 42, w18_setup 76 / 71, w18_Av 48 / 46).  The requests cost registers, so the
-// passes are compiled for the eight blocks per CU that the window's LDS allows (64 registers): left at 72 to
-// 80 they gained nothing.
+// pass requests everything that depends on nothing first -- win_prefetch and its row's data -- then the
+// index words of a tile that has a window (loc_prefetch) together with the records that it stages (1M rows,
+// us before / after: ip_pack 62 / 53, ip_rhs 52 / 47, cg_JT 47 / 42, w18_setup 76 / 71, w18_Av 48 / 46).  The
+// requests cost registers, so the passes are compiled for eight blocks per CU (pass_blocks): left at 72
+// to 80 registers they gained nothing.
 struct WinPre {
     int nw;      // ids in the tile's window (-1: none)
     int id[2];   // the thread's first two (not valid past nw)
@@ -327,25 +361,24 @@ __device__ __forceinline__ WinPre win_prefetch(const Rows& R, int tile) {
     return p;
 }
 
-// The row's first LOC_PF index words (tile windows); the first LOC_EAGER without waiting for the
-// number of slots to walk
-constexpr int LOC_EAGER = 4;
+// The row's first LOC_PF index words, if its tile has a window: asked for before that is known, they came
+// no sooner where it has one and cost a tile without one 2 to 4 KB (a 256 x 256 x 16 block, whose cross
+// section leaves 97 % of the tiles without: ip_pack 122 / 111 us, prj_tail 114 / 103)
 template <class FM, int G>
-__device__ __forceinline__ LocPre loc_prefetch(const Rows& R, int i, int g) {
+__device__ __forceinline__ LocPre loc_prefetch(const Rows& R, const WinPre& pre, int i, int g) {
     LocPre p;
 #pragma unroll
     for (int k = 0; k < LOC_PF; ++k) p.q[k] = 0u;
     if constexpr (has_windows<FM, G>()) {
         if (R.win_n != nullptr) {
-            const uint32_t* l = R.loc + (size_t)(i >> 6) * (size_t)R.Cs * 32u + 4u * (uint32_t)(i & (WAVE - 1)) + (uint32_t)g;
             const int wl = R.wave_len[i >> 4];
+            if (__builtin_amdgcn_readfirstlane(pre.nw) >= 0) {
+                const uint32_t* l = R.loc + (size_t)(i >> 6) * (size_t)R.Cs * 32u + 4u * (uint32_t)(i & (WAVE - 1)) + (uint32_t)g;
+                const int tl = __builtin_amdgcn_readfirstlane(wl);
 #pragma unroll
-            for (int k = 0; k < LOC_EAGER; ++k)
-                if (8 * k < R.Cs) p.q[k] = __builtin_nontemporal_load(l + k * 256);
-            const int tl = __builtin_amdgcn_readfirstlane(wl);
-#pragma unroll
-            for (int k = LOC_EAGER; k < LOC_PF; ++k)
-                if (8 * k < tl) p.q[k] = __builtin_nontemporal_load(l + k * 256);
+                for (int k = 0; k < LOC_PF; ++k)
+                    if (8 * k < tl) p.q[k] = __builtin_nontemporal_load(l + k * 256);
+            }
         }
     }
     return p;
@@ -384,17 +417,17 @@ __device__ __forceinline__ Vec<NB> vec_of(const float4& b) {
     return B;
 }
 
-template <class FM, int NB, int G, class LA, class LB, class F>
+template <class FM, int NB, int G, int U = PASS_UNROLL, class LA, class LB, class F>
 __device__ __forceinline__ void row_pairs_w(bool win, const WinLds<FM, G>& w, const LocPre& lp, const Rows& R, int i,
                                             float4 xi, LA&& loadA, LB&& loadB, F&& f, int g) {
     if constexpr (has_windows<FM, G>()) {
         if (win) {
-            row_pairs<FM, NB, G, PASS_UNROLL, true>(R, i, xi, [&](int k) { return w.A[k]; },
+            row_pairs<FM, NB, G, U, true>(R, i, xi, [&](int k) { return w.A[k]; },
                                                     [&](int k) { return vec_of<NB>(w.B[k]); }, f, g, lp);
             return;
         }
     }
-    row_pairs<FM, NB, G, PASS_UNROLL>(R, i, xi, loadA, loadB, f, g);
+    row_pairs<FM, NB, G, U>(R, i, xi, loadA, loadB, f, g);
 }
 
 // ---- IP ------------------------------------------------------------------------------------
@@ -462,7 +495,7 @@ __device__ __forceinline__ bool cg_stopped(const SolverState* st) { return st->a
 // (math_utils.py:76-91, pressure_base.py:187-203, 413-423).  J d in the form of
 // compute_J_x_kernel (pressure_base.py:111-127): sum_j m_j dot(d_i - d_j, gradW_ij) + dot(d_i, S_i).
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_pack(PackArgs a) {
+__global__ __launch_bounds__(BLOCK, (pass_blocks<FM, G>())) void k_ip_pack(PackArgs a) {
     constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.gate && !cg_stopped(a.gate)) return;
     if (!SC && a.mark && blockIdx.x == 0 && threadIdx.x == 0) *a.mark = wall_clock64();
@@ -492,7 +525,7 @@ __global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_
         own();
         tail();
     }
-    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, G>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.d4[j]; });
     double err = 0.0, nact = 0.0, npairs = 0.0;
     float acc = 0.0f;
@@ -549,7 +582,7 @@ struct RhsArgs {
 // x = 0, r = b, rr = r.r, p = r) is part of the pass; as a launch of its own with its own finalize
 // it took 18 us at 1M rows and 5 at 8k.
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_rhs(RhsArgs a) {
+__global__ __launch_bounds__(BLOCK, (pass_blocks<FM, G>())) void k_ip_rhs(RhsArgs a) {
     constexpr bool EAGER = eager_loads<FM, SC, G>();
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row<G>(blk), g = pass_lane<G>();
@@ -584,7 +617,7 @@ __global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_ip_
         own();
         tail();
     }
-    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, G>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.q4[j]; });
     double touched = 0.0, tpairs = 0.0, rr = 0.0;
     if (gt.on) {
@@ -640,7 +673,7 @@ struct CGJArgs {
 // compute_Jx_pcg (ip.py:19-60): y_i = dfdt_i k_i (J p)_i on rows with dfdt > 0, J p in the form
 // sum_j dot(p_i - p_j, m_j gradW_ij) + dot(p_i, S_i) (ip.py:51-58)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_J(CGJArgs a) {
+__global__ __launch_bounds__(BLOCK, (pass_blocks<FM, G>())) void k_cg_J(CGJArgs a) {
     constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -670,7 +703,7 @@ __global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_
     if constexpr (has_windows<FM, G>()) {
         // a tile without active rows neither stages nor walks
         if (!__syncthreads_or(sk != 0.0f)) return;
-        if (sk != 0.0f) lp = loc_prefetch<FM, G>(a.R, i, g);
+        if (sk != 0.0f) lp = loc_prefetch<FM, G>(a.R, wp, i, g);
         win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.p4[j]; });
     }
     if (sk == 0.0f) return;
@@ -705,7 +738,7 @@ struct CGJTArgs {
 // compute_Ax_part1 + compute_Ax_part2 (ip.py:63-121) in gather form, fused with p.Ap
 // (ip.py:307)
 template <class FM, bool SC, int G = lanes_for<SC>()>
-__global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_JT(CGJTArgs a) {
+__global__ __launch_bounds__(BLOCK, (pass_blocks<FM, G>())) void k_cg_JT(CGJTArgs a) {
     constexpr bool EAGER = eager_loads<FM, SC, G>();
     if (!SC && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -742,7 +775,7 @@ __global__ __launch_bounds__(BLOCK, (!SC || G == PASS_LANES) ? 8 : 1) void k_cg_
     if constexpr (has_windows<FM, G>()) {
         // a tile without touched rows stages nothing (its rows only write m p)
         if (__syncthreads_or(touched)) {
-            if (touched) lp = loc_prefetch<FM, G>(a.R, i, g);
+            if (touched) lp = loc_prefetch<FM, G>(a.R, wp, i, g);
             win = stage_window(a.R, blk, wp, w, loadA, [&](int j) {
                 const float2 y = a.y2[j];
                 return make_float4(y.x, y.y, 0.0f, 0.0f);
@@ -1027,7 +1060,7 @@ __global__ __launch_bounds__(BLOCK) void k_prj_init(int nd, float dt, const floa
 
 // pj_head_fused (prj.py:17-59); also the head of solve_df (prj.py:243-253)
 template <class FM>
-__global__ __launch_bounds__(BLOCK, 8) void k_prj_head(PrjArgs a) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_prj_head(PrjArgs a) {
     if (a.st->active == 0) return;
     if (a.mark0 && blockIdx.x == 0 && threadIdx.x == 0) *a.mark0 = wall_clock64();
     constexpr int G = PASS_LANES;
@@ -1049,7 +1082,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_prj_head(PrjArgs a) {
     const float4 xi = a.R.pos[ic];
     const float s0 = a.Ss[3 * ic + 0], s1 = a.Ss[3 * ic + 1], s2 = a.Ss[3 * ic + 2];
     const float v0 = a.v0[3 * ic + 0], v1 = a.v0[3 * ic + 1], v2 = a.v0[3 * ic + 2];
-    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, G>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) {
         const float2 l = a.lam[j];
         return make_float4(l.x, l.y, 0.0f, 0.0f);
@@ -1075,7 +1108,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_prj_head(PrjArgs a) {
 // pj_tail_fused (prj.py:62-115); DF: the pass of solve_df (prj.py:255-283: J v masked by the
 // active rows, D^-1 J v, lambda + omega D^-1 J v, max(., 0), error of J v / rho0)
 template <class FM, bool DF>
-__global__ __launch_bounds__(BLOCK, 8) void k_prj_tail(PrjArgs a) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_prj_tail(PrjArgs a) {
     if (a.st->active == 0) return;
     constexpr int G = PASS_LANES;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -1092,7 +1125,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_prj_tail(PrjArgs a) {
     const float lam = a.lam[ic].x, kk = a.kk[ic], cc = DF ? 0.0f : a.cc[ic];
     const int tot = DF ? a.rowtot[ic] : 0;
     float rho0 = a.rho0[ic];
-    const LocPre lp = loc_prefetch<FM, G>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, G>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.d4[j]; });
     double err = 0.0;
     if (on) {
@@ -1182,7 +1215,7 @@ __global__ __launch_bounds__(BLOCK) void k_prj_save(int nd, const float2* __rest
 // viscosity.py:62-108 with Jacobi reads.  Neighbour record: A = (x, y, z, m_j), m_j = 0 for a
 // non-fluid neighbour (its term is then exactly 0, as the reference's skip), B = (v_j, rho_j).
 template <class FM, bool ALLFLUID>
-__global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt, int fluid,
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_visc(Rows R, float coeff, float dt, int fluid,
                                                 const float4* __restrict__ v4, const float* __restrict__ rho0,
                                                 const int* __restrict__ mat, float* __restrict__ vel, NextIn next) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -1206,7 +1239,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt
     const int ic = i < R.nd ? i : R.nd - 1;
     const float4 xi = R.pos[ic], vi = v4[ic];
     const float rho_i = vi.w, rho0_i = rho0[ic];
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(R, wp, i, g);
     const bool win = stage_window(R, blk, wp, w, loadA, [&](int j) { return v4[j]; });
     if (i >= R.nd) return;
     if (!ALLFLUID && mat[i] != fluid) {   // v stays
@@ -1216,7 +1249,8 @@ __global__ __launch_bounds__(BLOCK, 8) void k_visc(Rows R, float coeff, float dt
     float eps2 = (0.01f * R.h) * (0.01f * R.h);
     float k_visc = 2.0f * (3.0f + 2.0f);
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    row_pairs_w<FM, 4, PASS_LANES>(win, w, lp, R, i, xi, loadA, loadB,
+    // (two slots in flight: with four the 64 registers spill, 105 -> 140 us on a 256 x 256 x 16 block)
+    row_pairs_w<FM, 4, PASS_LANES, 2>(win, w, lp, R, i, xi, loadA, loadB,
                          [&](const float4& xj, const Vec<4>& vj, float gx, float gy, float gz) {
                              float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
                              float rn = len3_rn(rx, ry, rz);
@@ -1355,7 +1389,7 @@ __device__ __forceinline__ float3 w18_Av_row(const W18Args& a, int i, float4 ui,
 // from the operator pass on p4 and k_w18_warm_init.  Without the preconditioner the blocks are
 // the identity, so z = P r is r exactly (apply_preconditioner's copy, weiler18.py:279-292).
 template <class FM, bool ALLFLUID, bool WARM = false>
-__global__ __launch_bounds__(BLOCK, 8) void k_w18_setup(W18Args a, float4* __restrict__ p4) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_w18_setup(W18Args a, float4* __restrict__ p4) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     auto loadA = [&](int j) { return w18_record<ALLFLUID>(a.R.pos, a.v4, a.mat, a.fluid, j); };
@@ -1365,7 +1399,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_setup(W18Args a, float4* __res
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
     const float4 vi = a.v4[ic], xi = a.R.pos[ic];
     const float f = a.fac[ic];
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.v4[j]; });
     double rz = 0.0;
     if (i < a.R.nd) {
@@ -1377,7 +1411,8 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_setup(W18Args a, float4* __res
         if (fl) {
             const float eps2 = 0.01f * a.R.h * a.R.h;
             const float dd = 10.0f;
-            row_pairs_w<FM, 3, PASS_LANES>(win, w, lp, a.R, i, xi, loadA, loadB,
+            // (two slots in flight: with four the 64 registers spill, 106 -> 127 us on a 256 x 256 x 16 block)
+            row_pairs_w<FM, 3, PASS_LANES, 2>(win, w, lp, a.R, i, xi, loadA, loadB,
                 [&](const float4& xj, const Vec<3>& uj, float gx, float gy, float gz) {
                     float x[3] = {xi.x - xj.x, xi.y - xj.y, xi.z - xj.z};
                     float v0 = vi.x - uj.v[0], v1 = vi.y - uj.v[1], v2 = vi.z - uj.v[2];
@@ -1555,7 +1590,7 @@ __device__ __forceinline__ bool p_step(const PStep& n, SolverState* st, int i, i
 // Ap = A p, p.Ap (weiler18.py:337-338).  Without CHECK (the warm-start residual) it runs
 // regardless of the solver state.
 template <class FM, bool ALLFLUID, bool CHECK = true, bool NEXT = false>
-__global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a, PStep n) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_w18_Av(W18Args a, PStep n) {
     if (CHECK && !NEXT && a.st->active == 0) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
@@ -1569,7 +1604,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_w18_Av(W18Args a, PStep n) {
     float4 pi = a.v4[ic];
     const float4 xi = a.R.pos[ic];
     const float f = a.fac[ic];
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, wp, i, g);
     if (NEXT && !p_step(n, a.st, i, a.R.nd, g, pi, &beta)) return;
     const bool win = stage_window(a.R, blk, wp, w, loadA, vec);
     double pap = 0.0;
@@ -1751,7 +1786,7 @@ struct StArgs {
 
 // compute_divergence_jeske23 (jeske23.py:73-112): div_i = sum_fluid m_j (v_i - v_j) . gradW_ij
 template <class FM, bool ALLFLUID>
-__global__ __launch_bounds__(BLOCK, 8) void k_st_div(StArgs a) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_st_div(StArgs a) {
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int i = pass_row(blk), g = pass_lane();
     auto loadA = [&](int j) {
@@ -1764,7 +1799,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_st_div(StArgs a) {
     const WinPre wp = win_prefetch<FM, PASS_LANES>(a.R, blk);
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
     const float4 ui = a.u4[ic], xi = a.R.pos[ic];
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, wp, i, g);
     const bool win = stage_window(a.R, blk, wp, w, loadA, [&](int j) { return a.u4[j]; });
     if (i >= a.R.nd) return;
     if (!ALLFLUID && a.mat[i] != a.fluid) {
@@ -1807,7 +1842,7 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
     const int ic = i < a.R.nd ? i : a.R.nd - 1;
     const float4 xi = a.R.pos[ic], ui = a.u4[ic];
     const float m_i = ui.w, rho_i = a.density[ic], div_i = a.div[ic];
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, wp, i, g);
     if constexpr (has_windows<FM, PASS_LANES>()) {
         const int nw = __builtin_amdgcn_readfirstlane(wp.nw);
         if (a.R.win_n != nullptr && nw >= 0) {
@@ -1925,7 +1960,7 @@ __global__ __launch_bounds__(BLOCK) void k_st_setup(StArgs a) {
 // RHS: out = u - M u + b (jeske23.py:637-647); otherwise out = M u and the block's p.Mp partial.
 // Only the ids and g~ are streamed and (u_j, m_j) gathered: positions are not needed.
 template <class FM, bool ALLFLUID, bool RHS, bool NEXT = false>
-__global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a, PStep n) {
+__global__ __launch_bounds__(BLOCK, pass_blocks<FM>()) void k_st_Av(StArgs a, PStep n) {
     if (!RHS && !NEXT && a.st->active == 0) return;
     constexpr unsigned REC = FM::REC;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -1937,7 +1972,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_st_Av(StArgs a, PStep n) {
     float4 ui = a.u4[ic];
     float beta = 0.0f;
     auto vec = [&](int j) { return NEXT ? n.at(j, beta) : a.u4[j]; };
-    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, i, g);
+    const LocPre lp = loc_prefetch<FM, PASS_LANES>(a.R, wp, i, g);
     if (NEXT && !p_step(n, a.st, i, a.R.nd, g, ui, &beta)) return;
     const bool win = stage_window(a.R, blk, wp, w, [](int) { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); }, vec);
     double pap = 0.0;
