@@ -1209,14 +1209,25 @@ struct WinBitmap {
 
 // Tile window of a 64-row tile by its 256 threads.  The window is the ascending list of the distinct
 // ids in the walked slots [0, tile_len) of the tile's valid rows (padding slots name the row
-// itself); v / on are the thread's word pairs of the tile, ix their ids' places in that list, 16 bits
-// each.  The ids are marked in an LDS bitmap over [lo, hi] of the tile's ids, and an id's place is
-// the number of marks below it.  Returns the list's length, or -1 for a tile whose range exceeds
+// itself); v / on are the thread's word pairs of the tile.  The ids are marked in an LDS bitmap over
+// [lo, hi] of the tile's ids, and an id's place in the list is the number of marks below it
+// (window_index).  Returns the list's length, or -1 for a tile whose range exceeds
 // WIN_SPAN_WORDS words or whose window exceeds the cap (at most WIN_MAX ids).  The result is
 // block-uniform; every thread of the block calls it.
+struct TileWindow {
+    int n, lo;
+};
+__device__ __forceinline__ uint32_t window_index(const WinBitmap& s, int lo, uint32_t j) {
+    const uint32_t p = j - (uint32_t)lo;
+    return (uint32_t)s.pre[p >> 5] + (uint32_t)__popc(s.bm[p >> 5] & ((1u << (p & 31)) - 1u));
+}
+// places of a word pair's two ids, 16 bits each
+__device__ __forceinline__ uint32_t window_pair(const WinBitmap& s, int lo, uint32_t x, uint32_t y) {
+    return window_index(s, lo, x) | (window_index(s, lo, y) << 16);
+}
 template <int PPT>
-__device__ __forceinline__ int tile_window(const uint32_t (&vx)[PPT], const uint32_t (&vy)[PPT], const bool (&on)[PPT],
-                                           int cap, WinBitmap& s, uint32_t (&ix)[PPT]) {
+__device__ __forceinline__ TileWindow tile_window(const uint32_t (&vx)[PPT], const uint32_t (&vy)[PPT], const bool (&on)[PPT],
+                                                  int cap, WinBitmap& s) {
     __shared__ int red[2 * WAVES_PER_BLOCK];
     int lo = 0x7fffffff, hi = -1;
 #pragma unroll
@@ -1235,9 +1246,9 @@ __device__ __forceinline__ int tile_window(const uint32_t (&vx)[PPT], const uint
     __syncthreads();
     lo = min(min(red[0], red[1]), min(red[2], red[3]));
     hi = max(max(red[4], red[5]), max(red[6], red[7]));
-    if (hi < 0) return 0;   // no walked slot
+    if (hi < 0) return TileWindow{0, 0};   // no walked slot
     const int words = ((hi - lo) >> 5) + 1;
-    if (words > WIN_SPAN_WORDS) return -1;
+    if (words > WIN_SPAN_WORDS) return TileWindow{-1, 0};
     for (int k = threadIdx.x; k < words; k += BLOCK) s.bm[k] = 0u;
     __syncthreads();
 #pragma unroll
@@ -1258,19 +1269,13 @@ __device__ __forceinline__ int tile_window(const uint32_t (&vx)[PPT], const uint
     for (int k = w0; k < w1; ++k) cnt += __popc(s.bm[k]);
     int total;
     int off = block_excl_scan(cnt, &total);
-    if (total > cap) return -1;
+    if (total > cap) return TileWindow{-1, 0};
     for (int k = w0; k < w1; ++k) {
         s.pre[k] = (uint16_t)off;
         off += __popc(s.bm[k]);
     }
     __syncthreads();
-    auto index = [&](uint32_t j) {
-        const uint32_t p = j - (uint32_t)lo;
-        return (uint32_t)s.pre[p >> 5] + (uint32_t)__popc(s.bm[p >> 5] & ((1u << (p & 31)) - 1u));
-    };
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) ix[k] = on[k] ? index(vx[k]) | (index(vy[k]) << 16) : 0u;
-    return total;
+    return TileWindow{total, lo};
 }
 
 // Four lanes of a row, one term each: acc + t0 + t1 + t2 + t3 in that order on every lane (the
@@ -1411,9 +1416,13 @@ __global__ __launch_bounds__(BLOCK, 8) void k_eval4(BuildArgs a) {
             vx[b] = min(vx[b], last);
             vy[b] = min(vy[b], last);
         }
-        nwin = tile_window<PPT>(vx, vy, on, a.win_cap, lds_w.s, ix);
+        const TileWindow tw = tile_window<PPT>(vx, vy, on, a.win_cap, lds_w.s);
+        nwin = tw.n;
         if (threadIdx.x == 0) a.win_n[tile] = nwin;
         if (nwin >= 0) {
+            // (an empty window has no bitmap to look up)
+#pragma unroll
+            for (int b = 0; b < PPT; ++b) ix[b] = nwin > 0 && on[b] ? window_pair(lds_w.s, tw.lo, vx[b], vy[b]) : 0u;
             __syncthreads();   // the bitmap has been read
             uint32_t* l32 = a.loc + (size_t)tile * (size_t)a.Cs * (WAVE / 2) + threadIdx.x;
 #pragma unroll
@@ -1537,7 +1546,8 @@ struct WinArgs {
 // Tile windows in a pass of their own (rows of more than 64 slots, and rows that the one-lane build
 // wrote), one block per 64-row tile; each walked slot's index goes 16 bits wide to the slot's id
 // word (the 8-byte word pair of slots g, g + 4 becomes one 32-bit word).  Each thread keeps its PPT
-// word pairs of the tile in registers from one coalesced load.
+// word pairs of the tile in registers from one coalesced load; a pair's places are looked up as it
+// is written (kept in registers as well, 1M rows of 256 slots took 145 us a build instead of 105).
 template <int PPT>
 __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -1548,7 +1558,7 @@ __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
     const size_t base = (size_t)t * (size_t)a.Cs * WAVE;
     const u32x2* ids2 = reinterpret_cast<const u32x2*>(a.nb + base);
     // word pair q of a tile: block q >> 8, row (q >> 2) & 63; thread pairs q = thread + BLOCK k
-    uint32_t vx[PPT], vy[PPT], ix[PPT];
+    uint32_t vx[PPT], vy[PPT];
     bool on[PPT];
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
@@ -1558,7 +1568,8 @@ __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
         vx[k] = v.x;
         vy[k] = v.y;
     }
-    const int total = tile_window<PPT>(vx, vy, on, a.cap, s, ix);
+    const TileWindow tw = tile_window<PPT>(vx, vy, on, a.cap, s);
+    const int total = tw.n;
     if (threadIdx.x == 0) a.win_n[t] = total;
     if (total <= 0) return;
     // every window id is named by some walked slot: each slot writes its id at its index (slots
@@ -1568,9 +1579,10 @@ __global__ __launch_bounds__(BLOCK) void k_window(WinArgs a) {
 #pragma unroll
     for (int k = 0; k < PPT; ++k)
         if (on[k]) {
-            wid[ix[k] & 0xffffu] = (int)vx[k];
-            wid[ix[k] >> 16] = (int)vy[k];
-            l32[threadIdx.x + BLOCK * k] = ix[k];
+            const uint32_t ix = window_pair(s, tw.lo, vx[k], vy[k]);
+            wid[ix & 0xffffu] = (int)vx[k];
+            wid[ix >> 16] = (int)vy[k];
+            l32[threadIdx.x + BLOCK * k] = ix;
         }
     // the build's partial row 1 (zeroed by the build's blocks; the sums are integers, exact in
     // any order)
