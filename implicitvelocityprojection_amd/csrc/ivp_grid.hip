@@ -944,6 +944,8 @@ inline size_t scan_cells_lds(int Cs) {
     return ((size_t)WAVE * (size_t)(Cs + 4) + WAVES_PER_BLOCK * SCAN_WAVE_LDS) * sizeof(uint32_t);
 }
 constexpr size_t SCAN_CELLS_LDS_MAX = 64 * 1024;
+constexpr size_t SCAN_CELLS_LDS_THREE = 160 * 1024 / 3;   // three blocks per CU
+constexpr int SCAN_CELLS_TWO = 2 * 256 * WAVE;            // rows whose tiles two blocks per CU hold
 
 // (at least four waves per SIMD: within 128 registers the matrix results stay in vector registers)
 template <int FMT, bool SCENES>
@@ -1910,13 +1912,18 @@ int grid_load(ivp_ctx* c, int n, const float* x, const float* v, const float* m,
 // staged rows fit the LDS, from 20k rows: scan alone, lanes per row (best count) against by cells,
 // us: 12k rows 12.3 / 14.7, 16k 13.5 / 15.7, 23k 17.5 / 15.2, 32k 21.2 / 16.6, 48k 27.1 / 17.8, 102k 43 /
 // 29, 262k 83 / 50, 1M 225 / 149; where it does not apply, the count's lanes per row (16 below 32k rows: 8 lanes
-// took 20 us from 1k to 23k rows against 16).
+// took 20 us from 1k to 23k rows against 16).  It needs three of its blocks per CU: rows of up to 168 slots
+// (lanes / by cells at 168 slots, 102k rows 43 / 36, 262k 79 / 67, 1M 249 / 220, and at 176, where two
+// fit, 42 / 46, 79 / 87, 244 / 300), or so few tiles that two per CU hold them all (27k rows of 216 slots
+// 20.4 / 17.6).
 static int lanes_by_count(int nd) { return nd >= (1 << 18) ? 2 : nd >= (1 << 15) ? 4 : 16; }
 
 int build_lanes_for(const ivp_ctx* c) {
     const int nd = c->nd;
-    const bool cells = c->rec_words == 64 && scan_cells_lds(c->Cs) <= SCAN_CELLS_LDS_MAX;
-    int G = c->build_lanes > 0 ? c->build_lanes : cells && nd >= 20480 ? 64 : lanes_by_count(nd);
+    const size_t lds = scan_cells_lds(c->Cs);
+    const bool cells = c->rec_words == 64 && lds <= SCAN_CELLS_LDS_MAX;
+    const bool pays = nd >= 20480 && (lds <= SCAN_CELLS_LDS_THREE || nd <= SCAN_CELLS_TWO);
+    int G = c->build_lanes > 0 ? c->build_lanes : cells && pays ? 64 : lanes_by_count(nd);
     if (G == 64 && !cells) G = lanes_by_count(nd);
     return G;
 }
