@@ -795,6 +795,57 @@ __device__ __forceinline__ SegRuns seg_runs(const BuildArgs& a, const Grid& g, i
     return SegRuns{inc - n, s0 - (inc - n), inc};
 }
 
+// The hits of one chunk decided from the positions as scan_ids decides them, for a segment with far
+// coordinates (particles outside the grid are in its border cells, at any distance).  A batch's positions go
+// to the LDS, where a lane reads the 16 of its quarter: gathered through the ids one after another
+// they took twice as long as the rest (104k rows, all outside the grid: build 526 -> 229 us; a third of
+// them 150 -> 107).
+__device__ __forceinline__ void far_chunk(const BuildArgs& a, const float4* __restrict__ ppos, const uint32_t* ids,
+                                          float* cand, int left, int nb, bool mine, float px, float py, float pz,
+                                          uint32_t (&W)[2]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const int q = lane >> 4, n = lane & 15;
+    const int base = 16 * nb * q;
+    float* cq = cand + SCAN_QUARTER * q;
+    unsigned long long hits = 0ull;
+#pragma unroll 1
+    for (int u = 0; u < nb; ++u) {
+        const int c = base + 16 * u + n;
+        const float4 p = ppos[ids[c < left ? c : left - 1]];
+        *reinterpret_cast<f32x4*>(cq + 4 * n) = f32x4{p.x, p.y, p.z, 0.0f};
+        wave_lds_sync();
+        uint32_t h = 0u, band = 0u;
+#pragma unroll 4
+        for (int k = 0; k < 16; ++k) {
+            const f32x4 pj = *reinterpret_cast<const f32x4*>(cq + 4 * k);
+            const float rx = px - pj.x, ry = py - pj.y, rz = pz - pj.z;
+            const float d2 = fmaf(rz, rz, fmaf(ry, ry, rx * rx));
+            h = h << 1 | (d2 < a.h2_lo ? 1u : 0u);
+            band = band << 1 | (d2 < a.h2_hi ? 1u : 0u);
+        }
+        const int valid = left - base - 16 * u;   // candidates of this lane's 16
+        const uint32_t in = !mine ? 0u : valid >= 16 ? 0xffffu : valid > 0 ? 0xffffu & ~(0xffffu >> valid) : 0u;
+        h &= in;
+        band &= in & ~h;
+        while (__builtin_amdgcn_ballot_w64(band != 0u)) {
+            if (band) {
+                const int k = __clz((int)band) - 16;
+                const uint32_t bit = 0x8000u >> k;
+                band &= ~bit;
+                const f32x4 pj = *reinterpret_cast<const f32x4*>(cq + 4 * k);
+                const float rx = px - pj.x, ry = py - pj.y, rz = pz - pj.z;
+                const float dd = rx * rx + ry * ry + rz * rz;
+                h = sqrtf(dd) < a.h ? (h | bit) : h;
+            }
+        }
+        wave_lds_sync();
+        hits |= (unsigned long long)h << (48 - 16 * u);
+    }
+    W[0] = (uint32_t)(hits >> 32);
+    W[1] = (uint32_t)hits;
+}
+
 // One population of a segment: rows rs .. re - 1 of the wave, whose positions lanes (q, n) hold for
 // row n.  found (every lane of row n) counts row n's hits of this population; the dynamic
 // population stores hit k at slot k while k < C (an overflowing row's hits past C all go to slot C,
@@ -850,13 +901,14 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             const int c = base + 16 * u + n;
-            if (u < nb) p[u] = ppos[ids[c < left ? c : left - 1]];
+            if (u < nb && !row_far) p[u] = ppos[ids[c < left ? c : left - 1]];
         }
         uint32_t W[2] = {0u, 0u};   // hits, first candidate in the highest bit, 32 per word
+        bool far = false;           // a candidate of the chunk with far coordinates
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             uint32_t w = W[u >> 1] << 16;
-            if (u < nb) {
+            if (u < nb && !row_far) {
                 const float bx = p[u].x - o.x, by = p[u].y - o.y, bz = p[u].z - o.z;
                 const float b2 = fmaf(bz, bz, fmaf(by, by, bx * bx));
                 const f32x4 rec = {bx, by, bz, base + 16 * u + n < left ? b2 : 1e30f};
@@ -875,18 +927,16 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
                     h = __builtin_amdgcn_alignbit(h, __float_as_uint(e), 31);   // h << 1 | sign
                     nearest = fminf(nearest, fabsf(e));
                 }
-                const bool far = !(b2 <= far2) || row_far;
-                if (__builtin_amdgcn_ballot_w64((mine && nearest < eps) || far)) {
-                    // candidates in the band (or, with far coordinates, all of them) by the exact test
-                    const bool all = __builtin_amdgcn_ballot_w64(far) != 0ull;
+                far = far || !(b2 <= far2);
+                if (__builtin_amdgcn_ballot_w64(mine && nearest < eps)) {
+                    // candidates in the band by the exact test
                     uint32_t band = 0u;
 #pragma unroll
                     for (int k = 0; k < 16; ++k)
                         band = __builtin_amdgcn_alignbit(band, __float_as_uint(fabsf(d[k >> 2][k & 3]) - eps), 31);
                     const int valid = left - base - 16 * u;   // candidates of this lane's 16
                     const uint32_t in = valid >= 16 ? 0xffffu : valid > 0 ? 0xffffu & ~(0xffffu >> valid) : 0u;
-                    h = all ? 0u : h;
-                    band = mine ? (all ? in : band & in) : 0u;
+                    band = mine ? band & in : 0u;
                     while (__builtin_amdgcn_ballot_w64(band != 0u)) {
                         if (band) {
                             const int k = __clz((int)band) - 16;
@@ -903,6 +953,7 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
             }
             W[u >> 1] = w;
         }
+        if (row_far || __builtin_amdgcn_ballot_w64(far)) far_chunk(a, ppos, ids, cand, left, nb, mine, px, py, pz, W);
         if (!mine) W[0] = W[1] = 0u;
         if (DYN) {   // the row itself: in run 4
             const int li = row0 + n - rb[4] - cb - base;
