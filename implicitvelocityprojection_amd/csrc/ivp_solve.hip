@@ -2756,7 +2756,6 @@ int prj_df_body(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* s
     if (nd == 0) return IVP_OK;
     const dim3 nb(blocks_for(nd));
     const float inv_dt = (float)(1.0 / (double)dt);
-    const long long tp = c->state_host->total_pairs;
     auto t1 = std::chrono::steady_clock::now();
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_prj_init<true>, nb, nd, dt, (const float*)c->density,
                    (const float*)c->rho0, (const float*)c->vel, (const float4*)c->pos, (const int*)c->uid,
@@ -2767,6 +2766,7 @@ int prj_df_body(ivp_ctx* c, float dt, const ivp_prj_params* prm, ivp_ip_stats* s
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_prj_save, nb, nd, (const float2*)c->prj_lam, (const int*)c->uid,
                    c->prj_df_prev));
     st.df_outer_iters = df_passes;
+    const long long tp = c->state_host->total_pairs;   // (reported with the loop's state)
     st.pairs_traversed += 2ll * (df_passes + 1) * tp;
     st.rows_traversed += 2ll * (df_passes + 1) * nd;
     IVP_TRY(launch(c, KC_GLUE, -1, 0.0, k_ip_finish, nb, nd, inv_dt, (const float4*)c->d4, (const float*)c->jd,
