@@ -116,9 +116,9 @@ class SceneBatch:
             self.ctx.build_lanes = min(build_ms, key=build_ms.get)
         for g in lanes:
             for k in chunks:
-                self.restore(snap)
                 self.ctx.scene_cg_chunk = k
-                self.ctx.scene_lanes = g
+                self.ctx.scene_lanes = g         # (before the rows are built: they follow it)
+                self.restore(snap)
                 self.step()                      # captures the replay graphs for this setting
                 self.restore(snap)
                 torch.cuda.synchronize()
