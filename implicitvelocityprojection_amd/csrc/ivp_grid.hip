@@ -532,7 +532,8 @@ __device__ __forceinline__ int scan_group(const Grid& g, const int* __restrict__
     const int x1 = cx < g.dims[0] - 1 ? cx + 1 : g.dims[0] - 1;
     const int wl = (int)(threadIdx.x & (WAVE - 1));
     const int base = wl & ~(G - 1);
-    const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1ull);
+    static_assert(G <= 8 && G * U <= POS_PAD, "16 lanes take scan_row16; a batch stays inside the position buffer's pad");
+    const unsigned long long gmask = (1ull << G) - 1ull;
     const unsigned long long below = (1ull << gl) - 1ull;
     int found = 0;
     for (int dz = -1; dz <= 1; ++dz) {
@@ -687,7 +688,6 @@ __global__ __launch_bounds__(BLOCK) void k_scan(BuildArgs a) {
     const int ic = on ? i : a.nd - 1;
     const float4 pi = a.pos[ic];
     const Grid g = SCENES ? a.grids[a.sid[ic]] : a.g;
-    int tot = 0, cnt = 0, cs = 0;
     // the k-th neighbour found (dynamic ones first) is stored when k < C
     Row16Runs rd = {0, 0}, rs = {0, 0};
     if constexpr (G == 16) {   // both populations' bounds in flight together
@@ -704,17 +704,13 @@ __global__ __launch_bounds__(BLOCK) void k_scan(BuildArgs a) {
     int nd_found = scan(a.dstart, a.pos, i, [&](int j, int rank, int before) {
         if (before + rank < C) tnb[slot_word<REC>(before + rank) + w0] = (uint32_t)j;
     });
-    cnt = nd_found < C ? nd_found : C;
-    tot = nd_found;
     int ns_found = scan(a.sstart, a.pos + a.nd, -1, [&](int j, int rank, int before) {
         const int k = nd_found + before + rank;
         if (k < C) tnb[slot_word<REC>(Cs - 1 - (before + rank)) + w0] = (uint32_t)j;
     });
-    tot += ns_found;
-    cs = (tot < C ? tot : C) - cnt;
-    (void)cs;
     if (on && gl == 0) {
-        a.rowcnt[i] = cnt;
+        const int tot = nd_found + ns_found;
+        a.rowcnt[i] = nd_found < C ? nd_found : C;
         a.rowtot[i] = tot;
         if (tot > C) atomicOr(a.err_flag, 1);
     }

@@ -2279,7 +2279,6 @@ int ip_solve_body(ivp_ctx* c, float dt, const ivp_ip_params* prm, ivp_ip_stats* 
     if (nd == 0) return IVP_OK;
     const dim3 nb(blocks_for(nd)), np = pass_grid(nd);
     const int stride = c->max_blocks;
-    const double pb = pair_bytes<FP>(), pbc = pair_bytes<FC>();
     Rows R = rows_of(c);
     float4* d4 = c->d4;
     IVP_TRY(stage_input(c, NEXT_IP, dt, 0.0f));
@@ -2526,7 +2525,6 @@ int weiler18_body(ivp_ctx* c, float coeff, float dt, int* iters_out) {
     const NextIn next = take_next(c);
     if (c->prof) IVP_TRY(build_fold(c));   // (the byte figures of the timed passes)
     const double pairs = (double)c->state_host->total_pairs;
-    const double pb = pair_bytes<FM>();
     W18Args wa{R, c->cfg.material_fluid, c->w_fac, c->mat, c->w_pinv, c->w_v4, c->w_rhs,
                c->w_dv, c->w_r, c->w_z, c->partials, stride, c->state, c->w18_precond ? 1 : 0, c->uid,
                c->w_dv_prev};
@@ -2654,7 +2652,7 @@ template <class FM, bool DF>
 int prj_loop(ivp_ctx* c, const ivp_prj_params* prm, double tol, int* passes, double* err, int* chunks) {
     const int nd = c->nd;
     const dim3 np = pass_grid(nd);
-    const double pb = pair_bytes<FM>(), pairs = (double)c->state_host->total_pairs;
+    const double pairs = (double)c->state_host->total_pairs;
     PrjArgs pa{rows_of(c), c->Ss, c->prj_v0, c->prj_lam, c->d4, c->cc, c->kk, c->rho0, c->rowtot, c->jd,
                prm->omega, c->C, prm->df_num_threshold, c->partials, c->max_blocks, c->state, nullptr};
     PrjFinArgs fa{c->partials, c->max_blocks, (int)np.x, c->state, tol, prm->max_iteration_opt,
