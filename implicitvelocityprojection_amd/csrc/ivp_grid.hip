@@ -883,6 +883,7 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
     for (int cb = 0; cb < T; cb += WAVE * NB) {
         const int left = T - cb < WAVE * NB ? T - cb : WAVE * NB;
         const int nb = (left + WAVE - 1) / WAVE;
+        const int nbm = row_far ? 0 : nb;   // batches for the matrix cores
         // the chunk's candidate ids in visiting order, run by run
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
@@ -897,14 +898,14 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             const int c = base + 16 * u + n;
-            if (u < nb && !row_far) p[u] = ppos[ids[c < left ? c : left - 1]];
+            if (u < nbm) p[u] = ppos[ids[c < left ? c : left - 1]];
         }
         uint32_t W[2] = {0u, 0u};   // hits, first candidate in the highest bit, 32 per word
         bool far = false;           // a candidate of the chunk with far coordinates
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             uint32_t w = W[u >> 1] << 16;
-            if (u < nb && !row_far) {
+            if (u < nbm) {
                 const float bx = p[u].x - o.x, by = p[u].y - o.y, bz = p[u].z - o.z;
                 const float b2 = fmaf(bz, bz, fmaf(by, by, bx * bx));
                 const f32x4 rec = {bx, by, bz, base + 16 * u + n < left ? b2 : 1e30f};
@@ -949,7 +950,8 @@ __device__ __forceinline__ void seg_pop_scan(const BuildArgs& a, const SegRuns& 
             }
             W[u >> 1] = w;
         }
-        if (row_far || __builtin_amdgcn_ballot_w64(far)) far_chunk(a, ppos, ids, cand, left, nb, mine, px, py, pz, W);
+        if (__builtin_expect(row_far || __builtin_amdgcn_ballot_w64(far) != 0ull, 0))
+            far_chunk(a, ppos, ids, cand, left, nb, mine, px, py, pz, W);
         if (!mine) W[0] = W[1] = 0u;
         if (DYN) {   // the row itself: in run 4
             const int li = row0 + n - rb[4] - cb - base;
