@@ -6,9 +6,9 @@
 //
 // Sort: a deterministic counting sort over cell keys.  count (atomic; a step's advection runs in
 // the same pass), exclusive scan, scatter (atomic slot), then every particle ranks itself inside
-// its cell by user id and moves to its place, so the resulting order -- (cell key, user id) -- depends on the positions only.  Cell keys are
-// x-fastest linear, so the three cells (cx-1..cx+1, cy, cz) of a stencil row are one contiguous
-// particle range: a query visits 9 ranges per population.
+// its cell by user id and moves to its place, so the resulting order -- (cell key, user id) -- depends on
+// the positions only.  Cell keys are x-fastest linear, so the three cells (cx-1..cx+1, cy, cz) of a stencil
+// row are one contiguous particle range: a query visits 9 ranges per population.
 #include <cmath>
 
 #include "ivp_internal.h"

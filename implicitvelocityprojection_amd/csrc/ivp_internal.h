@@ -44,8 +44,9 @@ int ivp_hip_fail(hipError_t e, const char* what, const char* file, int line);
 
 namespace ivp {
 
-// Device-resident solver state.  Reducing kernels write per-block partials; a one-block
-// finalize kernel folds them in a fixed order and updates these fields.
+// Device-resident solver state.  Reducing kernels write per-block partials, which are folded in a fixed
+// order by a one-block finalize kernel, or by every block of the pass that needs the sum, one of which
+// updates these fields.
 struct SolverState {
     double rr_old;      // r.r (IP) / r.z (Weiler18) of the current iteration
     double rr_new;
@@ -297,7 +298,10 @@ struct ivp_ctx {
     int prj_guess = 8;            // first launch chunk of the next pass loop
 
     // reductions
-    double* partials = nullptr;   // 4 * max_blocks
+    // PARTIAL_ROWS rows of max_blocks, then PARTIAL_ROWS rows of PREFOLD (k_prefold's output).  Rows BUILD_ROW
+    // and BUILD_ROW + 1 hold the last build's sums until build_fold or the next pressure solve's first
+    // sums have folded them: no other pass writes there
+    double* partials = nullptr;
     int max_blocks = 0;
     ivp::SolverState* state = nullptr;      // device
     // pinned, written by the device: a kernel that ends a stage stores the state there itself, and the

@@ -7,11 +7,10 @@
 
 namespace ivp {
 
-// Launch `kernel` (256-thread blocks) on the context's stream.  When timing is enabled for its
-// class the launch goes through hipExtLaunchKernelGGL with two events that the dispatch itself
-// stamps at kernel start and end, so the recorded time is the kernel's own execution time.
-// kclass < 0 marks helper launches that are never timed.
-// `shmem` bytes of dynamic LDS per block.
+// Launch `kernel` on the context's stream in blocks of `threads` threads with `shmem` bytes of dynamic LDS
+// (launch_shm and launch: 256 threads).  When timing is enabled for its class the launch goes through
+// hipExtLaunchKernelGGL with two events that the dispatch itself stamps at kernel start and end, so the
+// recorded time is the kernel's own execution time.  kclass < 0 marks helper launches that are never timed.
 template <typename... KArgs, typename... Args>
 inline int launch_any(ivp_ctx* c, int kclass, int tag, double bytes, void (*kernel)(KArgs...), dim3 grid, int threads,
                       unsigned shmem, Args... args) {

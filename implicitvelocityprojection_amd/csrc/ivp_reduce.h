@@ -220,11 +220,15 @@ __global__ __launch_bounds__(FIN_BLOCK) void k_finalize(FinArgs a) {
 // pass folds them itself, all to the same bits, and one block writes the state; above it the folds take
 // longer than the launch that they save, and k_prefold first reduces each row to PREFOLD partials in
 // one short launch of many blocks (15 625 partials: 4.6 us, what the one-block finalize took; the pass
-// that folds the rest is then no dependent launch of its own).  p.Ap has nd / 64 partials, an update's sums
-// nd / 256, and both are read by nd / 256 blocks.  us per implicit viscosity solve, prefolded /
-// folded by the readers: p.Ap at 133k rows 420 / 390, 176k 506 / 480, 262k (4.2 million reads) 879 / 861,
-// 350k (7.5 million) 1079 / 1108; the sums at 500k (3.8 million) 1378 / 1359, 750k (8.6 million) 1908 / 1956, 1M
-// 2371 / 2535.
+// that folds the rest is then no dependent launch of its own).
+// p.Ap has nd / 64 partials, an update's sums one per block of vec_grid, and vec_grid's blocks read both (the
+// operator pass's where it forms p).  Up to VEC_MAX rows that is 4.2 million reads at most (16 384 partials
+// by 256 blocks), so the readers fold; one row more, back at 256-thread blocks, it is 68 million for p.Ap and
+// 17 million for the sums, so in the CG k_prefold runs above VEC_MAX only (elsewhere: finalizes of more
+// than FIN_MAX partials).  The line between was measured with 256-thread vector blocks throughout, us per
+// implicit viscosity solve, prefolded / folded by the readers: p.Ap at 133k rows 420 / 390, 176k
+// 506 / 480, 262k (4.2 million reads) 879 / 861, 350k (7.5 million) 1079 / 1108; the sums at 500k (3.8 million)
+// 1378 / 1359, 750k (8.6 million) 1908 / 1956, 1M 2371 / 2535.
 constexpr long long FOLD_READS = 5ll << 20;
 // Partials (all rows) that the one-block finalize folds alone, us: three rows of 4096 4.3 and 6.9 with a
 // prefold; three of 15 625 9.1 and 9.7; six of 15 625 9.7 with one
@@ -277,9 +281,11 @@ __global__ __launch_bounds__(BLOCK) void k_prefold(const double* __restrict__ p,
 // Blocks of a CG's vector passes (update, p): 256 threads of one row each, or between VEC_MIN and VEC_MAX rows at
 // most 256 blocks -- one per CU -- of 1024 threads with as many rows each as that takes, all in flight:
 // then both the partials they write and the blocks that fold the operator pass's are few, and no
-// k_prefold is needed (us per implicit viscosity solve, 256-thread blocks / these: 90k rows 294 /
-// 302, 133k 377 / 371, 262k
-// 860 / 843, 350k 1071 / 1025, 500k 1351 / 1287, 1M 2374 / 2283; IP solve at 262k 331 / 315, 700k 652 (750k) / 609).
+// k_prefold is needed (us per implicit viscosity solve, 256-thread blocks / these: 90k rows 294 / 302, 133k
+// 377 / 371, 262k 860 / 843, 350k 1071 / 1025, 500k 1351 / 1287, 1M 2374 / 2283; IP solve at 262k 331 / 315).
+// VEC_MAX is what VEC_ROWS rows per thread in registers reach, not where 256-thread blocks become better;
+// above it a solve has its 256-thread form with k_prefold (1.06M to 4.1M rows: 1.0 to 1.27 times as fast as with
+// one-block finalizes between the passes).
 constexpr int VEC_THREADS = 1024, VEC_BLOCKS = 256, VEC_ROWS = 4;
 constexpr int VEC_MIN = 1 << 17, VEC_MAX = VEC_THREADS * VEC_BLOCKS * VEC_ROWS;
 struct VecGrid {

@@ -2976,14 +2976,14 @@ int ip_solve_scenes(ivp_ctx* c, float dt, const ivp_ip_params* prm) {
     return IVP_OK;
 }
 
-// v + g dt into the second velocity buffer, which becomes the first; the previous velocities stay
-// in the second until the next re-sort, so a step that must not start can restore them
 NextIn next_in(ivp_ctx* c, NextKind kind, float dt, float coeff) {
     if (kind == NEXT_NONE) return NextIn{};
     float4* out = kind == NEXT_IP ? c->d4 : kind == NEXT_VISC ? c->v4 : c->w_v4;
     return NextIn{kind, dt, coeff, c->pos, c->density, c->rho0, out, c->w_fac};
 }
 
+// v + g dt into the second velocity buffer, which becomes the first; the previous velocities stay
+// in the second until the next re-sort, so a step that must not start can restore them
 int glue_gravity(ivp_ctx* c, const float g[3], float dt) {
     if (!c->loaded) return IVP_ERR_STATE;
     if (c->nd == 0) return IVP_OK;
