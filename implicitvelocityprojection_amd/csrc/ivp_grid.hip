@@ -228,6 +228,9 @@ struct KeysArgs {
     AdvectArgs adv;
 };
 
+constexpr int KEY_SLOTS = 32;    // chunks that a block adds up itself
+constexpr int KEY_ROUNDS = 8;    // chunks of one wave
+
 // Cell keys and counts; with ADVECT the particle first moves (the step's advection reads and writes
 // the position that its key needs).
 template <bool SCENES, bool ADVECT>
@@ -250,23 +253,38 @@ __global__ __launch_bounds__(BLOCK) void k_keys(KeysArgs a) {
     KeyRun r = key_run(k, valid);
     if (r.head) atomicAdd(&a.ccount[k], r.len);
     if (a.bsum) {
-        // chunk totals: a block's particles mostly share the chunk of its first one, so that chunk
-        // takes one atomic per block (one per wave serialised on few addresses: 6 -> 26 us at 1M
-        // rows) and other chunks one per run
-        __shared__ int first, same[WAVES_PER_BLOCK];
-        const int c = valid ? k / SCAN_CHUNK : -1;
-        if (threadIdx.x == 0) first = c;
-        __syncthreads();
-        const bool in = valid && c == first;
-        const int n = __popcll(__ballot(in));
-        if ((threadIdx.x & (WAVE - 1)) == 0) same[threadIdx.x >> 6] = n;
-        const unsigned long long rest = __ballot(valid && !in);
-        if (rest) {
-            KeyRun t = key_run(c, valid);
-            if (t.head && !in) atomicAdd(&a.bsum[c], t.len);
+        // chunk totals: a block's particles lie in a few chunks, but rarely in runs (every second one of a
+        // lattice crosses into the next row of cells at once), so each wave adds up its own, one chunk a
+        // round, into the block's table, and a chunk takes one global atomic per block.  1M rows: 6 us without
+        // totals, 26 with an atomic per wave for the first particle's chunk; with one per block for that chunk
+        // and one per run for the others 19 us on a disordered state, but 35 on average and 153 at most in the
+        // dam break's steps; so 16.
+        __shared__ int tag[KEY_SLOTS], num[KEY_SLOTS];
+        if (threadIdx.x < KEY_SLOTS) {
+            tag[threadIdx.x] = -1;
+            num[threadIdx.x] = 0;
         }
         __syncthreads();
-        if (threadIdx.x == 0) atomicAdd(&a.bsum[first], (same[0] + same[1]) + (same[2] + same[3]));
+        const int c = valid ? k / SCAN_CHUNK : -1;
+        const int lane = (int)(threadIdx.x & (WAVE - 1));
+        unsigned long long rest = __ballot(valid);
+        for (int t = 0; rest && t < KEY_ROUNDS; ++t) {
+            const int lead = (int)__builtin_ctzll(rest);
+            const int c0 = __builtin_amdgcn_readlane(c, lead);
+            const unsigned long long m = __ballot(c == c0);
+            rest &= ~m;
+            if (lane == lead) {
+                const int q = c0 % KEY_SLOTS, n = (int)__popcll(m);
+                const int old = atomicCAS(&tag[q], -1, c0);
+                atomicAdd(old == -1 || old == c0 ? &num[q] : &a.bsum[c0], n);
+            }
+        }
+        if (rest) {   // particles in no order: an atomic per run
+            KeyRun t = key_run(c, valid);
+            if (t.head && ((rest >> lane) & 1ull)) atomicAdd(&a.bsum[c], t.len);
+        }
+        __syncthreads();
+        if (threadIdx.x < KEY_SLOTS && num[threadIdx.x] > 0) atomicAdd(&a.bsum[tag[threadIdx.x]], num[threadIdx.x]);
     }
 }
 
@@ -1353,7 +1371,7 @@ __device__ __forceinline__ void quad_sub(float& acc, float t) {
 // g + 4 of every 8-slot block (one 8-byte id load), forms their terms with the expressions of
 // build_eval, and the row's sums take the four lanes' terms in slot order, so rho, Aii, S and k are
 // bitwise those of the one-thread pass.  A block is one 64-row tile; block partials are per tile.
-// With PPT > 0 (one scene, rows of at most 8 PPT slots) the block also finds its tile's window
+// With PPT > 0 (rows of at most 8 PPT slots) the block also finds its tile's window
 // (tile_window): the thread's ids, loaded at once, are the word pairs that the search needs, the
 // window's (x, m) and 1/m go to the LDS, where the pairs read them, and the pass writes the list and
 // the slots' indices.  As two passes the ids were read twice and every pair gathered 20 B from

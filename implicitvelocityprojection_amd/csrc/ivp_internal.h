@@ -228,7 +228,7 @@ struct ivp_ctx {
                                // twice the word index of the slot's id
     int* tile_len = nullptr;
     int* wave_len = nullptr;   // slots to walk per 16 rows (after the tile lengths in one allocation)
-    // tile windows (ids-only layout, one scene): per 64-row tile its distinct neighbour ids in
+    // tile windows (ids-only layout; one scene, or scenes with four lanes per row): per 64-row tile its distinct neighbour ids in
     // ascending order (win_ids, WIN_MAX per tile) and their count (win_n, -1: the tile has no
     // window); per walked slot of a valid row the index of its id in the window, 16 bits at the
     // slot's id word (loc).  win_built: the last build wrote them.
