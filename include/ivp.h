@@ -291,8 +291,9 @@ int ivp_scene_history(ivp_ctx *ctx, int scene, int capacity, double *density_err
  * 382-383; default 1: the 3x3 block-Jacobi preconditioner). */
 #define IVP_OPT_W18_WARM_START 6
 #define IVP_OPT_W18_PRECONDITIONER 7
-/* Tile windows (1, default; ids-only and float16 rows, one scene): each neighbour build also
- * lists, per 64-row tile, the distinct neighbours of its rows, and the pair passes load them into
+/* Tile windows (1, default; ids-only and float16 rows; one scene, or independent scenes whose
+ * passes run four lanes per row): each neighbour build also lists, per 64-row tile, the distinct
+ * neighbours of its rows, and the pair passes load them into
  * on-chip memory once per tile instead of gathering each pair's neighbour from memory.  Results
  * are bitwise the same either way; 0 turns them off from the next build on, and a value v > 1
  * keeps windows of at most v neighbours only (tiles with more gather from memory). */
